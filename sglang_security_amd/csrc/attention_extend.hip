@@ -5,25 +5,23 @@
 // tokens themselves (the same rows of k_extend / v_extend, under the causal mask).  One online softmax
 // runs over both ranges (triton_ops/extend_attention.py:306-438 does the same in two loops).
 //
-// Fast path (16-bit, D = Dv = 128): one block per (sequence, query head, 64*NC query rows); the four waves
-// share every 32-token K/V tile through LDS and each multiplies it against NC tiles of 16 query rows on
-// the matrix cores.  Everything else takes a wave-per-(query row, head) kernel.
+// Pools of the query type with head sizes 64 and 128 run extend_tile_kernel (extend_tile.h).  An fp8 pool with head
+// size 128 runs extend_attention_kv8: one block per (sequence, query head, 64 query rows); the four waves share every
+// 32-token K/V tile through LDS, widened on the way in, and each multiplies it against 16 query rows on the matrix
+// cores.  Everything else takes a wave-per-(query row, head) kernel.
 #include <type_traits>
 
 #include "attention_tile.h"
 #include "common.h"
+#include "extend_tile.h"
 
 namespace sglk {
 namespace {
 
-constexpr int kNC = 2;
-#ifndef SGLK_EXTEND_PF
-#define SGLK_EXTEND_PF 1
-#endif
-constexpr int kExtPF = SGLK_EXTEND_PF;  // K / V tiles in flight ahead of the one being multiplied
+constexpr int kExtPF = 1;  // K / V tiles in flight ahead of the one being multiplied
 
-template <typename T, int NC, typename KV = T>
-__global__ void __launch_bounds__(256) extend_attention_mfma128(
+template <typename T, typename KV>
+__global__ void __launch_bounds__(256) extend_attention_kv8(
     const void* __restrict__ q_extend, const void* __restrict__ k_extend, const void* __restrict__ v_extend,
     void* __restrict__ o_extend, const void* __restrict__ k_buffer, const void* __restrict__ v_buffer,
     const int32_t* __restrict__ qo_indptr, const int32_t* __restrict__ kv_indptr,
@@ -35,6 +33,8 @@ __global__ void __launch_bounds__(256) extend_attention_mfma128(
   // cached prefix, the last split also the new tokens; every split leaves a normalised fp32 partial + log-sum-exp per
   // (query row, head) in part_o [T, Hq, kv_splits, 128] / part_lse [T, Hq, kv_splits] for extend_merge_kernel.  A
   // single request's short extend over a long prefix has too few (query block, head) pairs to fill the chip otherwise.
+  constexpr int NC = 1;
+  constexpr bool KV8 = true;
   extern __shared__ __attribute__((aligned(16))) char lds[];
   const int b = blockIdx.z, h = blockIdx.y;
   const int q0 = qo_indptr[b];
@@ -42,10 +42,9 @@ __global__ void __launch_bounds__(256) extend_attention_mfma128(
   const int split = kv_splits > 1 ? (int)blockIdx.x % kv_splits : 0;
   const int block_q0 = (kv_splits > 1 ? (int)blockIdx.x / kv_splits : (int)blockIdx.x) * 64 * NC;
   if (block_q0 >= ext_len) return;  // block-uniform
-  // fp8 pool: code -> value table behind the two stages (visible after the barrier that opens every run())
-  constexpr bool KV8 = !std::is_same<KV, T>::value;
-  [[maybe_unused]] uint16_t* lut = reinterpret_cast<uint16_t*>(lds + kBlockAttnLds);
-  if constexpr (KV8) lut[threadIdx.x] = Conv<T>::from_f32(KvElem<KV>::value(threadIdx.x));  // 256 threads, 256 codes
+  // code -> value table behind the two stages (visible after the barrier that opens every run())
+  uint16_t* lut = reinterpret_cast<uint16_t*>(lds + kBlockAttnLds);
+  lut[threadIdx.x] = Conv<T>::from_f32(KvElem<KV>::value(threadIdx.x));  // 256 threads, 256 codes
   const int pstart = kv_indptr[b];
   const int plen = kv_indptr[b + 1] - pstart;
   const int kvh = h / (Hq / Hkv);
@@ -75,10 +74,9 @@ __global__ void __launch_bounds__(256) extend_attention_mfma128(
     const int shift = plen - ext_len;
 #pragma unroll
     for (int c = 0; c < NC; ++c) qpos[c] += shift;
-    // (an fp8 pool: byte pointers and byte strides, carried in the 16-bit pointer type of run())
-    constexpr int kEl = KV8 ? 1 : 2;
-    const uint16_t* kb = reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(k_buffer) + (int64_t)kvh * k_stride_h * kEl);
-    const uint16_t* vb = reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(v_buffer) + (int64_t)kvh * v_stride_h * kEl);
+    // (byte pointers and byte strides, carried in the 16-bit pointer type of run())
+    const uint16_t* kb = reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(k_buffer) + (int64_t)kvh * k_stride_h);
+    const uint16_t* vb = reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(v_buffer) + (int64_t)kvh * v_stride_h);
     if (causal) {
       const int t_end = min(plen, shift + block_q0 + 64 * NC);
       if (t_end > 0)
@@ -98,10 +96,9 @@ __global__ void __launch_bounds__(256) extend_attention_mfma128(
     p1 = min(p0 + per, plen);
   }
   if (p1 > p0) {
-    constexpr int kEl = KV8 ? 1 : 2;
     st.template run<false, true, kExtPF, typename BlockAttn<T, NC>::NoHook, KV8>(
-        lds, reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(k_buffer) + (int64_t)kvh * k_stride_h * kEl),
-        reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(v_buffer) + (int64_t)kvh * v_stride_h * kEl),
+        lds, reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(k_buffer) + (int64_t)kvh * k_stride_h),
+        reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(v_buffer) + (int64_t)kvh * v_stride_h),
         k_stride_n, v_stride_n, kv_indices + pstart, p0, p1, qpos, wave_qmax, sm_scale, logit_cap,
         typename BlockAttn<T, NC>::NoHook(), lut);
   }
@@ -157,13 +154,13 @@ __global__ void __launch_bounds__(128) extend_merge_kernel(const float* __restri
                                                          int64_t o_stride_h, const int32_t* __restrict__ qo_indptr, int B) {
   const int64_t t = blockIdx.x;
   if (t >= qo_indptr[B]) return;  // rows of an over-allocated q_extend hold no partials: leave their output alone
-  const int h = blockIdx.y, d = threadIdx.x;
+  const int h = blockIdx.y, d = threadIdx.x, D = blockDim.x;
   const int64_t row0 = (t * Hq + h) * kv_splits;
   float e_max = -INFINITY, e_sum = 0.f, acc = 0.f;
   for (int s = 0; s < kv_splits; ++s) {
     const float l = part_lse[row0 + s];
     if (l > -INFINITY) {
-      const float v = part_o[(row0 + s) * 128 + d];
+      const float v = part_o[(row0 + s) * D + d];
       const float n_max = fmaxf(l, e_max);
       const float old = expf(e_max - n_max), w = expf(l - n_max);
       acc = acc * old + w * v;
@@ -305,41 +302,53 @@ static int extend_attention_impl(const void* q_extend, const void* k_extend, con
   // the pool side of the tile kernel's requirements: 16-byte row pieces of 16-bit elements, or 8-byte pieces of codes
   const bool pool_ok = (kvf ? (al8(k_buffer) && al8(v_buffer)) : (aligned16(k_buffer) && aligned16(v_buffer))) &&
                        mult8(k_stride_n) && mult8(k_stride_h) && mult8(v_stride_n) && mult8(v_stride_h);
-  const bool fast = !custom_mask && window <= 0 && (dtype == SGLK_F16 || dtype == SGLK_BF16) && D == 128 && Dv == 128 &&
-                    aligned16(q_extend) && (paged || (aligned16(k_extend) && aligned16(v_extend))) && pool_ok &&
-                    ((uintptr_t)o_extend % 8 == 0) && mult8(q_stride_t) && mult8(q_stride_h) && mult8(ke_stride_t) &&
-                    mult8(ke_stride_h) && mult8(ve_stride_t) && mult8(ve_stride_h) && o_stride_t % 4 == 0 &&
-                    o_stride_h % 4 == 0;
-  // One column tile per wave (64 query rows per block) keeps the kernel at two blocks per CU; two tiles per wave
-  // halve the K/V re-reads but run at one wave per SIMD and measured 25 % slower (SGLK_EXTEND_NC=2 selects them).
-  const char* env_nc = getenv("SGLK_EXTEND_NC");
-  const size_t tile_lds = kBlockAttnLds + (kvf ? kKv8LutBytes : 0);
-#define SGLK_EXT_TILE(NCV, GRID, SPLITS, PO, PL)                                                                       \
-  SGLK_DISPATCH_HALF(dtype, T, {                                                                                       \
-    SGLK_DISPATCH_KV(kvf, T, KV, {                                                                                     \
-      hipLaunchKernelGGL((extend_attention_mfma128<T, NCV, KV>), GRID, dim3(256), tile_lds, s, q_extend, k_extend,      \
-                         v_extend, o_extend, k_buffer, v_buffer, qo_indptr, kv_indptr, kv_indices, Hq, Hkv, q_stride_t, \
-                         q_stride_h, ke_stride_t, ke_stride_h, ve_stride_t, ve_stride_h, o_stride_t, o_stride_h,        \
-                         k_stride_n, k_stride_h, v_stride_n, v_stride_h, sm_scale, logit_cap, causal, SPLITS, PO, PL);  \
-    });                                                                                                                \
+  const bool rows_ok = !custom_mask && window <= 0 && (dtype == SGLK_F16 || dtype == SGLK_BF16) && D == Dv &&
+                       aligned16(q_extend) && (paged || (aligned16(k_extend) && aligned16(v_extend))) && pool_ok &&
+                       ((uintptr_t)o_extend % 8 == 0) && mult8(q_stride_t) && mult8(q_stride_h) && mult8(ke_stride_t) &&
+                       mult8(ke_stride_h) && mult8(ve_stride_t) && mult8(ve_stride_h) && o_stride_t % 4 == 0 &&
+                       o_stride_h % 4 == 0;
+  const int64_t row_blocks = ((int64_t)max_extend_len * (Hq / Hkv) + kExtRows - 1) / kExtRows;
+  auto row32 = [](int64_t v) { return v >= 0 && v < (1ll << 31); };  // twice that, in bytes, fits 32 bits
+  const bool tile = rows_ok && kvf == 0 && (D == 128 || D == 64) && row_blocks <= 65535 && (int64_t)Hkv * B < (1ll << 31) &&
+                    row32(k_stride_n) && row32(v_stride_n) && row32(ke_stride_t) && row32(ve_stride_t);
+  const bool fast8 = rows_ok && kvf != 0 && D == 128;
+  if (kv_splits > 1 && (!(tile || fast8) || paged))
+    return fail(SGLK_EUNSUP, "extend_attention_split: 16-bit types with head size 64 or 128 (an fp8 pool: 128) and contiguous new tokens only");
+  float* part_o = kv_splits > 1 ? split_ws : nullptr;
+  float* part_lse = kv_splits > 1 ? split_ws + total_rows * Hq * kv_splits * D : nullptr;
+  if (tile) {
+    auto u16 = [](const void* p) { return reinterpret_cast<const uint16_t*>(p); };
+    const ExtendArgs a{u16(q_extend), u16(k_extend), u16(v_extend), u16(k_buffer), u16(v_buffer),
+                       reinterpret_cast<uint16_t*>(o_extend), qo_indptr, kv_indptr, kv_indices, Hq, Hkv, q_stride_t, q_stride_h,
+                       ke_stride_h, ve_stride_h, o_stride_t, o_stride_h, k_stride_h, v_stride_h, (uint32_t)(2 * ke_stride_t),
+                       (uint32_t)(2 * ve_stride_t), (uint32_t)(2 * k_stride_n), (uint32_t)(2 * v_stride_n), sm_scale, logit_cap,
+                       causal, kv_splits, part_o, part_lse};
+    // kv heads run fastest: with eight of them the blocks of one head share an XCD's L2
+    const dim3 grid(Hkv * B, (unsigned)row_blocks, kv_splits);
+#define SGLK_EXT(DV, PRE)                                                                    \
+  SGLK_DISPATCH_HALF(dtype, T, {                                                             \
+    if (int rc = ensure_lds<extend_tile_kernel<T, DV, PRE>>(4 * kExtTokens * 2 * DV)) return rc; \
+    hipLaunchKernelGGL((extend_tile_kernel<T, DV, PRE>), grid, dim3(256), 4 * kExtTokens * 2 * DV, s, a); \
   })
-  if (kv_splits > 1) {
-    if (!fast || paged)
-      return fail(SGLK_EUNSUP, "extend_attention_split: 16-bit types with head size 128 and contiguous new tokens only");
-    float* part_o = split_ws;
-    float* part_lse = split_ws + total_rows * Hq * kv_splits * 128;
-    dim3 grid(((max_extend_len + 63) / 64) * kv_splits, Hq, B);
-    SGLK_EXT_TILE(1, grid, kv_splits, part_o, part_lse);
-    SGLK_LAUNCH_CHECK();
-    SGLK_DISPATCH_HALF(dtype, T,
-                       hipLaunchKernelGGL((extend_merge_kernel<T>), dim3((unsigned)total_rows, Hq), dim3(128), 0, s, part_o,
-                                          part_lse, o_extend, Hq, kv_splits, o_stride_t, o_stride_h, qo_indptr, B));
-  } else if (fast && !(env_nc && atoi(env_nc) == 2)) {
-    dim3 grid((max_extend_len + 63) / 64, Hq, B);
-    SGLK_EXT_TILE(1, grid, 1, (float*)nullptr, (float*)nullptr);
-  } else if (fast) {
-    dim3 grid((max_extend_len + 64 * kNC - 1) / (64 * kNC), Hq, B);
-    SGLK_EXT_TILE(kNC, grid, 1, (float*)nullptr, (float*)nullptr);
+    const bool pre = logit_cap > 0.f || !(sm_scale > 0.f);
+    if (D == 128) {
+      if (pre) SGLK_EXT(128, true) else SGLK_EXT(128, false)
+    } else {
+      if (pre) SGLK_EXT(64, true) else SGLK_EXT(64, false)
+    }
+#undef SGLK_EXT
+  } else if (fast8) {
+    const dim3 grid(((max_extend_len + 63) / 64) * kv_splits, Hq, B);
+    SGLK_DISPATCH_HALF(dtype, T, {
+      SGLK_DISPATCH_KV(kvf, T, KV, {
+        if constexpr (!std::is_same<KV, T>::value)
+          hipLaunchKernelGGL((extend_attention_kv8<T, KV>), grid, dim3(256), kBlockAttnLds + kKv8LutBytes, s, q_extend, k_extend,
+                             v_extend, o_extend, k_buffer, v_buffer, qo_indptr, kv_indptr, kv_indices, Hq, Hkv, q_stride_t,
+                             q_stride_h, ke_stride_t, ke_stride_h, ve_stride_t, ve_stride_h, o_stride_t, o_stride_h,
+                             k_stride_n, k_stride_h, v_stride_n, v_stride_h, sm_scale, logit_cap, causal, kv_splits, part_o,
+                             part_lse);
+      });
+    });
   } else {
     dim3 grid(max_extend_len, Hq, B);
     const size_t lds = (size_t)D * sizeof(float);
@@ -373,7 +382,12 @@ static int extend_attention_impl(const void* q_extend, const void* k_extend, con
 #undef SGLK_GEN_ANY
 #undef SGLK_GEN
   }
-#undef SGLK_EXT_TILE
+  if (kv_splits > 1) {
+    SGLK_LAUNCH_CHECK();
+    SGLK_DISPATCH_HALF(dtype, T,
+                       hipLaunchKernelGGL((extend_merge_kernel<T>), dim3((unsigned)total_rows, Hq), dim3(D), 0, s, part_o,
+                                          part_lse, o_extend, Hq, kv_splits, o_stride_t, o_stride_h, qo_indptr, B));
+  }
   SGLK_LAUNCH_CHECK();
   return SGLK_OK;
 }

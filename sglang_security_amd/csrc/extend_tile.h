@@ -1,0 +1,292 @@
+// Extend attention over 16-bit K / V rows, head sizes 64 and 128 (gfx950).
+//
+// Rows are (token, query head) pairs of one kv head, token-major: a block owns 128 consecutive ones, a wave 32.  The
+// query heads that share a kv head so sit in one block whatever their number, every wave of a block sees nearly the
+// same tokens, and the K / V rows are fetched once for all of them.  Scores are formed transposed on the 32x32x16
+// matrix instruction, S^T = K . Q^T: a lane's accumulators are 16 tokens of ONE row, so a row's maximum takes one
+// exchange between the two half waves, and the same registers, rounded, are the P^T operand of O^T += V^T . P^T (the
+// order of the tokens inside a k-step is free as long as V is read in the same order).
+//
+// Bound: the matrix pipe and the LDS share the tile evenly (64 tokens x 128 rows: 1024 matrix cycles per SIMD, 32 KiB
+// written and 128 KiB read), with the exponentials of the co-resident block in between: two blocks per CU.  Head size 64
+// carries its probabilities as the sum of two 16-bit numbers (the wave-per-row kernel it replaces kept them in fp32:
+// 0.00166 off the 64-bit result both, 0.0023 with one number); head size 128 rounds them once, as before.
+//
+// Measured (bf16, launch alone): 8 prompts of 768 to 1152 tokens, 32 / 8 heads of 128: 264 us (one block per 64 rows of
+// one head, 32-token tiles on 16x16x32) -> 124 us, 525 TFLOP/s; one prompt of 1152 tokens: 69 -> 36 us; 128 tokens over
+// 1024 cached, split 8 ways: 20.1 -> 14.6 us; 4 prompts of 667 to 1000 tokens over 683 to 1024 cached, 14 / 2 heads of
+// 64: 3.24 ms (wave per row) -> 0.056 ms.
+#pragma once
+#include "attention_tile.h"
+
+namespace sglk {
+
+template <typename T>
+struct Mfma32;
+template <>
+struct Mfma32<bf16_t> {
+  static __device__ __forceinline__ float16v mma(short8 a, short8 b, float16v c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bfloat8, a), __builtin_bit_cast(bfloat8, b), c, 0, 0, 0);
+  }
+};
+template <>
+struct Mfma32<f16_t> {
+  static __device__ __forceinline__ float16v mma(short8 a, short8 b, float16v c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0, 0);
+  }
+};
+
+struct ExtendArgs {
+  const uint16_t *q, *ke, *ve, *kb, *vb;  // ke == nullptr: every token is in the pool (paged form)
+  uint16_t* o;
+  const int32_t *qo_indptr, *kv_indptr, *kv_indices;
+  int Hq, Hkv;
+  int64_t q_st, q_sh, ke_sh, ve_sh, o_st, o_sh, kb_sh, vb_sh;
+  uint32_t ke_row, ve_row, kb_row, vb_row;  // bytes from row to row (below 2^32: one 32 x 32 + 64-bit product an address)
+  float sm_scale, logit_cap;
+  int causal, kv_splits;
+  float *part_o, *part_lse;  // kv_splits > 1: [T, Hq, kv_splits, D] and [T, Hq, kv_splits]
+};
+
+constexpr int kExtTokens = 64;  // per tile
+constexpr int kExtRows = 128;   // per block
+
+// 16-byte chunk c of K row r: 16 rows of one chunk (an operand read) fall on 16 different slots of 256 bytes
+template <int D>
+__device__ __forceinline__ int ext_k_off(int r, int c) {
+  return D == 128 ? r * 256 + ((c ^ (r & 15)) << 4) : r * 128 + ((c ^ ((r >> 1) & 7)) << 4);
+}
+// 64-byte granule of V row r: the four rows of a transposed read fall on four different granules
+template <int D>
+__device__ __forceinline__ int ext_v_off(int r, int byte) {
+  const int sw = D == 128 ? (r & 3) : ((r >> 1) & 1);
+  return r * 2 * D + ((((byte >> 6) ^ sw) << 6) | (byte & 63));
+}
+
+// kv_splits > 1: blockIdx.z is the split; split s walks its slice of the cached prefix, the last one also the new
+// tokens, and leaves normalised fp32 rows + log-sum-exps (a short extend over a long prefix has too few rows to fill
+// the chip otherwise).
+// PRE: scores are finished (scale, cap) before their maximum is taken: a capped call, or a scale that is not positive.
+template <typename T, int D, bool PRE>
+__global__ void __launch_bounds__(256, 2) extend_tile_kernel(ExtendArgs a) {
+  constexpr int KS = D / 16, NV = D / 32, NP = D / 32;  // k-steps, 32-wide value blocks, 16-byte pieces per thread
+  constexpr int kStage = kExtTokens * 2 * D;            // K (or V) bytes of a stage
+  constexpr int kTpr = D / 8;                           // threads (chunks) per row
+  constexpr float LOG2E = 1.4426950408889634f;
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int kvh = blockIdx.x % a.Hkv, b = blockIdx.x / a.Hkv;
+  const int share = a.Hq / a.Hkv;
+  const int q0 = a.qo_indptr[b], ext = a.qo_indptr[b + 1] - q0;
+  const int nrows = ext * share;
+  const int R0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * kExtRows;  // the rows that see most start first
+  if (R0 >= nrows) return;                                           // block-uniform
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  const int l31 = lane & 31, hi = lane >> 5;
+  const bool paged = a.ke == nullptr;
+  const int pstart = a.kv_indptr[b], plen = a.kv_indptr[b + 1] - pstart;
+  const int shift = paged ? plen - ext : 0;
+
+  // this lane's row
+  const int R = R0 + 32 * wid + l31;
+  const bool row_ok = R < nrows;
+  const int Rc = min(R, nrows - 1);
+  const int tok = Rc / share, head = kvh * share + Rc - tok * share;
+  // the new tokens this lane, and any lane of this wave, may see (as positions of the causal stage)
+  const int w_first = min(R0 + 32 * wid, nrows - 1) / share + shift;
+  const int w_last = min(R0 + 32 * wid + 31, nrows - 1) / share + shift;
+  const bool w_idle = R0 + 32 * wid >= nrows;
+  const int b_last = min(R0 + kExtRows - 1, nrows - 1) / share;
+
+  short8 qf[KS];
+  {
+    const uint16_t* qr = a.q + (int64_t)(q0 + tok) * a.q_st + (int64_t)head * a.q_sh + 8 * hi;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const short8*>(qr + 16 * ks);
+  }
+
+  // ranges: tokens p0 .. p1 of the index list, then tokens 0 .. e1 of the new ones
+  int p0 = 0, p1 = plen, e1 = 0;
+  const int split = blockIdx.z;
+  if (paged) {
+    if (a.causal) p1 = min(plen, shift + b_last + 1);
+  } else {
+    if (a.kv_splits > 1) {
+      const int per = (((plen + a.kv_splits - 1) / a.kv_splits) + 31) / 32 * 32;
+      p0 = min(per * split, plen);
+      p1 = min(p0 + per, plen);
+    }
+    if (split == a.kv_splits - 1) e1 = a.causal ? b_last + 1 : ext;
+  }
+  const int nt1 = p1 > p0 ? (p1 - p0 + kExtTokens - 1) / kExtTokens : 0;
+  const int nt = nt1 + (e1 + kExtTokens - 1) / kExtTokens;
+
+  const uint16_t* kb = a.kb + (int64_t)kvh * a.kb_sh;
+  const uint16_t* vb = a.vb + (int64_t)kvh * a.vb_sh;
+  const uint16_t* ke = paged ? nullptr : a.ke + (int64_t)q0 * (a.ke_row >> 1) + (int64_t)kvh * a.ke_sh;
+  const uint16_t* ve = paged ? nullptr : a.ve + (int64_t)q0 * (a.ve_row >> 1) + (int64_t)kvh * a.ve_sh;
+  const int32_t* idx = a.kv_indices + pstart;
+
+  // a thread moves 16-byte piece `chunk` of rows frow + i * 256 / kTpr
+  const int frow = tid / kTpr, chunk = tid % kTpr;
+  int4v kreg[NP], vreg[NP];
+  int slot[NP];
+  auto fetch_idx = [&](int j) {  // pool rows of tile j (rows past the end re-read the last one; their scores are masked)
+    if (j < nt1) {
+#pragma unroll
+      for (int i = 0; i < NP; ++i) slot[i] = idx[min(p0 + j * kExtTokens + frow + i * (256 / kTpr), p1 - 1)];
+    }
+  };
+  auto fetch = [&](int j) {
+    const bool pool = j < nt1;  // block-uniform
+    const char* kp = reinterpret_cast<const char*>(pool ? kb : ke);
+    const char* vp = reinterpret_cast<const char*>(pool ? vb : ve);
+    const uint32_t ks = pool ? a.kb_row : a.ke_row, vs = pool ? a.vb_row : a.ve_row;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const uint32_t r = pool ? slot[i] : min((j - nt1) * kExtTokens + frow + i * (256 / kTpr), e1 - 1);
+      kreg[i] = *reinterpret_cast<const int4v*>(kp + ((uint64_t)r * ks + chunk * 16));
+      vreg[i] = *reinterpret_cast<const int4v*>(vp + ((uint64_t)r * vs + chunk * 16));
+    }
+  };
+
+  float m = -INFINITY, lsum = 0.f;  // running maximum (log2 domain) and this lane's share of the running sum
+  float16v oacc[NV];
+#pragma unroll
+  for (int n = 0; n < NV; ++n)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) oacc[n][r] = 0.f;
+  const float c = PRE ? 1.f : a.sm_scale * LOG2E;
+
+  if (nt > 0) {
+    fetch_idx(0);
+    fetch(0);
+    fetch_idx(1);
+  }
+  for (int j = 0; j < nt; ++j) {
+    char* kl = lds + (j & 1) * 2 * kStage;
+    char* vl = kl + kStage;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      const int r = frow + i * (256 / kTpr);
+      *reinterpret_cast<int4v*>(kl + ext_k_off<D>(r, chunk)) = kreg[i];
+      *reinterpret_cast<int4v*>(vl + ext_v_off<D>(r, chunk * 16)) = vreg[i];
+    }
+    __syncthreads();  // also: nobody reads the other stage any more once the next tile is parked
+    if (j + 1 < nt) {
+      fetch(j + 1);
+      fetch_idx(j + 2);
+    }
+    const bool pool = j < nt1;
+    const int t0 = pool ? p0 + j * kExtTokens : (j - nt1) * kExtTokens;
+    const int t_end = pool ? p1 : e1;
+    const bool diag = a.causal && (paged || !pool);
+    if (w_idle || (diag && t0 > w_last)) continue;  // wave-uniform: nothing of this tile is visible here
+
+    float16v s[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) s[u][r] = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const short8 kf = *reinterpret_cast<const short8*>(kl + ext_k_off<D>(32 * u + l31, 2 * ks + hi));
+        s[u] = Mfma32<T>::mma(kf, qf[ks], s[u]);
+      }
+    }
+    if constexpr (PRE) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const float v = s[u][r] * a.sm_scale;
+          s[u][r] = (a.logit_cap > 0.f ? a.logit_cap * tanhf(v / a.logit_cap) : v) * LOG2E;
+        }
+    }
+    if (t0 + kExtTokens > t_end || (diag && t0 + kExtTokens - 1 > w_first)) {  // wave-uniform
+      const int lim = diag ? min(tok + shift, t_end - 1) : t_end - 1;          // last token this row sees
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (t0 + 32 * u + 8 * (r >> 2) + 4 * hi + (r & 3) > lim) s[u][r] = -INFINITY;
+    }
+    float tmax = s[0][0];
+#pragma unroll
+    for (int r = 1; r < 16; ++r) tmax = fmaxf(tmax, s[0][r]);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, s[1][r]);
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64)) * c;
+    // The maximum only keeps the exponentials in range.  Probabilities that are rounded to 16 bits need it exact (the
+    // largest one is then 1 and has no rounding error); split ones let it lag by 2^8 and save most of the rescaling.
+    constexpr bool P2 = D == 64;
+    if (__any(tmax > m + (P2 ? 8.f : 0.f))) {
+      const float m_new = fmaxf(m, tmax);
+      const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - m_new);
+      m = m_new;
+      lsum *= alpha;
+#pragma unroll
+      for (int n = 0; n < NV; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) oacc[n][r] *= alpha;
+    }
+    const float m_use = m == -INFINITY ? 0.f : m;  // nothing visible yet: everything stays zero
+    short8 pf[4], pl[P2 ? 4 : 1];
+    float psum = 0.f;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float p = __builtin_amdgcn_exp2f(fmaf(s[u][r], c, -m_use));
+        psum += p;
+        const uint16_t ph = Conv<T>::from_f32(p);
+        pf[2 * u + (r >> 3)][r & 7] = (short)ph;
+        if constexpr (P2) pl[2 * u + (r >> 3)][r & 7] = (short)Conv<T>::from_f32(p - Conv<T>::to_f32(ph));
+      }
+    lsum += psum;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int row = 16 * k + 4 * hi + ((lane & 15) >> 2);
+#pragma unroll
+      for (int n = 0; n < NV; ++n) {
+        const int byte = 64 * n + 32 * ((lane >> 4) & 1) + 8 * (lane & 3);
+        const short4v lo = lds_read_tr16(vl + ext_v_off<D>(row, byte));
+        const short4v up = lds_read_tr16(vl + ext_v_off<D>(row + 8, byte));
+        const short8 vf = short8{lo[0], lo[1], lo[2], lo[3], up[0], up[1], up[2], up[3]};
+        oacc[n] = Mfma32<T>::mma(vf, pf[k], oacc[n]);
+        if constexpr (P2) oacc[n] = Mfma32<T>::mma(vf, pl[k], oacc[n]);
+      }
+    }
+  }
+
+  const float tot = lsum + __shfl_xor(lsum, 32, 64);
+  if (!row_ok) return;
+  const float inv = tot == 0.f ? 0.f : 1.0f / tot;
+  // lane (row, hi) holds elements 32 n + 8 g + 4 hi + 0 .. 3 of its row
+  if (a.kv_splits > 1) {
+    const int64_t row = ((int64_t)(q0 + tok) * a.Hq + head) * a.kv_splits + split;
+    float* dst = a.part_o + row * D + 4 * hi;
+#pragma unroll
+    for (int n = 0; n < NV; ++n)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        float4v v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = oacc[n][4 * g + r] * inv;
+        *reinterpret_cast<float4v*>(dst + 32 * n + 8 * g) = v;
+      }
+    if (hi == 0) a.part_lse[row] = tot == 0.f ? -INFINITY : (m + log2f(tot)) * 0.6931471805599453f;
+    return;
+  }
+  uint16_t* dst = a.o + (int64_t)(q0 + tok) * a.o_st + (int64_t)head * a.o_sh + 4 * hi;
+#pragma unroll
+  for (int n = 0; n < NV; ++n)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      short4v v;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = (short)Conv<T>::from_f32(oacc[n][4 * g + r] * inv);
+      *reinterpret_cast<short4v*>(dst + 32 * n + 8 * g) = v;
+    }
+}
+
+}  // namespace sglk

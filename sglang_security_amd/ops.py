@@ -386,6 +386,8 @@ def extend_attention_fwd(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buf
         total_prefix = kv_indices.numel() if kv_indptr.numel() > 1 else 0
     splits = extend_attention_split_plan(T, Hq, B, max_len_extend, int(total_prefix), D,
                                          q_extend.dtype) if (D == Dv and k_buffer is not None) else 1
+    if splits > 1 and D == 64 and not _tile_rows(q_extend, k_extend, v_extend, k_buffer, v_buffer):
+        splits = 1
     if splits > 1:
         return extend_attention_split(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buffer, qo_indptr, kv_indptr,
                                       kv_indices, max_len_extend, sm_scale, logit_cap, is_causal, splits)
@@ -399,10 +401,15 @@ def extend_attention_fwd(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buf
         _attn_dtype(q_extend, k_buffer, v_buffer), _stream(q_extend)), "extend_attention")
 
 
+def _tile_rows(q, *rows) -> bool:
+    """Whether rows of q's type lie as the tile kernels read them (16-byte pieces)."""
+    return all(t.dtype == q.dtype and t.data_ptr() % 16 == 0 and t.stride(0) % 8 == 0 and t.stride(1) % 8 == 0 for t in (q, *rows))
+
+
 def extend_attention_split_plan(T, Hq, B, max_len_extend, total_prefix, head_dim, dtype) -> int:
     """How many ways to split the cached prefix (1 = the plain kernel): only where one block per (sequence, query block,
     head) would leave most CUs without work and the prefixes are long enough to be worth a merge launch."""
-    if head_dim != 128 or dtype not in (torch.float16, torch.bfloat16) or B <= 0 or total_prefix <= 0:
+    if head_dim not in (64, 128) or dtype not in (torch.float16, torch.bfloat16) or B <= 0 or total_prefix <= 0:
         return 1
     blocks = ((int(max_len_extend) + 63) // 64) * Hq * B
     avg_prefix = total_prefix // B

@@ -1,0 +1,80 @@
+"""GPU: the extend kernel over (token, head) rows at the sizes where its tiles end: 64-token K/V tiles, 128-row blocks of
+token-major (token, query head) pairs, prefix and new tokens in any mix, both head sizes, every way it is called."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+# probabilities and results are rounded to the 16-bit type once each (2^-9 or 2^-12 of values up to about four)
+TOL = {torch.bfloat16: 2e-2, torch.float16: 4e-3}
+
+
+def _case(Hq, Hkv, D, pre, ext, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    n, T = sum(pre) + 5, sum(ext)
+    rows = lambda n, h: torch.randn(n, h, D, generator=g).to(dtype)
+    ptr = lambda v: torch.tensor([0] + list(torch.tensor(v).cumsum(0)), dtype=torch.int32)
+    return (rows(T, Hq), rows(T, Hkv), rows(T, Hkv), rows(n, Hkv), rows(n, Hkv), ptr(ext), ptr(pre),
+            (torch.randperm(n - 1, generator=g)[: sum(pre)] + 1).to(torch.int32))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Hq,Hkv,pre,ext,causal,cap,scale", [
+    (14, 2, [0, 64, 65], [130, 64, 63], True, 0.0, 1.0),      # seven heads a group: a token's rows straddle waves and blocks
+    (8, 1, [200], [1], True, 0.0, 1.0),                       # fewer rows than a wave
+    (3, 3, [1, 0], [129, 257], True, 0.0, 1.0),               # a head of its own per group
+    (40, 8, [127, 128, 129], [5, 31, 33], True, 0.0, 1.0),
+    (8, 2, [70, 0], [100, 65], False, 0.0, 1.0),              # every new token seen
+    (8, 2, [70, 0], [100, 65], True, 5.0, 1.0),               # capped scores
+    (4, 4, [40], [70], True, 0.0, -0.5),                      # a scale that turns the order of the scores round
+    (4, 2, [40], [70], True, 0.0, 0.0),
+    (130, 1, [3], [3], True, 0.0, 1.0),                       # more heads in a group than rows in a block
+])
+def test_rows_tiles_and_ranges(dtype, D, Hq, Hkv, pre, ext, causal, cap, scale):
+    import oracle
+    from sglang_security_amd import ops
+
+    t = _case(Hq, Hkv, D, pre, ext, dtype, seed=Hq + sum(pre) + sum(ext))
+    sm = scale / math.sqrt(D)
+    want = oracle.extend_attention(*t, sm, cap, causal)
+    q, ke, ve, kb, vb, qo, kp, ki = (x.to(DEV) for x in t)
+    for splits in (1, 3):
+        o = torch.full(q.shape, float("nan"), dtype=dtype, device=DEV)
+        ops.extend_attention_split(q, ke, ve, o, kb, vb, qo, kp, ki, max(ext), sm, cap, causal, splits)
+        assert (o.float().cpu() - want).abs().max().item() < TOL[dtype]
+    # the same rows as views with gaps, and one index list over a pool that holds every token
+    wide = lambda x: torch.nn.functional.pad(x, (0, 24)).transpose(0, 1).contiguous().transpose(0, 1)[..., :D]
+    o = torch.full_like(q, float("nan"))
+    ops.extend_attention_fwd(wide(q), wide(ke), wide(ve), o, wide(kb), wide(vb), qo, kp, ki, None, causal, None, max(ext), sm, cap)
+    assert (o.float().cpu() - want).abs().max().item() < TOL[dtype]
+    if causal:
+        pool_k, pool_v, at = torch.cat([kb, ke]), torch.cat([vb, ve]), kb.shape[0]
+        lists = [torch.cat([ki[kp[b]: kp[b + 1]], torch.arange(int(qo[b]), int(qo[b + 1]), dtype=torch.int32, device=DEV) + at])
+                 for b in range(len(ext))]
+        o = torch.full_like(q, float("nan"))
+        ops.prefill_attention_paged(q, o, pool_k, pool_v, qo, kp + qo, torch.cat(lists), max(ext), sm, cap)
+        assert (o.float().cpu() - want).abs().max().item() < TOL[dtype]
+
+
+def test_sums_outgrow_the_first_maximum():
+    """Scores that rise along the context: the running maximum, which may lag, has to move several times; and a row whose
+    first tile holds only scores of minus infinity."""
+    from sglang_security_amd import ops
+
+    T, D = 300, 128
+    g = torch.Generator().manual_seed(0)
+    q = torch.ones(T, 1, D).to(torch.bfloat16)
+    k = (torch.arange(T).view(T, 1, 1) / 64.0 * torch.ones(1, 1, D)).to(torch.bfloat16)     # q k: 0 .. 600
+    k[:70] = -math.inf
+    v = torch.randn(T, 1, D, generator=g).to(torch.bfloat16)
+    s = torch.einsum("thd,shd->hts", q.double(), k.double()) / math.sqrt(D)
+    p = torch.softmax(s.masked_fill(torch.ones(T, T, dtype=torch.bool).triu(1), -math.inf), -1)
+    want = torch.einsum("hts,shd->thd", torch.nan_to_num(p), v.double())
+    d = lambda x: x.to(DEV)
+    o, ptr = torch.empty_like(d(q)), torch.tensor([0, T], dtype=torch.int32, device=DEV)
+    none = torch.zeros(2, dtype=torch.int32, device=DEV)
+    ops.extend_attention_fwd(d(q), d(k), d(v), o, d(k), d(v), ptr, none, none[:1], None, True, None, T)
+    assert (o.double().cpu() - want)[70:].abs().max().item() < 2e-2
