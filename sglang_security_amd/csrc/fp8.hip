@@ -13,6 +13,7 @@
 #include <cstdlib>
 
 #include "common.h"
+#include "fp8_tile.h"
 
 namespace sglk {
 namespace {
@@ -618,6 +619,57 @@ int launch_mm(const MmArgs& p, hipStream_t s, int batch = 1) {
   return SGLK_OK;
 }
 
+template <typename TO, int BM, int BN, int WM, int WN, int ST>
+int launch_fp8_tile(const MmArgs& p, hipStream_t s) {
+  constexpr int lds = ST * (BM + BN) * 128;
+  if (int rc = ensure_lds<fp8_tile_kernel<TO, BM, BN, WM, WN, ST>>(lds)) return rc;
+  const Fp8TileArgs t{p.a, p.b, p.sa, p.sb, p.bias, p.out, p.M, p.N, p.K, (p.M + BM - 1) / BM, (p.N + BN - 1) / BN,
+                      p.a_stride, p.b_stride, p.out_stride};
+  hipLaunchKernelGGL((fp8_tile_kernel<TO, BM, BN, WM, WN, ST>), dim3((unsigned)t.mt * t.nt), dim3(64 * WM * WN), lds, s, t);
+  SGLK_LAUNCH_CHECK();
+  return SGLK_OK;
+}
+
+// Which tile form multiplies [M, K] x [N, K] fastest (0: the form of this call that is not tiled).  Estimates in
+// microseconds, fitted to launches on weights that come from memory (N, K of the 8B model's projections and of the 70B
+// model's on one of eight ranks; M = 1 .. 2048): a form needs its time per k-block of 128 for every round of blocks.
+// Measured against the register kernel and the streaming kernel, M x N x K: 2048 x 28672 x 4096: 1190 -> 214 (streaming
+// 788); 2048 x 4096 x 14336: 593 -> 110 (349); 256 x 4096 x 14336: 79 -> 37 (68); 128 x 28672 x 4096: 83 -> 33 (57);
+// 128 x 4096 x 4096: 14.6 -> 12.9 (16.5); 64 x 28672 x 4096 without the streaming copy: 50 -> 30.
+static int fp8_tile_choice(int64_t M, int64_t N, int64_t K, bool streaming) {
+  if (M <= 0 || K % 128 != 0 || N % 16 != 0 || getenv("SGLK_FP8_SPLITS") || getenv("SGLK_FP8_WAVES")) return 0;
+  auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  auto rounds = [&](int bm, int bn, int per_round) { return (double)up(up(M, bm) * up(N, bn), per_round); };
+  const double cost[5] = {1.5 * rounds(256, 256, 256), 1.17 * rounds(128, 128, 512), 0.62 * rounds(128, 128, 256),
+                          0.47 * rounds(64, 128, 256), 0.31 * rounds(64, 64, 256)};
+  int best = 0;
+  for (int i = 1; i < 5; ++i)
+    if (cost[i] < cost[best]) best = i;
+  const double tiled = cost[best] * (K / 128) + 3.5, passes = (double)up(M, 64), mb = (double)N * K * 1e-6;
+  // up to 64 rows the streaming kernel, which leaves the weights out of the caches, is the faster one in a layer's
+  // sequence of products (28672 x 4096 tiled: a pass of four products 106 us against 100); up to 32 the register
+  // kernel's smaller tiles keep up with the memory
+  const double other = streaming ? (M <= 64 ? 0.0 : 5 + 2 * passes + 0.19 * passes * mb)
+                                 : (M <= 32 ? 0.0 : 2 + 2 * passes + (0.08 + 0.31 * passes) * mb);
+  return tiled < other ? best + 1 : 0;
+}
+
+static bool fp8_tile_rows(const MmArgs& p) {
+  return p.out_stride % 8 == 0 && aligned16(p.out) && aligned16(p.sb) && (reinterpret_cast<uintptr_t>(p.bias) & 7) == 0 &&
+         p.a_stride < (1 << 24) && p.b_stride < (1 << 24);  // row offsets inside a tile are 32-bit
+}
+
+template <typename TO>
+int launch_fp8_tiled(int form, const MmArgs& p, hipStream_t s) {
+  switch (form) {
+    case 1: return launch_fp8_tile<TO, 256, 256, 2, 4, 2>(p, s);  // one block a CU
+    case 2: return launch_fp8_tile<TO, 128, 128, 2, 2, 2>(p, s);  // two
+    case 3: return launch_fp8_tile<TO, 128, 128, 2, 2, 4>(p, s);  // one, three stages ahead
+    case 4: return launch_fp8_tile<TO, 64, 128, 1, 4, 6>(p, s);
+    default: return launch_fp8_tile<TO, 64, 64, 1, 2, 4>(p, s);
+  }
+}
+
 
 // ---- streaming form of the per-token / per-channel scaled product at decode batch sizes --------------------------
 // out[M, N] = (x[M, K] . W[N, K]^T) * sa[m] * sb[n] (+ bias) with the weight re-laid-out once at load time
@@ -1027,9 +1079,15 @@ int sglk_fp8_scaled_mm(const void* a, const void* b_nk, const float* scales_a, c
   if (M == 0) return SGLK_OK;
   MmArgs p{(const uint8_t*)a, (const uint8_t*)b_nk, scales_a, scales_b, bias, out, M, N, K, a_stride, b_stride,
            out_stride,        0,                    0,        0,        0};
-  SGLK_DISPATCH_HALF(out_dtype, TO, return (launch_mm<TO, false>(p, (hipStream_t)stream)));
+  const int form = fp8_tile_rows(p) ? fp8_tile_choice(M, N, K, false) : 0;
+  SGLK_DISPATCH_HALF(out_dtype, TO, {
+    if (form) return (launch_fp8_tiled<TO>(form, p, (hipStream_t)stream));
+    return (launch_mm<TO, false>(p, (hipStream_t)stream));
+  });
   return SGLK_OK;
 }
+
+int sglk_fp8_tiled(int M, int N, int K) { return fp8_tile_choice(M, N, K, true) != 0; }
 
 int64_t sglk_fp8_mm_workspace_bytes(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
@@ -1156,7 +1214,9 @@ int sglk_fp8_scaled_mm_ws(const void* a, const void* b_nk, const float* scales_a
                           void* out, int M, int N, int K, int64_t a_stride, int64_t b_stride, int64_t out_stride,
                           void* workspace, int64_t workspace_bytes, int out_dtype, void* stream) {
   const int splits = (M > 0 && N > 0 && K > 0) ? fp8_splits(M, N, K) : 1;
-  if (splits <= 1 || !workspace || workspace_bytes < sglk_fp8_mm_workspace_bytes(M, N, K) || !aligned16(workspace))
+  const MmArgs shape{nullptr, nullptr, nullptr, scales_b, bias, out, M, N, K, a_stride, b_stride, out_stride};
+  if (splits <= 1 || !workspace || workspace_bytes < sglk_fp8_mm_workspace_bytes(M, N, K) || !aligned16(workspace) ||
+      (fp8_tile_rows(shape) && fp8_tile_choice(M, N, K, false)))
     return sglk_fp8_scaled_mm(a, b_nk, scales_a, scales_b, bias, out, M, N, K, a_stride, b_stride, out_stride, out_dtype,
                               stream);
   SGLK_CHECK(a && b_nk && scales_a && scales_b && out, "fp8_scaled_mm: null pointer");

@@ -1002,6 +1002,11 @@ def fp8_blockwise_scaled_mm_packed(mat_a, packed, scales_a, scales_b, out_dtype,
     return out
 
 
+def fp8_tiled(M, N, K) -> bool:
+    """Whether fp8_scaled_mm on a row-major weight is expected to beat fp8_scaled_mm_packed on its streaming copy."""
+    return bool(lib().sglk_fp8_tiled(M, N, K))
+
+
 def fp8_mm_packed_partial_splits(M, N, K) -> int:
     return int(lib().sglk_fp8_mm_packed_partial_splits(M, N, K))
 

@@ -115,7 +115,7 @@ class W8A8Fp8LinearMethod:
         xs = torch.empty(m, dtype=torch.float32, device=x.device)
         ops.per_token_quant_fp8(x2, xq, xs)
         ws = self._workspace(layer, m, x.device)
-        if layer.sglk_packed is not None and m <= self.streaming_max_tokens:
+        if layer.sglk_packed is not None and m <= self.streaming_max_tokens and not ops.fp8_tiled(m, n, k):
             out = ops.fp8_scaled_mm_packed(xq, layer.sglk_packed, xs, layer.weight_scale, x.dtype, bias, None, ws)
         else:
             out = ops.fp8_scaled_mm(xq, layer.weight, xs, layer.weight_scale, x.dtype, bias, None, ws)
