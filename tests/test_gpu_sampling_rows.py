@@ -1,0 +1,96 @@
+"""GPU: the sampling filters' radix selection where its shortcuts end: rows of peaked, flat, tied and unnormalised
+values, lists that overflow, thresholds below the mean, vocabularies that are no multiple of a load or a chunk, and rows
+that are not aligned.  Values are sums of few powers of two, so that every mass is exact and so is the kept set."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _rows(kind, n, g):
+    e = {"peaked": lambda: torch.randint(-20, 1, (n,), generator=g), "flat": lambda: torch.zeros(n, dtype=torch.long),
+         "two": lambda: torch.randint(-1, 1, (n,), generator=g) * 9,
+         "steep": lambda: -(torch.arange(n) * 22 // n)[torch.randperm(n, generator=g)]}[kind]()
+    x = 2.0 ** e.double()
+    if kind == "peaked":
+        x = x * (1 + torch.randint(0, 8, (n,), generator=g) / 8)
+    return x * 2.0 ** -30       # far from a mass of one: the guess of what can be skipped is checked
+
+
+def _threshold(x, k, p, joint):
+    thr = 0.0
+    s = x.sort(descending=True).values
+    if 0 < k < len(x):
+        thr = s[k - 1].item()
+    if p < 1:
+        lo = thr if (0 < k < len(x) and not joint) else 0.0
+        v = x[x >= lo].sort().values
+        target = (1 - p) * v.sum()
+        at = torch.nonzero(v.cumsum(0) >= target)
+        thr = max(thr, v[at[0, 0]].item() if len(at) else v[-1].item())
+    return thr
+
+
+@pytest.mark.parametrize("kind", ["peaked", "flat", "two", "steep"])
+@pytest.mark.parametrize("n", [1, 3, 255, 4099, 40000, 128259])
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** 15])
+def test_kept_sets(kind, n, scale):
+    import sglang_security_amd.sgl_kernel as sk
+    from sglang_security_amd import ops
+
+    g = torch.Generator().manual_seed(n)
+    x = _rows(kind, n, g) * scale
+    B = 6
+    wide = torch.zeros(B, n + 5, device=DEV)
+    wide[:, 1: n + 1] = x.float().to(DEV)
+    aligned = torch.zeros(B, (n + 3) // 4 * 4, device=DEV)
+    aligned[:, :n] = x.float().to(DEV)
+    ks = [0, 1, min(50, n), n // 2, n - 1, n]
+    ps = [0.75, 0.5, 0.875, 0.0, 1.0, 0.9375]       # exact in fp32
+    kt, pt = torch.tensor(ks, dtype=torch.int32, device=DEV), torch.tensor(ps, device=DEV)
+    for rows in (wide[:, 1: n + 1], aligned[:, :n]):
+        got_p = sk.top_p_renorm_probs(rows, pt).cpu().double()
+        got_k = sk.top_k_renorm_probs(rows, kt).cpu().double()
+        for b in range(B):
+            for got, want in ((got_p, _threshold(x, 0, ps[b], True)), (got_k, _threshold(x, ks[b], 1.0, True))):
+                kept = torch.where(x >= want, x, 0.0)
+                assert torch.equal(got[b] > 0, kept > 0)
+                assert torch.allclose(got[b], kept / kept.sum(), rtol=1e-5, atol=0)
+        for joint in (True, False):
+            for u in (0.0, 0.3, 0.999999):
+                ids = ops.sampling_from_probs(rows, torch.full((B,), u, device=DEV), kt, pt, 0.0, joint).cpu().long()
+                for b in range(B):
+                    kept = torch.where(x >= _threshold(x, ks[b], ps[b], joint), x, 0.0)
+                    cum = kept.cumsum(0) / kept.sum()
+                    i = int(ids[b])
+                    assert kept[i] > 0
+                    # the running sum passes u at the chosen index, up to the rounding of fp32 sums
+                    assert cum[i] >= u - 1e-5 and (i == 0 or cum[i - 1] <= u + 1e-5)
+
+
+def test_rows_without_mass():
+    """All zeros, and values that are not numbers or negative beside one that is."""
+    from sglang_security_amd import ops
+
+    x = torch.zeros(3, 1000, device=DEV)
+    x[1, 17] = 0.5
+    x[2] = float("nan")
+    x[2, ::2] = -1.0
+    x[2, 400] = 0.25
+    u = torch.full((3,), 0.5, device=DEV)
+    k, p = torch.full((3,), 10, dtype=torch.int32, device=DEV), torch.full((3,), 0.9, device=DEV)
+    for joint in (True, False):
+        ids = ops.sampling_from_probs(x, u, k, p, 0.0, joint).tolist()
+        assert ids == [999, 17, 400]
+
+
+def test_rows_of_infinite_mass():
+    """The k largest are found where masses say nothing."""
+    import sglang_security_amd.sgl_kernel as sk
+
+    x = (torch.arange(3000, device=DEV) % 997).float()[None] + 1
+    x[0, 5] = float("inf")
+    got = sk.top_k_renorm_probs(x, 20)
+    assert torch.equal(torch.nan_to_num(got, nan=1.0)[0] != 0, x[0] == float("inf"))
+    assert got[0].isnan().sum() == 1            # inf / inf; the other kept values over infinity are zeros
