@@ -813,8 +813,8 @@ SGLK_API int sglk_top_k_renorm_probs(const float* probs, float* out, const int32
                                      int top_k_val, int batch, int vocab, int64_t in_stride,
                                      int64_t out_stride, void* stream);
 /* Drop the longest ascending run of entries whose cumulative mass stays below 1 - top_p, renormalise the rest:
- * top_p_renorm_probs, sampling.py:69-102.  The cumulative masses are fp32 sums whose order is not fixed: an entry
- * whose cumulative mass sits within rounding of 1 - top_p may fall on either side of the cut from run to run. */
+ * top_p_renorm_probs, sampling.py:69-102.  The cumulative masses are sums in fixed point (2^-44 of the row's
+ * mass at 128256 entries); those of the least entries are fp32 sums. */
 SGLK_API int sglk_top_p_renorm_probs(const float* probs, float* out, const float* top_p_arr,
                                      float top_p_val, int batch, int vocab, int64_t in_stride,
                                      int64_t out_stride, void* stream);
@@ -828,6 +828,21 @@ SGLK_API int sglk_sampling_from_probs(const float* probs, const float* uniform, 
                                       const float* top_p_arr, float top_p_val,
                                       const float* min_p_arr, float min_p_val, int joint, int batch,
                                       int vocab, int64_t in_stride, void* stream);
+/* The same with a caller's workspace (16-byte aligned, contents of no matter before and after;
+ * sglk_sampling_workspace_bytes(batch, vocab), 0 where it would not be used): rows are spread over several blocks in
+ * four launches.  Without one, or a smaller one, every row is one block's. */
+SGLK_API int64_t sglk_sampling_workspace_bytes(int batch, int vocab);
+SGLK_API int sglk_top_k_renorm_probs_ws(const float* probs, float* out, const int32_t* top_k_arr,
+                                        int top_k_val, int batch, int vocab, int64_t in_stride,
+                                        int64_t out_stride, void* workspace, int64_t workspace_bytes, void* stream);
+SGLK_API int sglk_top_p_renorm_probs_ws(const float* probs, float* out, const float* top_p_arr,
+                                        float top_p_val, int batch, int vocab, int64_t in_stride,
+                                        int64_t out_stride, void* workspace, int64_t workspace_bytes, void* stream);
+SGLK_API int sglk_sampling_from_probs_ws(const float* probs, const float* uniform, int32_t* out,
+                                         const int32_t* top_k_arr, int top_k_val, const float* top_p_arr,
+                                         float top_p_val, const float* min_p_arr, float min_p_val, int joint,
+                                         int batch, int vocab, int64_t in_stride, void* workspace,
+                                         int64_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------------ draft-tree helpers -------- */
 

@@ -9,9 +9,11 @@
 // is wide enough (sixteen bins an octave) that the chosen bins fit an LDS list, and the other digits are taken from
 // there; rows are read in 16-byte pieces, eight in flight a thread.
 //
-// Measured, 64 rows of 128256, top-k and top-p together: sampling 555 -> 81 us, top-p renormalisation 390 -> 66 us (256
-// bins for four 8-bit digits each, a float atomic on a handful of exponents for every element, and a thread's elements
-// 500 bytes from the next thread's).
+// Measured, 64 rows of 128256, top-k and top-p together: sampling 555 us (256 bins for four 8-bit digits each, a float
+// atomic on a handful of exponents for every element, a thread's elements 500 bytes from the next thread's) -> 81 us with
+// a block a row, 45 us with its rows spread over four blocks; top-p renormalisation 390 -> 66 -> 44 us.
+#include <algorithm>
+
 #include "common.h"
 
 namespace sglk {
@@ -28,11 +30,13 @@ struct SampShared {
     float chunk[kBins];
   };
   uint32_t list[2][kList];  // bit patterns: candidates of the top-k cut, of the top-p cut
+  u64 digit[2][128];
+  uint32_t cut[2];
   float red[16];
   u64 ured[16];
   uint32_t fill[2];
-  int pick, last;
-  u64 below, below_last;
+  int pick;
+  u64 below;
   uint32_t need;
 };
 
@@ -92,12 +96,11 @@ __device__ __forceinline__ V bscan(V v, V* red, V& total) {
   return base + incl - v;
 }
 
-// f(value) for every element of the row
-template <bool VEC, typename F>
+// f(value) for every element of the row, U loads in flight
+template <bool VEC, int U = 8, typename F>
 __device__ __forceinline__ void each(const float* __restrict__ x, int n, F f) {
   if constexpr (VEC) {
     const int n4 = n >> 2;
-    constexpr int U = 8;  // loads in flight
     for (int i0 = threadIdx.x; i0 < n4; i0 += U * kSampThreads) {
       float4v r[U];
 #pragma unroll
@@ -139,38 +142,40 @@ __device__ __forceinline__ int pick_count(SampShared& sh, const Fixed& fx, uint3
 }
 
 // first bin with mass at which the mass, `below` included, reaches `target`; if the target lies beyond the total, the last
-// bin with mass.  sh.below: the mass in front of the bin
+// bin with mass (0 if there is none).  sh.below: the mass in front of the bin
 template <int PER>
 __device__ __forceinline__ int pick_mass(SampShared& sh, const Fixed& fx, u64 below, u64 target) {
-  if (threadIdx.x == 0) {
-    sh.pick = kBins;
-    sh.last = -1;
-  }
   u64 m[PER], own = 0, total;
 #pragma unroll
   for (int j = 0; j < PER; ++j) own += m[j] = fx.mass(sh.bin[threadIdx.x * PER + j]);
-  u64 run = below + bscan<u64>(own, sh.ured, total);  // also: pick and last are set
-  int first = kBins, last = -1;
-  u64 at_first = run, at_last = run;
+  u64 run = below + bscan<u64>(own, sh.ured, total);
+  if (target == 0) target = 1;
+  if (below + total >= target) {  // block-uniform: whole numbers, one bin passes the target
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      if (m[j] > 0 && (run < target || run == below) && run + m[j] >= target) {
+        sh.pick = threadIdx.x * PER + j;
+        sh.below = run;
+      }
+      run += m[j];
+    }
+    __syncthreads();
+    return sh.pick;
+  }
+  if (threadIdx.x == 0) sh.pick = 0;
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < PER; ++j)
+    if (m[j] > 0) atomicMax(&sh.pick, (int)threadIdx.x * PER + j);
+  if (threadIdx.x == 0) sh.below = below;
+  __syncthreads();
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
-    if (m[j] > 0) {
-      if (run + m[j] >= target && first == kBins) first = threadIdx.x * PER + j, at_first = run;
-      last = threadIdx.x * PER + j, at_last = run;
-    }
+    if (m[j] > 0 && sh.pick == (int)threadIdx.x * PER + j) sh.below = run;
     run += m[j];
   }
-  if (first < kBins) atomicMin(&sh.pick, first);
-  if (last >= 0) atomicMax(&sh.last, last);
   __syncthreads();
-  if (sh.pick == first && first < kBins) sh.below = at_first;
-  if (sh.last == last && last >= 0) sh.below_last = at_last;
-  __syncthreads();
-  const bool found = sh.pick < kBins;
-  const int d = found ? sh.pick : max(sh.last, 0);
-  if (!found && threadIdx.x == 0) sh.below = sh.last >= 0 ? sh.below_last : below;
-  __syncthreads();
-  return d;
+  return sh.pick;
 }
 
 __device__ __forceinline__ void clear_bins(SampShared& sh, int bins) {
@@ -207,6 +212,62 @@ __device__ uint32_t refine(const float* __restrict__ x, int n, SampShared& sh, c
       below = sh.below;
     }
     __syncthreads();
+    prefix |= (uint32_t)d << shift;
+    bits = shift;
+  }
+  return prefix;
+}
+
+// The same from a list, by one wave: digits of 6, 6 and 7 bits, two bins a lane, no block barrier.
+template <bool COUNT>
+__device__ uint32_t refine_list(u64* bins, const Fixed& fx, const uint32_t* list, int listed, int bin, uint32_t rank, u64 below, u64 target,
+                                uint32_t lo) {
+  const int lane = threadIdx.x & 63;
+  uint32_t prefix = (uint32_t)bin << 19;
+  int bits = 19;
+  if (!COUNT && target == 0) target = 1;
+#pragma unroll
+  for (int digit = 0; digit < 3; ++digit) {
+    const int take = digit < 2 ? 6 : 7, shift = bits - take;
+    bins[2 * lane] = bins[2 * lane + 1] = 0;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // one wave: its LDS accesses are done in order
+    for (int i = lane; i < listed; i += 64) {
+      const uint32_t b = list[i];
+      if ((b >> bits) == (prefix >> bits) && b >= lo) atomicAdd(&bins[(b >> shift) & ((1u << take) - 1)], (1ull << fx.bits) + fx.of(b));
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    const u64 w0 = bins[2 * lane], w1 = bins[2 * lane + 1];
+    u64 incl = w0 + w1;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const u64 v = __shfl_up(incl, o, 64);
+      if (lane >= o) incl += v;
+    }
+    const u64 total = __shfl(incl, 63, 64), before = incl - (w0 + w1);
+    int d = -1;
+    if (COUNT) {
+      const uint32_t c0 = fx.count(w0), c1 = fx.count(w1);
+      uint32_t above = fx.count(total) - fx.count(before) - c0 - c1;
+      uint32_t need = 0;
+      if (above < rank && rank <= above + c1) d = 2 * lane + 1, need = rank - above;
+      above += c1;
+      if (above < rank && rank <= above + c0) d = 2 * lane, need = rank - above;
+      const u64 who = __ballot(d >= 0);
+      const int src = who ? __ffsll(who) - 1 : 0;
+      d = max(__shfl(d, src, 64), 0);
+      rank = __shfl(need, src, 64);
+    } else {
+      const u64 m0 = fx.mass(w0), m1 = fx.mass(w1);
+      const bool reach = below + fx.mass(total) >= target;  // else: the last bin with mass
+      u64 at = below + fx.mass(before), run = at;
+      if (m0 > 0 && (reach ? run + m0 >= target : true)) d = 2 * lane, at = run;
+      run += m0;
+      if (m1 > 0 && (reach ? d < 0 && run + m1 >= target : true)) d = 2 * lane + 1, at = run;
+      const u64 who = __ballot(d >= 0);
+      const int src = !who ? 0 : reach ? __ffsll(who) - 1 : 63 - __clzll(who);
+      d = max(__shfl(d, src, 64), 0);
+      if (who) below = __shfl(at, src, 64);
+    }
     prefix |= (uint32_t)d << shift;
     bits = shift;
   }
@@ -303,6 +364,7 @@ __device__ float row_threshold(const float* __restrict__ x, int n, const RowPara
       target = goal(low + mass_of(0));
       pbin = pick_mass<PER>(sh, fx, low, target);
       below = sh.below;
+      __syncthreads();
     }
     const int kcount = kbin >= 0 ? (int)fx.count(sh.bin[kbin]) : 0;
     int pcount = pbin >= 0 ? (int)fx.count(sh.bin[pbin]) : 0;
@@ -363,6 +425,7 @@ __device__ float row_threshold(const float* __restrict__ x, int n, const RowPara
       target = goal(above + part);
       pbin = pick_mass<PER>(sh, fx, 0, target);
       below = sh.below;
+      __syncthreads();
       int plist = 0;
       pcount = kcount;
       if (pbin != kbin) {
@@ -389,34 +452,8 @@ __device__ float row_threshold(const float* __restrict__ x, int n, const RowPara
   return thr;
 }
 
-__device__ __forceinline__ RowParams load_params(int row, const int32_t* k_arr, int k_val, const float* p_arr, float p_val,
-                                                 const float* m_arr, float m_val, int joint) {
-  RowParams rp;
-  rp.top_k = k_arr ? k_arr[row] : k_val;
-  rp.top_p = p_arr ? p_arr[row] : p_val;
-  rp.min_p = m_arr ? m_arr[row] : m_val;
-  rp.joint = joint;
-  return rp;
-}
-
 template <bool VEC>
-__global__ void __launch_bounds__(kSampThreads) renorm_kernel(const float* __restrict__ probs, float* __restrict__ out,
-                                                             int n, int64_t in_stride, int64_t out_stride,
-                                                             const int32_t* k_arr, int k_val, const float* p_arr,
-                                                             float p_val) {
-  __shared__ SampShared sh;
-  const int row = blockIdx.x;
-  const float* x = probs + (int64_t)row * in_stride;
-  const RowParams rp = load_params(row, k_arr, k_val, p_arr, p_val, nullptr, 0.f, 1);
-  float kept;
-  const float thr = row_threshold<VEC>(x, n, rp, sh, kept);
-  if (!(kept > 0.f)) {
-    float s = 0.f;
-    each<VEC>(x, n, [&](float v) { s += v >= thr ? v : 0.f; });
-    kept = bsum(s, sh.red);
-  }
-  const float inv = 1.0f / kept;
-  float* o = out + (int64_t)row * out_stride;
+__device__ __forceinline__ void write_renormed(const float* __restrict__ x, float* __restrict__ o, int n, float thr, float inv) {
   if constexpr (VEC) {
     for (int i = threadIdx.x; i < n >> 2; i += kSampThreads) {
       float4v v = *reinterpret_cast<const float4v*>(x + 4 * (int64_t)i);
@@ -431,56 +468,67 @@ __global__ void __launch_bounds__(kSampThreads) renorm_kernel(const float* __res
   }
 }
 
-// Inverse CDF over the kept elements in index order: the first kept index whose running sum exceeds u * total.  The row
-// is summed in chunks of whole waves; the chunk that holds the target is walked again by one wave.
 template <bool VEC>
-__global__ void __launch_bounds__(kSampThreads) sample_kernel(const float* __restrict__ probs,
-                                                             const float* __restrict__ uniform, int32_t* __restrict__ out,
-                                                             int n, int64_t in_stride, const int32_t* k_arr, int k_val,
-                                                             const float* p_arr, float p_val, const float* m_arr,
-                                                             float m_val, int joint) {
-  __shared__ SampShared sh;
-  const int row = blockIdx.x, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  const float* x = probs + (int64_t)row * in_stride;
-  const RowParams rp = load_params(row, k_arr, k_val, p_arr, p_val, m_arr, m_val, joint);
+__device__ void renorm_row(const float* __restrict__ x, float* __restrict__ o, int n, const RowParams& rp, SampShared& sh) {
   float kept;
   const float thr = row_threshold<VEC>(x, n, rp, sh, kept);
-  auto four = [&](int64_t i) {  // kept values of elements i .. i + 3
-    float4v v = {0.f, 0.f, 0.f, 0.f};
-    if (VEC && i + 4 <= n) {
-      v = *reinterpret_cast<const float4v*>(x + i);
-    } else {
+  if (!(kept > 0.f)) {
+    float s = 0.f;
+    each<VEC>(x, n, [&](float v) { s += v >= thr ? v : 0.f; });
+    kept = bsum(s, sh.red);
+  }
+  write_renormed<VEC>(x, o, n, thr, 1.0f / kept);
+}
+
+// kept values of elements i .. i + 3
+template <bool VEC>
+__device__ __forceinline__ float4v kept_four(const float* __restrict__ x, int n, int64_t i, float thr) {
+  float4v v = {0.f, 0.f, 0.f, 0.f};
+  if (VEC && i + 4 <= n) {
+    v = *reinterpret_cast<const float4v*>(x + i);
+  } else {
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
-        if (i + e < n) v[e] = x[i + e];
-    }
+    for (int e = 0; e < 4; ++e)
+      if (i + e < n) v[e] = x[i + e];
+  }
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = v[e] >= thr ? v[e] : 0.f;
-    return v;
-  };
-  const int64_t chunk = 256 * (((int64_t)n + 256 * kBins - 1) / (256 * kBins));  // at most kBins chunks
-  const int chunks = (int)((n + chunk - 1) / chunk);
-  __syncthreads();
-  for (int i = threadIdx.x; i < kBins; i += kSampThreads) sh.chunk[i] = 0.f;
-  __syncthreads();
-  for (int c0 = wid; c0 < chunks; c0 += 64) {
+  for (int e = 0; e < 4; ++e) v[e] = v[e] >= thr ? v[e] : 0.f;
+  return v;
+}
+
+// elements a chunk has: at most kBins chunks a row
+__host__ __device__ inline int64_t chunk_of(int64_t n) { return 256 * ((n + 256 * kBins - 1) / (256 * kBins)); }
+
+// masses of the kept elements of chunks c0 .. c1 - 1, whole waves at a time
+template <bool VEC>
+__device__ __forceinline__ void sum_chunks(const float* __restrict__ x, int n, float thr, int64_t chunk, int first, int last,
+                                           float* __restrict__ sums) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  for (int c0 = first + wid; c0 < last; c0 += 64) {
     float s[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       s[u] = 0.f;
       const int64_t c = c0 + 16 * u;
-      if (c < chunks)
+      if (c < last)
         for (int64_t i = c * chunk; i < (c + 1) * chunk; i += 256) {
-          const float4v v = four(i + 4 * lane);
+          const float4v v = kept_four<VEC>(x, n, i + 4 * lane, thr);
           s[u] += (v[0] + v[1]) + (v[2] + v[3]);
         }
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
       s[u] = wave_sum(s[u]);
-      if (lane == 0 && c0 + 16 * u < chunks) sh.chunk[c0 + 16 * u] = s[u];
+      if (lane == 0 && c0 + 16 * u < last) sums[c0 + 16 * u] = s[u];
     }
   }
+}
+
+// Inverse CDF over the kept elements in index order: the first kept index whose running sum exceeds u * total.  The
+// chunks' masses stand in sh.chunk (zeros behind the last); the chunk that holds the target is walked by one wave.
+template <bool VEC>
+__device__ void choose(const float* __restrict__ x, int n, float thr, int64_t chunk, float u, int32_t* __restrict__ out, SampShared& sh) {
+  const int lane = threadIdx.x & 63;
   if (threadIdx.x == 0) sh.pick = kBins;
   __syncthreads();
   constexpr int PER = kBins / kSampThreads;
@@ -488,7 +536,7 @@ __global__ void __launch_bounds__(kSampThreads) sample_kernel(const float* __res
 #pragma unroll
   for (int j = 0; j < PER; ++j) own += m[j] = sh.chunk[threadIdx.x * PER + j];
   float run = bscan<float>(own, sh.red, total);
-  const float target = uniform[row] * total;
+  const float target = u * total;
   int first = kBins;
   float at_first = 0.f;
 #pragma unroll
@@ -501,19 +549,19 @@ __global__ void __launch_bounds__(kSampThreads) sample_kernel(const float* __res
   const int c = sh.pick;
   if (c == first && first < kBins) sh.red[0] = at_first;
   __syncthreads();
-  if (wid != 0) return;
+  if (threadIdx.x >= 64) return;
   int pick = -1;
   if (c < kBins) {
     run = sh.red[0];
     int last = -1;
     for (int64_t i = c * chunk; i < (c + 1) * chunk && pick < 0; i += 256) {
-      const float4v v = four(i + 4 * lane);
+      const float4v v = kept_four<VEC>(x, n, i + 4 * lane, thr);
       const float sum = (v[0] + v[1]) + (v[2] + v[3]);
       float incl = sum;
 #pragma unroll
       for (int o = 1; o < 64; o <<= 1) {
-        const float u = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += u;
+        const float w = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += w;
       }
       float r = run + (incl - sum);
       int at = 1 << 30, mine = -1;
@@ -542,8 +590,350 @@ __global__ void __launch_bounds__(kSampThreads) sample_kernel(const float* __res
         if (x[i] >= thr) pick = i;
       if (pick < 0) pick = 0;
     }
-    out[row] = pick;
+    *out = pick;
   }
+}
+
+template <bool VEC>
+__device__ void sample_row(const float* __restrict__ x, int n, const RowParams& rp, float u, int32_t* __restrict__ out, SampShared& sh) {
+  float kept;
+  const float thr = row_threshold<VEC>(x, n, rp, sh, kept);
+  const int64_t chunk = chunk_of(n);
+  __syncthreads();
+  for (int i = threadIdx.x; i < kBins; i += kSampThreads) sh.chunk[i] = 0.f;
+  __syncthreads();
+  sum_chunks<VEC>(x, n, thr, chunk, 0, (int)((n + chunk - 1) / chunk), sh.chunk);
+  __syncthreads();
+  choose<VEC>(x, n, thr, chunk, u, out, sh);
+}
+
+struct SampArgs {
+  const float* probs;
+  float* out;               // renormalised rows, or nullptr
+  const float* uniform;
+  int32_t* ids;
+  int n;
+  int64_t in_stride, out_stride;
+  const int32_t* k_arr;
+  const float *p_arr, *m_arr;
+  int k_val;
+  float p_val, m_val;
+  int joint;
+  int slices, slice;        // blocks a row is spread over, elements each
+  char* ws;
+};
+
+__device__ __forceinline__ RowParams load_params(const SampArgs& a, int row) {
+  RowParams rp;
+  rp.top_k = a.k_arr ? a.k_arr[row] : a.k_val;
+  rp.top_p = a.p_arr ? a.p_arr[row] : a.p_val;
+  rp.min_p = a.m_arr ? a.m_arr[row] : a.m_val;
+  rp.joint = a.joint;
+  return rp;
+}
+
+// one block per row
+template <bool VEC>
+__global__ void __launch_bounds__(kSampThreads) filter_rows_kernel(SampArgs a) {
+  __shared__ SampShared sh;
+  const int row = blockIdx.x;
+  const float* x = a.probs + (int64_t)row * a.in_stride;
+  const RowParams rp = load_params(a, row);
+  if (a.out)
+    renorm_row<VEC>(x, a.out + (int64_t)row * a.out_stride, a.n, rp, sh);
+  else
+    sample_row<VEC>(x, a.n, rp, a.uniform[row], a.ids + row, sh);
+}
+
+// ---- rows spread over several blocks --------------------------------------------------------------------------------
+// A unit streams about 20 bytes a clock of a row that the caches do not hold, and a batch of 64 rows leaves three of four
+// units idle.  The same selection in launches that meet at their ends: bins per slice; every block adds its row's bins up
+// and collects its slice's candidates; every block finishes the threshold and writes (or sums) its slice; one block per
+// row picks.  The first digit has a window of 1024 bins (2^64 of the least value binned).  Rows the guess of mass one does
+// not hold for, or whose candidates overflow a list, are done whole by one block of the last launch.
+constexpr int kWindow = 1024;
+constexpr int kMaxSlices = 16;
+struct SliceStat {
+  float under, over, vmax, pad;
+};
+struct RowState {
+  u64 below, target, above;
+  int valid, kbin, pbin, kcount, pcount;
+  uint32_t rank;
+  float vmax, thr;
+};
+struct SampWs {  // of one row
+  u64* bins;        // [slices][kWindow]
+  SliceStat* stat;  // [slices]
+  RowState* state;
+  uint32_t* fill;   // [2]
+  uint32_t* list;   // [2][kList]
+  float* chunk;     // [kBins]
+};
+__host__ __device__ inline int64_t samp_ws_row(int slices) {
+  return (int64_t)slices * (kWindow * 8 + 16) + 128 + 16 + 2 * kList * 4 + kBins * 4;
+}
+__device__ __forceinline__ SampWs samp_ws(const SampArgs& a, int row) {
+  char* w = a.ws + (int64_t)row * samp_ws_row(a.slices);
+  SampWs r;
+  r.bins = reinterpret_cast<u64*>(w);
+  w += (int64_t)a.slices * kWindow * 8;
+  r.state = reinterpret_cast<RowState*>(w);
+  w += 128;
+  r.stat = reinterpret_cast<SliceStat*>(w);
+  w += a.slices * 16;
+  r.fill = reinterpret_cast<uint32_t*>(w);
+  w += 16;
+  r.list = reinterpret_cast<uint32_t*>(w);
+  w += 2 * kList * 4;
+  r.chunk = reinterpret_cast<float*>(w);
+  return r;
+}
+static_assert(sizeof(RowState) <= 128, "");
+
+struct Guess {  // what a row of mass one can leave unbinned
+  bool use_k, use_p;
+  float least;
+  Fixed fx;
+  int base;
+};
+__device__ __forceinline__ Guess guess_of(const RowParams& rp, int n) {
+  Guess g;
+  g.use_k = rp.top_k > 0 && rp.top_k < n;
+  g.use_p = rp.top_p < 1.0f;
+  const float share = 0.999f * (1.0f - rp.top_p) / (float)n, mean = 1.0f / (float)n;
+  g.least = g.use_p ? (g.use_k ? fminf(mean, share) : share) : mean;
+  if (!(g.least >= 0.f)) g.least = 0.f;
+  g.fx.bits = 32 + __clz(n) - 1;
+  g.fx.scale = g.fx.bits - 2;
+  g.base = (int)(__float_as_uint(g.least) >> 19);
+  return g;
+}
+
+template <bool VEC>
+__global__ void __launch_bounds__(kSampThreads) slice_bins_kernel(SampArgs a) {
+  __shared__ SampShared sh;
+  const int slice = blockIdx.x, row = blockIdx.y, lo = slice * a.slice, n = min(a.slice, a.n - lo);
+  const float* x = a.probs + (int64_t)row * a.in_stride + lo;
+  const RowParams rp = load_params(a, row);
+  const Guess g = guess_of(rp, a.n);
+  const SampWs w = samp_ws(a, row);
+  clear_bins(sh, kWindow);
+  float s = 0.f, o = 0.f, mx = 0.f;
+  const bool bin = g.use_k || g.use_p;
+  each<VEC, 4>(x, n, [&](float raw) {
+    const float v = fmaxf(raw, 0.f);
+    const uint32_t b = __float_as_uint(v);
+    const bool in = bin && v >= g.least;
+    mx = fmaxf(mx, v);
+    s += in ? 0.f : v;
+    o += in ? v : 0.f;
+    if (in) atomicAdd(&sh.bin[min((int)(b >> 19) - g.base, kWindow - 1)], (1ull << g.fx.bits) + g.fx.of(b));
+  });
+  mx = bmax(mx, sh.red);
+  s = bsum(s, sh.red);
+  o = bsum(o, sh.red);
+  if (threadIdx.x == 0) w.stat[slice] = SliceStat{s, o, mx, 0.f};
+  if (slice == 0 && threadIdx.x < 2) w.fill[threadIdx.x] = 0;
+  if (bin) w.bins[slice * kWindow + threadIdx.x] = sh.bin[threadIdx.x];
+}
+
+template <bool VEC>
+__global__ void __launch_bounds__(kSampThreads) slice_collect_kernel(SampArgs a) {
+  __shared__ SampShared sh;
+  const int slice = blockIdx.x, row = blockIdx.y, lo = slice * a.slice, n = min(a.slice, a.n - lo);
+  const float* x = a.probs + (int64_t)row * a.in_stride + lo;
+  const RowParams rp = load_params(a, row);
+  const SampWs w = samp_ws(a, row);
+  const Guess g = guess_of(rp, a.n);
+  const bool bin = g.use_k || g.use_p;
+  // everything the slices left is asked for at once: one trip to memory
+  u64 word[kMaxSlices];
+  float4v stat[kMaxSlices];
+#pragma unroll
+  for (int t = 0; t < kMaxSlices; ++t) {
+    if (t < a.slices) {
+      stat[t] = *reinterpret_cast<const float4v*>(w.stat + t);
+      if (bin) word[t] = w.bins[t * kWindow + threadIdx.x];
+    }
+  }
+  RowState st{};
+  double under = 0.0, total = 0.0;
+#pragma unroll
+  for (int t = 0; t < kMaxSlices; ++t)
+    if (t < a.slices) {
+      under += stat[t][0];
+      total += (double)stat[t][0] + (double)stat[t][1];
+      st.vmax = fmaxf(st.vmax, stat[t][2]);
+    }
+  st.valid = 1;
+  st.kbin = st.pbin = -1;
+  if (bin) {
+    u64 sum = 0;
+#pragma unroll
+    for (int t = 0; t < kMaxSlices; ++t) sum += t < a.slices ? word[t] : 0;
+    sh.bin[threadIdx.x] = sum;
+    __syncthreads();
+    // counts and masses in front of this thread's bin in one scan of the packed words
+    u64 words;
+    const u64 before = bscan<u64>(sum, sh.ured, words);
+    const uint32_t all = g.fx.count(words), c = g.fx.count(sum), behind = all - g.fx.count(before) - c;
+    const u64 low = (u64)ldexp(under, g.fx.scale), m = g.fx.mass(sum), run = low + g.fx.mass(before);
+    st.target = max((u64)fmin(ceil((double)(1.0f - rp.top_p) * (double)(low + g.fx.mass(words))), 4e18), (u64)1);
+    // the whole-row form's checks, and the window's
+    st.valid = total > 0.2 && total < 1.99 && st.vmax < 2.f && all > 0 && (!g.use_k || (int)all >= rp.top_k) &&
+               (!g.use_p || (under < (double)(1.0f - rp.top_p) * total && low + g.fx.mass(words) >= st.target && low < st.target));
+    if (st.valid && g.use_k && behind < (uint32_t)rp.top_k && (uint32_t)rp.top_k <= behind + c) {
+      sh.cut[0] = threadIdx.x;
+      sh.need = rp.top_k - behind;
+    }
+    if (st.valid && g.use_p && m > 0 && run < st.target && run + m >= st.target) {
+      sh.cut[1] = threadIdx.x;
+      sh.below = run;
+    }
+    __syncthreads();
+    if (st.valid && g.use_k) {
+      st.kbin = sh.cut[0];
+      st.rank = sh.need;
+      st.kcount = (int)g.fx.count(sh.bin[st.kbin]);
+    }
+    if (st.valid && g.use_p) {
+      st.pbin = sh.cut[1];
+      st.below = sh.below;
+      st.pcount = (int)g.fx.count(sh.bin[st.pbin]);
+    }
+    if (st.kcount > kList || st.pcount > kList) st.valid = 0;
+    // for the kept mass: of the bins behind the cut
+    if (st.valid && (int)threadIdx.x == (g.use_k ? st.kbin : st.pbin)) sh.ured[0] = g.fx.mass(words) - g.fx.mass(before) - m;
+    __syncthreads();
+    st.above = sh.ured[0];
+  }
+  if (slice == 0 && threadIdx.x == 0) *w.state = st;
+  if (!bin || !st.valid) return;  // block-uniform, the same in every block of the row (no fill is read then)
+  if (threadIdx.x < 2) sh.fill[threadIdx.x] = 0;
+  __syncthreads();
+  const uint32_t from = __float_as_uint(g.least);
+  each<VEC, 4>(x, n, [&](float raw) {
+    const uint32_t bits = value_bits(raw);
+    const int d = bits >= from ? min((int)(bits >> 19) - g.base, kWindow - 1) : -2;
+    if (d == st.kbin) sh.list[0][atomicAdd(&sh.fill[0], 1u)] = bits;
+    if (d == st.pbin) sh.list[1][atomicAdd(&sh.fill[1], 1u)] = bits;
+  });
+  __syncthreads();
+  // a place in the row's lists (in any order: what is taken from them does not depend on it)
+  if (threadIdx.x < 2) sh.cut[threadIdx.x] = sh.fill[threadIdx.x] ? atomicAdd(&w.fill[threadIdx.x], sh.fill[threadIdx.x]) : 0u;
+  __syncthreads();
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+    for (int i = threadIdx.x; i < (int)sh.fill[t]; i += kSampThreads) w.list[t * kList + sh.cut[t] + i] = sh.list[t][i];
+}
+
+template <bool VEC>
+__global__ void __launch_bounds__(kSampThreads) slice_apply_kernel(SampArgs a) {
+  __shared__ SampShared sh;
+  const int slice = blockIdx.x, row = blockIdx.y, lo = slice * a.slice, n = min(a.slice, a.n - lo);
+  const float* x = a.probs + (int64_t)row * a.in_stride;
+  const SampWs w = samp_ws(a, row);
+  uint32_t got[2][kList / kSampThreads];  // (whatever stands behind the lists' ends is not looked at)
+#pragma unroll
+  for (int t = 0; t < 2; ++t)
+#pragma unroll
+    for (int j = 0; j < kList / kSampThreads; ++j) got[t][j] = w.list[t * kList + threadIdx.x + j * kSampThreads];
+  const RowParams rp = load_params(a, row);
+  const Guess g = guess_of(rp, a.n);
+  const RowState st = *w.state;
+  if (!st.valid) return;  // block-uniform
+  float thr = 0.f, kept = -1.f;
+  if (g.use_k || g.use_p) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int j = 0; j < kList / kSampThreads; ++j) sh.list[t][threadIdx.x + j * kSampThreads] = got[t][j];
+    __syncthreads();
+    const uint32_t from = __float_as_uint(g.least);
+    if (threadIdx.x < 2) sh.cut[threadIdx.x] = 0;
+    __syncthreads();
+    const int wid = threadIdx.x >> 6;
+    if (wid == 0 && g.use_k)
+      sh.cut[0] = refine_list<true>(sh.digit[0], g.fx, sh.list[0], st.kcount, st.kbin + g.base, st.rank, 0, 0, from);
+    if (wid == 1 && g.use_p)
+      sh.cut[1] = refine_list<false>(sh.digit[1], g.fx, sh.list[1], st.pcount, st.pbin + g.base, 0u, st.below, st.target, from);
+    __syncthreads();
+    thr = fmaxf(__uint_as_float(sh.cut[0]), __uint_as_float(sh.cut[1]));
+    if (g.use_k != g.use_p) {
+      u64 part = 0, all;
+      for (int i = threadIdx.x; i < (g.use_k ? st.kcount : st.pcount); i += kSampThreads) {
+        const uint32_t b = sh.list[g.use_k ? 0 : 1][i];
+        if (__uint_as_float(b) >= thr) part += g.fx.of(b);
+      }
+      bscan<u64>(part, sh.ured, all);
+      kept = (float)ldexp((double)(st.above + all), -g.fx.scale);
+    }
+  }
+  if (rp.min_p > 0.f) thr = fmaxf(thr, rp.min_p * st.vmax);
+  if (a.out) {
+    if (!(kept > 0.f)) {  // no filter: the whole row's mass
+      kept = 0.f;
+      for (int t = 0; t < a.slices; ++t) kept += w.stat[t].under + w.stat[t].over;
+    }
+    write_renormed<VEC>(x + lo, a.out + (int64_t)row * a.out_stride + lo, n, thr, 1.0f / kept);
+    return;
+  }
+  if (slice == 0 && threadIdx.x == 0) w.state->thr = thr;
+  sum_chunks<VEC>(x, a.n, thr, 256, lo / 256, (lo + n + 255) / 256, w.chunk);
+}
+
+template <bool VEC>
+__global__ void __launch_bounds__(kSampThreads) slice_choose_kernel(SampArgs a) {
+  __shared__ SampShared sh;
+  const int row = blockIdx.x;
+  const float* x = a.probs + (int64_t)row * a.in_stride;
+  const SampWs w = samp_ws(a, row);
+  if (!w.state->valid) {
+    const RowParams rp = load_params(a, row);
+    if (a.out)
+      renorm_row<VEC>(x, a.out + (int64_t)row * a.out_stride, a.n, rp, sh);
+    else
+      sample_row<VEC>(x, a.n, rp, a.uniform[row], a.ids + row, sh);
+    return;
+  }
+  if (a.out) return;
+  const int chunks = (a.n + 255) / 256;
+  for (int i = threadIdx.x; i < kBins; i += kSampThreads) sh.chunk[i] = i < chunks ? w.chunk[i] : 0.f;
+  __syncthreads();
+  choose<VEC>(x, a.n, w.state->thr, 256, a.uniform[row], a.ids + row, sh);
+}
+
+// Blocks a row is spread over: at least 8192 elements each, and one block a unit at most (what a block scans and waits for
+// does not shrink with its share: 64 rows over 512 blocks took 155 us for sampling and renormalisation, over 256 85 us,
+// unspread 152 us).
+static int samp_slices(int64_t batch, int64_t n) {
+  if (batch <= 0 || n > 256 * kBins) return 1;
+  const int64_t s = std::min<int64_t>({kMaxSlices, n / 8192, 256 / batch});
+  return (int)std::max<int64_t>(s, 1);
+}
+
+static int launch_filters(SampArgs a, int batch, void* workspace, int64_t workspace_bytes, void* stream) {
+  hipStream_t s = (hipStream_t)stream;
+  const bool vec = aligned16(a.probs) && a.in_stride % 4 == 0 && (!a.out || (aligned16(a.out) && a.out_stride % 4 == 0));
+  const bool both_in_turn = !a.joint && (a.k_arr || a.k_val > 0) && (a.p_arr || a.p_val < 1.f);  // top-p over the k largest
+  a.slices = samp_slices(batch, a.n);
+  if (a.slices < 2 || both_in_turn || batch > 65535 || !workspace || (reinterpret_cast<uintptr_t>(workspace) & 15) ||
+      workspace_bytes < samp_ws_row(a.slices) * batch) {
+    hipLaunchKernelGGL(vec ? filter_rows_kernel<true> : filter_rows_kernel<false>, dim3(batch), dim3(kSampThreads), 0, s, a);
+    SGLK_LAUNCH_CHECK();
+    return SGLK_OK;
+  }
+  a.slice = (int)(((int64_t)a.n + a.slices * 256 - 1) / (a.slices * 256) * 256);
+  a.slices = (a.n + a.slice - 1) / a.slice;
+  a.ws = (char*)workspace;
+  const dim3 grid(a.slices, batch), block(kSampThreads);
+  hipLaunchKernelGGL(vec ? slice_bins_kernel<true> : slice_bins_kernel<false>, grid, block, 0, s, a);
+  hipLaunchKernelGGL(vec ? slice_collect_kernel<true> : slice_collect_kernel<false>, grid, block, 0, s, a);
+  hipLaunchKernelGGL(vec ? slice_apply_kernel<true> : slice_apply_kernel<false>, grid, block, 0, s, a);
+  hipLaunchKernelGGL(vec ? slice_choose_kernel<true> : slice_choose_kernel<false>, dim3(batch), block, 0, s, a);
+  SGLK_LAUNCH_CHECK();
+  return SGLK_OK;
 }
 
 }  // namespace
@@ -553,40 +943,60 @@ using namespace sglk;
 
 extern "C" {
 
-int sglk_top_k_renorm_probs(const float* probs, float* out, const int32_t* top_k_arr, int top_k_val, int batch, int vocab,
-                            int64_t in_stride, int64_t out_stride, void* stream) {
+int64_t sglk_sampling_workspace_bytes(int batch, int vocab) {
+  const int slices = vocab > 0 ? samp_slices(batch, vocab) : 1;
+  return slices < 2 ? 0 : samp_ws_row(slices) * batch;
+}
+
+int sglk_top_k_renorm_probs_ws(const float* probs, float* out, const int32_t* top_k_arr, int top_k_val, int batch, int vocab,
+                               int64_t in_stride, int64_t out_stride, void* workspace, int64_t workspace_bytes, void* stream) {
   SGLK_CHECK(batch >= 0 && vocab > 0 && in_stride >= vocab && out_stride >= vocab, "top_k_renorm_probs: bad shape");
   if (batch == 0) return SGLK_OK;
   SGLK_CHECK(probs && out, "top_k_renorm_probs: null pointer");
-  const bool vec = aligned16(probs) && aligned16(out) && in_stride % 4 == 0 && out_stride % 4 == 0;
-  hipLaunchKernelGGL(vec ? renorm_kernel<true> : renorm_kernel<false>, dim3(batch), dim3(kSampThreads), 0, (hipStream_t)stream,
-                     probs, out, vocab, in_stride, out_stride, top_k_arr, top_k_val, (const float*)nullptr, 1.0f);
-  SGLK_LAUNCH_CHECK();
-  return SGLK_OK;
+  SampArgs a{};
+  a.probs = probs, a.out = out, a.n = vocab, a.in_stride = in_stride, a.out_stride = out_stride;
+  a.k_arr = top_k_arr, a.k_val = top_k_val, a.p_val = 1.0f, a.joint = 1;
+  return launch_filters(a, batch, workspace, workspace_bytes, stream);
+}
+
+int sglk_top_k_renorm_probs(const float* probs, float* out, const int32_t* top_k_arr, int top_k_val, int batch, int vocab,
+                            int64_t in_stride, int64_t out_stride, void* stream) {
+  return sglk_top_k_renorm_probs_ws(probs, out, top_k_arr, top_k_val, batch, vocab, in_stride, out_stride, nullptr, 0, stream);
+}
+
+int sglk_top_p_renorm_probs_ws(const float* probs, float* out, const float* top_p_arr, float top_p_val, int batch, int vocab,
+                               int64_t in_stride, int64_t out_stride, void* workspace, int64_t workspace_bytes, void* stream) {
+  SGLK_CHECK(batch >= 0 && vocab > 0 && in_stride >= vocab && out_stride >= vocab, "top_p_renorm_probs: bad shape");
+  if (batch == 0) return SGLK_OK;
+  SGLK_CHECK(probs && out, "top_p_renorm_probs: null pointer");
+  SampArgs a{};
+  a.probs = probs, a.out = out, a.n = vocab, a.in_stride = in_stride, a.out_stride = out_stride;
+  a.p_arr = top_p_arr, a.p_val = top_p_val, a.joint = 1;
+  return launch_filters(a, batch, workspace, workspace_bytes, stream);
 }
 
 int sglk_top_p_renorm_probs(const float* probs, float* out, const float* top_p_arr, float top_p_val, int batch, int vocab,
                             int64_t in_stride, int64_t out_stride, void* stream) {
-  SGLK_CHECK(batch >= 0 && vocab > 0 && in_stride >= vocab && out_stride >= vocab, "top_p_renorm_probs: bad shape");
-  if (batch == 0) return SGLK_OK;
-  SGLK_CHECK(probs && out, "top_p_renorm_probs: null pointer");
-  const bool vec = aligned16(probs) && aligned16(out) && in_stride % 4 == 0 && out_stride % 4 == 0;
-  hipLaunchKernelGGL(vec ? renorm_kernel<true> : renorm_kernel<false>, dim3(batch), dim3(kSampThreads), 0, (hipStream_t)stream,
-                     probs, out, vocab, in_stride, out_stride, (const int32_t*)nullptr, 0, top_p_arr, top_p_val);
-  SGLK_LAUNCH_CHECK();
-  return SGLK_OK;
+  return sglk_top_p_renorm_probs_ws(probs, out, top_p_arr, top_p_val, batch, vocab, in_stride, out_stride, nullptr, 0, stream);
 }
 
-int sglk_sampling_from_probs(const float* probs, const float* uniform, int32_t* out, const int32_t* top_k_arr,
-                             int top_k_val, const float* top_p_arr, float top_p_val, const float* min_p_arr,
-                             float min_p_val, int joint, int batch, int vocab, int64_t in_stride, void* stream) {
+int sglk_sampling_from_probs_ws(const float* probs, const float* uniform, int32_t* out, const int32_t* top_k_arr, int top_k_val,
+                                const float* top_p_arr, float top_p_val, const float* min_p_arr, float min_p_val, int joint,
+                                int batch, int vocab, int64_t in_stride, void* workspace, int64_t workspace_bytes, void* stream) {
   SGLK_CHECK(batch >= 0 && vocab > 0 && in_stride >= vocab, "sampling_from_probs: bad shape");
   if (batch == 0) return SGLK_OK;
   SGLK_CHECK(probs && uniform && out, "sampling_from_probs: null pointer");
-  const bool vec = aligned16(probs) && in_stride % 4 == 0;
-  hipLaunchKernelGGL(vec ? sample_kernel<true> : sample_kernel<false>, dim3(batch), dim3(kSampThreads), 0, (hipStream_t)stream,
-                     probs, uniform, out, vocab, in_stride, top_k_arr, top_k_val, top_p_arr, top_p_val, min_p_arr, min_p_val, joint ? 1 : 0);
-  SGLK_LAUNCH_CHECK();
-  return SGLK_OK;
+  SampArgs a{};
+  a.probs = probs, a.uniform = uniform, a.ids = out, a.n = vocab, a.in_stride = in_stride;
+  a.k_arr = top_k_arr, a.k_val = top_k_val, a.p_arr = top_p_arr, a.p_val = top_p_val, a.m_arr = min_p_arr, a.m_val = min_p_val;
+  a.joint = joint ? 1 : 0;
+  return launch_filters(a, batch, workspace, workspace_bytes, stream);
+}
+
+int sglk_sampling_from_probs(const float* probs, const float* uniform, int32_t* out, const int32_t* top_k_arr, int top_k_val,
+                             const float* top_p_arr, float top_p_val, const float* min_p_arr, float min_p_val, int joint,
+                             int batch, int vocab, int64_t in_stride, void* stream) {
+  return sglk_sampling_from_probs_ws(probs, uniform, out, top_k_arr, top_k_val, top_p_arr, top_p_val, min_p_arr, min_p_val, joint,
+                                     batch, vocab, in_stride, nullptr, 0, stream);
 }
 }

@@ -1401,12 +1401,19 @@ def _per_row(v, batch, dtype, name):
     return None, v
 
 
+def _filter_workspace(probs):
+    """(tensor or None, bytes): rows spread over several blocks meet there."""
+    need = int(lib().sglk_sampling_workspace_bytes(probs.shape[0], probs.shape[1]))
+    return (torch.empty(need, dtype=torch.uint8, device=probs.device) if need else None), need
+
+
 def top_k_renorm_probs(probs, top_k):
     B, V = _probs2d(probs, "top_k_renorm_probs")
     arr, val = _per_row(top_k, B, torch.int32, "top_k_renorm_probs")
     out = torch.empty_like(probs)
-    check(lib().sglk_top_k_renorm_probs(_ptr(probs), _ptr(out), _ptr(arr), int(val), B, V, probs.stride(0), out.stride(0),
-                                        _stream(probs)), "top_k_renorm_probs")
+    ws, need = _filter_workspace(probs)
+    check(lib().sglk_top_k_renorm_probs_ws(_ptr(probs), _ptr(out), _ptr(arr), int(val), B, V, probs.stride(0), out.stride(0),
+                                           _ptr(ws), need, _stream(probs)), "top_k_renorm_probs")
     return out
 
 
@@ -1414,8 +1421,9 @@ def top_p_renorm_probs(probs, top_p):
     B, V = _probs2d(probs, "top_p_renorm_probs")
     arr, val = _per_row(top_p, B, torch.float32, "top_p_renorm_probs")
     out = torch.empty_like(probs)
-    check(lib().sglk_top_p_renorm_probs(_ptr(probs), _ptr(out), _ptr(arr), float(val), B, V, probs.stride(0),
-                                        out.stride(0), _stream(probs)), "top_p_renorm_probs")
+    ws, need = _filter_workspace(probs)
+    check(lib().sglk_top_p_renorm_probs_ws(_ptr(probs), _ptr(out), _ptr(arr), float(val), B, V, probs.stride(0),
+                                           out.stride(0), _ptr(ws), need, _stream(probs)), "top_p_renorm_probs")
     return out
 
 
@@ -1429,9 +1437,10 @@ def sampling_from_probs(probs, uniform, top_k=0, top_p=1.0, min_p=0.0, joint=Tru
     pa, pv = _per_row(top_p, B, torch.float32, "sampling_from_probs")
     ma, mv = _per_row(min_p, B, torch.float32, "sampling_from_probs")
     out = torch.empty(B, dtype=torch.int32, device=probs.device)
-    check(lib().sglk_sampling_from_probs(_ptr(probs), _ptr(uniform), _ptr(out), _ptr(ka), int(kv), _ptr(pa), float(pv),
-                                         _ptr(ma), float(mv), 1 if joint else 0, B, V, probs.stride(0), _stream(probs)),
-          "sampling_from_probs")
+    ws, need = _filter_workspace(probs)
+    check(lib().sglk_sampling_from_probs_ws(_ptr(probs), _ptr(uniform), _ptr(out), _ptr(ka), int(kv), _ptr(pa), float(pv),
+                                            _ptr(ma), float(mv), 1 if joint else 0, B, V, probs.stride(0), _ptr(ws), need,
+                                            _stream(probs)), "sampling_from_probs")
     return out
 
 

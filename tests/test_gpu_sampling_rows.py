@@ -1,6 +1,8 @@
 """GPU: the sampling filters' radix selection where its shortcuts end: rows of peaked, flat, tied and unnormalised
 values, lists that overflow, thresholds below the mean, vocabularies that are no multiple of a load or a chunk, and rows
 that are not aligned.  Values are sums of few powers of two, so that every mass is exact and so is the kept set."""
+import math
+
 import pytest
 import torch
 
@@ -15,7 +17,7 @@ def _rows(kind, n, g):
     x = 2.0 ** e.double()
     if kind == "peaked":
         x = x * (1 + torch.randint(0, 8, (n,), generator=g) / 8)
-    return x * 2.0 ** -30       # far from a mass of one: the guess of what can be skipped is checked
+    return x
 
 
 def _threshold(x, k, p, joint):
@@ -34,13 +36,14 @@ def _threshold(x, k, p, joint):
 
 @pytest.mark.parametrize("kind", ["peaked", "flat", "two", "steep"])
 @pytest.mark.parametrize("n", [1, 3, 255, 4099, 40000, 128259])
-@pytest.mark.parametrize("scale", [1.0, 2.0 ** 15])
+@pytest.mark.parametrize("scale", [None, 2.0 ** -30, 2.0 ** 12])   # None: a mass between one half and one, as probabilities have
 def test_kept_sets(kind, n, scale):
     import sglang_security_amd.sgl_kernel as sk
     from sglang_security_amd import ops
 
     g = torch.Generator().manual_seed(n)
-    x = _rows(kind, n, g) * scale
+    x = _rows(kind, n, g)
+    x = x * (scale or 2.0 ** -math.ceil(math.log2(x.sum().item())))
     B = 6
     wide = torch.zeros(B, n + 5, device=DEV)
     wide[:, 1: n + 1] = x.float().to(DEV)
@@ -94,3 +97,19 @@ def test_rows_of_infinite_mass():
     got = sk.top_k_renorm_probs(x, 20)
     assert torch.equal(torch.nan_to_num(got, nan=1.0)[0] != 0, x[0] == float("inf"))
     assert got[0].isnan().sum() == 1            # inf / inf; the other kept values over infinity are zeros
+
+
+def test_one_block_and_several_agree():
+    """A row alone (spread over sixteen blocks) and in a batch too large to spread give the same tokens and rows."""
+    import sglang_security_amd.sgl_kernel as sk
+    from sglang_security_amd import ops
+
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.softmax(3 * torch.randn(1, 50257, device=DEV, generator=g), -1)
+    many = x.repeat(600, 1)
+    u = torch.rand(600, device=DEV, generator=g)
+    for kw in (dict(top_k=40, top_p=0.9), dict(top_p=0.99), dict(top_k=500), dict(min_p=0.1), dict()):
+        ids = ops.sampling_from_probs(many, u, **kw)
+        assert torch.equal(ids[:50], torch.cat([ops.sampling_from_probs(x, u[i: i + 1], **kw) for i in range(50)]))
+    assert torch.equal(sk.top_p_renorm_probs(many, 0.9)[7:8], sk.top_p_renorm_probs(x, 0.9))
+    assert torch.equal(sk.top_k_renorm_probs(many, 77)[7:8], sk.top_k_renorm_probs(x, 77))
