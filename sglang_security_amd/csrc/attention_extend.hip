@@ -309,8 +309,9 @@ static int extend_attention_impl(const void* q_extend, const void* k_extend, con
                        o_stride_h % 4 == 0;
   const int64_t row_blocks = ((int64_t)max_extend_len * (Hq / Hkv) + kExtRows - 1) / kExtRows;
   auto row32 = [](int64_t v) { return v >= 0 && v < (1ll << 31); };  // twice that, in bytes, fits 32 bits
+  const int64_t span = D == 64 ? 32 : 1;  // head size 64 adds up to 32 rows of new tokens in 32 bits
   const bool tile = rows_ok && kvf == 0 && (D == 128 || D == 64) && row_blocks <= 65535 && (int64_t)Hkv * B < (1ll << 31) &&
-                    row32(k_stride_n) && row32(v_stride_n) && row32(ke_stride_t) && row32(ve_stride_t);
+                    row32(k_stride_n) && row32(v_stride_n) && row32(span * ke_stride_t) && row32(span * ve_stride_t);
   const bool fast8 = rows_ok && kvf != 0 && D == 128;
   if (kv_splits > 1 && (!(tile || fast8) || paged))
     return fail(SGLK_EUNSUP, "extend_attention_split: 16-bit types with head size 64 or 128 (an fp8 pool: 128) and contiguous new tokens only");

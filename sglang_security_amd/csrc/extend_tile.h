@@ -15,7 +15,8 @@
 // Measured (bf16, launch alone): 8 prompts of 768 to 1152 tokens, 32 / 8 heads of 128: 264 us (one block per 64 rows of
 // one head, 32-token tiles on 16x16x32) -> 124 us, 525 TFLOP/s; one prompt of 1152 tokens: 69 -> 36 us; 128 tokens over
 // 1024 cached, split 8 ways: 20.1 -> 14.6 us; 4 prompts of 667 to 1000 tokens over 683 to 1024 cached, 14 / 2 heads of
-// 64: 3.24 ms (wave per row) -> 0.056 ms.
+// 64: 3.24 ms (wave per row) -> 0.052 ms.  Operand reads are spelled out ahead of the products that use them: the
+// compiler's own order waits for each (8 prompts: 137.5 -> 134.5 us of a call with its copies, one box).
 #pragma once
 #include "attention_tile.h"
 
@@ -136,14 +137,28 @@ __global__ void __launch_bounds__(256, 2) extend_tile_kernel(ExtendArgs a) {
       for (int i = 0; i < NP; ++i) slot[i] = idx[min(p0 + j * kExtTokens + frow + i * (256 / kTpr), p1 - 1)];
     }
   };
+  // D = 64 has half the work per tile to hide the addresses behind: a whole tile of new tokens has a uniform base and one
+  // 32-bit offset a lane there (4 prompts of 667 to 1000 tokens, 14 / 2 heads: a call 62 -> 57 us; at D = 128 the same form gains nothing)
+  const uint32_t ke_off = (uint32_t)frow * a.ke_row + chunk * 16, ve_off = (uint32_t)frow * a.ve_row + chunk * 16;
   auto fetch = [&](int j) {
+    const int t0 = (j - nt1) * kExtTokens;
+    if (D == 64 && j >= nt1 && t0 + kExtTokens <= e1) {
+      const char* kp = reinterpret_cast<const char*>(ke) + (uint64_t)(uint32_t)t0 * a.ke_row;
+      const char* vp = reinterpret_cast<const char*>(ve) + (uint64_t)(uint32_t)t0 * a.ve_row;
+#pragma unroll
+      for (int i = 0; i < NP; ++i) {
+        kreg[i] = *reinterpret_cast<const int4v*>(kp + (uint64_t)(i * (256 / kTpr)) * a.ke_row + ke_off);
+        vreg[i] = *reinterpret_cast<const int4v*>(vp + (uint64_t)(i * (256 / kTpr)) * a.ve_row + ve_off);
+      }
+      return;
+    }
     const bool pool = j < nt1;  // block-uniform
     const char* kp = reinterpret_cast<const char*>(pool ? kb : ke);
     const char* vp = reinterpret_cast<const char*>(pool ? vb : ve);
     const uint32_t ks = pool ? a.kb_row : a.ke_row, vs = pool ? a.vb_row : a.ve_row;
 #pragma unroll
     for (int i = 0; i < NP; ++i) {
-      const uint32_t r = pool ? slot[i] : min((j - nt1) * kExtTokens + frow + i * (256 / kTpr), e1 - 1);
+      const uint32_t r = pool ? slot[i] : min(t0 + frow + i * (256 / kTpr), e1 - 1);
       kreg[i] = *reinterpret_cast<const int4v*>(kp + ((uint64_t)r * ks + chunk * 16));
       vreg[i] = *reinterpret_cast<const int4v*>(vp + ((uint64_t)r * vs + chunk * 16));
     }
@@ -184,15 +199,27 @@ __global__ void __launch_bounds__(256, 2) extend_tile_kernel(ExtendArgs a) {
 
     float16v s[2];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int r = 0; r < 16; ++r) s[u][r] = 0.f;
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
         const short8 kf = *reinterpret_cast<const short8*>(kl + ext_k_off<D>(32 * u + l31, 2 * ks + hi));
         s[u] = Mfma32<T>::mma(kf, qf[ks], s[u]);
       }
+    // operand reads run kAhead products ahead of the matrix unit (left to itself the compiler waits for each)
+    constexpr int kAhead = 4;
+    __builtin_amdgcn_sched_group_barrier(0x100, kAhead, 0);
+#pragma unroll
+    for (int i = 0; i < 2 * KS - kAhead; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
+    __builtin_amdgcn_sched_group_barrier(0x8, kAhead, 0);
+    __builtin_amdgcn_sched_barrier(0);
     if constexpr (PRE) {
 #pragma unroll
       for (int u = 0; u < 2; ++u)
@@ -256,6 +283,14 @@ __global__ void __launch_bounds__(256, 2) extend_tile_kernel(ExtendArgs a) {
         if constexpr (P2) oacc[n] = Mfma32<T>::mma(vf, pl[k], oacc[n]);
       }
     }
+    constexpr int kPer = P2 ? 2 : 1, kAheadV = 3;  // products a value operand, operands read ahead
+    __builtin_amdgcn_sched_group_barrier(0x100, 2 * kAheadV, 1);
+#pragma unroll
+    for (int i = 0; i < 4 * NV - kAheadV; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x8, kPer, 1);
+      __builtin_amdgcn_sched_group_barrier(0x100, 2, 1);
+    }
+    __builtin_amdgcn_sched_group_barrier(0x8, kPer * kAheadV, 1);
   }
 
   const float tot = lsum + __shfl_xor(lsum, 32, 64);
