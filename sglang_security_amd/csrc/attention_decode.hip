@@ -291,6 +291,33 @@ __global__ void __launch_bounds__(64) decode_stage1_generic(
   if (lane == 0) attn_lse[ob] = m + logf(l);
 }
 
+// How many ways request b's context is split.  units == 0: as the caller says.  Otherwise a split of every request is
+// `units` blocks for the chip's kMlaPlaces (two a unit), and of 1 .. the caller's number the one is taken that makes
+// rounds x (tokens of a split + 32 for its start and its merge) least, counted as if all requests were like this one.  A
+// last round that leaves every unit one block or none counts 0.65, any other that is not full 0.95 (a block that has
+// its unit to itself is that much faster).  A request half as long again as the batch's average keeps what it was given:
+// alone in the last round, it would end the launch.
+constexpr int kMlaPlaces = 512;
+__device__ __forceinline__ int splits_of(const int32_t* __restrict__ num_kv_splits, const int32_t* __restrict__ kv_indptr, int b, int B,
+                                         int len, int max_splits, int units) {
+  const int most = max(num_kv_splits[b], 1);
+  if (units == 0 || most > max_splits || (int64_t)units * most <= kMlaPlaces) return most;
+  if (2 * (int64_t)len * B > 3 * ((int64_t)kv_indptr[B] - kv_indptr[0])) return most;
+  int best = 1;
+  int64_t best_cost = 0;  // times 20 and `best`
+  for (int n = 1; n <= most; ++n) {
+    const int64_t blocks = (int64_t)units * n;
+    const int rest = (int)(blocks % kMlaPlaces);
+    const int64_t rounds = 20 * (blocks / kMlaPlaces) + (rest == 0 ? 0 : rest <= kMlaPlaces / 2 ? 13 : 19);
+    const int64_t cost = rounds * (len + 32 * n);
+    if (n == 1 || cost * best < best_cost * n) {
+      best = n;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
 // ---------------------------------------------------------------------------------------------
 // stage 2: LSE merge of the split partials (decode_attention.py:497-557)
 // ---------------------------------------------------------------------------------------------
@@ -301,12 +328,12 @@ __global__ void __launch_bounds__(128) decode_stage2(const float* __restrict__ a
                                                      const int32_t* __restrict__ num_kv_splits, int max_kv_splits,
                                                      int Hq, int Dv, int64_t o_stride_b, int64_t o_stride_h,
                                                      float* __restrict__ xsum_out, int64_t xs_stride,
-                                                     const int32_t* __restrict__ gate = nullptr) {
+                                                     const int32_t* __restrict__ gate = nullptr, int units = 0) {
   __shared__ float xs_red[2];
   if (gate && *gate != 0) return;  // see decode_stage1_mfma128
   const int b = blockIdx.x, h = blockIdx.y;
   const int len = kv_indptr[b + 1] - kv_indptr[b];
-  const int splits = max(num_kv_splits[b], 1);
+  const int splits = splits_of(num_kv_splits, kv_indptr, b, gridDim.x, len, max_kv_splits, units);
   const int per_split = cdiv_i(cdiv_i(len, splits), kMinBlockKV) * kMinBlockKV;
   const int64_t base = ((int64_t)b * Hq + h) * max_kv_splits;
   if (Dv % 512 == 0 && !xsum_out && (reinterpret_cast<uintptr_t>(attn_logits) & 15) == 0) {
@@ -501,7 +528,7 @@ __global__ void __launch_bounds__(256, HT == 1 ? 3 : 2) decode_stage1_mla(
     const int32_t* __restrict__ kv_indices, float* __restrict__ attn_logits, float* __restrict__ attn_lse,
     const int32_t* __restrict__ num_kv_splits, int max_kv_splits, int Hq, int Hkv, int head_tiles, int64_t q_stride_b,
     int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h, float sm_scale, float logit_cap,
-    const int32_t* __restrict__ gate = nullptr) {
+    const int32_t* __restrict__ gate, int units) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   if (gate && *gate != 0) return;  // see decode_stage1_mfma128
   const int lane = threadIdx.x & 63;
@@ -512,7 +539,7 @@ __global__ void __launch_bounds__(256, HT == 1 ? 3 : 2) decode_stage1_mla(
   const int group = Hq / Hkv;
   const int start = kv_indptr[b];
   const int len = kv_indptr[b + 1] - start;
-  const int splits = max(num_kv_splits[b], 1);
+  const int splits = splits_of(num_kv_splits, kv_indptr, b, gridDim.x, len, max_kv_splits, units);
   const int per_split = cdiv_i(cdiv_i(len, splits), kMinBlockKV) * kMinBlockKV;
   const int s0 = per_split * split, s1 = min(s0 + per_split, len);
   if (s1 <= s0) return;  // block-uniform
@@ -1659,6 +1686,7 @@ static int decode_attention_impl(const void* q, const void* k_buffer, const void
   if (B == 0) return SGLK_OK;
   hipStream_t s = (hipStream_t)stream;
   const int group = Hq / Hkv;
+  int units = 0;  // blocks of one split of every request, where their number is weighed (splits_of)
   const bool fast = kvf == 0 && (dtype == SGLK_F16 || dtype == SGLK_BF16) && D == 128 && Dv == 128 && aligned16(q) &&
                     aligned16(k_buffer) && aligned16(v_buffer) && aligned16(attn_logits) && (q_stride_b % 8 == 0) &&
                     (q_stride_h % 8 == 0) && (k_stride_n % 8 == 0) && (k_stride_h % 8 == 0) && (v_stride_n % 8 == 0) &&
@@ -1692,13 +1720,19 @@ static int decode_attention_impl(const void* q, const void* k_buffer, const void
       });
     });
   } else if (mla) {
-    if (group >= 32) {  // two tiles of 16 heads per block
+    // Splits that spill the grid into a nearly empty round cost more than they spread.  128 heads, a call before -> after
+    // (splits): 64 requests of 768 to 1152 tokens 87 (3) -> 75 us (2), 32 of them 58 (5) -> 48 (4), 20 of 2731 to 4096
+    // tokens 91 (8) -> 77 (6); 75 of 768 to 1152 stay at 2 (104 us; 116 with one), 75 of up to 4096 at 3 (255; 338 with
+    // one).  Up to 31 heads a group the copy rate bounds the launch and a short last round is nearly free (100 requests of
+    // up to 2048 tokens, 16 heads: 49.9 us with 8 splits, 51.5 with 7): there the caller's number stands.
+    if (group >= 32) {  // two tiles of 16 heads per block, two blocks a unit
       const int head_tiles = (group + 31) / 32;
+      if ((int64_t)B * Hkv * head_tiles < (1 << 20)) units = B * Hkv * head_tiles;
       dim3 grid(B, Hkv * head_tiles, max_kv_splits);
 #define SGLK_MLA_LAUNCH(HT, CAP)                                                                                         \
   hipLaunchKernelGGL((decode_stage1_mla<T, HT, CAP>), grid, dim3(256), kMlaTileBytes + HT * kMlaScoreBytes, s, q, k_buffer, \
                      kv_indptr, kv_indices, attn_logits, attn_lse, num_kv_splits, max_kv_splits, Hq, Hkv, head_tiles,      \
-                     q_stride_b, q_stride_h, k_stride_n, k_stride_h, sm_scale, logit_cap, gate)
+                     q_stride_b, q_stride_h, k_stride_n, k_stride_h, sm_scale, logit_cap, gate, units)
       SGLK_DISPATCH_HALF(dtype, T, {
         if (logit_cap > 0.f)
           SGLK_MLA_LAUNCH(2, true);
@@ -1770,7 +1804,7 @@ static int decode_attention_impl(const void* q, const void* k_buffer, const void
   SGLK_DISPATCH_FLOAT(dtype, T,
                       hipLaunchKernelGGL((decode_stage2<T>), dim3(B, Hq), dim3(128), 0, s, attn_logits, attn_lse, o,
                                          kv_indptr, num_kv_splits, max_kv_splits, Hq, Dv, o_stride_b, o_stride_h,
-                                         xsum_out, xs_stride, gate));
+                                         xsum_out, xs_stride, gate, units));
   SGLK_LAUNCH_CHECK();
   return SGLK_OK;
 }
