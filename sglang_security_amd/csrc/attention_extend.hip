@@ -313,6 +313,8 @@ static int extend_attention_impl(const void* q_extend, const void* k_extend, con
   const bool tile = rows_ok && kvf == 0 && (D == 128 || D == 64) && row_blocks <= 65535 && (int64_t)Hkv * B < (1ll << 31) &&
                     row32(k_stride_n) && row32(v_stride_n) && row32(span * ke_stride_t) && row32(span * ve_stride_t);
   const bool fast8 = rows_ok && kvf != 0 && D == 128;
+  // strides or row counts past the tile kernel's 32-bit range: not split, whole rows on the kernel below
+  if (!tile && !paged && rows_ok && kvf == 0 && (D == 128 || D == 64)) kv_splits = 1;
   if (kv_splits > 1 && (!(tile || fast8) || paged))
     return fail(SGLK_EUNSUP, "extend_attention_split: 16-bit types with head size 64 or 128 (an fp8 pool: 128) and contiguous new tokens only");
   float* part_o = kv_splits > 1 ? split_ws : nullptr;

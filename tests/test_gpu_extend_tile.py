@@ -78,3 +78,18 @@ def test_sums_outgrow_the_first_maximum():
     none = torch.zeros(2, dtype=torch.int32, device=DEV)
     ops.extend_attention_fwd(d(q), d(k), d(v), o, d(k), d(v), ptr, none, none[:1], None, True, None, T)
     assert (o.double().cpu() - want)[70:].abs().max().item() < 2e-2
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_split_call_past_32_bit_strides(D):
+    """One new token whose (unused) row stride is past the tile kernel's range: the split call gives the rows all the same."""
+    from sglang_security_amd import ops
+
+    q, ke, ve, kb, vb, qo, kp, ki = (t.to(DEV) for t in _case(4, 2, D, [150], [1], torch.bfloat16, 5))
+    far = lambda t: torch.as_strided(t, t.shape, (2**31, D, 1))
+    sm, got = 1.0 / math.sqrt(D), []
+    for k, v in ((ke, ve), (far(ke), far(ve))):
+        o = torch.full_like(q, float("nan"))
+        ops.extend_attention_split(q, k, v, o, kb, vb, qo, kp, ki, 1, sm, 0.0, True, 3)
+        got.append(o.float().cpu())
+    assert (got[0] - got[1]).abs().max().item() < TOL[torch.bfloat16]
