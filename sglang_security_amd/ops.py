@@ -386,7 +386,7 @@ def extend_attention_fwd(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buf
         total_prefix = kv_indices.numel() if kv_indptr.numel() > 1 else 0
     splits = extend_attention_split_plan(T, Hq, B, max_len_extend, int(total_prefix), D,
                                          q_extend.dtype) if (D == Dv and k_buffer is not None) else 1
-    if splits > 1 and D == 64 and not _tile_rows(q_extend, k_extend, v_extend, k_buffer, v_buffer):
+    if splits > 1 and not _split_rows(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buffer):
         splits = 1
     if splits > 1:
         return extend_attention_split(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buffer, qo_indptr, kv_indptr,
@@ -401,9 +401,13 @@ def extend_attention_fwd(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buf
         _attn_dtype(q_extend, k_buffer, v_buffer), _stream(q_extend)), "extend_attention")
 
 
-def _tile_rows(q, *rows) -> bool:
-    """Whether rows of q's type lie as the tile kernels read them (16-byte pieces)."""
-    return all(t.dtype == q.dtype and t.data_ptr() % 16 == 0 and t.stride(0) % 8 == 0 and t.stride(1) % 8 == 0 for t in (q, *rows))
+def _split_rows(q, k, v, o, k_buffer, v_buffer) -> bool:
+    """Whether the rows lie as the split form takes them: 16-byte pieces of q, k, v and of a 16-bit pool, 8-byte pieces of
+    the output and of an fp8 pool, which only head size 128 has a tile kernel for."""
+    pool8 = k_buffer.element_size() == 1
+    lies = lambda t, ptr, stride: t.data_ptr() % ptr == 0 and t.stride(0) % stride == 0 and t.stride(1) % stride == 0
+    return (all(lies(t, 16, 8) for t in (q, k, v)) and lies(o, 8, 4) and
+            all(lies(t, 8 if pool8 else 16, 8) for t in (k_buffer, v_buffer)) and not (pool8 and q.shape[2] != 128))
 
 
 def extend_attention_split_plan(T, Hq, B, max_len_extend, total_prefix, head_dim, dtype) -> int:

@@ -93,3 +93,29 @@ def test_split_call_past_32_bit_strides(D):
         ops.extend_attention_split(q, k, v, o, kb, vb, qo, kp, ki, 1, sm, 0.0, True, 3)
         got.append(o.float().cpu())
     assert (got[0] - got[1]).abs().max().item() < TOL[torch.bfloat16]
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("odd", ["output stride", "output start", "key stride", "pool start", "none"])
+def test_prefix_long_enough_to_split_with_any_rows(D, odd):
+    """Rows that do not lie as the split form reads or writes them: the call is not split, and gives the same rows."""
+    import oracle
+    from sglang_security_amd import ops
+
+    t = _case(4, 2, D, [600], [9], torch.bfloat16, 11)
+    want = oracle.extend_attention(*t, 1.0 / math.sqrt(D), 0.0, True)
+    q, ke, ve, kb, vb, qo, kp, ki = (x.to(DEV) for x in t)
+    assert ops.extend_attention_split_plan(9, 4, 1, 9, 600, D, torch.bfloat16) > 1
+
+    def shift(x, at, gap):     # the same rows, `at` elements into a buffer, `gap` elements between tokens
+        n, h, _ = x.shape
+        buf = torch.full((at + n * (h * D + gap),), float("nan"), dtype=x.dtype, device=DEV)
+        view = buf[at:].as_strided((n, h, D), (h * D + gap, D, 1))
+        view.copy_(x)
+        return view
+
+    o = shift(torch.zeros_like(q), 1 if odd == "output start" else 0, 2 if odd == "output stride" else 0)
+    ke = shift(ke, 0, 4 if odd == "key stride" else 0)
+    kb = shift(kb, 4 if odd == "pool start" else 0, 0)
+    ops.extend_attention_fwd(q, ke, ve, o, kb, vb, qo, kp, ki, None, True, None, 9)
+    assert (o.float().cpu() - want).abs().max().item() < TOL[torch.bfloat16]
