@@ -18,6 +18,8 @@
 // 64: 3.24 ms (wave per row) -> 0.052 ms.  Operand reads are spelled out ahead of the products that use them: the
 // compiler's own order waits for each (8 prompts: 137.5 -> 134.5 us of a call with its copies, one box).
 #pragma once
+#include <type_traits>
+
 #include "attention_tile.h"
 
 namespace sglk {
@@ -35,6 +37,11 @@ struct Mfma32<f16_t> {
   static __device__ __forceinline__ float16v mma(short8 a, short8 b, float16v c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0, 0);
   }
+};
+
+template <typename T>
+struct Special {  // the type's infinity and one
+  static constexpr uint16_t kInf = std::is_same<T, bf16_t>::value ? 0x7F80 : 0x7C00, kOne = std::is_same<T, bf16_t>::value ? 0x3F80 : 0x3C00;
 };
 
 struct ExtendArgs {
@@ -68,8 +75,10 @@ __device__ __forceinline__ int ext_v_off(int r, int byte) {
 // tokens, and leaves normalised fp32 rows + log-sum-exps (a short extend over a long prefix has too few rows to fill
 // the chip otherwise).
 // PRE: scores are finished (scale, cap) before their maximum is taken: a capped call, or a scale that is not positive.
-template <typename T, int D, bool PRE>
-__global__ void __launch_bounds__(256, 2) extend_tile_kernel(ExtendArgs a) {
+// A block's walk over its ranges: rows leave where `mine`, unless a result of theirs is not finite; returns whether one of
+// this lane's row is not.  CAREFUL: values that are not finite stay out of the matrix products, and all rows leave.
+template <typename T, int D, bool PRE, bool CAREFUL>
+__device__ __forceinline__ bool extend_walk(const ExtendArgs& a, const int tid, bool mine) {
   constexpr int KS = D / 16, NV = D / 32, NP = D / 32;  // k-steps, 32-wide value blocks, 16-byte pieces per thread
   constexpr int kStage = kExtTokens * 2 * D;            // K (or V) bytes of a stage
   constexpr int kTpr = D / 8;                           // threads (chunks) per row
@@ -80,8 +89,8 @@ __global__ void __launch_bounds__(256, 2) extend_tile_kernel(ExtendArgs a) {
   const int q0 = a.qo_indptr[b], ext = a.qo_indptr[b + 1] - q0;
   const int nrows = ext * share;
   const int R0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * kExtRows;  // the rows that see most start first
-  if (R0 >= nrows) return;                                           // block-uniform
-  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  if (R0 >= nrows) return false;                                     // block-uniform
+  const int lane = tid & 63, wid = tid >> 6;
   const int l31 = lane & 31, hi = lane >> 5;
   const bool paged = a.ke == nullptr;
   const int pstart = a.kv_indptr[b], plen = a.kv_indptr[b + 1] - pstart;
@@ -164,20 +173,25 @@ __global__ void __launch_bounds__(256, 2) extend_tile_kernel(ExtendArgs a) {
     }
   };
 
+  const float c = PRE ? 1.f : a.sm_scale * LOG2E;
+  if (!CAREFUL) mine = row_ok;
   float m = -INFINITY, lsum = 0.f;  // running maximum (log2 domain) and this lane's share of the running sum
   float16v oacc[NV];
 #pragma unroll
   for (int n = 0; n < NV; ++n)
 #pragma unroll
     for (int r = 0; r < 16; ++r) oacc[n][r] = 0.f;
-  const float c = PRE ? 1.f : a.sm_scale * LOG2E;
 
-  if (nt > 0) {
+  if (!CAREFUL && nt > 0) {
     fetch_idx(0);
     fetch(0);
     fetch_idx(1);
   }
   for (int j = 0; j < nt; ++j) {
+    if constexpr (CAREFUL) {  // none ahead: the registers are needed below
+      fetch_idx(j);
+      fetch(j);
+    }
     char* kl = lds + (j & 1) * 2 * kStage;
     char* vl = kl + kStage;
 #pragma unroll
@@ -187,7 +201,7 @@ __global__ void __launch_bounds__(256, 2) extend_tile_kernel(ExtendArgs a) {
       *reinterpret_cast<int4v*>(vl + ext_v_off<D>(r, chunk * 16)) = vreg[i];
     }
     __syncthreads();  // also: nobody reads the other stage any more once the next tile is parked
-    if (j + 1 < nt) {
+    if (!CAREFUL && j + 1 < nt) {
       fetch(j + 1);
       fetch_idx(j + 2);
     }
@@ -229,13 +243,17 @@ __global__ void __launch_bounds__(256, 2) extend_tile_kernel(ExtendArgs a) {
           s[u][r] = (a.logit_cap > 0.f ? a.logit_cap * tanhf(v / a.logit_cap) : v) * LOG2E;
         }
     }
+    [[maybe_unused]] uint32_t hidden = 0;
     if (t0 + kExtTokens > t_end || (diag && t0 + kExtTokens - 1 > w_first)) {  // wave-uniform
       const int lim = diag ? min(tok + shift, t_end - 1) : t_end - 1;          // last token this row sees
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
         for (int r = 0; r < 16; ++r)
-          if (t0 + 32 * u + 8 * (r >> 2) + 4 * hi + (r & 3) > lim) s[u][r] = -INFINITY;
+          if (t0 + 32 * u + 8 * (r >> 2) + 4 * hi + (r & 3) > lim) {
+            s[u][r] = -INFINITY;
+            if constexpr (CAREFUL) hidden |= 1u << (16 * u + r);
+          }
     }
     float tmax = s[0][0];
 #pragma unroll
@@ -246,7 +264,7 @@ __global__ void __launch_bounds__(256, 2) extend_tile_kernel(ExtendArgs a) {
     // The maximum only keeps the exponentials in range.  Probabilities that are rounded to 16 bits need it exact (the
     // largest one is then 1 and has no rounding error); split ones let it lag by 2^8 and save most of the rescaling.
     constexpr bool P2 = D == 64;
-    if (__any(tmax > m + (P2 ? 8.f : 0.f))) {
+    if (__any(tmax > m + (P2 && !CAREFUL ? 8.f : 0.f))) {
       const float m_new = fmaxf(m, tmax);
       const float alpha = m_new == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - m_new);
       m = m_new;
@@ -265,16 +283,75 @@ __global__ void __launch_bounds__(256, 2) extend_tile_kernel(ExtendArgs a) {
       for (int r = 0; r < 16; ++r) {
         const float p = __builtin_amdgcn_exp2f(fmaf(s[u][r], c, -m_use));
         psum += p;
+        if constexpr (CAREFUL) {
+          s[u][r] = p;
+          continue;
+        }
         const uint16_t ph = Conv<T>::from_f32(p);
         pf[2 * u + (r >> 3)][r & 7] = (short)ph;
         if constexpr (P2) pl[2 * u + (r >> 3)][r & 7] = (short)Conv<T>::from_f32(p - Conv<T>::to_f32(ph));
       }
     lsum += psum;
+    if constexpr (CAREFUL) {
+      // A value that is not finite counts as zero in the product; two more products count those of a row's 16 tokens on
+      // either side (a NaN, and an infinity of weight zero, is one on both), and one infinity stands for a side.
+      auto value = [&](int k, int n) {  // V^T operand: 16 tokens from 16 k on, elements 32 n .. 32 n + 31
+        const int row = 16 * k + 4 * hi + ((lane & 15) >> 2);
+        const int byte = 64 * n + 32 * ((lane >> 4) & 1) + 8 * (lane & 3);
+        const short4v lo = lds_read_tr16(vl + ext_v_off<D>(row, byte));
+        const short4v up = lds_read_tr16(vl + ext_v_off<D>(row + 8, byte));
+        return short8{lo[0], lo[1], lo[2], lo[3], up[0], up[1], up[2], up[3]};
+      };
+      constexpr int kInf = Special<T>::kInf, kOne = Special<T>::kOne;
+      if (m == -INFINITY) hidden = ~0u;  // (nothing of weight so far: the row takes nothing)
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int row = 16 * k + 4 * hi + ((lane & 15) >> 2);
+      for (int k = 0; k < 4; ++k) {
+        short8 hp, lp, on, off;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float p = s[k >> 1][8 * (k & 1) + e];
+          const int seen = hidden >> (8 * k + e) & 1 ? 0 : kOne;
+          const uint16_t ph = Conv<T>::from_f32(p);
+          hp[e] = (short)ph;
+          lp[e] = (short)Conv<T>::from_f32(p - Conv<T>::to_f32(ph));
+          on[e] = (short)(p == 0.f ? 0 : seen);
+          off[e] = (short)(p == 0.f ? seen : 0);
+        }
+#pragma unroll
+        for (int n = 0; n < NV; ++n) {
+          __builtin_amdgcn_sched_barrier(0);
+          const short8 vf = value(k, n);
+          short8 fin, any, side[2];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const int sign = vf[e] >> 15, mag = vf[e] & 0x7FFF;
+            const int odd = (kInf - 1 - mag) >> 31, nan = (kInf - mag) >> 31;  // all ones or zeros
+            fin[e] = (short)(vf[e] & ~odd);
+            any[e] = (short)(odd & kOne);
+            side[0][e] = (short)((nan | (odd & ~sign)) & kOne);
+            side[1][e] = (short)((nan | (odd & sign)) & kOne);
+          }
+          oacc[n] = Mfma32<T>::mma(fin, hp, oacc[n]);
+          if constexpr (P2) oacc[n] = Mfma32<T>::mma(fin, lp, oacc[n]);
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            float16v count;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) count[r] = 0.f;
+            count = Mfma32<T>::mma(side[t], on, Mfma32<T>::mma(any, off, count));
+#pragma unroll
+            for (int r = 0; r < 16; ++r) oacc[n][r] += count[r] == 0.f ? 0.f : t == 0 ? INFINITY : -INFINITY;
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+      }
+      continue;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
+        const int row = 16 * k + 4 * hi + ((lane & 15) >> 2);
         const int byte = 64 * n + 32 * ((lane >> 4) & 1) + 8 * (lane & 3);
         const short4v lo = lds_read_tr16(vl + ext_v_off<D>(row, byte));
         const short4v up = lds_read_tr16(vl + ext_v_off<D>(row + 8, byte));
@@ -282,7 +359,6 @@ __global__ void __launch_bounds__(256, 2) extend_tile_kernel(ExtendArgs a) {
         oacc[n] = Mfma32<T>::mma(vf, pf[k], oacc[n]);
         if constexpr (P2) oacc[n] = Mfma32<T>::mma(vf, pl[k], oacc[n]);
       }
-    }
     constexpr int kPer = P2 ? 2 : 1, kAheadV = 3;  // products a value operand, operands read ahead
     __builtin_amdgcn_sched_group_barrier(0x100, 2 * kAheadV, 1);
 #pragma unroll
@@ -294,8 +370,15 @@ __global__ void __launch_bounds__(256, 2) extend_tile_kernel(ExtendArgs a) {
   }
 
   const float tot = lsum + __shfl_xor(lsum, 32, 64);
-  if (!row_ok) return;
   const float inv = tot == 0.f ? 0.f : 1.0f / tot;
+  float zero[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int n = 0; n < NV; ++n)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) zero[r & 3] = fmaf(oacc[n][r], 0.f, zero[r & 3]);
+  const float nan = (zero[0] + zero[1]) + (zero[2] + zero[3]);
+  const bool odd = nan != 0.f || __shfl_xor(nan, 32, 64) != 0.f;
+  if (!mine || (odd && !CAREFUL)) return mine && odd;
   // lane (row, hi) holds elements 32 n + 8 g + 4 hi + 0 .. 3 of its row
   if (a.kv_splits > 1) {
     const int64_t row = ((int64_t)(q0 + tok) * a.Hq + head) * a.kv_splits + split;
@@ -310,7 +393,7 @@ __global__ void __launch_bounds__(256, 2) extend_tile_kernel(ExtendArgs a) {
         *reinterpret_cast<float4v*>(dst + 32 * n + 8 * g) = v;
       }
     if (hi == 0) a.part_lse[row] = tot == 0.f ? -INFINITY : (m + log2f(tot)) * 0.6931471805599453f;
-    return;
+    return false;
   }
   uint16_t* dst = a.o + (int64_t)(q0 + tok) * a.o_st + (int64_t)head * a.o_sh + 4 * hi;
 #pragma unroll
@@ -322,6 +405,27 @@ __global__ void __launch_bounds__(256, 2) extend_tile_kernel(ExtendArgs a) {
       for (int r = 0; r < 4; ++r) v[r] = (short)Conv<T>::from_f32(oacc[n][4 * g + r] * inv);
       *reinterpret_cast<short4v*>(dst + 32 * n + 8 * g) = v;
     }
+  return false;
+}
+
+template <typename T, int D, bool PRE>
+__global__ void __launch_bounds__(256, 2) extend_tile_kernel(ExtendArgs a) {
+  // A value that is not finite spoils, times a probability of zero, the rows that do not see it as well (and, at head size
+  // 64, times the second part of a probability, those that do; there also sums that overflow under a lagging maximum).
+  // Rows whose result is not finite are walked once more.  To the others that costs a multiplication a result and a
+  // barrier at the end: 0.2 us of a launch alone, 118.2 -> 118.9 us for the 8 prompts above.
+  int tid = threadIdx.x;
+  const bool again = extend_walk<T, D, PRE, false>(a, tid, false);
+  __shared__ int spoilt[4];
+  if ((tid & 63) == 0) spoilt[tid >> 6] = 0;
+  if (again) spoilt[tid >> 6] = 1;
+  __syncthreads();  // also: nobody reads a stage any more
+  if (__builtin_expect((spoilt[0] | spoilt[1] | spoilt[2] | spoilt[3]) == 0, 1)) return;
+  // the second walk takes everything from the arguments again: what the first keeps in registers for it slows its loop
+  // (head size 128: by a quarter)
+  auto args = __builtin_amdgcn_kernarg_segment_ptr();  // the kernel's one argument
+  asm volatile("" : "+s"(args), "+v"(tid));
+  extend_walk<T, D, PRE, true>(*(const ExtendArgs*)args, tid, again);
 }
 
 }  // namespace sglk

@@ -119,3 +119,84 @@ def test_prefix_long_enough_to_split_with_any_rows(D, odd):
     kb = shift(kb, 4 if odd == "pool start" else 0, 0)
     ops.extend_attention_fwd(q, ke, ve, o, kb, vb, qo, kp, ki, None, True, None, 9)
     assert (o.float().cpu() - want).abs().max().item() < TOL[torch.bfloat16]
+
+
+def _dense(q, ke, ve, kb, vb, qo, kp, ki, sm, causal=True):
+    """Rows as double sums over the tokens they see."""
+    out = torch.empty(*q.shape[:2], ve.shape[2], dtype=torch.float64)
+    share = q.shape[1] // ke.shape[1]
+    for b in range(len(qo) - 1):
+        idx = ki[kp[b]: kp[b + 1]].long()
+        k = torch.cat([kb[idx], ke[qo[b]: qo[b + 1]]]).double().repeat_interleave(share, 1)
+        v = torch.cat([vb[idx], ve[qo[b]: qo[b + 1]]]).double().repeat_interleave(share, 1)
+        for i in range(int(qo[b]), int(qo[b + 1])):
+            n = len(idx) + (i - int(qo[b]) + 1 if causal else int(qo[b + 1] - qo[b]))
+            p = torch.softmax(torch.einsum("hd,thd->ht", q[i].double(), k[:n]) * sm, -1)
+            out[i] = (p.unsqueeze(-1) * v[:n].transpose(0, 1)).sum(1)
+    return out
+
+
+def _agree(got, want, tol):
+    got = got.double().cpu()
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got == math.inf, want == math.inf) and torch.equal(got == -math.inf, want == -math.inf)
+    ok = want.isfinite()
+    assert (got[ok] - want[ok]).abs().max().item() < tol
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_values_that_are_not_finite(dtype, D, splits):
+    """Infinities and NaNs among the values: rows that see them take them as sums of doubles do, rows in front of them
+    (in the same tile, the same block, in a wave of their own) are those of finite values."""
+    from sglang_security_amd import ops
+
+    t = list(_case(8, 2, D, [70, 65, 0], [150, 20, 33], dtype, 3))
+    sm = 1.0 / math.sqrt(D)
+    g = [x.to(DEV) for x in t]
+    run = lambda: ops.extend_attention_split(*g[:3], o, *g[3:], 150, sm, 0.0, True, splits)
+    o = torch.full_like(g[0], float("nan"))
+    run()
+    clean = o.clone()
+    ve, vb, ki = t[2], t[4], t[7].long()
+    ve[149, 0, 3], ve[140, 1, 5], ve[139, 1, 5] = math.nan, math.inf, -math.inf       # the first request's last tokens
+    ve[70, 0, 7] = -math.inf                                                          # seen from its middle on
+    ve[150 + 19, 1, 0] = math.inf                                                     # the second one's last token
+    vb[ki[70 + 64], 0, 2], vb[ki[70 + 1], 1, 9] = math.inf, math.nan                  # its prefix: every row of it sees them
+    ve[150 + 20 + 32, :, 1] = math.nan
+    g[2], g[4] = ve.to(DEV), vb.to(DEV)
+    o = torch.full_like(g[0], float("nan"))
+    run()
+    want = _dense(*t, sm)
+    _agree(o, want, TOL[dtype])
+    blind = want.isfinite().all(-1)          # rows (token, head) that see none of them
+    assert blind.sum() > 150 * 4
+    if D == 128:                             # (head size 64 lets its maximum lag where every result is finite)
+        assert torch.equal(o.cpu()[blind], clean.cpu()[blind])
+    if splits == 1:                          # the paged form, and every new token seen
+        pool = [torch.cat([g[3], g[1]]), torch.cat([g[4], g[2]])]
+        qo, kp, at = t[5], t[6], t[3].shape[0]
+        idx = torch.cat([torch.cat([t[7][kp[b]: kp[b + 1]], torch.arange(int(qo[b]), int(qo[b + 1]), dtype=torch.int32) + at]) for b in range(3)])
+        o = torch.full_like(g[0], float("nan"))
+        ops.prefill_attention_paged(g[0], o, *pool, g[5], g[6] + g[5], idx.to(DEV), 150, sm, 0.0)
+        _agree(o, want, TOL[dtype])
+        o = torch.full_like(g[0], float("nan"))
+        ops.extend_attention_fwd(*g[:3], o, *g[3:], None, False, None, 150, sm, 0.0)
+        _agree(o, _dense(*t, sm, causal=False), TOL[dtype])
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_values_near_the_end_of_the_range(D):
+    """Values of 2^120 under scores that rise by less than 2^8: sums stay finite as long as probabilities stay below one."""
+    from sglang_security_amd import ops
+
+    T = 200
+    q, k, v = torch.zeros(T, 1, D), torch.zeros(T, 1, D), torch.full((T, 1, D), 2.0**120)
+    q[..., 0] = 1.0
+    k[64:, :, 0] = 5.0                       # exp(5) = 2^7.2
+    d = lambda x: x.to(torch.bfloat16).to(DEV)
+    o, ptr = torch.empty_like(d(q)), torch.tensor([0, T], dtype=torch.int32, device=DEV)
+    none = torch.zeros(2, dtype=torch.int32, device=DEV)
+    ops.extend_attention_fwd(d(q), d(k), d(v), o, d(k), d(v), ptr, none, none[:1], None, True, None, T, 1.0)
+    assert ((o.double() / 2.0**120 - 1).abs() < 2.0**-7).all()
