@@ -126,7 +126,7 @@ __global__ void __launch_bounds__(256) extend_attention_kv8(
       float* dst = part_o + row * 128;
 #pragma unroll
       for (int n = 0; n < 8; ++n) *reinterpret_cast<float4v*>(dst + 16 * n + 4 * g) = st.oacc[c][n] * inv;
-      if (g == 0) part_lse[row] = tot > 0.f ? (st.m[c] + log2f(tot)) * 0.6931471805599453f : -INFINITY;
+      if (g == 0) part_lse[row] = tot == 0.f ? -INFINITY : (st.m[c] + log2f(tot)) * 0.6931471805599453f;
     }
     return;
   }
@@ -159,7 +159,7 @@ __global__ void __launch_bounds__(128) extend_merge_kernel(const float* __restri
   float e_max = -INFINITY, e_sum = 0.f, acc = 0.f;
   for (int s = 0; s < kv_splits; ++s) {
     const float l = part_lse[row0 + s];
-    if (l > -INFINITY) {
+    if (l != -INFINITY) {  // (a NaN takes part)
       const float v = part_o[(row0 + s) * D + d];
       const float n_max = fmaxf(l, e_max);
       const float old = expf(e_max - n_max), w = expf(l - n_max);
@@ -168,7 +168,7 @@ __global__ void __launch_bounds__(128) extend_merge_kernel(const float* __restri
       e_max = n_max;
     }
   }
-  st<T>(o, t * o_stride_t + (int64_t)h * o_stride_h + d, e_sum > 0.f ? acc / e_sum : 0.f);
+  st<T>(o, t * o_stride_t + (int64_t)h * o_stride_h + d, e_sum == 0.f ? 0.f : acc / e_sum);
 }
 
 // one wave per (query row, head): any head size, any float type

@@ -200,3 +200,17 @@ def test_values_near_the_end_of_the_range(D):
     none = torch.zeros(2, dtype=torch.int32, device=DEV)
     ops.extend_attention_fwd(d(q), d(k), d(v), o, d(k), d(v), ptr, none, none[:1], None, True, None, T, 1.0)
     assert ((o.double() / 2.0**120 - 1).abs() < 2.0**-7).all()
+
+
+@pytest.mark.parametrize("D,pool", [(64, torch.bfloat16), (128, torch.bfloat16), (128, torch.float8_e4m3fn)])
+def test_a_split_without_a_sum_is_not_lost(D, pool):
+    """A key that is not a number makes its rows NaN however the prefix is split; the rows of other requests stay."""
+    from sglang_security_amd import ops
+
+    q, ke, ve, kb, vb, qo, kp, ki = (x.to(DEV) for x in _case(4, 2, D, [300, 40], [7, 9], torch.bfloat16, 2))
+    kb[ki[150].long(), 0, 3] = math.nan
+    kb, vb = kb.to(pool), vb.to(pool)
+    for splits in (1, 3):
+        o = torch.zeros_like(q)
+        ops.extend_attention_split(q, ke, ve, o, kb, vb, qo, kp, ki, 9, 1.0 / math.sqrt(D), 0.0, True, splits)
+        assert o[:7, :2].isnan().all() and o[:7, 2:].isfinite().all() and o[7:].isfinite().all()
