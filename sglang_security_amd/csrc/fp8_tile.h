@@ -99,8 +99,9 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) fp8_tile_kernel(Fp8TileArgs p
 #pragma unroll
   for (int i = 0; i < ST - 1; ++i) issue(i);
   for (int kb = 0; kb < nk; ++kb) {
-    // this wave's pieces of the stage have landed; behind the barrier everyone's have, and the stage before is free
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * U * (ST - 2)) : "memory");
+    // this wave's pieces of the stage have landed and its operands of the stage before have arrived; behind the barrier
+    // everyone's have, and the stage before is free
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(2 * U * (ST - 2)) : "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (ST > 2 || kb + 1 < nk) issue(kb + ST - 1);
