@@ -730,8 +730,9 @@ SGLK_API int sglk_fp8_blockwise_scaled_mm_packed(const void* a, const void* pack
  * and carry on (fused add + norm + per-token quantisation; rotation + pool write).  row_scale may alias the `scales`
  * output of sglk_rmsnorm_quant_fp8_partial.  No counterpart in the reference, which runs these steps as separate ops. */
 SGLK_API int sglk_fp8_mm_packed_partial_splits(int M, int N, int K);
-/* 1 where sglk_fp8_scaled_mm multiplies an [M, K] x [N, K] product by the tile kernels and they are expected to be
- * faster than sglk_fp8_scaled_mm_packed (callers that hold both layouts of a weight), else 0. */
+/* 1 where sglk_fp8_scaled_mm, with a workspace and without, multiplies an [M, K] x [N, K] product by the tile kernels (rows,
+ * scales and bias aligned as they take them) and they are expected to be faster than sglk_fp8_scaled_mm_packed (callers
+ * that hold both layouts of a weight), else 0. */
 SGLK_API int sglk_fp8_tiled(int M, int N, int K);
 SGLK_API int sglk_fp8_mm_packed_partial(const void* a, const void* packed, float* partial, int M, int N, int K,
                                         int64_t a_stride, void* stream);

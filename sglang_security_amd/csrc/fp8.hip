@@ -630,28 +630,49 @@ int launch_fp8_tile(const MmArgs& p, hipStream_t s) {
   return SGLK_OK;
 }
 
-// Which tile form multiplies [M, K] x [N, K] fastest (0: the form of this call that is not tiled).  Estimates in
-// microseconds, fitted to launches on weights that come from memory (N, K of the 8B model's projections and of the 70B
-// model's on one of eight ranks; M = 1 .. 2048): a form needs its time per k-block of 128 for every round of blocks.
-// Measured against the register kernel and the streaming kernel, M x N x K: 2048 x 28672 x 4096: 1190 -> 214 (streaming
-// 788); 2048 x 4096 x 14336: 593 -> 110 (349); 256 x 4096 x 14336: 79 -> 37 (68); 128 x 28672 x 4096: 83 -> 33 (57);
-// 128 x 4096 x 4096: 14.6 -> 12.9 (16.5); 64 x 28672 x 4096 without the streaming copy: 50 -> 30.
-static int fp8_tile_choice(int64_t M, int64_t N, int64_t K, bool streaming) {
+static int fp8_stream_splits(int M, int N, int K);
+
+enum class Fp8Other { kRegister, kSplit, kStreaming };  // what a call falls back on; a later one could also take the earlier
+
+// Which tile form multiplies [M, K] x [N, K] fastest (0: none, the call falls back on `other`).  Estimates in
+// microseconds, fitted to launches on weights that come from memory: a tile form needs its time per k-block of 128 for
+// every round of blocks; the others take the lesser of an estimate by work and one by rounds (narrow outputs spread K
+// over idle units, which the tiles do not).  Measured against the register kernel, the split and the streaming one:
+//   N, K of the 8B model's projections and of the 70B model's on one of eight ranks, M = 1 .. 2048: 2048 x 28672 x 4096
+//   1190 -> 214 (streaming 788); 2048 x 4096 x 14336 593 -> 110 (349); 256 x 4096 x 14336 79 -> 37 (68); 128 x 28672 x
+//   4096 83 -> 33 (57); 128 x 4096 x 4096 14.6 -> 12.9 (16.5); 64 x 28672 x 4096 without the streaming copy 50 -> 30;
+//   M = 33 .. 2048, N = 32 .. 8192, K = 512 .. 14336, 1008 sizes: no call on tiles is slower than its fallback by more
+//   than 4 % (33 x 6144 x 14336), none that stays would gain more than 11 % (the same, against the split kernel).
+//   Narrow ones that stay: 1024 x 128 x 14336 split 18.9, streaming 15.8, tiled 30.9; 512 x 256 x 7168 13.8, 11.8, 17.4.
+static int fp8_tile_choice(int64_t M, int64_t N, int64_t K, Fp8Other other) {
   if (M <= 0 || K % 128 != 0 || N % 16 != 0 || getenv("SGLK_FP8_SPLITS") || getenv("SGLK_FP8_WAVES")) return 0;
-  auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
-  auto rounds = [&](int bm, int bn, int per_round) { return (double)up(up(M, bm) * up(N, bn), per_round); };
-  const double cost[5] = {1.5 * rounds(256, 256, 256), 1.17 * rounds(128, 128, 512), 0.62 * rounds(128, 128, 256),
-                          0.47 * rounds(64, 128, 256), 0.31 * rounds(64, 64, 256)};
-  int best = 0;
-  for (int i = 1; i < 5; ++i)
-    if (cost[i] < cost[best]) best = i;
-  const double tiled = cost[best] * (K / 128) + 3.5, passes = (double)up(M, 64), mb = (double)N * K * 1e-6;
   // up to 64 rows the streaming kernel, which leaves the weights out of the caches, is the faster one in a layer's
   // sequence of products (28672 x 4096 tiled: a pass of four products 106 us against 100); up to 32 the register
   // kernel's smaller tiles keep up with the memory
-  const double other = streaming ? (M <= 64 ? 0.0 : 5 + 2 * passes + 0.19 * passes * mb)
-                                 : (M <= 32 ? 0.0 : 2 + 2 * passes + (0.08 + 0.31 * passes) * mb);
-  return tiled < other ? best + 1 : 0;
+  if (M <= (other == Fp8Other::kStreaming ? 64 : 32)) return 0;
+  auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  auto rounds = [&](int bm, int bn, int per_round) { return (double)up(up(M, bm) * up(N, bn), per_round); };
+  const double small = M <= 64 && N >= 8192 ? 0.35 : 0.28;  // one row of blocks: 128 units ask memory for all the weights
+  const double cost[5] = {1.35 * rounds(256, 256, 256), 1.05 * rounds(128, 128, 512), 0.56 * rounds(128, 128, 256),
+                          0.42 * rounds(64, 128, 256), small * rounds(64, 64, 256)};
+  int best = 0;
+  for (int i = 1; i < 5; ++i)
+    if (cost[i] < cost[best]) best = i;
+  const double tiled = cost[best] * (K / 128) + 3.15, passes = (double)up(M, 64), mb = (double)N * K * 1e-6;
+  auto by_rounds = [&](int splits, int bn, double per_block, double partial) {  // partial: us a million sums left by a split
+    const double per = (double)up(K / 128, splits), blocks = (double)up(N, bn) * passes * splits;
+    return (splits > 1 ? 1.3 + partial * 1e-6 * splits * M * N : 0.0) + per_block * per * std::max(1.0, blocks / 256);
+  };
+  const double rows = 0.34 * (0.75 + 0.25 * (double)std::min<int64_t>(M, 64) / 64);
+  const double by_work = 2 + 2 * passes + (0.08 + 0.31 * passes) * mb;
+  double least = std::min(by_work, 4.0 + by_rounds(1, 32, rows, 0));
+  if (other != Fp8Other::kRegister) least = std::min(least, 4.0 + by_rounds(fp8_splits((int)M, (int)N, (int)K), 32, rows, 4.1));
+  if (other == Fp8Other::kStreaming) {
+    const int splits = fp8_stream_splits((int)M, (int)N, (int)K);
+    least = std::min({least, 5 + 2 * passes + 0.19 * passes * mb,
+                      4.4 + by_rounds(splits, 64, 0.34, 1.7) + 0.18 * (double)up(K / 128, splits) + 0.033 * mb});
+  }
+  return tiled < least ? best + 1 : 0;
 }
 
 static bool fp8_tile_rows(const MmArgs& p) {
@@ -1079,7 +1100,7 @@ int sglk_fp8_scaled_mm(const void* a, const void* b_nk, const float* scales_a, c
   if (M == 0) return SGLK_OK;
   MmArgs p{(const uint8_t*)a, (const uint8_t*)b_nk, scales_a, scales_b, bias, out, M, N, K, a_stride, b_stride,
            out_stride,        0,                    0,        0,        0};
-  const int form = fp8_tile_rows(p) ? fp8_tile_choice(M, N, K, false) : 0;
+  const int form = fp8_tile_rows(p) ? fp8_tile_choice(M, N, K, Fp8Other::kRegister) : 0;
   SGLK_DISPATCH_HALF(out_dtype, TO, {
     if (form) return (launch_fp8_tiled<TO>(form, p, (hipStream_t)stream));
     return (launch_mm<TO, false>(p, (hipStream_t)stream));
@@ -1087,7 +1108,7 @@ int sglk_fp8_scaled_mm(const void* a, const void* b_nk, const float* scales_a, c
   return SGLK_OK;
 }
 
-int sglk_fp8_tiled(int M, int N, int K) { return fp8_tile_choice(M, N, K, true) != 0; }
+int sglk_fp8_tiled(int M, int N, int K) { return fp8_tile_choice(M, N, K, Fp8Other::kStreaming) != 0; }
 
 int64_t sglk_fp8_mm_workspace_bytes(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
@@ -1216,7 +1237,7 @@ int sglk_fp8_scaled_mm_ws(const void* a, const void* b_nk, const float* scales_a
   const int splits = (M > 0 && N > 0 && K > 0) ? fp8_splits(M, N, K) : 1;
   const MmArgs shape{nullptr, nullptr, nullptr, scales_b, bias, out, M, N, K, a_stride, b_stride, out_stride};
   if (splits <= 1 || !workspace || workspace_bytes < sglk_fp8_mm_workspace_bytes(M, N, K) || !aligned16(workspace) ||
-      (fp8_tile_rows(shape) && fp8_tile_choice(M, N, K, false)))
+      (fp8_tile_rows(shape) && fp8_tile_choice(M, N, K, Fp8Other::kSplit)))
     return sglk_fp8_scaled_mm(a, b_nk, scales_a, scales_b, bias, out, M, N, K, a_stride, b_stride, out_stride, out_dtype,
                               stream);
   SGLK_CHECK(a && b_nk && scales_a && scales_b && out, "fp8_scaled_mm: null pointer");
