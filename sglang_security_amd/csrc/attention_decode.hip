@@ -291,31 +291,25 @@ __global__ void __launch_bounds__(64) decode_stage1_generic(
   if (lane == 0) attn_lse[ob] = m + logf(l);
 }
 
-// How many ways request b's context is split.  units == 0: as the caller says.  Otherwise a split of every request is
-// `units` blocks for the chip's kMlaPlaces (two a unit), and of 1 .. the caller's number the one is taken that makes
-// rounds x (tokens of a split + 32 for its start and its merge) least, counted as if all requests were like this one.  A
-// last round that leaves every unit one block or none counts 0.65, any other that is not full 0.95 (a block that has
-// its unit to itself is that much faster).  A request half as long again as the batch's average keeps what it was given:
-// alone in the last round, it would end the launch.
-constexpr int kMlaPlaces = 512;
-__device__ __forceinline__ int splits_of(const int32_t* __restrict__ num_kv_splits, const int32_t* __restrict__ kv_indptr, int b, int B,
-                                         int len, int max_splits, int units) {
+// How many ways request b's context is split: as the caller says, or, where `fewer` names a number for that many and a batch
+// of such a mean context (64 tokens and up, by powers of two), as it says (mla_fewer_splits).  A request twice as long as
+// the mean keeps what it was given: alone in the last round, it would end the launch.
+constexpr int kMeans = 7;
+struct FewerSplits {
+  int batch;  // 0: always as the caller says
+  uint64_t pick[kMeans];  // four bits a number of splits, 1 .. 16; 0: as the caller says
+};
+__device__ __forceinline__ int splits_of(const int32_t* __restrict__ num_kv_splits, const int32_t* __restrict__ kv_indptr, int b, int len,
+                                         int max_splits, const FewerSplits& fewer) {
   const int most = max(num_kv_splits[b], 1);
-  if (units == 0 || most > max_splits || (int64_t)units * most <= kMlaPlaces) return most;
-  if (2 * (int64_t)len * B > 3 * ((int64_t)kv_indptr[B] - kv_indptr[0])) return most;
-  int best = 1;
-  int64_t best_cost = 0;  // times 20 and `best`
-  for (int n = 1; n <= most; ++n) {
-    const int64_t blocks = (int64_t)units * n;
-    const int rest = (int)(blocks % kMlaPlaces);
-    const int64_t rounds = 20 * (blocks / kMlaPlaces) + (rest == 0 ? 0 : rest <= kMlaPlaces / 2 ? 13 : 19);
-    const int64_t cost = rounds * (len + 32 * n);
-    if (n == 1 || cost * best < best_cost * n) {
-      best = n;
-      best_cost = cost;
-    }
-  }
-  return best;
+  if (fewer.batch == 0 || most > min(max_splits, 16)) return most;
+  const float mean = (float)(kv_indptr[fewer.batch] - kv_indptr[0]) * __builtin_amdgcn_rcpf((float)fewer.batch);
+  if (!(mean >= 64.f) || (float)len > 2.f * mean) return most;
+  uint64_t picks = fewer.pick[0];
+#pragma unroll
+  for (int k = 1; k < kMeans; ++k) picks = mean < (float)(64 << k) ? picks : fewer.pick[k];
+  const int n = (int)(picks >> (4 * (most - 1))) & 15;
+  return n ? n : most;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -328,12 +322,12 @@ __global__ void __launch_bounds__(128) decode_stage2(const float* __restrict__ a
                                                      const int32_t* __restrict__ num_kv_splits, int max_kv_splits,
                                                      int Hq, int Dv, int64_t o_stride_b, int64_t o_stride_h,
                                                      float* __restrict__ xsum_out, int64_t xs_stride,
-                                                     const int32_t* __restrict__ gate = nullptr, int units = 0) {
+                                                     const int32_t* __restrict__ gate = nullptr, FewerSplits fewer = {}) {
   __shared__ float xs_red[2];
   if (gate && *gate != 0) return;  // see decode_stage1_mfma128
   const int b = blockIdx.x, h = blockIdx.y;
   const int len = kv_indptr[b + 1] - kv_indptr[b];
-  const int splits = splits_of(num_kv_splits, kv_indptr, b, gridDim.x, len, max_kv_splits, units);
+  const int splits = splits_of(num_kv_splits, kv_indptr, b, len, max_kv_splits, fewer);
   const int per_split = cdiv_i(cdiv_i(len, splits), kMinBlockKV) * kMinBlockKV;
   const int64_t base = ((int64_t)b * Hq + h) * max_kv_splits;
   if (Dv % 512 == 0 && !xsum_out && (reinterpret_cast<uintptr_t>(attn_logits) & 15) == 0) {
@@ -528,7 +522,7 @@ __global__ void __launch_bounds__(256, HT == 1 ? 3 : 2) decode_stage1_mla(
     const int32_t* __restrict__ kv_indices, float* __restrict__ attn_logits, float* __restrict__ attn_lse,
     const int32_t* __restrict__ num_kv_splits, int max_kv_splits, int Hq, int Hkv, int head_tiles, int64_t q_stride_b,
     int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h, float sm_scale, float logit_cap,
-    const int32_t* __restrict__ gate, int units) {
+    const int32_t* __restrict__ gate, FewerSplits fewer) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   if (gate && *gate != 0) return;  // see decode_stage1_mfma128
   const int lane = threadIdx.x & 63;
@@ -539,7 +533,7 @@ __global__ void __launch_bounds__(256, HT == 1 ? 3 : 2) decode_stage1_mla(
   const int group = Hq / Hkv;
   const int start = kv_indptr[b];
   const int len = kv_indptr[b + 1] - start;
-  const int splits = splits_of(num_kv_splits, kv_indptr, b, gridDim.x, len, max_kv_splits, units);
+  const int splits = splits_of(num_kv_splits, kv_indptr, b, len, max_kv_splits, fewer);
   const int per_split = cdiv_i(cdiv_i(len, splits), kMinBlockKV) * kMinBlockKV;
   const int s0 = per_split * split, s1 = min(s0 + per_split, len);
   if (s1 <= s0) return;  // block-uniform
@@ -1667,6 +1661,50 @@ int sglk_common_prefix_len(const int32_t* req_to_token, int64_t row_stride, cons
   return SGLK_OK;
 }
 
+// Where fewer splits than the caller's make a latent launch of up to 16 faster.  `units` blocks are one split of every
+// request, for 512 places (two a unit of the chip).  An estimate in microseconds: blocks take 0.086 a token of the mean
+// context, a last round that leaves every unit one block or none a part of that; the partials a time per round of blocks.
+// Of the numbers that leave at most a tenth of a round's places empty, the one with the least estimate is taken if that is
+// below 0.87 of the caller's; one above 0.8 of the caller's has to save a round and to fill those left.  Below 256 tokens
+// the partials are what counts: up to 0.7, any number of places, below 0.95.  Fitted to 664 batches (1 to 256 requests of
+// 32, 40, 64 and 128 heads, contexts of 100 to 16000 tokens, even ones and spread from a quarter up) timed with 1 to 16
+// splits.  Calls with the caller's number -> with the rule's, 128 heads: 64 requests of 768 to 1152 tokens 75.6 us (3 splits)
+// -> 66.8 (2), 98.6 (8) -> 70.3; 32 of them 56.0 (8) -> 44.8 (4); 20 of 2731 to 4096 tokens 85.4 (8) -> 75.7 (6); 100 of 150
+// to 300 tokens 88.4 (8) -> 49.8 (1); 75 of 768 to 1152 keep 2 (98), of 1024 to 4096 keep 3 (216).  Of 3984 calls 1039 are
+// more than 4 % faster; calls that keep their number pay up to 1 us of a pair of launches for asking (45 of them more than
+// 4 %).  An estimate weighed in every block cost more than it gave: 5 to 20 us of 25600 merge blocks.
+static FewerSplits mla_fewer_splits(int B, int64_t units, int max_splits) {
+  constexpr int kPlaces = 512;
+  FewerSplits f{};
+  if (units * max_splits <= kPlaces || units >= (1 << 20)) return f;
+  const int last = std::min(max_splits, 16);
+  for (int k = 0; k < kMeans; ++k) {
+    const int mean = (int)(90.5 * (1 << k));  // the middle of the range
+    const bool few = mean < 256;
+    double cost[17];
+    int64_t blocks[17], rounds[17];
+    for (int n = 1; n <= last; ++n) {
+      const int per = ((mean + n - 1) / n + kMinBlockKV - 1) / kMinBlockKV * kMinBlockKV;
+      blocks[n] = units * ((mean + per - 1) / per), rounds[n] = (blocks[n] + kPlaces - 1) / kPlaces;
+      const int64_t full = blocks[n] / kPlaces, rest = blocks[n] % kPlaces;
+      const double part = rest == 0 ? 0.0 : rest > kPlaces / 2 ? 1.0 : few ? 0.9 : 0.8;
+      cost[n] = 4 + 0.086 * per * ((double)full + part) + (few ? 16.0 : 12.0) * blocks[n] / kPlaces;
+    }
+    for (int most = 2; most <= last; ++most) {
+      if (units * most <= kPlaces) continue;
+      double least = (few ? 0.95 : 0.87) * cost[most];
+      int pick = 0;
+      for (int n = few ? 7 * most / 10 : most - 1; n >= 1 && (few || 10 * units * n >= 9 * kPlaces); --n) {
+        if (10 * n > 8 * most && (rounds[n] == rounds[most] || 100 * blocks[n] < 92 * kPlaces * rounds[n])) continue;
+        if (cost[n] < least) pick = n, least = cost[n];
+      }
+      f.pick[k] |= (uint64_t)pick << (4 * (most - 1));
+      if (pick) f.batch = B;
+    }
+  }
+  return f;
+}
+
 static int decode_attention_impl(const void* q, const void* k_buffer, const void* v_buffer, void* o, const int32_t* kv_indptr,
                              const int32_t* kv_indices, float* attn_logits, float* attn_lse, const int32_t* num_kv_splits,
                              int max_kv_splits, int B, int Hq, int Hkv, int D, int Dv, int64_t q_stride_b,
@@ -1686,7 +1724,7 @@ static int decode_attention_impl(const void* q, const void* k_buffer, const void
   if (B == 0) return SGLK_OK;
   hipStream_t s = (hipStream_t)stream;
   const int group = Hq / Hkv;
-  int units = 0;  // blocks of one split of every request, where their number is weighed (splits_of)
+  FewerSplits fewer{};
   const bool fast = kvf == 0 && (dtype == SGLK_F16 || dtype == SGLK_BF16) && D == 128 && Dv == 128 && aligned16(q) &&
                     aligned16(k_buffer) && aligned16(v_buffer) && aligned16(attn_logits) && (q_stride_b % 8 == 0) &&
                     (q_stride_h % 8 == 0) && (k_stride_n % 8 == 0) && (k_stride_h % 8 == 0) && (v_stride_n % 8 == 0) &&
@@ -1720,19 +1758,17 @@ static int decode_attention_impl(const void* q, const void* k_buffer, const void
       });
     });
   } else if (mla) {
-    // Splits that spill the grid into a nearly empty round cost more than they spread.  128 heads, a call before -> after
-    // (splits): 64 requests of 768 to 1152 tokens 87 (3) -> 75 us (2), 32 of them 58 (5) -> 48 (4), 20 of 2731 to 4096
-    // tokens 91 (8) -> 77 (6); 75 of 768 to 1152 stay at 2 (104 us; 116 with one), 75 of up to 4096 at 3 (255; 338 with
-    // one).  Up to 31 heads a group the copy rate bounds the launch and a short last round is nearly free (100 requests of
-    // up to 2048 tokens, 16 heads: 49.9 us with 8 splits, 51.5 with 7): there the caller's number stands.
+    // Splits that spill the grid into a nearly empty round cost more than they spread (mla_fewer_splits).
+    // Up to 31 heads a group the copy rate bounds the launch and a short last round is nearly free (100 requests of up to
+    // 2048 tokens, 16 heads: 49.9 us with 8 splits, 51.5 with 7): there the caller's number stands.
     if (group >= 32) {  // two tiles of 16 heads per block, two blocks a unit
       const int head_tiles = (group + 31) / 32;
-      if ((int64_t)B * Hkv * head_tiles < (1 << 20)) units = B * Hkv * head_tiles;
+      fewer = mla_fewer_splits(B, (int64_t)B * Hkv * head_tiles, max_kv_splits);
       dim3 grid(B, Hkv * head_tiles, max_kv_splits);
 #define SGLK_MLA_LAUNCH(HT, CAP)                                                                                         \
   hipLaunchKernelGGL((decode_stage1_mla<T, HT, CAP>), grid, dim3(256), kMlaTileBytes + HT * kMlaScoreBytes, s, q, k_buffer, \
                      kv_indptr, kv_indices, attn_logits, attn_lse, num_kv_splits, max_kv_splits, Hq, Hkv, head_tiles,      \
-                     q_stride_b, q_stride_h, k_stride_n, k_stride_h, sm_scale, logit_cap, gate, units)
+                     q_stride_b, q_stride_h, k_stride_n, k_stride_h, sm_scale, logit_cap, gate, fewer)
       SGLK_DISPATCH_HALF(dtype, T, {
         if (logit_cap > 0.f)
           SGLK_MLA_LAUNCH(2, true);
@@ -1804,7 +1840,7 @@ static int decode_attention_impl(const void* q, const void* k_buffer, const void
   SGLK_DISPATCH_FLOAT(dtype, T,
                       hipLaunchKernelGGL((decode_stage2<T>), dim3(B, Hq), dim3(128), 0, s, attn_logits, attn_lse, o,
                                          kv_indptr, num_kv_splits, max_kv_splits, Hq, Dv, o_stride_b, o_stride_h,
-                                         xsum_out, xs_stride, gate, units));
+                                         xsum_out, xs_stride, gate, fewer));
   SGLK_LAUNCH_CHECK();
   return SGLK_OK;
 }
