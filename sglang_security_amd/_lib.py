@@ -255,6 +255,9 @@ def lib():
     return _lib
 
 
+EUNSUP = -3  # SGLK_EUNSUP: a valid request there is no kernel for
+
+
 def check(rc: int, what: str = ""):
     if rc != 0:
         msg = lib().sglk_last_error().decode(errors="replace")

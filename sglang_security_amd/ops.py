@@ -12,7 +12,7 @@ from typing import Optional
 import torch
 
 from . import _lib
-from ._lib import SglkError, check, dtype_code, lib
+from ._lib import EUNSUP, SglkError, check, dtype_code, lib
 
 
 def _ptr(t: Optional[torch.Tensor]) -> int:
@@ -386,11 +386,13 @@ def extend_attention_fwd(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buf
         total_prefix = kv_indices.numel() if kv_indptr.numel() > 1 else 0
     splits = extend_attention_split_plan(T, Hq, B, max_len_extend, int(total_prefix), D,
                                          q_extend.dtype) if (D == Dv and k_buffer is not None) else 1
-    if splits > 1 and not _split_rows(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buffer):
-        splits = 1
     if splits > 1:
-        return extend_attention_split(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buffer, qo_indptr, kv_indptr,
-                                      kv_indices, max_len_extend, sm_scale, logit_cap, is_causal, splits)
+        # rows that do not lie as the split form takes them (or a pool it has no kernel for) run unsplit: the launcher, which
+        # has the pointers and strides, says so before it launches anything (asking here as well took 2.5 us of 17.5 a call)
+        rc = _extend_split(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buffer, qo_indptr, kv_indptr, kv_indices,
+                           max_len_extend, sm_scale, logit_cap, is_causal, splits, None)
+        if rc != EUNSUP:
+            return check(rc, "extend_attention_split")
     check(lib().sglk_extend_attention(
         _ptr(q_extend), _ptr(k_extend), _ptr(v_extend), _ptr(o_extend), _ptr(k_buffer), _ptr(v_buffer),
         _ptr(qo_indptr), _ptr(kv_indptr), _ptr(kv_indices), B, Hq, Hkv, D, Dv,
@@ -399,15 +401,6 @@ def extend_attention_fwd(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buf
         k_buffer.stride(0), k_buffer.stride(1), v_buffer.stride(0), v_buffer.stride(1),
         int(max_len_extend), float(sm_scale), float(logit_cap), 1 if is_causal else 0,
         _attn_dtype(q_extend, k_buffer, v_buffer), _stream(q_extend)), "extend_attention")
-
-
-def _split_rows(q, k, v, o, k_buffer, v_buffer) -> bool:
-    """Whether the rows lie as the split form takes them: 16-byte pieces of q, k, v and of a 16-bit pool, 8-byte pieces of
-    the output and of an fp8 pool, which only head size 128 has a tile kernel for."""
-    pool8 = k_buffer.element_size() == 1
-    lies = lambda t, ptr, stride: t.data_ptr() % ptr == 0 and t.stride(0) % stride == 0 and t.stride(1) % stride == 0
-    return (all(lies(t, 16, 8) for t in (q, k, v)) and lies(o, 8, 4) and
-            all(lies(t, 8 if pool8 else 16, 8) for t in (k_buffer, v_buffer)) and not (pool8 and q.shape[2] != 128))
 
 
 def extend_attention_split_plan(T, Hq, B, max_len_extend, total_prefix, head_dim, dtype) -> int:
@@ -426,6 +419,12 @@ def extend_attention_split(q_extend, k_extend, v_extend, o_extend, k_buffer, v_b
                            max_len_extend, sm_scale, logit_cap, is_causal, kv_splits, workspace=None):
     """extend_attention_fwd with the cached prefix split kv_splits ways and a merge launch (sglk_extend_attention_split)."""
     _need_gpu(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buffer, qo_indptr, kv_indptr, kv_indices)
+    check(_extend_split(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buffer, qo_indptr, kv_indptr, kv_indices,
+                        max_len_extend, sm_scale, logit_cap, is_causal, kv_splits, workspace), "extend_attention_split")
+
+
+def _extend_split(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buffer, qo_indptr, kv_indptr, kv_indices,
+                  max_len_extend, sm_scale, logit_cap, is_causal, kv_splits, workspace) -> int:
     T, Hq, D = q_extend.shape
     Hkv, Dv = v_extend.shape[1], v_extend.shape[2]
     B = qo_indptr.shape[0] - 1
@@ -434,14 +433,14 @@ def extend_attention_split(q_extend, k_extend, v_extend, o_extend, k_buffer, v_b
         workspace = torch.empty(need // 4, dtype=torch.float32, device=q_extend.device)
     elif workspace.numel() * workspace.element_size() < need:
         raise SglkError(f"extend_attention_split: workspace too small ({need} bytes needed)")
-    check(lib().sglk_extend_attention_split(
+    return lib().sglk_extend_attention_split(
         _ptr(q_extend), _ptr(k_extend), _ptr(v_extend), _ptr(o_extend), _ptr(k_buffer), _ptr(v_buffer),
         _ptr(qo_indptr), _ptr(kv_indptr), _ptr(kv_indices), B, Hq, Hkv, D, Dv,
         q_extend.stride(0), q_extend.stride(1), k_extend.stride(0), k_extend.stride(1),
         v_extend.stride(0), v_extend.stride(1), o_extend.stride(0), o_extend.stride(1),
         k_buffer.stride(0), k_buffer.stride(1), v_buffer.stride(0), v_buffer.stride(1),
         int(max_len_extend), float(sm_scale), float(logit_cap), 1 if is_causal else 0, int(kv_splits), _ptr(workspace), T,
-        _attn_dtype(q_extend, k_buffer, v_buffer), _stream(q_extend)), "extend_attention_split")
+        _attn_dtype(q_extend, k_buffer, v_buffer), _stream(q_extend))
 
 
 # ------------------------------------------------------------------------------------------- A3
