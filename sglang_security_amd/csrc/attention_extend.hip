@@ -9,6 +9,7 @@
 // size 128 runs extend_attention_kv8: one block per (sequence, query head, 64 query rows); the four waves share every
 // 32-token K/V tile through LDS, widened on the way in, and each multiplies it against 16 query rows on the matrix
 // cores.  Everything else takes a wave-per-(query row, head) kernel.
+#include <algorithm>
 #include <type_traits>
 
 #include "attention_tile.h"
@@ -310,11 +311,11 @@ static int extend_attention_impl(const void* q_extend, const void* k_extend, con
   const int64_t row_blocks = ((int64_t)max_extend_len * (Hq / Hkv) + kExtRows - 1) / kExtRows;
   auto row32 = [](int64_t v) { return v >= 0 && v < (1ll << 31); };  // twice that, in bytes, fits 32 bits
   const int64_t span = D == 64 ? 32 : 1;  // head size 64 adds up to 32 rows of new tokens in 32 bits
-  const bool tile = rows_ok && kvf == 0 && (D == 128 || D == 64) && row_blocks <= 65535 && (int64_t)Hkv * B < (1ll << 31) &&
+  const bool tile = rows_ok && kvf == 0 && (D == 128 || D == 64) && row_blocks < (1 << 24) - 65536 && (int64_t)Hkv * B < (1ll << 31) &&
                     row32(k_stride_n) && row32(v_stride_n) && row32(span * ke_stride_t) && row32(span * ve_stride_t);
   const bool fast8 = rows_ok && kvf != 0 && D == 128;
-  // strides or row counts past the tile kernel's 32-bit range: not split, whole rows on the kernel below
-  if (!tile && !paged && rows_ok && kvf == 0 && (D == 128 || D == 64)) kv_splits = 1;
+  // strides or row counts past the tile kernel's 32-bit range, or past one dimension of a grid: not split
+  if ((!tile || row_blocks > 65535) && !paged && rows_ok && kvf == 0 && (D == 128 || D == 64)) kv_splits = 1;
   if (kv_splits > 1 && (!(tile || fast8) || paged))
     return fail(SGLK_EUNSUP, "extend_attention_split: 16-bit types with head size 64 or 128 (an fp8 pool: 128) and contiguous new tokens only");
   float* part_o = kv_splits > 1 ? split_ws : nullptr;
@@ -327,7 +328,8 @@ static int extend_attention_impl(const void* q_extend, const void* k_extend, con
                        (uint32_t)(2 * ve_stride_t), (uint32_t)(2 * k_stride_n), (uint32_t)(2 * v_stride_n), sm_scale, logit_cap,
                        causal, kv_splits, part_o, part_lse};
     // kv heads run fastest: with eight of them the blocks of one head share an XCD's L2
-    const dim3 grid(Hkv * B, (unsigned)row_blocks, kv_splits);
+    const unsigned gy = (unsigned)std::min<int64_t>(row_blocks, 65535);
+    const dim3 grid(Hkv * B, gy, kv_splits > 1 ? kv_splits : (unsigned)((row_blocks + gy - 1) / gy));
 #define SGLK_EXT(DV, PRE)                                                                    \
   SGLK_DISPATCH_HALF(dtype, T, {                                                             \
     if (int rc = ensure_lds<extend_tile_kernel<T, DV, PRE>>(4 * kExtTokens * 2 * DV)) return rc; \

@@ -88,8 +88,12 @@ __device__ __forceinline__ bool extend_walk(const ExtendArgs& a, const int tid, 
   const int share = a.Hq / a.Hkv;
   const int q0 = a.qo_indptr[b], ext = a.qo_indptr[b + 1] - q0;
   const int nrows = ext * share;
-  const int R0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * kExtRows;  // the rows that see most start first
-  if (R0 >= nrows) return false;                                     // block-uniform
+  // unsplit, more blocks of rows than one dimension of a grid holds go on in the next
+  const bool whole = a.kv_splits == 1;
+  const int split = whole ? 0 : blockIdx.z;
+  const int after = whole ? (gridDim.z - blockIdx.z) * gridDim.y - blockIdx.y - 1 : gridDim.y - blockIdx.y - 1;
+  const int R0 = after * kExtRows;    // the rows that see most start first
+  if (R0 >= nrows) return false;      // block-uniform
   const int lane = tid & 63, wid = tid >> 6;
   const int l31 = lane & 31, hi = lane >> 5;
   const bool paged = a.ke == nullptr;
@@ -116,7 +120,6 @@ __device__ __forceinline__ bool extend_walk(const ExtendArgs& a, const int tid, 
 
   // ranges: tokens p0 .. p1 of the index list, then tokens 0 .. e1 of the new ones
   int p0 = 0, p1 = plen, e1 = 0;
-  const int split = blockIdx.z;
   if (paged) {
     if (a.causal) p1 = min(plen, shift + b_last + 1);
   } else {

@@ -96,6 +96,22 @@ def test_split_call_past_32_bit_strides(D):
 
 
 @pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("blocks", [65535, 65536, 140000])
+def test_more_row_blocks_than_one_grid_dimension(D, blocks):
+    """A longest extend that asks for that many blocks of 128 (token, head) rows: the same kernel, so the same bits, as with
+    the true length."""
+    from sglang_security_amd import ops
+
+    q, ke, ve, kb, vb, qo, kp, ki = (t.to(DEV) for t in _case(16, 1, D, [70, 0], [150, 40], torch.bfloat16, 6))
+    got = []
+    for most in (150, blocks * 8):
+        o = torch.full_like(q, float("nan"))
+        ops.extend_attention_fwd(q, ke, ve, o, kb, vb, qo, kp, ki, None, True, None, most)
+        got.append(o)
+    assert not got[0].isnan().any() and torch.equal(*got)
+
+
+@pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("odd", ["output stride", "output start", "key stride", "pool start", "none"])
 def test_prefix_long_enough_to_split_with_any_rows(D, odd):
     """Rows that do not lie as the split form reads or writes them: the call is not split, and gives the same rows."""
