@@ -282,11 +282,11 @@ struct RowParams {
 };
 
 // Threshold of the kept set {x >= thr} for the row's filters.  kept: its mass where one filter was applied and the chosen
-// bin's elements were listed, else negative
-template <bool VEC>
+// bin's elements were listed, else negative.  FILTER: the call may have a top-k or top-p
+template <bool VEC, bool FILTER>
 __device__ float row_threshold(const float* __restrict__ x, int n, const RowParams& rp, SampShared& sh, float& kept) {
   constexpr int PER = kBins / kSampThreads;
-  const bool use_k = rp.top_k > 0 && rp.top_k < n, use_p = rp.top_p < 1.0f;
+  const bool use_k = FILTER && rp.top_k > 0 && rp.top_k < n, use_p = FILTER && rp.top_p < 1.0f;
   float thr = 0.f, vmax = 0.f;
   kept = -1.f;
   if (use_k || use_p) {
@@ -468,10 +468,10 @@ __device__ __forceinline__ void write_renormed(const float* __restrict__ x, floa
   }
 }
 
-template <bool VEC>
+template <bool VEC, bool FILTER>
 __device__ void renorm_row(const float* __restrict__ x, float* __restrict__ o, int n, const RowParams& rp, SampShared& sh) {
   float kept;
-  const float thr = row_threshold<VEC>(x, n, rp, sh, kept);
+  const float thr = row_threshold<VEC, FILTER>(x, n, rp, sh, kept);
   if (!(kept > 0.f)) {
     float s = 0.f;
     each<VEC>(x, n, [&](float v) { s += v >= thr ? v : 0.f; });
@@ -524,35 +524,14 @@ __device__ __forceinline__ void sum_chunks(const float* __restrict__ x, int n, f
   }
 }
 
-// Inverse CDF over the kept elements in index order: the first kept index whose running sum exceeds u * total.  The
-// chunks' masses stand in sh.chunk (zeros behind the last); the chunk that holds the target is walked by one wave.
+// Inverse CDF over the kept elements in index order: the first kept index whose running sum exceeds u * total.  One wave
+// walks the chunk that holds the target from the mass in front of it; c < 0: none does.
 template <bool VEC>
-__device__ void choose(const float* __restrict__ x, int n, float thr, int64_t chunk, float u, int32_t* __restrict__ out, SampShared& sh) {
+__device__ void walk_chunk(const float* __restrict__ x, int n, float thr, int64_t chunk, int c, float run, float target,
+                           int32_t* __restrict__ out) {
   const int lane = threadIdx.x & 63;
-  if (threadIdx.x == 0) sh.pick = kBins;
-  __syncthreads();
-  constexpr int PER = kBins / kSampThreads;
-  float m[PER], own = 0.f, total;
-#pragma unroll
-  for (int j = 0; j < PER; ++j) own += m[j] = sh.chunk[threadIdx.x * PER + j];
-  float run = bscan<float>(own, sh.red, total);
-  const float target = u * total;
-  int first = kBins;
-  float at_first = 0.f;
-#pragma unroll
-  for (int j = 0; j < PER; ++j) {
-    if (m[j] > 0.f && first == kBins && target < run + m[j]) first = threadIdx.x * PER + j, at_first = run;
-    run += m[j];
-  }
-  if (first < kBins) atomicMin(&sh.pick, first);
-  __syncthreads();
-  const int c = sh.pick;
-  if (c == first && first < kBins) sh.red[0] = at_first;
-  __syncthreads();
-  if (threadIdx.x >= 64) return;
   int pick = -1;
-  if (c < kBins) {
-    run = sh.red[0];
+  if (c >= 0) {
     int last = -1;
     for (int64_t i = c * chunk; i < (c + 1) * chunk && pick < 0; i += 256) {
       const float4v v = kept_four<VEC>(x, n, i + 4 * lane, thr);
@@ -594,10 +573,37 @@ __device__ void choose(const float* __restrict__ x, int n, float thr, int64_t ch
   }
 }
 
+// The chunks' masses stand in sh.chunk (zeros behind the last).
 template <bool VEC>
+__device__ void choose(const float* __restrict__ x, int n, float thr, int64_t chunk, float u, int32_t* __restrict__ out, SampShared& sh) {
+  if (threadIdx.x == 0) sh.pick = kBins;
+  __syncthreads();
+  constexpr int PER = kBins / kSampThreads;
+  float m[PER], own = 0.f, total;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) own += m[j] = sh.chunk[threadIdx.x * PER + j];
+  float run = bscan<float>(own, sh.red, total);
+  const float target = u * total;
+  int first = kBins;
+  float at_first = 0.f;
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    if (m[j] > 0.f && first == kBins && target < run + m[j]) first = threadIdx.x * PER + j, at_first = run;
+    run += m[j];
+  }
+  if (first < kBins) atomicMin(&sh.pick, first);
+  __syncthreads();
+  const int c = sh.pick;
+  if (c == first && first < kBins) sh.red[0] = at_first;
+  __syncthreads();
+  if (threadIdx.x >= 64) return;
+  walk_chunk<VEC>(x, n, thr, chunk, c < kBins ? c : -1, sh.red[0], target, out);
+}
+
+template <bool VEC, bool FILTER>
 __device__ void sample_row(const float* __restrict__ x, int n, const RowParams& rp, float u, int32_t* __restrict__ out, SampShared& sh) {
   float kept;
-  const float thr = row_threshold<VEC>(x, n, rp, sh, kept);
+  const float thr = row_threshold<VEC, FILTER>(x, n, rp, sh, kept);
   const int64_t chunk = chunk_of(n);
   __syncthreads();
   for (int i = threadIdx.x; i < kBins; i += kSampThreads) sh.chunk[i] = 0.f;
@@ -632,17 +638,77 @@ __device__ __forceinline__ RowParams load_params(const SampArgs& a, int row) {
   return rp;
 }
 
-// one block per row
-template <bool VEC>
+// One block per row.  Calls without a top-k or top-p have a kernel of their own: the selection's 128 registers leave room for
+// one block a unit (512 rows of 4096, sampling without a filter: 17 us with them, 8.3 without).
+template <bool VEC, bool FILTER>
 __global__ void __launch_bounds__(kSampThreads) filter_rows_kernel(SampArgs a) {
   __shared__ SampShared sh;
   const int row = blockIdx.x;
   const float* x = a.probs + (int64_t)row * a.in_stride;
   const RowParams rp = load_params(a, row);
   if (a.out)
-    renorm_row<VEC>(x, a.out + (int64_t)row * a.out_stride, a.n, rp, sh);
+    renorm_row<VEC, FILTER>(x, a.out + (int64_t)row * a.out_stride, a.n, rp, sh);
   else
-    sample_row<VEC>(x, a.n, rp, a.uniform[row], a.ids + row, sh);
+    sample_row<VEC, FILTER>(x, a.n, rp, a.uniform[row], a.ids + row, sh);
+}
+
+// Short rows without a selection: a block of four waves, a chunk of 256 elements a wave at a time, the choice by one wave of
+// a lane a chunk.  Such a row is a handful of loads, and what a block of 1024 threads starts, clears and meets for is most of
+// its launch (sampling without a filter, 1024 threads and 256: 512 rows of 4096 8.5 and 5.0 us, with a min-p 11.2 and 5.9;
+// one row 5.8 and 4.2.  From 16384 elements on four waves are too few for a row: 64 rows 7.4 and 8.3 us).
+constexpr int kShort = 8192;
+template <bool VEC>
+__global__ void __launch_bounds__(256) short_rows_kernel(SampArgs a) {
+  __shared__ float chunk[64], red[4];
+  const int row = blockIdx.x, lane = threadIdx.x & 63, wid = threadIdx.x >> 6, n = a.n, chunks = (n + 255) / 256;
+  const float* x = a.probs + (int64_t)row * a.in_stride;
+  const float min_p = load_params(a, row).min_p;
+  float thr = 0.f;
+  if (threadIdx.x < 64) chunk[threadIdx.x] = 0.f;
+  if (min_p > 0.f) {  // block-uniform
+    float mx = 0.f;
+    for (int c0 = wid; c0 < chunks; c0 += 16) {
+      float4v v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = kept_four<VEC>(x, n, (c0 + 4 * j) * 256 + 4 * lane, 0.f);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) mx = fmaxf(fmaxf(mx, fmaxf(v[j][0], v[j][1])), fmaxf(v[j][2], v[j][3]));
+    }
+    mx = wave_max(mx);
+    if (lane == 0) red[wid] = mx;
+  }
+  __syncthreads();
+  if (min_p > 0.f) thr = fmaxf(0.f, min_p * fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
+  for (int c0 = wid; c0 < chunks; c0 += 16) {
+    float4v v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = kept_four<VEC>(x, n, (c0 + 4 * j) * 256 + 4 * lane, thr);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float sum = wave_sum((v[j][0] + v[j][1]) + (v[j][2] + v[j][3]));
+      if (lane == 0 && c0 + 4 * j < chunks) chunk[c0 + 4 * j] = sum;
+    }
+  }
+  __syncthreads();
+  const float m = chunk[lane];
+  float incl = m;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const float w = __shfl_up(incl, o, 64);
+    if (lane >= o) incl += w;
+  }
+  const float total = __shfl(incl, 63, 64);
+  if (a.out) {
+    float* o = a.out + (int64_t)row * a.out_stride;
+    const float inv = 1.0f / total;
+    for (int i = threadIdx.x; i < n; i += 256) o[i] = x[i] >= thr ? x[i] * inv : 0.f;
+    return;
+  }
+  if (wid) return;
+  const float target = a.uniform[row] * total;
+  const u64 past = __ballot(m > 0.f && target < incl);
+  const int c = past ? __ffsll(past) - 1 : -1;
+  walk_chunk<VEC>(x, n, thr, 256, c, __shfl(incl - m, max(c, 0), 64), target, a.ids + row);
 }
 
 // ---- rows spread over several blocks --------------------------------------------------------------------------------
@@ -892,9 +958,9 @@ __global__ void __launch_bounds__(kSampThreads) slice_choose_kernel(SampArgs a) 
   if (!w.state->valid) {
     const RowParams rp = load_params(a, row);
     if (a.out)
-      renorm_row<VEC>(x, a.out + (int64_t)row * a.out_stride, a.n, rp, sh);
+      renorm_row<VEC, true>(x, a.out + (int64_t)row * a.out_stride, a.n, rp, sh);
     else
-      sample_row<VEC>(x, a.n, rp, a.uniform[row], a.ids + row, sh);
+      sample_row<VEC, true>(x, a.n, rp, a.uniform[row], a.ids + row, sh);
     return;
   }
   if (a.out) return;
@@ -917,10 +983,21 @@ static int launch_filters(SampArgs a, int batch, void* workspace, int64_t worksp
   hipStream_t s = (hipStream_t)stream;
   const bool vec = aligned16(a.probs) && a.in_stride % 4 == 0 && (!a.out || (aligned16(a.out) && a.out_stride % 4 == 0));
   const bool both_in_turn = !a.joint && (a.k_arr || a.k_val > 0) && (a.p_arr || a.p_val < 1.f);  // top-p over the k largest
+  const bool filter = a.k_arr || (a.k_val > 0 && a.k_val < a.n) || a.p_arr || a.p_val < 1.f;
   a.slices = samp_slices(batch, a.n);
-  if (a.slices < 2 || both_in_turn || batch > 65535 || !workspace || (reinterpret_cast<uintptr_t>(workspace) & 15) ||
+  // Without a selection to share out, one block a row is the faster one up to 65536 elements (sampling, spread and not: 64
+  // rows of 32000 16.5 and 9.7 us, of 65536 19.2 and 14.4, of 128256 23.5 and 25.2; one row 14.5 and 9.1, 15.3 and 12.6,
+  // 15.8 and 20.5).
+  if (a.slices < 2 || (!filter && a.n <= 65536) || both_in_turn || batch > 65535 || !workspace || (reinterpret_cast<uintptr_t>(workspace) & 15) ||
       workspace_bytes < samp_ws_row(a.slices) * batch) {
-    hipLaunchKernelGGL(vec ? filter_rows_kernel<true> : filter_rows_kernel<false>, dim3(batch), dim3(kSampThreads), 0, s, a);
+    if (!filter && a.n <= kShort) {
+      hipLaunchKernelGGL(vec ? short_rows_kernel<true> : short_rows_kernel<false>, dim3(batch), dim3(256), 0, s, a);
+      SGLK_LAUNCH_CHECK();
+      return SGLK_OK;
+    }
+    const auto kernel = filter ? (vec ? filter_rows_kernel<true, true> : filter_rows_kernel<false, true>)
+                               : (vec ? filter_rows_kernel<true, false> : filter_rows_kernel<false, false>);
+    hipLaunchKernelGGL(kernel, dim3(batch), dim3(kSampThreads), 0, s, a);
     SGLK_LAUNCH_CHECK();
     return SGLK_OK;
   }

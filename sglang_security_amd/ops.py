@@ -1404,8 +1404,10 @@ def _per_row(v, batch, dtype, name):
     return None, v
 
 
-def _filter_workspace(probs):
-    """(tensor or None, bytes): rows spread over several blocks meet there."""
+def _filter_workspace(probs, filtered=True):
+    """(tensor or None, bytes): rows spread over several blocks meet there.  Rows that never are do not ask (1 us of 9 a call)."""
+    if probs.shape[1] < 16384 or (not filtered and probs.shape[1] <= 65536):
+        return None, 0
     need = int(lib().sglk_sampling_workspace_bytes(probs.shape[0], probs.shape[1]))
     return (torch.empty(need, dtype=torch.uint8, device=probs.device) if need else None), need
 
@@ -1440,7 +1442,7 @@ def sampling_from_probs(probs, uniform, top_k=0, top_p=1.0, min_p=0.0, joint=Tru
     pa, pv = _per_row(top_p, B, torch.float32, "sampling_from_probs")
     ma, mv = _per_row(min_p, B, torch.float32, "sampling_from_probs")
     out = torch.empty(B, dtype=torch.int32, device=probs.device)
-    ws, need = _filter_workspace(probs)
+    ws, need = _filter_workspace(probs, ka is not None or kv > 0 or pa is not None or pv < 1.0)
     check(lib().sglk_sampling_from_probs_ws(_ptr(probs), _ptr(uniform), _ptr(out), _ptr(ka), int(kv), _ptr(pa), float(pv),
                                             _ptr(ma), float(mv), 1 if joint else 0, B, V, probs.stride(0), _ptr(ws), need,
                                             _stream(probs)), "sampling_from_probs")

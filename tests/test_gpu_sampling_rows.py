@@ -72,6 +72,35 @@ def test_kept_sets(kind, n, scale):
                     assert cum[i] >= u - 1e-5 and (i == 0 or cum[i - 1] <= u + 1e-5)
 
 
+@pytest.mark.parametrize("n", [1, 3, 255, 4099, 8192, 8193, 65536, 65537])
+@pytest.mark.parametrize("B", [5, 300])
+@pytest.mark.parametrize("min_p", [0.0, 0.5])
+def test_rows_without_top_k_and_top_p(n, B, min_p):
+    """The kernel without a selection, and the spread rows: multiples of 2^-10, so every mass is exact."""
+    import sglang_security_amd.sgl_kernel as sk
+    from sglang_security_amd import ops
+
+    g = torch.Generator().manual_seed(n + B)
+    x = torch.randint(0, 9, (B, n), generator=g).float()
+    x[:, n // 2] = 8.0
+    u = torch.randint(0, 1024, (B,), generator=g) / 1024
+    kept = torch.where(x >= min_p * 8, x, 0.0).double()
+    cum = kept.cumsum(1)
+    wide = torch.zeros(B, n + 5, device=DEV)
+    wide[:, 1: n + 1] = x.to(DEV) / 1024
+    aligned = torch.zeros(B, (n + 3) // 4 * 4, device=DEV)
+    aligned[:, :n] = x.to(DEV) / 1024
+    for rows in (wide[:, 1: n + 1], aligned[:, :n]):
+        ids = ops.sampling_from_probs(rows, u.to(DEV), 0, 1.0, min_p).cpu().long()
+        target = u.double() * cum[:, -1]                # the product is rounded once to fp32
+        assert (kept.gather(1, ids[:, None]) > 0).all()
+        at = cum.gather(1, ids[:, None])[:, 0]
+        assert (at * (1 + 2.0**-23) >= target).all()
+        assert (((at - kept.gather(1, ids[:, None])[:, 0]) * (1 - 2.0**-23)) <= target).all()
+        got = sk.top_p_renorm_probs(rows, 1.0).cpu().double()
+        assert torch.allclose(got, x.double() / x.double().sum(1, keepdim=True), rtol=1e-6, atol=0)
+
+
 def test_rows_without_mass():
     """All zeros, and values that are not numbers or negative beside one that is."""
     from sglang_security_amd import ops
