@@ -53,6 +53,7 @@ struct ExtendArgs {
   uint32_t ke_row, ve_row, kb_row, vb_row;  // bytes from row to row (below 2^32: one 32 x 32 + 64-bit product an address)
   float sm_scale, logit_cap;
   int causal, kv_splits;
+  int last_block, z_blocks;  // of rows, over the grid's second dimension and, unsplit, its third (blocks a step of it has, else 0)
   float *part_o, *part_lse;  // kv_splits > 1: [T, Hq, kv_splits, D] and [T, Hq, kv_splits]
 };
 
@@ -88,12 +89,9 @@ __device__ __forceinline__ bool extend_walk(const ExtendArgs& a, const int tid, 
   const int share = a.Hq / a.Hkv;
   const int q0 = a.qo_indptr[b], ext = a.qo_indptr[b + 1] - q0;
   const int nrows = ext * share;
-  // unsplit, more blocks of rows than one dimension of a grid holds go on in the next
-  const bool whole = a.kv_splits == 1;
-  const int split = whole ? 0 : blockIdx.z;
-  const int after = whole ? (gridDim.z - blockIdx.z) * gridDim.y - blockIdx.y - 1 : gridDim.y - blockIdx.y - 1;
-  const int R0 = after * kExtRows;    // the rows that see most start first
-  if (R0 >= nrows) return false;      // block-uniform
+  const int split = a.z_blocks ? 0 : blockIdx.z;
+  const int R0 = (a.last_block - (int)blockIdx.y - a.z_blocks * (int)blockIdx.z) * kExtRows;  // the rows that see most start first
+  if (R0 >= nrows) return false;  // block-uniform
   const int lane = tid & 63, wid = tid >> 6;
   const int l31 = lane & 31, hi = lane >> 5;
   const bool paged = a.ke == nullptr;
