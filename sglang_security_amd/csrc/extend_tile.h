@@ -10,7 +10,9 @@
 // Bound: the matrix pipe and the LDS share the tile evenly (64 tokens x 128 rows: 1024 matrix cycles per SIMD, 32 KiB
 // written and 128 KiB read), with the exponentials of the co-resident block in between: two blocks per CU.  Head size 64
 // carries its probabilities as the sum of two 16-bit numbers (the wave-per-row kernel it replaces kept them in fp32:
-// 0.00166 off the 64-bit result both, 0.0023 with one number); head size 128 rounds them once, as before.
+// 0.00166 off the 64-bit result both, 0.0023 with one number); head size 128 rounds them once and divides by the sum of the
+// rounded ones, whose errors cancel in part (700 tokens, 32 / 8 heads: 0.00196 off; 0.00198 over the sum of the others, and
+// 0.00197 with that on tiles of 32 tokens, which had more probabilities of exactly one).
 //
 // Measured (bf16, launch alone): 8 prompts of 768 to 1152 tokens, 32 / 8 heads of 128: 264 us (one block per 64 rows of
 // one head, 32-token tiles on 16x16x32) -> 124 us, 525 TFLOP/s; one prompt of 1152 tokens: 69 -> 36 us; 128 tokens over
@@ -38,6 +40,20 @@ struct Mfma32<f16_t> {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0, 0);
   }
 };
+
+// acc + the two numbers of a word
+template <typename T>
+__device__ __forceinline__ float add_pair(short lo, short hi, float acc) {
+  typedef short short2v __attribute__((ext_vector_type(2)));
+  const short2v v = {lo, hi};
+  if constexpr (std::is_same<T, bf16_t>::value) {
+    typedef __bf16 two __attribute__((ext_vector_type(2)));
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(two, v), two{(__bf16)1.f, (__bf16)1.f}, acc, false);
+  } else {
+    typedef _Float16 two __attribute__((ext_vector_type(2)));
+    return __builtin_amdgcn_fdot2(__builtin_bit_cast(two, v), two{(_Float16)1.f, (_Float16)1.f}, acc, false);
+  }
+}
 
 template <typename T>
 struct Special {  // the type's infinity and one
@@ -283,7 +299,7 @@ __device__ __forceinline__ bool extend_walk(const ExtendArgs& a, const int tid, 
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
         const float p = __builtin_amdgcn_exp2f(fmaf(s[u][r], c, -m_use));
-        psum += p;
+        if constexpr (P2) psum += p;
         if constexpr (CAREFUL) {
           s[u][r] = p;
           continue;
@@ -292,6 +308,12 @@ __device__ __forceinline__ bool extend_walk(const ExtendArgs& a, const int tid, 
         pf[2 * u + (r >> 3)][r & 7] = (short)ph;
         if constexpr (P2) pl[2 * u + (r >> 3)][r & 7] = (short)Conv<T>::from_f32(p - Conv<T>::to_f32(ph));
       }
+    // two rounded probabilities an instruction, added as exactly as one
+    if constexpr (!P2 && !CAREFUL)
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int e = 0; e < 8; e += 2) psum = add_pair<T>(pf[k][e], pf[k][e + 1], psum);
     lsum += psum;
     if constexpr (CAREFUL) {
       // A value that is not finite counts as zero in the product; two more products count those of a row's 16 tokens on
@@ -318,6 +340,9 @@ __device__ __forceinline__ bool extend_walk(const ExtendArgs& a, const int tid, 
           on[e] = (short)(p == 0.f ? 0 : seen);
           off[e] = (short)(p == 0.f ? seen : 0);
         }
+        if constexpr (!P2)
+#pragma unroll
+          for (int e = 0; e < 8; e += 2) lsum = add_pair<T>(hp[e], hp[e + 1], lsum);
 #pragma unroll
         for (int n = 0; n < NV; ++n) {
           __builtin_amdgcn_sched_barrier(0);
