@@ -293,7 +293,9 @@ SGLK_API int sglk_extend_attention_masked(const void* q_extend, const void* k_ex
  * request extending a short tail over a long cached prefix, the shape of a radix-cache hit -- where one block per pair
  * leaves most of the chip idle and walks the whole prefix serially.  No counterpart in the reference, whose kernel
  * walks the prefix once per query block (extend_attention.py:96-210); same result within fp tolerance (the merge is
- * merge_state arithmetic in split order).  16-bit types, head size 128, contiguous new tokens, no mask.
+ * merge_state arithmetic in split order).  16-bit types, head sizes 64 and 128 (an fp8 pool: 128), rows aligned as the tile
+ * kernels read and write them (q, k, v and a 16-bit pool by 16 bytes, the output and an fp8 pool by 8), contiguous new
+ * tokens, no mask; SGLK_EUNSUP otherwise, with nothing launched.
  * workspace: sglk_extend_attention_split_workspace_bytes(total_rows, Hq, kv_splits) bytes, 16-byte aligned, where
  * total_rows = qo_indptr[B] (the number of query rows); kv_splits == 1 is sglk_extend_attention. */
 SGLK_API int64_t sglk_extend_attention_split_workspace_bytes(int64_t total_rows, int Hq, int kv_splits);
@@ -831,7 +833,8 @@ SGLK_API int sglk_sampling_from_probs(const float* probs, const float* uniform, 
                                       int vocab, int64_t in_stride, void* stream);
 /* The same with a caller's workspace (16-byte aligned, contents of no matter before and after;
  * sglk_sampling_workspace_bytes(batch, vocab), 0 where it would not be used): rows are spread over several blocks in
- * four launches.  Without one, or a smaller one, every row is one block's. */
+ * four launches.  Without one, or a smaller one, or where no top-k or top-p is given and rows are short, every row is
+ * one block's. */
 SGLK_API int64_t sglk_sampling_workspace_bytes(int batch, int vocab);
 SGLK_API int sglk_top_k_renorm_probs_ws(const float* probs, float* out, const int32_t* top_k_arr,
                                         int top_k_val, int batch, int vocab, int64_t in_stride,

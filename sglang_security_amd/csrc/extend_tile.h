@@ -7,8 +7,9 @@
 // exchange between the two half waves, and the same registers, rounded, are the P^T operand of O^T += V^T . P^T (the
 // order of the tokens inside a k-step is free as long as V is read in the same order).
 //
-// Bound: the matrix pipe and the LDS share the tile evenly (64 tokens x 128 rows: 1024 matrix cycles per SIMD, 32 KiB
-// written and 128 KiB read), with the exponentials of the co-resident block in between: two blocks per CU.  Head size 64
+// Bound: the issue port.  A tile of 64 tokens x 128 rows is 1024 matrix cycles per SIMD beside 32 KiB written to and 128 KiB
+// read from the LDS, but the matrix pipe is busy a third of the time (counters; no bank conflicts): maxima, exponentials and
+// conversions stand between the products, and two blocks per CU do not hide them.  Head size 64
 // carries its probabilities as the sum of two 16-bit numbers (the wave-per-row kernel it replaces kept them in fp32:
 // 0.00166 off the 64-bit result both, 0.0023 with one number); head size 128 rounds them once and divides by the sum of the
 // rounded ones, whose errors cancel in part (700 tokens, 32 / 8 heads: 0.00196 off; 0.00198 over the sum of the others, and

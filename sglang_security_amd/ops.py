@@ -404,8 +404,9 @@ def extend_attention_fwd(q_extend, k_extend, v_extend, o_extend, k_buffer, v_buf
 
 
 def extend_attention_split_plan(T, Hq, B, max_len_extend, total_prefix, head_dim, dtype) -> int:
-    """How many ways to split the cached prefix (1 = the plain kernel): only where one block per (sequence, query block,
-    head) would leave most CUs without work and the prefixes are long enough to be worth a merge launch."""
+    """How many ways to split the cached prefix (1 = the plain kernel): only where few rows would leave most CUs without work
+    and the prefixes are long enough to be worth a merge launch.  Counted in blocks of 64 tokens a head, as the fp8-pool
+    kernel has them; the 16-bit kernel's are 128 (token, head) rows of a kv head, half as many or fewer."""
     if head_dim not in (64, 128) or dtype not in (torch.float16, torch.bfloat16) or B <= 0 or total_prefix <= 0:
         return 1
     blocks = ((int(max_len_extend) + 63) // 64) * Hq * B
