@@ -432,6 +432,9 @@ SGLK_API int sglk_gptq_repack(const int32_t* qweight, const int32_t* qzeros, int
  * (for the prefill path once the reference-layout qweight has been dropped).  K % 128 == 0, N % 16 == 0. */
 SGLK_API int sglk_awq_dequantize_packed(const int32_t* packed, const void* scales, const int32_t* qzeros,
                                         void* out, int K, int N, int group_size, int dtype, void* stream);
+/* the same values transposed: out [N, K], the operand a library product reads contiguously along K; 16-byte aligned */
+SGLK_API int sglk_awq_dequantize_packed_nk(const int32_t* packed, const void* scales, const int32_t* qzeros,
+                                           void* out, int K, int N, int group_size, int dtype, void* stream);
 
 /* out[M,N] = x[M,K] @ dequant(W) (+bias) with the int4 weights dequantised in registers and fed to
  * the matrix cores; W in the sglk_awq_repack layout.  Fuses AWQLinearMethod.apply,

@@ -219,6 +219,48 @@ __global__ void __launch_bounds__(256) awq_dequant_packed_tile_kernel(const int3
   }
 }
 
+// The same as W^T [N, K]: what a library product reads fastest, both operands contiguous along K.  A packed word holds
+// eight consecutive k of a column, so it becomes one 16-byte store without a transposition: a wave takes a strip of 16 columns
+// and 128 k, four columns an instruction, a column's 256 bytes from 16 adjacent lanes; a block's four waves take
+// neighbouring k groups (1 KiB of a row).  Bound by its writes.
+template <typename T>
+__global__ void __launch_bounds__(256) awq_dequant_packed_nk_kernel(const int32_t* __restrict__ packed,
+                                                                    const uint16_t* __restrict__ scales,
+                                                                    const int32_t* __restrict__ qzeros,
+                                                                    uint16_t* __restrict__ out, int K, int N,
+                                                                    int group_size) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int nstrips = N / 16, qcols = N / 8, kblocks = K / 128, kchunks = (kblocks + 3) / 4;
+  const int64_t jobs = (int64_t)kchunks * nstrips;
+  const int oct = lane & 15;  // k octet of the tile: its word is piece oct >> 2 of lane group oct & 3
+  for (int64_t job = blockIdx.x; job < jobs; job += gridDim.x) {
+    const int nb = (int)(job / kchunks), kb = (int)(job % kchunks) * 4 + wid;
+    if (kb >= kblocks) continue;
+    const int32_t* tile = packed + ((int64_t)kb * nstrips + nb) * 256;
+    const int k0 = 128 * kb + 8 * oct, gq = k0 / group_size;
+    uint32_t w[4], z[4];
+    float s[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int i = 4 * t + (lane >> 4), n = 16 * nb + i;
+      w[t] = (uint32_t)tile[((oct & 3) * 16 + i) * 4 + (oct >> 2)];
+      z[t] = ((uint32_t)qzeros[(int64_t)gq * qcols + (n >> 3)] >> (4 * kAwqOrd[n & 7])) & 0xF;
+      s[t] = Conv<T>::to_f32(scales[(int64_t)gq * N + n]);
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int n = 16 * nb + 4 * t + (lane >> 4);
+      int4v o;
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {  // nibbles e / 2 and e / 2 + 4
+        const float v0 = (float)((int)((w[t] >> (2 * e)) & 0xF) - (int)z[t]) * s[t];
+        const float v1 = (float)((int)((w[t] >> (2 * e + 16)) & 0xF) - (int)z[t]) * s[t];
+        o[e >> 1] = (int)((uint32_t)Conv<T>::from_f32(v0) | ((uint32_t)Conv<T>::from_f32(v1) << 16));
+      }
+      *reinterpret_cast<int4v*>(out + (int64_t)n * K + k0) = o;
+    }
+  }
+}
 
 // x tile in LDS: 16-byte chunk c of row r at slot c ^ (r & 15) (conflict-free row reads, as the K tile
 // of the attention kernel)
@@ -1518,6 +1560,21 @@ int sglk_awq_dequantize_packed(const int32_t* packed, const void* scales, const 
   if (blocks > 16384) blocks = 16384;
   SGLK_DISPATCH_HALF(dtype, T,
                      hipLaunchKernelGGL((awq_dequant_packed_kernel<T>), dim3(blocks), dim3(256), 0, (hipStream_t)stream,
+                                        packed, (const uint16_t*)scales, qzeros, (uint16_t*)out, K, N, group_size));
+  SGLK_LAUNCH_CHECK();
+  return SGLK_OK;
+}
+
+int sglk_awq_dequantize_packed_nk(const int32_t* packed, const void* scales, const int32_t* qzeros, void* out, int K, int N,
+                                  int group_size, int dtype, void* stream) {
+  SGLK_CHECK(packed && scales && qzeros && out, "awq_dequantize_packed_nk: null pointer");
+  SGLK_CHECK(K > 0 && N > 0 && K % 128 == 0 && N % 16 == 0, "awq_dequantize_packed_nk: K %% 128 and N %% 16 must be 0");
+  SGLK_CHECK(group_size > 0 && K % group_size == 0 && group_size % 8 == 0, "awq_dequantize_packed_nk: bad group size");
+  SGLK_CHECK(aligned16(out), "awq_dequantize_packed_nk: out must be 16-byte aligned");
+  const int64_t jobs = (int64_t)((K / 128 + 3) / 4) * (N / 16);
+  const int blocks = (int)(jobs < 16384 ? jobs : 16384);
+  SGLK_DISPATCH_HALF(dtype, T,
+                     hipLaunchKernelGGL((awq_dequant_packed_nk_kernel<T>), dim3(blocks), dim3(256), 0, (hipStream_t)stream,
                                         packed, (const uint16_t*)scales, qzeros, (uint16_t*)out, K, N, group_size));
   SGLK_LAUNCH_CHECK();
   return SGLK_OK;

@@ -610,6 +610,20 @@ def awq_dequantize_packed(packed, scales, qzeros, out=None):
     return out
 
 
+def awq_dequantize_packed_nk(packed, scales, qzeros, out=None):
+    """The values of awq_dequantize_packed as W^T [N, K]: x @ out.t() is the product that the library runs fastest."""
+    _need_gpu(packed, scales, qzeros)
+    K, N = packed.shape[0], packed.shape[1] * 8
+    group = K // scales.shape[0]
+    if out is None:
+        out = torch.empty((N, K), dtype=scales.dtype, device=packed.device)
+    elif out.shape != (N, K) or out.dtype != scales.dtype or not out.is_contiguous() or out.device != packed.device:
+        raise SglkError("awq_dequantize_packed_nk: out must be a contiguous [N, K] tensor of the scale dtype")
+    check(lib().sglk_awq_dequantize_packed_nk(_ptr(packed), _ptr(scales), _ptr(qzeros), _ptr(out), K, N, group,
+                                              dtype_code(scales.dtype), _stream(packed)), "awq_dequantize_packed_nk")
+    return out
+
+
 def awq_gemm_workspace_bytes(M, N, K) -> int:
     return int(lib().sglk_awq_gemm_workspace_bytes(M, N, K))
 

@@ -36,7 +36,7 @@ class LlamaPrefill:
     def __init__(self, dec: LlamaDecoder, kv_pool: MHATokenToKVPool, max_tokens: int, use_graph: bool = True,
                  resident_bf16: bool = False, prefill_gemm: str = "library", overlap_dequant: bool = False):
         """prefill_gemm: what multiplies batches of DEQUANT_GEMM_MIN_TOKENS rows or more.  "library": dequantise the
-        int4 weight (sglk_awq_dequantize_packed), then torch.matmul = hipBLASLt -- the faster of the two today;
+        int4 weight (sglk_awq_dequantize_packed_nk), then torch.matmul = hipBLASLt -- the faster of the two today;
         "fused": the hand-written tile kernels of this package (sglk_awq_gemm_prefill dequantises inside the GEMM and
         writes no dequantised copy; sglk_dense_gemm_prefill for 16-bit weights).
 
@@ -119,10 +119,10 @@ class LlamaPrefill:
                 if self.resident_bf16:
                     wd = self._dense.get(id(w))
                     if wd is None:
-                        wd = self._dense[id(w)] = ops.awq_dequantize_packed(w.packed, w.scales, w.qzeros)
+                        wd = self._dense[id(w)] = ops.awq_dequantize_packed_nk(w.packed, w.scales, w.qzeros)
                 else:
-                    wd = ops.awq_dequantize_packed(w.packed, w.scales, w.qzeros)
-                torch.matmul(x, wd, out=out)
+                    wd = ops.awq_dequantize_packed_nk(w.packed, w.scales, w.qzeros)
+                torch.matmul(x, wd.t(), out=out)
             else:
                 ops.awq_gemm(x, w.packed, w.scales, w.qzeros, None, out, self.workspace)
         elif isinstance(w, _DenseLinear):
@@ -164,7 +164,7 @@ class LlamaPrefill:
         if j >= self._RING:
             self._side.wait_event(self._free[slot])      # the product that read this buffer last
         with torch.cuda.stream(self._side):
-            ops.awq_dequantize_packed(w.packed, w.scales, w.qzeros, out=self._ring[slot][: w.K * w.N].view(w.K, w.N))
+            ops.awq_dequantize_packed_nk(w.packed, w.scales, w.qzeros, out=self._ring[slot][: w.K * w.N].view(w.N, w.K))
             self._ready[slot].record(self._side)
 
     def _pipe_matmul(self, w, x, out):
@@ -175,7 +175,7 @@ class LlamaPrefill:
         self._pipe_issue(j + 1)
         main = torch.cuda.current_stream(self.dec.device)
         main.wait_event(self._ready[slot])
-        torch.matmul(x, self._ring[slot][: w.K * w.N].view(w.K, w.N), out=out)
+        torch.matmul(x, self._ring[slot][: w.K * w.N].view(w.N, w.K).t(), out=out)
         self._free[slot].record(main)
         self._pipe = j + 1
         return out

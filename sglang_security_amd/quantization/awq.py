@@ -119,7 +119,7 @@ class AWQLinearMethod:
         if layer.qweight is not None:
             w = ops.awq_dequantize(layer.qweight, layer.scales, layer.qzeros)
         else:
-            w = ops.awq_dequantize_packed(layer.sglk_packed, layer.scales, layer.qzeros)
+            w = ops.awq_dequantize_packed_nk(layer.sglk_packed, layer.scales, layer.qzeros).t()
         out = torch.matmul(x2, w)
         if bias is not None:
             out.add_(bias)

@@ -133,7 +133,7 @@ class GPTQLinearMethod:
             out = ops.awq_gemm(x2.contiguous(), layer.sglk_packed, layer.scales, layer.sglk_zeros, bias, None,
                                self._workspace(layer, m, x.device))
             return out.reshape(out_shape)
-        out = torch.matmul(x2, ops.awq_dequantize_packed(layer.sglk_packed, layer.scales, layer.sglk_zeros))
+        out = torch.matmul(x2, ops.awq_dequantize_packed_nk(layer.sglk_packed, layer.scales, layer.sglk_zeros).t())
         if bias is not None:
             out.add_(bias)
         return out.reshape(out_shape)

@@ -383,6 +383,22 @@ def test_awq_dequantize_packed_matches_reference_layout(K, N, group, dtype):
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
 
 
+@pytest.mark.parametrize("K,N,group", [(128, 16, 8), (128, 64, 128), (384, 48, 64), (640, 112, 128), (1024, 192, 256)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_awq_dequantize_packed_nk_is_the_transpose(K, N, group, dtype):
+    """Bit for bit the transpose of awq_dequantize: fewer k groups than a block's four waves, strips that are no multiple
+    of four, groups below and above a tile's 128."""
+    from sglang_security_amd import ops
+
+    g = torch.Generator().manual_seed(K + N)
+    qw = torch.randint(-(2 ** 31), 2 ** 31 - 1, (K, N // 8), dtype=torch.int32, generator=g).to("cuda")
+    qz = torch.randint(-(2 ** 31), 2 ** 31 - 1, (K // group, N // 8), dtype=torch.int32, generator=g).to("cuda")
+    sc = (torch.rand(K // group, N, generator=g) * 0.02).to(dtype).to("cuda")
+    want = ops.awq_dequantize(qw, sc, qz)
+    got = ops.awq_dequantize_packed_nk(ops.awq_repack(qw), sc, qz)
+    assert torch.equal(got.t().contiguous().view(torch.int16), want.view(torch.int16))
+
+
 # ---------------------------------------------------------------------------------------------- large-M (prefill) GEMMs
 @pytest.mark.parametrize("M,K,N", [(256, 256, 128), (300, 512, 256), (1152, 1024, 384), (77, 4096, 128)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
