@@ -19,15 +19,11 @@
 // (triton_ops/decode_attention.py:497-557).
 #include <type_traits>
 
-#include "attention_mla.h"
+#include "latent_wave.h"
 #include "attention_tile.h"
 #include "common.h"
 
 namespace sglk {
-
-static constexpr int kMinBlockKV = 32;  // decode_attention.py:40 (_MIN_BLOCK_KV)
-
-__host__ __device__ __forceinline__ int cdiv_i(int a, int b) { return (a + b - 1) / b; }
 
 // ---------------------------------------------------------------------------------------------
 // metadata
@@ -291,27 +287,6 @@ __global__ void __launch_bounds__(64) decode_stage1_generic(
   if (lane == 0) attn_lse[ob] = m + logf(l);
 }
 
-// How many ways request b's context is split: as the caller says, or, where `fewer` names a number for that many and a batch
-// of such a mean context (64 tokens and up, by powers of two), as it says (mla_fewer_splits).  A request twice as long as
-// the mean keeps what it was given: alone in the last round, it would end the launch.
-constexpr int kMeans = 7;
-struct FewerSplits {
-  int batch;  // 0: always as the caller says
-  uint64_t pick[kMeans];  // four bits a number of splits, 1 .. 16; 0: as the caller says
-};
-__device__ __forceinline__ int splits_of(const int32_t* __restrict__ num_kv_splits, const int32_t* __restrict__ kv_indptr, int b, int len,
-                                         int max_splits, const FewerSplits& fewer) {
-  const int most = max(num_kv_splits[b], 1);
-  if (fewer.batch == 0 || most > min(max_splits, 16)) return most;
-  const float mean = (float)(kv_indptr[fewer.batch] - kv_indptr[0]) * __builtin_amdgcn_rcpf((float)fewer.batch);
-  if (!(mean >= 64.f) || (float)len > 2.f * mean) return most;
-  uint64_t picks = fewer.pick[0];
-#pragma unroll
-  for (int k = 1; k < kMeans; ++k) picks = mean < (float)(64 << k) ? picks : fewer.pick[k];
-  const int n = (int)(picks >> (4 * (most - 1))) & 15;
-  return n ? n : most;
-}
-
 // ---------------------------------------------------------------------------------------------
 // stage 2: LSE merge of the split partials (decode_attention.py:497-557)
 // ---------------------------------------------------------------------------------------------
@@ -322,12 +297,12 @@ __global__ void __launch_bounds__(128) decode_stage2(const float* __restrict__ a
                                                      const int32_t* __restrict__ num_kv_splits, int max_kv_splits,
                                                      int Hq, int Dv, int64_t o_stride_b, int64_t o_stride_h,
                                                      float* __restrict__ xsum_out, int64_t xs_stride,
-                                                     const int32_t* __restrict__ gate = nullptr, FewerSplits fewer = {}) {
+                                                     const int32_t* __restrict__ gate = nullptr) {
   __shared__ float xs_red[2];
   if (gate && *gate != 0) return;  // see decode_stage1_mfma128
   const int b = blockIdx.x, h = blockIdx.y;
   const int len = kv_indptr[b + 1] - kv_indptr[b];
-  const int splits = splits_of(num_kv_splits, kv_indptr, b, len, max_kv_splits, fewer);
+  const int splits = max(num_kv_splits[b], 1);
   const int per_split = cdiv_i(cdiv_i(len, splits), kMinBlockKV) * kMinBlockKV;
   const int64_t base = ((int64_t)b * Hq + h) * max_kv_splits;
   if (Dv % 512 == 0 && !xsum_out && (reinterpret_cast<uintptr_t>(attn_logits) & 15) == 0) {
@@ -522,7 +497,7 @@ __global__ void __launch_bounds__(256, HT == 1 ? 3 : 2) decode_stage1_mla(
     const int32_t* __restrict__ kv_indices, float* __restrict__ attn_logits, float* __restrict__ attn_lse,
     const int32_t* __restrict__ num_kv_splits, int max_kv_splits, int Hq, int Hkv, int head_tiles, int64_t q_stride_b,
     int64_t q_stride_h, int64_t k_stride_n, int64_t k_stride_h, float sm_scale, float logit_cap,
-    const int32_t* __restrict__ gate, FewerSplits fewer) {
+    const int32_t* __restrict__ gate) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   if (gate && *gate != 0) return;  // see decode_stage1_mfma128
   const int lane = threadIdx.x & 63;
@@ -533,7 +508,7 @@ __global__ void __launch_bounds__(256, HT == 1 ? 3 : 2) decode_stage1_mla(
   const int group = Hq / Hkv;
   const int start = kv_indptr[b];
   const int len = kv_indptr[b + 1] - start;
-  const int splits = splits_of(num_kv_splits, kv_indptr, b, len, max_kv_splits, fewer);
+  const int splits = max(num_kv_splits[b], 1);
   const int per_split = cdiv_i(cdiv_i(len, splits), kMinBlockKV) * kMinBlockKV;
   const int s0 = per_split * split, s1 = min(s0 + per_split, len);
   if (s1 <= s0) return;  // block-uniform
@@ -1758,34 +1733,55 @@ static int decode_attention_impl(const void* q, const void* k_buffer, const void
       });
     });
   } else if (mla) {
-    // Splits that spill the grid into a nearly empty round cost more than they spread (mla_fewer_splits).
+    // Splits that spill the grid into a nearly empty round cost more than they spread (mla_fewer_splits); the kernel of 32 heads
+    // a block folds those left into blocks (latent_plan).
     // Up to 31 heads a group the copy rate bounds the launch and a short last round is nearly free (100 requests of up to
     // 2048 tokens, 16 heads: 49.9 us with 8 splits, 51.5 with 7): there the caller's number stands.
-    if (group >= 32) {  // two tiles of 16 heads per block, two blocks a unit
-      const int head_tiles = (group + 31) / 32;
-      fewer = mla_fewer_splits(B, (int64_t)B * Hkv * head_tiles, max_kv_splits);
-      dim3 grid(B, Hkv * head_tiles, max_kv_splits);
+    const int64_t units = (int64_t)B * Hkv * ((group + 31) / 32);
+    const int64_t blocks = 8 * (int64_t)Hkv * ((group + 31) / 32) * (((int64_t)B * max_kv_splits + 7) / 8);
+    // Where every split of every request has a unit of the chip to itself the launch is a chain of trips, and a block of waves that
+    // share each tile starts and ends sooner than one of waves that meet at the end: 8 requests, 128 heads, 64 / 300 / 1152 / 4096
+    // tokens: 19.9 / 22.7 / 30.4 / 53.0 us against 21.0 / 24.4 / 29.1 / 40.7; one request 19.5 / 21.9 / 28.4 / 49.2 against
+    // 20.9 / 24.4 / 26.6 / 35.8.  (How long the requests are is not known here.)  A launch holds fewer than 2^32 threads.
+    if (units * max_kv_splits > 256 && group >= 32 && blocks < (1 << 24) && (int64_t)B * max_kv_splits < INT32_MAX) {
+      fewer = mla_fewer_splits(B, units, max_kv_splits);
+      const LatentArgs la{(const uint16_t*)q, (const uint16_t*)k_buffer, kv_indptr, kv_indices, num_kv_splits, gate, attn_logits, attn_lse, o, B, Hq,
+                          Hkv, (group + 31) / 32, max_kv_splits, q_stride_b, q_stride_h, k_stride_n, k_stride_h, o_stride_b, o_stride_h, sm_scale, logit_cap};
+      SGLK_DISPATCH_HALF(dtype, T, {
+        if (logit_cap > 0.f) {
+          if (int rc = ensure_lds<latent_decode_kernel<T, true>>(kLatLds)) return rc;
+          hipLaunchKernelGGL((latent_decode_kernel<T, true>), dim3((unsigned)blocks), dim3(256), kLatLds, s, la, fewer);
+        } else {
+          if (int rc = ensure_lds<latent_decode_kernel<T, false>>(kLatLds)) return rc;
+          hipLaunchKernelGGL((latent_decode_kernel<T, false>), dim3((unsigned)blocks), dim3(256), kLatLds, s, la, fewer);
+        }
+        SGLK_LAUNCH_CHECK();
+        hipLaunchKernelGGL((latent_merge_kernel<T>), dim3(B, (Hq + 3) / 4), dim3(256), 0, s, la, fewer);
+      });
+      SGLK_LAUNCH_CHECK();
+      return SGLK_OK;
+    }
+    const int per_block = group >= 32 ? 32 : 16;  // heads: a latent tile in LDS serves two tiles of them where there are as many
+    const int head_tiles = (group + per_block - 1) / per_block;
+    dim3 grid(B, Hkv * head_tiles, max_kv_splits);
 #define SGLK_MLA_LAUNCH(HT, CAP)                                                                                         \
   hipLaunchKernelGGL((decode_stage1_mla<T, HT, CAP>), grid, dim3(256), kMlaTileBytes + HT * kMlaScoreBytes, s, q, k_buffer, \
                      kv_indptr, kv_indices, attn_logits, attn_lse, num_kv_splits, max_kv_splits, Hq, Hkv, head_tiles,      \
-                     q_stride_b, q_stride_h, k_stride_n, k_stride_h, sm_scale, logit_cap, gate, fewer)
-      SGLK_DISPATCH_HALF(dtype, T, {
+                     q_stride_b, q_stride_h, k_stride_n, k_stride_h, sm_scale, logit_cap, gate)
+    SGLK_DISPATCH_HALF(dtype, T, {
+      if (per_block == 32) {
         if (logit_cap > 0.f)
           SGLK_MLA_LAUNCH(2, true);
         else
           SGLK_MLA_LAUNCH(2, false);
-      });
-    } else {
-      const int head_tiles = (group + 15) / 16;
-      dim3 grid(B, Hkv * head_tiles, max_kv_splits);
-      SGLK_DISPATCH_HALF(dtype, T, {
+      } else {
         if (logit_cap > 0.f)
           SGLK_MLA_LAUNCH(1, true);
         else
           SGLK_MLA_LAUNCH(1, false);
-      });
+      }
+    });
 #undef SGLK_MLA_LAUNCH
-    }
   } else if (fast) {
     const int head_tiles = (group + 15) / 16;
     dim3 grid(B, Hkv * head_tiles, (max_kv_splits + kWavesPerBlock - 1) / kWavesPerBlock);
@@ -1840,7 +1836,7 @@ static int decode_attention_impl(const void* q, const void* k_buffer, const void
   SGLK_DISPATCH_FLOAT(dtype, T,
                       hipLaunchKernelGGL((decode_stage2<T>), dim3(B, Hq), dim3(128), 0, s, attn_logits, attn_lse, o,
                                          kv_indptr, num_kv_splits, max_kv_splits, Hq, Dv, o_stride_b, o_stride_h,
-                                         xsum_out, xs_stride, gate, fewer));
+                                         xsum_out, xs_stride, gate));
   SGLK_LAUNCH_CHECK();
   return SGLK_OK;
 }
