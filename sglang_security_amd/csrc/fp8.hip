@@ -99,6 +99,42 @@ __global__ __launch_bounds__(256) void per_token_quant_kernel(const void* __rest
   }
 }
 
+// Rows of up to 16384 elements: a thread holds its NV vectors between the maximum and the codes, all requested at once (the loop
+// above reads a row twice, a trip to memory per vector).  Three launches of 4096 elements and one of 14336: 2048 rows 53.1 -> 49.6 us,
+// 64 rows 16.9 -> 15.2.
+template <typename T, int NV>
+__global__ __launch_bounds__(256) void per_token_quant_held_kernel(const void* __restrict__ x, uint8_t* __restrict__ q,
+                                                                   float* __restrict__ scales, int hidden) {
+  __shared__ float red[4];
+  const int64_t row = blockIdx.x;
+  const int64_t base = row * hidden;
+  float v[NV][8];
+  float amax = 0.f;
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[k][j] = 0.f;
+    const int i = (threadIdx.x + 256 * k) * 8;
+    if (i < hidden) load8<T>(x, base + i, v[k]);
+  }
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[k][j]));
+  amax = block_max_256(amax, red);
+  const float scale = amax / kFp8Max;
+  if (threadIdx.x == 0) scales[row] = scale;
+  const float inv = 1.0f / scale;
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const int i = (threadIdx.x + 256 * k) * 8;
+    if (i >= hidden) break;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[k][j] = clamp_sym(v[k][j] * inv, -kFp8Max, kFp8Max);
+    *reinterpret_cast<uint2*>(q + base + i) = cvt8(v[k]);
+  }
+}
+
 // ---- producers that quantise on the way out: the 16-bit tensor the plain op sequence would write in between is
 // formed (and rounded) in registers only.  One block of 1024 threads per row, up to four 8-element vectors a thread.
 __device__ __forceinline__ float block_sum_1024(float v, float* red) {
@@ -905,14 +941,24 @@ int sglk_per_token_quant_fp8(const void* x, void* q, float* scales, int64_t rows
   if (rows == 0) return SGLK_OK;
   const bool vec = hidden % 8 == 0 && aligned16(x) && ((uintptr_t)q & 7) == 0;
   hipStream_t s = (hipStream_t)stream;
+#define SGLK_HELD(NV) hipLaunchKernelGGL((per_token_quant_held_kernel<T, NV>), dim3((unsigned)rows), dim3(256), 0, s, x, (uint8_t*)q, scales, hidden)
   SGLK_DISPATCH_FLOAT(dtype, T, {
-    if (vec)
+    if (vec && hidden <= 2048)
+      SGLK_HELD(1);
+    else if (vec && hidden <= 4096)
+      SGLK_HELD(2);
+    else if (vec && hidden <= 8192)
+      SGLK_HELD(4);
+    else if (vec && hidden <= 16384)
+      SGLK_HELD(8);
+    else if (vec)
       hipLaunchKernelGGL((per_token_quant_kernel<T, true>), dim3((unsigned)rows), dim3(256), 0, s, x, (uint8_t*)q, scales,
                          hidden);
     else
       hipLaunchKernelGGL((per_token_quant_kernel<T, false>), dim3((unsigned)rows), dim3(256), 0, s, x, (uint8_t*)q,
                          scales, hidden);
   });
+#undef SGLK_HELD
   SGLK_LAUNCH_CHECK();
   return SGLK_OK;
 }

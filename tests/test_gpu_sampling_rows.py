@@ -72,6 +72,31 @@ def test_kept_sets(kind, n, scale):
                     assert cum[i] >= u - 1e-5 and (i == 0 or cum[i - 1] <= u + 1e-5)
 
 
+@pytest.mark.parametrize("B,n", [(64, 128259), (64, 163843), (100, 128259), (128, 81923), (20, 8195 * 12)])
+def test_spread_rows_around_the_held_elements(B, n):
+    """Slices of fewer elements than a block holds in registers, of just as many and of more, and a row's last three."""
+    import sglang_security_amd.sgl_kernel as sk
+    from sglang_security_amd import ops
+
+    g = torch.Generator().manual_seed(n + B)
+    x = _rows("peaked", n, g)
+    x[-2] = 2.0                                     # the last elements are kept ones
+    x = x * 2.0 ** -math.ceil(math.log2(x.sum().item()))
+    rows = torch.zeros(B, (n + 3) // 4 * 4, device=DEV)[:, :n]
+    rows[:] = x.float().to(DEV)
+    ps = torch.tensor([0.75, 0.5, 0.875, 0.9375][: 4] * (B // 4 + 1), device=DEV)[:B]
+    got = sk.top_p_renorm_probs(rows, ps).cpu().double()
+    ids = ops.sampling_from_probs(rows, torch.full((B,), 0.999999, device=DEV), 0, ps, 0.0, True).cpu().long()
+    for b in range(4):
+        kept = torch.where(x >= _threshold(x, 0, ps[b].item(), True), x, 0.0)
+        cum = kept.cumsum(0) / kept.sum()
+        for r in range(b, B, 4):
+            assert torch.equal(got[r] > 0, kept > 0)
+            assert torch.allclose(got[r], kept / kept.sum(), rtol=1e-5, atol=0)
+            i = int(ids[r])
+            assert kept[i] > 0 and cum[i] >= 0.999999 - 1e-5
+
+
 @pytest.mark.parametrize("n", [1, 3, 255, 4099, 8192, 8193, 65536, 65537])
 @pytest.mark.parametrize("B", [5, 300])
 @pytest.mark.parametrize("min_p", [0.0, 0.5])
