@@ -396,7 +396,10 @@ __host__ __device__ inline int tail_blocks(int len, int tmax, int first_blocks) 
 // the pair64 heads of its first kv head followed by the pair64 heads of its second.  A query row is placed in the half
 // of the 128-wide operand that faces its own kv head, the other half is zero, so S is exactly q . k of its own head;
 // O = P . [v_first, v_second] holds the head's output in the same half, which alone is stored (rows of 64).
-template <typename T, typename KV = T>
+//
+// SHARE: a block takes one split, its waves a quarter of the split's tiles each, and their states meet in the LDS; else a wave
+// takes a split of its own.  A wave's chain of tiles bounds the launch (1.5 us a tile) where there are few blocks.
+template <typename T, typename KV = T, bool SHARE = false>
 __global__ void __launch_bounds__(256, 2) decode_stage1_mfma128(
     const void* __restrict__ q, const void* __restrict__ k_buffer, const void* __restrict__ v_buffer,
     const int32_t* __restrict__ kv_indptr, const int32_t* __restrict__ kv_indices, float* __restrict__ attn_logits,
@@ -420,15 +423,22 @@ __global__ void __launch_bounds__(256, 2) decode_stage1_mfma128(
 
   const int b = blockIdx.x;
   const int kvh = blockIdx.y / head_tiles, ht = blockIdx.y - kvh * head_tiles;
-  const int split = blockIdx.z * kWavesPerBlock + wid;
+  const int split = SHARE ? blockIdx.z : blockIdx.z * kWavesPerBlock + wid;
   const int group = Hq / Hkv;
   const int start = kv_indptr[b];
   const int len = kv_indptr[b + 1] - start;
   const int splits = max(num_kv_splits[b], 1);
   const int per_split = cdiv_i(cdiv_i(len, splits), kMinBlockKV) * kMinBlockKV;
-  const int s0 = per_split * split;
-  const int s1 = min(s0 + per_split, len);
-  if (split >= max_kv_splits || s1 <= s0) return;  // wave-uniform; no block-level synchronisation is used
+  int s0 = per_split * split;
+  int s1 = min(s0 + per_split, len);
+  if (split >= max_kv_splits || s1 <= s0) return;  // wave-uniform (SHARE: block-uniform); else no block-level synchronisation is used
+  const bool together = SHARE && s1 - s0 > kTile;  // block-uniform; one tile is one wave's
+  if constexpr (SHARE) {
+    if (!together && wid != 0) return;
+    const int per_wave = cdiv_i(cdiv_i(s1 - s0, kTile), kWavesPerBlock) * kTile;
+    s0 += per_wave * wid;
+    s1 = min(s0 + per_wave, s1);  // (none left: an empty range, and a state of nothing)
+  }
 
   const int hl = lane & 15;  // operand column: query head within this head tile
   const int g = lane >> 4;   // 16-lane group
@@ -453,11 +463,38 @@ __global__ void __launch_bounds__(256, 2) decode_stage1_mfma128(
     wa.run8(kl, vl, lut, reinterpret_cast<const uint8_t*>(k_buffer) + (int64_t)kvh * k_stride_h,
             reinterpret_cast<const uint8_t*>(v_buffer) + (int64_t)kvh * v_stride_h, k_stride_n, v_stride_n,
             kv_indices + start, s0, s1, sm_scale, logit_cap);
-  const float m = wa.m;
-  const float4v(&oacc)[8] = wa.oacc;
+  float m = wa.m;
+  float4v(&oacc)[8] = wa.oacc;
 
   // ---- epilogue: total sum over the four lane groups, normalise, store partial
-  const float lsum = wa.total();
+  float lsum = wa.total();
+  if (SHARE && together) {  // the waves' states, over their tiles; wave w is left with output elements 32 w .. + 31
+    float4v* parts = reinterpret_cast<float4v*>(lds_all);                   // [4 waves][8][64 lanes]
+    float2v* states = reinterpret_cast<float2v*>(parts + 4 * 8 * 64);  // [4 waves][16 columns]
+    __syncthreads();  // nobody reads a tile any more
+#pragma unroll
+    for (int n = 0; n < 8; ++n) parts[(wid * 8 + n) * 64 + lane] = oacc[n];
+    if (g == 0) states[wid * 16 + hl] = float2v{m, lsum};
+    __syncthreads();
+    float top = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) top = fmaxf(top, states[w * 16 + hl][0]);
+    float sum = 0.f;
+    float4v mine[2] = {float4v{0.f, 0.f, 0.f, 0.f}, float4v{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const float2v st = states[w * 16 + hl];
+      const float f = st[1] == 0.f ? 0.f : exp2f(st[0] - top);
+      sum += f * st[1];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) mine[i] += parts[(w * 8 + 2 * wid + i) * 64 + lane] * f;
+    }
+    m = top;
+    lsum = sum;
+#pragma unroll
+    for (int n = 0; n < 8; ++n)
+      if (n >> 1 == wid) oacc[n] = mine[n & 1];
+  }
   if (head_ok) {
     const float inv = 1.0f / lsum;
     const int64_t ob = ((int64_t)b * Hq + head) * max_kv_splits + split;
@@ -465,16 +502,16 @@ __global__ void __launch_bounds__(256, 2) decode_stage1_mfma128(
       float* dst = attn_logits + ob * 64;
 #pragma unroll
       for (int n = 0; n < 8; ++n)
-        if ((n >> 2) == half) *reinterpret_cast<float4v*>(dst + 16 * (n & 3) + 4 * g) = oacc[n] * inv;
+        if ((n >> 2) == half && (!together || n >> 1 == wid)) *reinterpret_cast<float4v*>(dst + 16 * (n & 3) + 4 * g) = oacc[n] * inv;
     } else {
       float* dst = attn_logits + ob * 128;
 #pragma unroll
       for (int n = 0; n < 8; ++n) {
         // lane (hl, g) holds O[head][16n + 4g + r], r = 0..3
-        *reinterpret_cast<float4v*>(dst + 16 * n + 4 * g) = oacc[n] * inv;
+        if (!together || n >> 1 == wid) *reinterpret_cast<float4v*>(dst + 16 * n + 4 * g) = oacc[n] * inv;
       }
     }
-    if (g == 0) attn_lse[ob] = (m + log2f(lsum)) * 0.6931471805599453f;
+    if (g == 0 && (!together || wid == 0)) attn_lse[ob] = (m + log2f(lsum)) * 0.6931471805599453f;
   }
 }
 
@@ -1720,13 +1757,20 @@ static int decode_attention_impl(const void* q, const void* k_buffer, const void
                      aligned16(attn_logits) && (q_stride_b % 8 == 0) && (q_stride_h % 8 == 0) && (k_stride_n % 8 == 0) &&
                      (k_stride_h % 8 == 0) && (v_stride_n % 8 == 0) && (v_stride_h % 8 == 0);
   SGLK_CHECK(!gate || fast || fast8 || pair64 || mla, "decode_attention: a gated launch needs one of the tile kernels");
+  // A split gets a block instead of a wave (decode_stage1_mfma128, SHARE) where that makes up to two blocks a unit.  Calls of 8 splits
+  // over 200 / 600 / 1152 / 4096 tokens, wave and block a split: one request, 8 kv heads of 128 9.9 / 12.8 / 16.0 / 31.0 and
+  // 10.0 / 10.5 / 11.9 / 15.5 us; eight (512 blocks) 8.8 / 12.5 / 17.7 / 33.2 and 9.1 / 10.6 / 15.7 / 31.7; sixteen 9.1 / 16.0 /
+  // 22.5 / 51.0 and 12.8 / 19.4 / 24.8 / 50.7.
+  auto few = [&](int64_t columns) { return max_kv_splits <= 65535 && B * columns * max_kv_splits <= 512; };
   if (fast8) {
     const int head_tiles = (group + 15) / 16;
-    dim3 grid(B, Hkv * head_tiles, (max_kv_splits + kWavesPerBlock - 1) / kWavesPerBlock);
+    const bool share = few(Hkv * head_tiles);
+    dim3 grid(B, Hkv * head_tiles, share ? max_kv_splits : (max_kv_splits + kWavesPerBlock - 1) / kWavesPerBlock);
     const size_t lds = (size_t)kWavesPerBlock * kLdsPerWave + 512;
     SGLK_DISPATCH_HALF(dtype, T, {
       SGLK_DISPATCH_KV(kvf, T, KV, {
-        hipLaunchKernelGGL((decode_stage1_mfma128<T, KV>), grid, dim3(64 * kWavesPerBlock), lds, s, q, k_buffer, v_buffer,
+        const auto kernel = share ? decode_stage1_mfma128<T, KV, true> : decode_stage1_mfma128<T, KV, false>;
+        hipLaunchKernelGGL(kernel, grid, dim3(64 * kWavesPerBlock), lds, s, q, k_buffer, v_buffer,
                            kv_indptr, kv_indices, attn_logits, attn_lse, num_kv_splits, max_kv_splits, Hq, Hkv, head_tiles,
                            q_stride_b, q_stride_h, k_stride_n, k_stride_h, v_stride_n, v_stride_h, sm_scale, logit_cap, 0,
                            gate);
@@ -1784,23 +1828,27 @@ static int decode_attention_impl(const void* q, const void* k_buffer, const void
 #undef SGLK_MLA_LAUNCH
   } else if (fast) {
     const int head_tiles = (group + 15) / 16;
-    dim3 grid(B, Hkv * head_tiles, (max_kv_splits + kWavesPerBlock - 1) / kWavesPerBlock);
+    const bool share = few(Hkv * head_tiles);
+    dim3 grid(B, Hkv * head_tiles, share ? max_kv_splits : (max_kv_splits + kWavesPerBlock - 1) / kWavesPerBlock);
     const size_t lds = (size_t)kWavesPerBlock * kLdsPerWave;
-    SGLK_DISPATCH_HALF(dtype, T,
-                       hipLaunchKernelGGL((decode_stage1_mfma128<T>), grid, dim3(64 * kWavesPerBlock), lds, s, q, k_buffer,
-                                          v_buffer, kv_indptr, kv_indices, attn_logits, attn_lse, num_kv_splits,
-                                          max_kv_splits, Hq, Hkv, head_tiles, q_stride_b, q_stride_h, k_stride_n,
-                                          k_stride_h, v_stride_n, v_stride_h, sm_scale, logit_cap, 0, gate));
+    SGLK_DISPATCH_HALF(dtype, T, {
+      const auto kernel = share ? decode_stage1_mfma128<T, T, true> : decode_stage1_mfma128<T, T, false>;
+      hipLaunchKernelGGL(kernel, grid, dim3(64 * kWavesPerBlock), lds, s, q, k_buffer, v_buffer, kv_indptr, kv_indices,
+                         attn_logits, attn_lse, num_kv_splits, max_kv_splits, Hq, Hkv, head_tiles, q_stride_b, q_stride_h,
+                         k_stride_n, k_stride_h, v_stride_n, v_stride_h, sm_scale, logit_cap, 0, gate);
+    });
   } else if (pair64) {
     // head size 64 on the 128-wide tile kernel: Hkv / 2 pairs of kv heads, 2 * group query heads per pair
     const int head_tiles = (2 * group + 15) / 16;
-    dim3 grid(B, (Hkv / 2) * head_tiles, (max_kv_splits + kWavesPerBlock - 1) / kWavesPerBlock);
+    const bool share = few((Hkv / 2) * head_tiles);
+    dim3 grid(B, (Hkv / 2) * head_tiles, share ? max_kv_splits : (max_kv_splits + kWavesPerBlock - 1) / kWavesPerBlock);
     const size_t lds = (size_t)kWavesPerBlock * kLdsPerWave;
-    SGLK_DISPATCH_HALF(dtype, T,
-                       hipLaunchKernelGGL((decode_stage1_mfma128<T>), grid, dim3(64 * kWavesPerBlock), lds, s, q, k_buffer,
-                                          v_buffer, kv_indptr, kv_indices, attn_logits, attn_lse, num_kv_splits,
-                                          max_kv_splits, Hq, Hkv / 2, head_tiles, q_stride_b, q_stride_h, k_stride_n,
-                                          (int64_t)128, v_stride_n, (int64_t)128, sm_scale, logit_cap, group, gate));
+    SGLK_DISPATCH_HALF(dtype, T, {
+      const auto kernel = share ? decode_stage1_mfma128<T, T, true> : decode_stage1_mfma128<T, T, false>;
+      hipLaunchKernelGGL(kernel, grid, dim3(64 * kWavesPerBlock), lds, s, q, k_buffer, v_buffer, kv_indptr, kv_indices,
+                         attn_logits, attn_lse, num_kv_splits, max_kv_splits, Hq, Hkv / 2, head_tiles, q_stride_b, q_stride_h,
+                         k_stride_n, (int64_t)128, v_stride_n, (int64_t)128, sm_scale, logit_cap, group, gate);
+    });
   } else {
     dim3 grid(B, Hq, max_kv_splits);
     const size_t lds = (size_t)D * sizeof(float);

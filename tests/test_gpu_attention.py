@@ -505,3 +505,36 @@ def test_mla_rope_and_store(dtype, neox, B, H):
 
     with pytest.raises(SglkError):
         ops.mla_rope_and_store(q[..., nope:], q_input[:, :, : lora + 8], qkv_a[:, 96:], pool, loc, cos_sin, positions, lora)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Hq,Hkv,D", [(32, 8, 128), (14, 2, 64), (40, 2, 128)])
+@pytest.mark.parametrize("lens,splits", [
+    ([1, 31, 32, 33], 1), ([64, 65, 127, 128], 1),         # a split of one tile (a wave's), of two, of a tile a wave
+    ([129, 500, 33, 1000], 2), ([700, 1, 64, 2000], 3),    # more tiles than waves, waves without any
+])
+def test_decode_splits_shared_by_a_block(Hq, Hkv, D, lens, splits, dtype):
+    """Few requests: a split is a block's, its waves' states meet; against float64."""
+    ops = _ops()
+    gen = torch.Generator().manual_seed(sum(lens) + Hq)
+    B, total = len(lens), sum(lens)
+    k = torch.randn(total + 3, Hkv, D, generator=gen).to(dtype).to(DEV)
+    v = torch.randn(total + 3, Hkv, D, generator=gen).to(dtype).to(DEV)
+    q = torch.randn(B, Hq, D, generator=gen).to(dtype).to(DEV)
+    ind = torch.randperm(total + 3, generator=gen)[:total].to(torch.int32).to(DEV)
+    ptr = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
+    ns = torch.full((B,), splits, dtype=torch.int32, device=DEV)
+    o = torch.full((B, Hq, D), float("nan"), dtype=dtype, device=DEV)
+    al = torch.full((B, Hq, 4, D), float("nan"), device=DEV)
+    lse = torch.full((B, Hq, 4), float("nan"), device=DEV)
+    ops.decode_attention_fwd(q, k, v, o, ptr, ind, al, lse, ns, 4, D**-0.5, 0.0)
+    eps = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
+    for b in range(B):
+        rows = ind[ptr[b]: ptr[b + 1]].long()
+        kb, vb = (t[rows].double().repeat_interleave(Hq // Hkv, 1) for t in (k, v))
+        s = (kb * q[b].double()).sum(-1) * D**-0.5             # [tokens, heads]
+        want = (torch.softmax(s, 0)[..., None] * vb).sum(0)
+        # probabilities are rounded once to the type (against |v| <= max|v|), and the result once
+        assert (o[b].double() - want).abs().max().item() <= eps * (vb.abs().max() + want.abs().max()).item() + 1e-4
+        got = torch.logsumexp(torch.where(lse[b].isnan(), torch.full_like(lse[b], -math.inf), lse[b]), -1)
+        assert (got.double() - torch.logsumexp(s, 0)).abs().max().item() <= 1e-4
