@@ -355,6 +355,11 @@ SGLK_API int sglk_merge_state(const void* v_a, const float* s_a, const void* v_b
 
 /* ------------------------------------------------------------------ P1: KV pool write --------- */
 
+/* dst[i][0 .. count[i]) = src[i][0 .. count[i]) for up to eight vectors of int32 or int64 (*_is64), in one launch; the
+ * arrays are host memory and may be reused when the call returns */
+SGLK_API int sglk_copy_indices(const void* const* src, void* const* dst, const int64_t* count,
+                               const int32_t* src_is64, const int32_t* dst_is64, int segments, void* stream);
+
 /* k_buffer[loc[t]] = k[t], v_buffer[loc[t]] = v[t]  (rows of Hkv*D / Hkv*Dv elements).
  * Replaces MHATokenToKVPool.set_kv_buffer, python/sglang/srt/mem_cache/memory_pool.py:378-412. */
 SGLK_API int sglk_set_kv_buffer(void* k_buffer, void* v_buffer, const void* k, const void* v,

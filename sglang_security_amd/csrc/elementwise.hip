@@ -312,6 +312,27 @@ __global__ void __launch_bounds__(1024) rope_store_partial_kernel(
   }
 }
 
+// Several index vectors of either width in one launch (the inputs of a captured extend: six copies of up to 5 KB were six launches
+// at their latency, 2.4 us each and the gaps between them, behind the wait for the prefix length: 128 tokens after 1024 cached
+// ones, two layers of Llama-3-8B, 345 -> 316 us).
+constexpr int kCopySegments = 8;
+struct CopyIndices {
+  const void* src[kCopySegments];
+  void* dst[kCopySegments];
+  int64_t n[kCopySegments];
+  int src64[kCopySegments], dst64[kCopySegments];
+};
+__global__ void __launch_bounds__(256) copy_indices_kernel(CopyIndices c) {
+  const int s = blockIdx.y;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < c.n[s]; i += (int64_t)gridDim.x * 256) {
+    const int64_t v = ld_idx(c.src[s], c.src64[s], i);
+    if (c.dst64[s])
+      reinterpret_cast<int64_t*>(c.dst[s])[i] = v;
+    else
+      reinterpret_cast<int32_t*>(c.dst[s])[i] = (int32_t)v;
+  }
+}
+
 // ---------------------------------------------------------------------------------------------
 // act_and_mul: out = act(x[:, :d]) * x[:, d:]; act rounded to T before the product
 // (activation.cu:22-50 of the reference: silu returns T, then T*T)
@@ -826,6 +847,25 @@ int sglk_rope_and_store_kv(void* qkv, const float* cos_sin_cache, const int64_t*
                                         (hipStream_t)stream, qkv, cos_sin_cache, positions, k_buffer, v_buffer, loc,
                                         loc_is64, q_heads, kv_heads, head_size, rot_dim, kbuf_stride_n, vbuf_stride_n,
                                         interleave));
+  SGLK_LAUNCH_CHECK();
+  return SGLK_OK;
+}
+
+int sglk_copy_indices(const void* const* src, void* const* dst, const int64_t* count, const int32_t* src_is64, const int32_t* dst_is64,
+                      int segments, void* stream) {
+  SGLK_CHECK(segments >= 0 && segments <= kCopySegments, "copy_indices: 0 to %d segments", kCopySegments);
+  if (segments == 0) return SGLK_OK;
+  SGLK_CHECK(src && dst && count && src_is64 && dst_is64, "copy_indices: null pointer");
+  CopyIndices c{};
+  int64_t most = 0;
+  for (int i = 0; i < segments; ++i) {
+    SGLK_CHECK(count[i] >= 0 && (count[i] == 0 || (src[i] && dst[i])), "copy_indices: bad segment");
+    c.src[i] = src[i], c.dst[i] = dst[i], c.n[i] = count[i], c.src64[i] = src_is64[i], c.dst64[i] = dst_is64[i];
+    most = count[i] > most ? count[i] : most;
+  }
+  if (most == 0) return SGLK_OK;
+  const int64_t blocks = (most + 255) / 256;
+  hipLaunchKernelGGL(copy_indices_kernel, dim3((unsigned)(blocks < 1024 ? blocks : 1024), segments), dim3(256), 0, (hipStream_t)stream, c);
   SGLK_LAUNCH_CHECK();
   return SGLK_OK;
 }

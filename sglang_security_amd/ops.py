@@ -37,6 +37,23 @@ def _is64(t: torch.Tensor) -> int:
     raise SglkError(f"index tensor must be int32 or int64, got {t.dtype}")
 
 
+def copy_indices(dst, src):
+    """dst[i].copy_(src[i]) for up to eight pairs of equally long contiguous int32 / int64 vectors, in one launch."""
+    n = len(dst)
+    if n != len(src) or n > 8:
+        raise SglkError("copy_indices: up to eight pairs")
+    for d, s in zip(dst, src):
+        _need_gpu(d, s)
+        if d.numel() != s.numel() or not (d.is_contiguous() and s.is_contiguous()):
+            raise SglkError("copy_indices: pairs must be contiguous and of one length")
+    if n == 0:
+        return
+    wide = C.c_int32 * n
+    check(lib().sglk_copy_indices((C.c_void_p * n)(*(t.data_ptr() for t in src)), (C.c_void_p * n)(*(t.data_ptr() for t in dst)),
+                                  (C.c_int64 * n)(*(t.numel() for t in src)), wide(*(_is64(t) for t in src)),
+                                  wide(*(_is64(t) for t in dst)), n, _stream(dst[0])), "copy_indices")
+
+
 # ------------------------------------------------------------------------------------------- A0
 def create_kv_indices(req_to_token, req_pool_indices, page_kernel_lens, kv_indptr, kv_start_idx, kv_indices):
     """create_flashinfer_kv_indices_triton[(bs,)](...) -- layers/attention/utils.py:5-41."""

@@ -196,16 +196,23 @@ class LlamaPrefill:
         single = qo_indptr.numel() == 2 and max_extend_len == T
         if not (single and T < DEQUANT_GEMM_MIN_TOKENS and kv_indices.numel() <= self.g_ki.numel()):
             return self._extend(input_ids, positions, out_cache_loc, qo_indptr, kv_indptr, kv_indices, max_extend_len)
-        pre = int(kv_indptr[-1].item())  # cached prefix tokens (kv_indices may be a one-element placeholder without any)
         fused = 0 < T <= self.fused_rows
         if not (self.use_graph or fused):
             return self._extend(input_ids, positions, out_cache_loc, qo_indptr, kv_indptr, kv_indices, max_extend_len)
-        self.g_ids[:T].copy_(input_ids)
-        self.g_pos[:T].copy_(positions)
-        self.g_loc[:T].copy_(out_cache_loc)
-        self.g_qo.copy_(qo_indptr)
-        self.g_kp.copy_(kv_indptr)
-        self.g_ki[:pre].copy_(kv_indices[:pre])
+        # the copies are on their way while the host waits for the number of cached prefix tokens (kv_indices may be a
+        # one-element placeholder without any, and longer than what kv_indptr says)
+        n = kv_indices.numel()
+        dst = (self.g_ids[:T], self.g_pos[:T], self.g_loc[:T], self.g_qo, self.g_kp, self.g_ki[:n])
+        src = (input_ids, positions, out_cache_loc, qo_indptr, kv_indptr, kv_indices)
+        if all(s.device == d.device and s.shape == d.shape and s.is_contiguous() and s.dtype in (torch.int32, torch.int64)
+               for d, s in zip(dst, src)):
+            ops.copy_indices(dst, src)
+        else:
+            for d, s in zip(dst, src):
+                d.copy_(s)
+        pre = int(kv_indptr[-1].item())
+        if pre > n:
+            self.g_ki[:pre].copy_(kv_indices[:pre])
         args = (self.g_ids[:T], self.g_pos[:T], self.g_loc[:T], self.g_qo, self.g_kp, self.g_ki, T)
         run = self._extend_fused if fused else self._extend
         if not self.use_graph:

@@ -215,3 +215,41 @@ def test_bench_tiny_line_and_ttft_block():
     out = ttft_experiment(_tiny("awq"), 1024, 16, pool_tokens=8192, repeats=1)
     assert out["public"]["cached_prefix_tokens_cold_other_owner"] == [0, 1024, 1024]
     assert out["private"]["cached_prefix_tokens_cold_other_owner"] == [0, 0, 1024]
+
+
+@pytest.mark.parametrize("counts", [(1,), (5, 0, 300), (128, 128, 128, 2, 2, 70000), (0, 0)])
+def test_copy_indices(counts):
+    """Vectors of both widths, empty ones and ones longer than a block, and nothing beside them is written."""
+    from sglang_security_amd import ops
+    from sglang_security_amd._lib import SglkError
+
+    g = torch.Generator().manual_seed(sum(counts))
+    kinds = [(torch.int32, torch.int32), (torch.int64, torch.int32), (torch.int32, torch.int64), (torch.int64, torch.int64)]
+    src = [torch.randint(-9, 2**31 - 1, (n,), generator=g).to(kinds[i % 4][0]).to(DEV) for i, n in enumerate(counts)]
+    whole = [torch.full((n + 2,), -77, dtype=kinds[i % 4][1], device=DEV) for i, n in enumerate(counts)]
+    ops.copy_indices([w[1:-1] for w in whole], src)
+    for w, s in zip(whole, src):
+        assert torch.equal(w[1:-1].long(), s.long()) and w[0] == -77 and w[-1] == -77
+    with pytest.raises(SglkError):
+        ops.copy_indices([whole[0]], [src[0]])
+
+
+def test_extend_refuses_more_cached_tokens_than_indices():
+    """kv_indptr beyond kv_indices is an error, and the next extend is right."""
+    from sglang_security_amd.mem_cache.memory_pool import MHATokenToKVPool
+    from sglang_security_amd.prefill_runner import LlamaPrefill
+
+    dec = _tiny()
+    c = dec.cfg
+    kv = MHATokenToKVPool(128, 1, torch.bfloat16, c.kv_heads, c.head_dim, c.layers, DEV)
+    model = LlamaPrefill(dec, kv, 64)
+    i32 = lambda *v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    ids, pos, loc = torch.arange(8, device=DEV), torch.arange(8, device=DEV), torch.arange(1, 9, device=DEV)
+    good = (ids, pos, loc, i32(0, 8), i32(0, 0), i32(0), 8)
+    want = [t.clone() for t in model.extend(*good)]
+    with pytest.raises(RuntimeError):
+        model.extend(ids, pos, loc, i32(0, 8), i32(0, 5), i32(20, 21, 22), 8)
+    assert all(torch.equal(a, b) for a, b in zip(model.extend(*good), want))
+    # vectors of other widths, and views with gaps, are copied one by one or converted
+    got = model.extend(ids.int(), pos.repeat_interleave(2)[::2], loc.int(), i32(0, 8).long(), i32(0, 0), i32(0).long(), 8)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
