@@ -93,6 +93,8 @@ __host__ __device__ inline int delta_step_lds(int dp, int vp) { return (2 * dp +
 
 // Block: one head of one sequence.  Thread (rg, cg) owns the columns 4 cg .. + 3 of the state's rows rg, rg + RG, ...; NR of
 // them per thread in registers (NR = 0: any number, the state stays in memory).  EXACT: every thread owns NR rows.
+// A chain of trips to memory beside the state's 131 KB: everything a row needs is asked for at its top, split sums eight at a
+// time (16 rows of 20 heads of 128 / 128, 5 splits: 14.1 us asked for where it is used, one split behind the other -> 12.0).
 template <typename T, int NR, bool EXACT>
 __global__ void __launch_bounds__(256) delta_step_kernel(DeltaRule a, int seq0) {
   extern __shared__ __attribute__((aligned(16))) float delta_lds[];
@@ -136,6 +138,16 @@ __global__ void __launch_bounds__(256) delta_step_kernel(DeltaRule a, int seq0) 
       sq += qv * qv;
       dot += kv * qv;
     }
+    constexpr int OV = 4;  // vp <= 1024
+    float vin[OV], zin[OV];  // the row's values and gate channels: asked for here, they arrive beside the rest
+#pragma unroll
+    for (int i = 0; i < OV; ++i) {
+      const int c = threadIdx.x + 256 * i;
+      vin[i] = zin[i] = 0.f;
+      if (c >= a.vp) continue;
+      vin[i] = ld<T>(a.u, uv + c);
+      zin[i] = source1<T>(a.src, m, h * a.vp + c);
+    }
     float log_g, beta;
     delta_gates<T>(a, m, h, log_g, beta);
     const float g = expf(log_g);
@@ -162,7 +174,6 @@ __global__ void __launch_bounds__(256) delta_step_kernel(DeltaRule a, int seq0) 
     }
     __syncthreads();
     float so = 0.f;
-    constexpr int OV = 4;  // vp <= 1024
     float o[OV];
 #pragma unroll
     for (int i = 0; i < OV; ++i) {
@@ -174,7 +185,7 @@ __global__ void __launch_bounds__(256) delta_step_kernel(DeltaRule a, int seq0) 
         s1 += part[r * a.vp + c];
         s2 += part[(RG + r) * a.vp + c];
       }
-      const float u = beta * (ld<T>(a.u, uv + c) - g * rk * s1);
+      const float u = beta * (vin[i] - g * rk * s1);
       ub[c] = u * rk;
       o[i] = g * rq * s2 + u * (dot * rk * rq);
       so += o[i] * o[i];
@@ -203,8 +214,7 @@ __global__ void __launch_bounds__(256) delta_step_kernel(DeltaRule a, int seq0) 
     for (int i = 0; i < OV; ++i) {
       const int c = threadIdx.x + 256 * i;
       if (c >= a.vp) continue;
-      const float z = source1<T>(a.src, m, h * a.vp + c);
-      const float gate = sizeof(typename Raw<T>::type) == 2 ? silu_fast(z) : activate(z, 3);
+      const float gate = sizeof(typename Raw<T>::type) == 2 ? silu_fast(zin[i]) : activate(zin[i], 3);
       st<T>(a.out, m * a.out_stride + h * a.vp + c, o[i] * inv * a.norm[c] * gate);
     }
     __syncthreads();  // the rows in LDS are read until here

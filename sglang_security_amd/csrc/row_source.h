@@ -58,12 +58,20 @@ __device__ __forceinline__ void source8(const RowSource& s, int64_t row, int col
     ld8<T>(s.p, row * s.stride + col, v);
 }
 
-// one element; the splits are added in the same order
+// one element; the splits are requested eight at a time and added in the same order
 template <typename T>
 __device__ __forceinline__ float source1(const RowSource& s, int64_t row, int col) {
   if (!s.f32) return ld<T>(s.p, row * s.stride + col);
   float v = 0.f;
-  for (int k = 0; k < s.splits; ++k) v += reinterpret_cast<const float*>(s.p)[k * s.part_stride + row * s.stride + col];
+  const float* p = reinterpret_cast<const float*>(s.p) + row * s.stride + col;
+  for (int first = 0; first < s.splits; first += 8) {
+    float part[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) part[u] = p[min(first + u, s.splits - 1) * s.part_stride];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (first + u < s.splits) v += part[u];
+  }
   return v;
 }
 
