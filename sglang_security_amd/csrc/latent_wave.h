@@ -303,13 +303,14 @@ __global__ void __launch_bounds__(256, 1) latent_decode_kernel(LatentArgs a, Few
     // probabilities as the sum of two 16-bit numbers: [hi, lo][head tile][pair]
     uint32_t w[2][2][2];
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < 2; ++u) {
+      const float from = m[u] == -INFINITY ? 0.f : m[u];  // nothing but scores of -inf so far: they weigh nothing
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         uint16_t first[2], second[2];
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-          const float x = __builtin_amdgcn_exp2f(sc[u][2 * h + e] - m[u]);
+          const float x = __builtin_amdgcn_exp2f(sc[u][2 * h + e] - from);
           lcur[u] += x;
           first[e] = Conv<T>::from_f32(x);
           second[e] = Conv<T>::from_f32(x - Conv<T>::to_f32(first[e]));
@@ -317,6 +318,7 @@ __global__ void __launch_bounds__(256, 1) latent_decode_kernel(LatentArgs a, Few
         w[0][u][h] = (uint32_t)first[0] | ((uint32_t)first[1] << 16);
         w[1][u][h] = (uint32_t)second[0] | ((uint32_t)second[1] << 16);
       }
+    }
     // P^T operands: lane holds head lane & 31, tokens 8 (lane >> 5) .. + 7
     short8 pf[2];
 #pragma unroll
@@ -365,7 +367,7 @@ __global__ void __launch_bounds__(256, 1) latent_decode_kernel(LatentArgs a, Few
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       const float2v x = st[w * 32];
-      sum += x[1] == 0.f ? 0.f : x[1] * __builtin_amdgcn_exp2f(x[0] - top);
+      sum += x[1] == 0.f ? 0.f : x[1] * __builtin_amdgcn_exp2f(x[0] - top);  // (the maximum of a wave without a weight is not asked)
     }
   };
   const int l31 = lane & 31, hi = lane >> 5;
@@ -388,7 +390,7 @@ __global__ void __launch_bounds__(256, 1) latent_decode_kernel(LatentArgs a, Few
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       const float2v own = state[w * 32 + hd];
-      share[w] = own[1] == 0.f ? 0.f : __builtin_amdgcn_exp2f(own[0] - top) * inv;
+      share[w] = (own[1] == 0.f ? 0.f : __builtin_amdgcn_exp2f(own[0] - top)) * inv;  // (NaN where nothing weighs anything)
     }
   }
 #pragma unroll

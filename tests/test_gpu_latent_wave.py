@@ -81,3 +81,18 @@ def test_more_splits_asked_for_than_there_is_room_for():
     kv, q = _data(lens, 128, torch.bfloat16, 5)
     o, lse, _, _ = _run(lens, 128, 2, torch.bfloat16, kv, q, splits=8)
     assert o.isfinite().all() and lse.isfinite().all()
+
+
+def test_scores_of_minus_infinity():
+    """A run of tokens whose key (beside the value part) makes their score -inf weighs nothing, wherever a wave meets it."""
+    lens = [96, 16 + 64] + [40] * 31
+    kv, q = _data(lens, 256, torch.bfloat16, 7)
+    ind = torch.randperm(sum(lens) + 5, generator=torch.Generator().manual_seed(sum(lens)))[: sum(lens)].to(DEV)
+    hidden = torch.zeros(sum(lens), dtype=torch.bool, device=DEV)
+    hidden[0:16] = hidden[64:80] = hidden[96 + 16: 96 + 80] = True      # first tiles of waves, and of one request all but a tile
+    kv[ind[hidden], 0, 575] = math.inf
+    q[..., 575] = -1.0
+    o, _, want, _ = _run(lens, 256, 1, torch.bfloat16, kv, q)
+    assert o.isfinite().all()
+    v = kv[..., :512].abs().max().double()
+    assert (o.double() - want).abs().max().item() <= 2.0**-8 * (v + want.abs().max()).item() + 1e-4
