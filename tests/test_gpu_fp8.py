@@ -52,6 +52,22 @@ def test_per_token_quant_bitexact(rows, hidden, dtype):
     assert torch.equal(_u8(q), wq.view(torch.uint8))
 
 
+@pytest.mark.parametrize("hidden", [8, 2048, 2056, 4096, 4104, 8192, 8200, 16384, 16392])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_per_token_quant_held_rows(hidden, dtype):
+    """Rows around the sizes up to which a thread holds one, two, four and eight vectors, and beyond."""
+    import oracle
+
+    torch.manual_seed(hidden)
+    x = (torch.randn(3, hidden) * 3).to(dtype)
+    wq, ws = oracle.per_token_quant_fp8(x)
+    q = torch.empty(3, hidden, dtype=F8, device=DEV)
+    s = torch.empty(3, 1, dtype=torch.float32, device=DEV)
+    _ops().per_token_quant_fp8(x.to(DEV), q, s)
+    assert torch.equal(s.cpu(), ws)
+    assert torch.equal(_u8(q), wq.view(torch.uint8))
+
+
 def test_per_token_quant_golden(golden):
     """Fixture minted from the reference formula (sgl-kernel/tests/test_per_token_quant_fp8.py:15-27)."""
     ops = _ops()

@@ -73,8 +73,8 @@ def test_kept_sets(kind, n, scale):
 
 
 @pytest.mark.parametrize("B,n", [(64, 128259), (64, 163843), (100, 128259), (128, 81923), (20, 8195 * 12)])
-def test_spread_rows_around_the_held_elements(B, n):
-    """Slices of fewer elements than a block holds in registers, of just as many and of more, and a row's last three."""
+def test_spread_rows_of_large_batches(B, n):
+    """Rows over two, four and twelve blocks with slices of 8192 to 64000 elements, and a row's last three."""
     import sglang_security_amd.sgl_kernel as sk
     from sglang_security_amd import ops
 
