@@ -211,8 +211,8 @@ class LlamaPrefill:
             for d, s in zip(dst, src):
                 d.copy_(s)
         pre = int(kv_indptr[-1].item())
-        if pre > n:
-            self.g_ki[:pre].copy_(kv_indices[:pre])
+        if pre > n:     # (what is in flight fills staging buffers that nobody reads before the next call has filled them anew)
+            raise RuntimeError(f"extend: kv_indptr names {pre} cached tokens, kv_indices holds {n}")
         args = (self.g_ids[:T], self.g_pos[:T], self.g_loc[:T], self.g_qo, self.g_kp, self.g_ki, T)
         run = self._extend_fused if fused else self._extend
         if not self.use_graph:

@@ -249,6 +249,10 @@ def test_extend_refuses_more_cached_tokens_than_indices():
     want = [t.clone() for t in model.extend(*good)]
     with pytest.raises(RuntimeError):
         model.extend(ids, pos, loc, i32(0, 8), i32(0, 5), i32(20, 21, 22), 8)
+    # ... also where a copy of the indices would fit: one that could be spread over all of them, and as many as the buffer holds
+    for pre, have in ((5, i32(20)), (65, torch.arange(1, 65, dtype=torch.int32, device=DEV))):
+        with pytest.raises(RuntimeError, match="cached tokens"):
+            model.extend(ids, pos, loc, i32(0, 8), i32(0, pre), have, 8)
     assert all(torch.equal(a, b) for a, b in zip(model.extend(*good), want))
     # vectors of other widths, and views with gaps, are copied one by one or converted
     got = model.extend(ids.int(), pos.repeat_interleave(2)[::2], loc.int(), i32(0, 8).long(), i32(0, 0), i32(0).long(), 8)
