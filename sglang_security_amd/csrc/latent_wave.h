@@ -386,11 +386,12 @@ __global__ void __launch_bounds__(256, 1) latent_decode_kernel(LatentArgs a, Few
   {
     float top, sum;
     meet(state + hd, top, sum);
-    const float inv = 1.f / sum;
+    // where nothing weighs anything: NaN if this is the request, nothing if other blocks may have what does (log-sum-exps of -inf)
+    const float inv = sum == 0.f && p.blocks > 1 ? 0.f : 1.f / sum;
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       const float2v own = state[w * 32 + hd];
-      share[w] = (own[1] == 0.f ? 0.f : __builtin_amdgcn_exp2f(own[0] - top)) * inv;  // (NaN where nothing weighs anything)
+      share[w] = (own[1] == 0.f ? 0.f : __builtin_amdgcn_exp2f(own[0] - top)) * inv;
     }
   }
 #pragma unroll

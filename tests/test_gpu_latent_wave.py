@@ -96,3 +96,25 @@ def test_scores_of_minus_infinity():
     assert o.isfinite().all()
     v = kv[..., :512].abs().max().double()
     assert (o.double() - want).abs().max().item() <= 2.0**-8 * (v + want.abs().max()).item() + 1e-4
+
+
+@pytest.mark.parametrize("splits", [32, 8])
+def test_blocks_of_minus_infinity(splits):
+    """Requests of several blocks (of two folded splits, and of one), some of which hold nothing but scores of -inf: the others'
+    rows are the result; with none left it is NaN, as a softmax over nothing."""
+    lens = [512, 512, 300] + [20] * 6
+    kv, q = _data(lens, 32, torch.bfloat16, 11)
+    ind = torch.randperm(sum(lens) + 5, generator=torch.Generator().manual_seed(sum(lens)))[: sum(lens)].to(DEV)
+    hidden = torch.zeros(sum(lens), dtype=torch.bool, device=DEV)
+    hidden[64:192] = hidden[448:512] = True             # of the first request: the second, third and last 64 tokens
+    hidden[512: 1024] = True                            # the whole second one
+    kv[ind[hidden], 0, 575] = math.inf
+    q[..., 575] = -1.0
+    o, lse, want, wlse = _run(lens, 32, 32, torch.bfloat16, kv, q, splits=splits)
+    assert o[1].isnan().all()
+    keep = [b for b in range(len(lens)) if b != 1]
+    assert o[keep].isfinite().all()
+    v = kv[..., :512].abs().max().double()
+    assert (o[keep].double() - want[keep]).abs().max().item() <= 2.0**-8 * (v + want[keep].abs().max()).item() + 1e-4
+    got = torch.logsumexp(torch.where(lse.isnan(), torch.full_like(lse, -math.inf), lse), -1)
+    assert (got[keep].double() - wlse[keep]).abs().max().item() <= 2.0**-8 + 1e-4
