@@ -290,6 +290,44 @@ __global__ void __launch_bounds__(64) decode_stage1_generic(
 // ---------------------------------------------------------------------------------------------
 // stage 2: LSE merge of the split partials (decode_attention.py:497-557)
 // ---------------------------------------------------------------------------------------------
+// Splits first .. first + N - 1 of a row's elements (those below `live`), all requested at once and merged in order.
+template <int N, typename V>
+__device__ __forceinline__ void merge_splits(const float* part, const float* lse, int first, int live, int Dv, V& acc, float& e_sum,
+                                             float& e_max) {
+  V tv[N];
+  float tl[N];
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    const int s = min(first + u, live - 1);
+    tv[u] = *reinterpret_cast<const V*>(part + (int64_t)s * Dv);
+    tl[u] = lse[s];
+  }
+#pragma unroll
+  for (int u = 0; u < N; ++u) asm volatile("" : "+v"(tv[u]), "+v"(tl[u]));  // (the compiler moves a load to where it is used)
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    if (first + u >= live) break;
+    const float n_max = fmaxf(tl[u], e_max);
+    const float old = expf(e_max - n_max), w = expf(tl[u] - n_max);
+    acc = acc * old + w * tv[u];
+    e_sum = e_sum * old + w;
+    e_max = n_max;
+  }
+}
+
+// Eight splits are requested at once (one at a time, each waits for the one before: 8 splits of one request of 600 / 1152 / 4096
+// tokens, 32 heads, replayed calls: 10.0 / 11.4 / 14.7 -> 8.3 / 9.5 / 13.0 us), and two where there are no more: short requests have
+// one or two, and eight requests for those cost 0.2 to 0.35 us a launch (16 requests of 32 / 64 tokens 6.6 / 7.0 -> 6.3 / 6.6).
+template <typename V>
+__device__ __forceinline__ void merge_row(const float* part, const float* lse, int live, int Dv, V& acc, float& e_sum) {
+  float e_max = -INFINITY;
+  if (live <= 2) {
+    if (live > 0) merge_splits<2>(part, lse, 0, live, Dv, acc, e_sum, e_max);
+    return;
+  }
+  for (int first = 0; first < live; first += 8) merge_splits<8>(part, lse, first, live, Dv, acc, e_sum, e_max);
+}
+
 template <typename T>
 __global__ void __launch_bounds__(128) decode_stage2(const float* __restrict__ attn_logits,
                                                      const float* __restrict__ attn_lse, void* __restrict__ o,
@@ -305,65 +343,23 @@ __global__ void __launch_bounds__(128) decode_stage2(const float* __restrict__ a
   const int splits = max(num_kv_splits[b], 1);
   const int per_split = cdiv_i(cdiv_i(len, splits), kMinBlockKV) * kMinBlockKV;
   const int64_t base = ((int64_t)b * Hq + h) * max_kv_splits;
-  // Eight splits are requested at once and then merged in order (one at a time, each waited for the one before: 8 splits of one
-  // request: calls of 600 / 1152 / 4096 tokens, 32 heads, 10.4 / 11.8 / 15.4 -> 9.1 / 10.3 / 14.0 us).  Splits have tokens up to the last of the request, so the first without any ends the walk.
-  constexpr int kAtOnce = 8;
+  // splits have tokens up to the last of the request: the first without any ends the walk
   const int live = per_split > 0 ? min(cdiv_i(len, per_split), max_kv_splits) : 0;
   if (Dv % 512 == 0 && !xsum_out && (reinterpret_cast<uintptr_t>(attn_logits) & 15) == 0) {
     // wide values (absorbed MLA): four consecutive elements a thread, a split's weights formed once per thread; the
     // same operations per element, in the same order, as the loop below
     for (int d = 4 * threadIdx.x; d < Dv; d += 512) {
-      float e_sum = 0.f, e_max = -INFINITY;
+      float e_sum = 0.f;
       float4v acc = float4v{0.f, 0.f, 0.f, 0.f};
-      for (int first = 0; first < live; first += kAtOnce) {
-        float4v tv[kAtOnce];
-        float tl[kAtOnce];
-#pragma unroll
-        for (int u = 0; u < kAtOnce; ++u) {
-          const int s = min(first + u, live - 1);
-          tv[u] = *reinterpret_cast<const float4v*>(attn_logits + (base + s) * Dv + d);
-          tl[u] = attn_lse[base + s];
-        }
-#pragma unroll
-        for (int u = 0; u < kAtOnce; ++u) asm volatile("" : "+v"(tv[u]), "+v"(tl[u]));  // (the compiler moves a load to where it is used)
-#pragma unroll
-        for (int u = 0; u < kAtOnce; ++u) {
-          if (first + u >= live) break;
-          const float n_max = fmaxf(tl[u], e_max);
-          const float old = expf(e_max - n_max), w = expf(tl[u] - n_max);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[r] = acc[r] * old + w * tv[u][r];
-          e_sum = e_sum * old + w;
-          e_max = n_max;
-        }
-      }
+      merge_row(attn_logits + base * Dv + d, attn_lse + base, live, Dv, acc, e_sum);
 #pragma unroll
       for (int r = 0; r < 4; ++r) st<T>(o, (int64_t)b * o_stride_b + (int64_t)h * o_stride_h + d + r, acc[r] / e_sum);
     }
     return;
   }
   for (int d = threadIdx.x; d < Dv; d += 128) {
-    float e_sum = 0.f, e_max = -INFINITY, acc = 0.f;
-    for (int first = 0; first < live; first += kAtOnce) {
-      float tv[kAtOnce], tl[kAtOnce];
-#pragma unroll
-      for (int u = 0; u < kAtOnce; ++u) {
-        const int s = min(first + u, live - 1);
-        tv[u] = attn_logits[(base + s) * Dv + d];
-        tl[u] = attn_lse[base + s];
-      }
-#pragma unroll
-      for (int u = 0; u < kAtOnce; ++u) asm volatile("" : "+v"(tv[u]), "+v"(tl[u]));
-#pragma unroll
-      for (int u = 0; u < kAtOnce; ++u) {
-        if (first + u >= live) break;
-        const float n_max = fmaxf(tl[u], e_max);
-        const float old = expf(e_max - n_max), w = expf(tl[u] - n_max);
-        acc = acc * old + w * tv[u];
-        e_sum = e_sum * old + w;
-        e_max = n_max;
-      }
-    }
+    float e_sum = 0.f, acc = 0.f;
+    merge_row(attn_logits + base * Dv + d, attn_lse + base, live, Dv, acc, e_sum);
     st<T>(o, (int64_t)b * o_stride_b + (int64_t)h * o_stride_h + d, acc / e_sum);
     if (xsum_out) {  // Dv == 128: one head is one 128-element block of the following projection's input row
       const float r = wave_sum(Conv<T>::to_f32(Conv<T>::from_f32(acc / e_sum)));
@@ -1787,10 +1783,10 @@ static int decode_attention_impl(const void* q, const void* k_buffer, const void
                      aligned16(attn_logits) && (q_stride_b % 8 == 0) && (q_stride_h % 8 == 0) && (k_stride_n % 8 == 0) &&
                      (k_stride_h % 8 == 0) && (v_stride_n % 8 == 0) && (v_stride_h % 8 == 0);
   SGLK_CHECK(!gate || fast || fast8 || pair64 || mla, "decode_attention: a gated launch needs one of the tile kernels");
-  // A split gets a block instead of a wave (decode_stage1_mfma128, SHARE) where that makes up to two blocks a unit.  Calls of 8 splits
-  // over 200 / 600 / 1152 / 4096 tokens, wave and block a split: one request, 8 kv heads of 128 9.9 / 12.8 / 16.0 / 31.0 and
-  // 10.0 / 10.5 / 11.9 / 15.5 us; eight (512 blocks) 8.8 / 12.5 / 17.7 / 33.2 and 9.1 / 10.6 / 15.7 / 31.7; sixteen 9.1 / 16.0 /
-  // 22.5 / 51.0 and 12.8 / 19.4 / 24.8 / 50.7.
+  // A split gets a block instead of a wave (decode_stage1_mfma128, SHARE) where that makes up to two blocks a unit.  Replayed calls of
+  // 8 splits over 32 / 64 / 200 / 600 / 1152 / 4096 tokens, wave and block a split: one request, 8 kv heads of 128 6.1 / 6.5 / 7.9 /
+  // 10.8 / 13.7 / 28.7 and 6.3 / 6.4 / 7.1 / 8.3 / 9.4 / 13.0 us; eight (512 blocks) 6.0 / 6.3 / 7.8 / 11.0 / 15.3 / 30.6 and 6.1 /
+  // 6.3 / 7.2 / 9.0 / 13.1 / 28.3; sixteen 6.3 / 6.7 / 8.4 / 13.9 / 20.4 / 47.8 and 6.5 / 6.7 / 10.7 / 16.9 / 22.5 / 48.1.
   auto few = [&](int64_t columns) { return max_kv_splits <= 65535 && B * columns * max_kv_splits <= 512; };
   if (fast8) {
     const int head_tiles = (group + 15) / 16;

@@ -538,3 +538,31 @@ def test_decode_splits_shared_by_a_block(Hq, Hkv, D, lens, splits, dtype):
         assert (o[b].double() - want).abs().max().item() <= eps * (vb.abs().max() + want.abs().max()).item() + 1e-4
         got = torch.logsumexp(torch.where(lse[b].isnan(), torch.full_like(lse[b], -math.inf), lse[b]), -1)
         assert (got.double() - torch.logsumexp(s, 0)).abs().max().item() <= 1e-4
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(8, 2, 128), (16, 1, 576)])
+@pytest.mark.parametrize("splits", [1, 2, 3, 8, 16])
+def test_merge_of_few_and_many_splits(Hq, Hkv, D, splits):
+    """Rows of one split, two, three to eight and more, each merged its own way; against float64."""
+    ops = _ops()
+    lens, Dv = [20, 64, 90, 0, 260, 600], 512 if D == 576 else D
+    gen = torch.Generator().manual_seed(splits + D)
+    B, total = len(lens), sum(lens)
+    k = torch.randn(total + 3, Hkv, D, generator=gen).to(torch.bfloat16).to(DEV)
+    v = k[..., :512] if D == 576 else torch.randn(total + 3, Hkv, D, generator=gen).to(torch.bfloat16).to(DEV)
+    q = torch.randn(B, Hq, D, generator=gen).to(torch.bfloat16).to(DEV)
+    ind = torch.randperm(total + 3, generator=gen)[:total].to(torch.int32).to(DEV)
+    ptr = torch.tensor([0] + torch.tensor(lens).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
+    ns = torch.full((B,), splits, dtype=torch.int32, device=DEV)
+    o = torch.full((B, Hq, Dv), 7.0, dtype=torch.bfloat16, device=DEV)
+    al = torch.full((B, Hq, splits, Dv), float("nan"), device=DEV)
+    lse = torch.full((B, Hq, splits), float("nan"), device=DEV)
+    ops.decode_attention_fwd(q, k, v, o, ptr, ind, al, lse, ns, splits, D**-0.5, 0.0)
+    for b, n in enumerate(lens):
+        if n == 0:
+            assert o[b].isnan().all()                        # a sum over nothing
+            continue
+        rows = ind[ptr[b]: ptr[b + 1]].long()
+        kb, vb = (t[rows].double().repeat_interleave(Hq // Hkv, 1) for t in (k, v))
+        want = (torch.softmax((kb * q[b].double()).sum(-1) * D**-0.5, 0)[..., None] * vb).sum(0)
+        assert (o[b].double() - want).abs().max().item() <= 2.0**-8 * (vb.abs().max() + want.abs().max()).item() + 1e-4
