@@ -1699,18 +1699,16 @@ int sglk_common_prefix_len(const int32_t* req_to_token, int64_t row_stride, cons
   return SGLK_OK;
 }
 
-// Where fewer splits than the caller's make a latent launch of up to 16 faster.  `units` blocks are one split of every
-// request, for 512 places (two a unit of the chip).  An estimate in microseconds: blocks take 0.086 a token of the mean
-// context, a last round that leaves every unit one block or none a part of that; the partials a time per round of blocks.
-// Of the numbers that leave at most a tenth of a round's places empty, the one with the least estimate is taken if that is
-// below 0.87 of the caller's; one above 0.8 of the caller's has to save a round and to fill those left.  Below 256 tokens
-// the partials are what counts: up to 0.7, any number of places, below 0.95.  Fitted to 664 batches (1 to 256 requests of
-// 32, 40, 64 and 128 heads, contexts of 100 to 16000 tokens, even ones and spread from a quarter up) timed with 1 to 16
-// splits.  Calls with the caller's number -> with the rule's, 128 heads: 64 requests of 768 to 1152 tokens 75.6 us (3 splits)
-// -> 66.8 (2), 98.6 (8) -> 70.3; 32 of them 56.0 (8) -> 44.8 (4); 20 of 2731 to 4096 tokens 85.4 (8) -> 75.7 (6); 100 of 150
-// to 300 tokens 88.4 (8) -> 49.8 (1); 75 of 768 to 1152 keep 2 (98), of 1024 to 4096 keep 3 (216).  Of 3984 calls 1039 are
-// more than 4 % faster; calls that keep their number pay up to 1 us of a pair of launches for asking (45 of them more than
-// 4 %).  An estimate weighed in every block cost more than it gave: 5 to 20 us of 25600 merge blocks.
+// Where a latent launch takes fewer splits than the caller's, up to 16: what its log-sum-exps are counted in.  `units` blocks are one
+// split of every request, for 512 places (two a unit of the chip): the rule is that of the kernel of waves that share a tile, fitted
+// when it served these calls too (664 batches of 1 to 256 requests of 32 to 128 heads and 100 to 16000 tokens), by an estimate in
+// microseconds: blocks take 0.086 a token of the mean context, a last round that leaves every unit one block or none a part of that;
+// the partials a time per round of blocks.  Of the numbers that leave at most a tenth of a round's places empty, the one with the
+// least estimate is taken if that is below 0.87 of the caller's; one above 0.8 of the caller's has to save a round and to fill those
+// left.  Below 256 tokens the partials are what counts: up to 0.7, any number of places, below 0.95.
+// The kernel of waves with tiles of their own chooses its blocks by itself (latent_plan) and folds these splits into them; what is
+// left of the rule there is how many log-sum-exps there are and how evenly they divide: 90 batches of 16 to 64 requests of up to 64 to
+// 4096 tokens take the caller's numbers 1 % faster on the whole, 24 of up to 2000 44.3 -> 40.6 us, 20 of up to 4096 53.1 -> 55.3.
 static FewerSplits mla_fewer_splits(int B, int64_t units, int max_splits) {
   constexpr int kPlaces = 512;
   FewerSplits f{};
@@ -1808,22 +1806,26 @@ static int decode_attention_impl(const void* q, const void* k_buffer, const void
     // Up to 31 heads a group the copy rate bounds the launch and a short last round is nearly free (100 requests of up to
     // 2048 tokens, 16 heads: 49.9 us with 8 splits, 51.5 with 7): there the caller's number stands.
     const int64_t units = (int64_t)B * Hkv * ((group + 31) / 32);
-    const int64_t blocks = 8 * (int64_t)Hkv * ((group + 31) / 32) * (((int64_t)B * max_kv_splits + 7) / 8);
     // Where every split of every request has a unit of the chip to itself the launch is a chain of trips, and a block of waves that
-    // share each tile starts and ends sooner than one of waves that meet at the end: 8 requests, 128 heads, 64 / 300 / 1152 / 4096
-    // tokens: 19.9 / 22.7 / 30.4 / 53.0 us against 21.0 / 24.4 / 29.1 / 40.7; one request 19.5 / 21.9 / 28.4 / 49.2 against
-    // 20.9 / 24.4 / 26.6 / 35.8.  (How long the requests are is not known here.)  A launch holds fewer than 2^32 threads.
-    if (units * max_kv_splits > 256 && group >= 32 && blocks < (1 << 24) && (int64_t)B * max_kv_splits < INT32_MAX) {
+    // share each tile starts and ends sooner than one of waves that meet at the end: 8 requests, 128 heads, up to 64 / 300 / 1152 / 4096
+    // tokens: 12.1 / 15.4 / 23.0 / 45.4 us against 12.9 / 16.9 / 21.4 / 31.6; one request 11.6 / 14.4 / 20.9 / 41.4 against 12.7 / 17.1 /
+    // 19.9 / 28.2.  (How long the requests are is not known here.)  From 9 requests on the other is within a few percent where it is
+    // not faster (16 of up to 64 / 128 / 300 / 1152: 13.5 / 15.5 / 20.5 / 31.5 against 13.0 / 16.4 / 18.5 / 27.0).  A launch holds fewer
+    // than 2^32 threads, and 65535 rows of blocks.
+    if (units * max_kv_splits > 256 && group >= 32 && units * max_kv_splits < (1 << 24) && (int64_t)B * max_kv_splits <= 500000 && units / B <= 65535) {
       fewer = mla_fewer_splits(B, units, max_kv_splits);
-      const LatentArgs la{(const uint16_t*)q, (const uint16_t*)k_buffer, kv_indptr, kv_indices, num_kv_splits, gate, attn_logits, attn_lse, o, B, Hq,
-                          Hkv, (group + 31) / 32, max_kv_splits, q_stride_b, q_stride_h, k_stride_n, k_stride_h, o_stride_b, o_stride_h, sm_scale, logit_cap};
+      LatentArgs la{(const uint16_t*)q, (const uint16_t*)k_buffer, kv_indptr, kv_indices, num_kv_splits, gate, attn_logits, attn_lse, o, B, Hq,
+                    Hkv, (group + 31) / 32, group, max_kv_splits, 0, 0, 0.f, q_stride_b, q_stride_h, k_stride_n, k_stride_h, o_stride_b, o_stride_h,
+                    sm_scale, logit_cap};
+      latent_places(la);
+      const dim3 grid(8, Hkv * la.head_tiles, (la.units + 7) / 8);
       SGLK_DISPATCH_HALF(dtype, T, {
         if (logit_cap > 0.f) {
           if (int rc = ensure_lds<latent_decode_kernel<T, true>>(kLatLds)) return rc;
-          hipLaunchKernelGGL((latent_decode_kernel<T, true>), dim3((unsigned)blocks), dim3(256), kLatLds, s, la, fewer);
+          hipLaunchKernelGGL((latent_decode_kernel<T, true>), grid, dim3(256), kLatLds, s, la, fewer);
         } else {
           if (int rc = ensure_lds<latent_decode_kernel<T, false>>(kLatLds)) return rc;
-          hipLaunchKernelGGL((latent_decode_kernel<T, false>), dim3((unsigned)blocks), dim3(256), kLatLds, s, la, fewer);
+          hipLaunchKernelGGL((latent_decode_kernel<T, false>), grid, dim3(256), kLatLds, s, la, fewer);
         }
         SGLK_LAUNCH_CHECK();
         hipLaunchKernelGGL((latent_merge_kernel<T>), dim3(B, (Hq + 3) / 4), dim3(256), 0, s, la, fewer);

@@ -118,3 +118,21 @@ def test_blocks_of_minus_infinity(splits):
     assert (o[keep].double() - want[keep]).abs().max().item() <= 2.0**-8 * (v + want[keep].abs().max()).item() + 1e-4
     got = torch.logsumexp(torch.where(lse.isnan(), torch.full_like(lse, -math.inf), lse), -1)
     assert (got[keep].double() - wlse[keep]).abs().max().item() <= 2.0**-8 + 1e-4
+
+
+@pytest.mark.parametrize("Hq,lens,most", [
+    (128, [300] * 3 + [40] * 8 + [700, 1] + [33] * 6, 8),      # more than the blocks every request has a place for, and fewer
+    (128, [1500] + [10] * 69, 8),                              # one long request among more than a wave's lanes
+    (64, [20] * 66 + [2000, 900, 0, 1200], 5),                 # ... behind them, and one without tokens
+    (32, [700, 30] * 8, 64),                                   # splits that have to be folded eight at a time
+    (72, [64, 128, 129, 640] * 6, 16),                         # 85 places of three head tiles
+])
+def test_blocks_are_found(Hq, lens, most):
+    """Requests with more and fewer blocks than they have a place for by their number: every row, and every log-sum-exp."""
+    kv, q = _data(lens, Hq, torch.bfloat16, len(lens) + Hq)
+    o, lse, want, wlse = _run(lens, Hq, most, torch.bfloat16, kv, q)
+    keep = [b for b, n in enumerate(lens) if n]
+    assert all(o[b].isnan().all() for b, n in enumerate(lens) if n == 0)
+    assert (o[keep].double() - want[keep]).abs().max().item() <= 2.0**-8 * (kv.abs().max().double() + want[keep].abs().max()).item() + 1e-4
+    got = torch.logsumexp(torch.where(lse.isnan(), torch.full_like(lse, -math.inf), lse), -1)
+    assert (got[keep].double() - wlse[keep]).abs().max().item() <= 2.0**-8 + 1e-4
