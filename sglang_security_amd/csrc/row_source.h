@@ -58,7 +58,7 @@ __device__ __forceinline__ void source8(const RowSource& s, int64_t row, int col
     ld8<T>(s.p, row * s.stride + col, v);
 }
 
-// one element; the splits are requested eight at a time and added in the same order
+// one element; the splits, as many as there are, are requested eight at a time and added in the same order
 template <typename T>
 __device__ __forceinline__ float source1(const RowSource& s, int64_t row, int col) {
   if (!s.f32) return ld<T>(s.p, row * s.stride + col);
@@ -67,7 +67,10 @@ __device__ __forceinline__ float source1(const RowSource& s, int64_t row, int co
   for (int first = 0; first < s.splits; first += 8) {
     float part[8];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) part[u] = p[min(first + u, s.splits - 1) * s.part_stride];
+    for (int u = 0; u < 8; ++u) {
+      part[u] = 0.f;
+      if (first + u < s.splits) part[u] = p[(first + u) * s.part_stride];  // (a scalar branch)
+    }
 #pragma unroll
     for (int u = 0; u < 8; ++u)
       if (first + u < s.splits) v += part[u];
