@@ -309,8 +309,14 @@ __device__ __forceinline__ void merge_splits(const float* part, const float* lse
     if (first + u >= live) break;
     const float n_max = fmaxf(tl[u], e_max);
     const float old = expf(e_max - n_max), w = expf(tl[u] - n_max);
-    acc = acc * old + w * tv[u];
-    e_sum = e_sum * old + w;
+    // (which product is rounded by itself is written out: the same rows whatever they are inlined into)
+    if constexpr (sizeof(V) == sizeof(float)) {
+      acc = fmaf(acc, old, w * tv[u]);
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[r] = fmaf(w, tv[u][r], acc[r] * old);
+    }
+    e_sum = fmaf(e_sum, old, w);
     e_max = n_max;
   }
 }
