@@ -161,7 +161,8 @@ __global__ void __launch_bounds__(256) gptq_repack_kernel(const int32_t* __restr
 // The same over whole tiles, with row-contiguous stores: a wave takes one 128-k group of 64 columns (four 1-KiB strip
 // tiles), parks the packed words in LDS with the eight column words of every (k-octet, 8-column half) side by side,
 // and each lane then builds 8 neighbouring columns of one row per step: two 16-byte LDS reads, one 16-byte store, a
-// row's 128 bytes from eight adjacent lanes.  Needs N % 64 == 0 and group_size % 128 == 0.
+// row's 128 bytes from eight adjacent lanes.  Needs N % 64 == 0 and group_size % 128 == 0.  (For callers that want the operand
+// as [K, N]; this package's own products read its transpose, below.)
 template <typename T>
 __global__ void __launch_bounds__(256) awq_dequant_packed_tile_kernel(const int32_t* __restrict__ packed,
                                                                       const uint16_t* __restrict__ scales,

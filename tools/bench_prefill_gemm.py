@@ -40,10 +40,9 @@ for name, K, N in [("qkv", 4096, 6144), ("o", 4096, 4096), ("gate_up", 4096, 286
     out = torch.empty(M, N, dtype=torch.bfloat16, device=dev)
     flops = 2.0 * M * K * N
     t_fused = timeit(lambda: ops.awq_gemm_prefill(x, packed, sc, qz, None, out))
-    wd = ops.awq_dequantize_packed(packed, sc, qz)
-    t_deq = timeit(lambda: ops.awq_dequantize_packed(packed, sc, qz))
-    t_lib = timeit(lambda: torch.matmul(x, wd, out=out))
-    wt = wd.t().contiguous()
+    wt = ops.awq_dequantize_packed_nk(packed, sc, qz)
+    t_deq = timeit(lambda: ops.awq_dequantize_packed_nk(packed, sc, qz))
+    t_lib = timeit(lambda: torch.matmul(x, wt.t(), out=out))
     t_dense = timeit(lambda: ops.dense_gemm_prefill(x, wt, None, out))
     print(f"{name:8s} M={M} K={K:6d} N={N:6d}  fused int4 {t_fused:8.1f} us ({flops / t_fused / 1e6:6.0f} TFLOP/s)   "
           f"dense hand-written {t_dense:8.1f} us ({flops / t_dense / 1e6:6.0f})   library {t_lib:8.1f} us "
