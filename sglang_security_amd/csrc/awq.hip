@@ -23,6 +23,7 @@
 #include <mutex>
 
 #include "awq_common.h"
+#include "awq_rows16.h"
 
 namespace sglk {
 
@@ -658,7 +659,8 @@ struct ZpOnMatrixCores<bf16_t> {
 // of being computed here: one barrier per stage instead of two.  partial_mode: every split stores its fp32 tile
 // row-major to partial[split][M][N] and returns; the consumer kernel adds the splits up.
 // MT: 32-row tiles of the 64-row block that are multiplied (batches of up to 32 rows skip the matrix work of the
-// rows they do not have; staging, reduction and stores keep the 64-row shape, the skipped tile is zeros).
+// rows they do not have; staging, reduction and stores keep the 64-row shape, the skipped tile is zeros).  Batches of at
+// most 16 rows come here only in a chain; alone they run on awq_rows16.h.
 //
 // One projection is a WideJob.  awq_gemm_wide_kernel runs one job, a block per (column tile, split, row block).
 // awq_chain_kernel (CHAIN) runs a list of jobs in ONE launch of persistent blocks, job j + 1 reading what job j wrote:
@@ -1515,6 +1517,10 @@ static int static_prepare_kernels() {
   if (int rc = ensure_lds<&awq_gemm_wide_kernel<T, false, 2>>(Wide::kLds)) return rc;
   if (int rc = ensure_lds<&awq_gemm_wide_kernel<T, true, 1>>(Wide::kLds)) return rc;
   if (int rc = ensure_lds<&awq_gemm_wide_kernel<T, true, 2>>(Wide::kLds)) return rc;
+  if (int rc = ensure_lds<&awq_rows16_kernel<T, 4, 1, 8>>(4 * AwqRows16::kTile * 4)) return rc;
+  if (int rc = ensure_lds<&awq_rows16_kernel<T, 4, 2, 8>>(4 * AwqRows16::kTile * 4)) return rc;
+  if (int rc = ensure_lds<&awq_rows16_kernel<T, 4, 2, 16>>(8 * AwqRows16::kTile * 4)) return rc;
+  if (int rc = ensure_lds<&awq_rows16_kernel<T, 8, 1, 8>>(8 * AwqRows16::kTile * 4)) return rc;
   if (int rc = ensure_lds<&awq_gemm_kernel<T, 4, 2, 6>>(GemmGeom<4, 2, 6>::kLds)) return rc;
   if (int rc = ensure_lds<&awq_gemm_kernel<T, 4, 1, 6>>(GemmGeom<4, 1, 6>::kLds)) return rc;
   if (int rc = ensure_lds<&awq_gemm_kernel<T, 4, 1, 4>>(GemmGeom<4, 1, 4>::kLds)) return rc;
@@ -1645,6 +1651,42 @@ static int launch_awq_wide(const WidePlan& wp, const void* x, const int32_t* pac
   return SGLK_OK;
 }
 
+// At most 16 rows on the wide kernel's blocks and splits (awq_rows16.h).
+static int launch_awq_rows16(const WidePlan& wp, const void* x, const int32_t* packed, const void* scales,
+                             const int32_t* qzeros, const void* bias, void* out, float* partial, int* tickets, int M, int N,
+                             int K, int64_t x_stride, int64_t out_stride, int dtype, int partial_mode, hipStream_t s,
+                             int act_mode = 0, float* xsum_out = nullptr, int64_t xs_out_stride = 0) {
+  const int groups = wp.stages_per_split * (Wide::kStageK / 128);
+  const dim3 grid(N / 128, wp.splits);
+  SGLK_DISPATCH_HALF(dtype, T, {
+    const AwqRows16Args<T> a{(const uint16_t*)x, packed, (const uint16_t*)scales, qzeros, (const uint16_t*)bias,
+                             (uint16_t*)out, partial, tickets, xsum_out, x_stride, out_stride, xs_out_stride, M, N, K,
+                             groups, wp.splits, partial_mode, act_mode};
+#define SGLK_ROWS16(S, R, NW)                                                                                    \
+  {                                                                                                              \
+    constexpr int kLds = NW * S / 8 * AwqRows16::kTile * 4;                                                      \
+    if (int rc = ensure_lds<&awq_rows16_kernel<T, S, R, NW>>(kLds)) return rc;                                   \
+    hipLaunchKernelGGL((awq_rows16_kernel<T, S, R, NW>), grid, dim3(64 * NW), kLds, s, a);                       \
+  }
+    // One or two groups a wave: all of them at once (4096 x 4096 in one-stage splits 7.7 -> 4.6 us, 4096 x 6144 in two-stage
+    // splits 9.3 -> 5.5; 16 waves 6.1).  Longer splits: 16 waves of two groups (one row, 4096 x 28672 23.2 -> 14.6, 14336 x
+    // 4096 14.4 -> 8.8; four groups and 8 waves 16.4 and 9.7) while x is small; from nine rows on a wave takes all 128 columns,
+    // so that x is read once a block instead of twice (16 rows 23.4 -> 16.7 and 14.5 -> 10.6, against 18.4 and 10.7; at 8 rows
+    // 15.9 and 9.8 against 15.4 and 9.2).
+    if (groups <= 4)
+      SGLK_ROWS16(4, 1, 8)
+    else if (groups <= 8)
+      SGLK_ROWS16(4, 2, 8)
+    else if (M <= 8)
+      SGLK_ROWS16(4, 2, 16)
+    else
+      SGLK_ROWS16(8, 1, 8)
+  });
+#undef SGLK_ROWS16
+  SGLK_LAUNCH_CHECK();
+  return SGLK_OK;
+}
+
 int sglk_awq_gemm_partial_splits(int M, int N, int K, int group_size) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   const WidePlan wp = plan_awq_wide(M, N, K, group_size, true);
@@ -1662,6 +1704,9 @@ int sglk_awq_gemm_partial(const void* x, const int32_t* packed, const void* scal
   if (!wp.ok)
     return fail(SGLK_EUNSUP, "awq_gemm_partial: needs K %% 512 == 0, N %% 128 == 0 and group size 128 (K=%d N=%d G=%d)", K,
                 N, group_size);
+  if (M <= AwqRows16::kRows)
+    return launch_awq_rows16(wp, x, packed, scales, qzeros, nullptr, nullptr, partial, nullptr, M, N, K, x_stride, N, dtype,
+                             1, (hipStream_t)stream);
   return launch_awq_wide(wp, x, packed, scales, qzeros, nullptr, nullptr, partial, nullptr, M, N, K, x_stride, N, dtype,
                          xsum, xs_stride, 1, (hipStream_t)stream);
 }
@@ -1681,6 +1726,9 @@ int sglk_awq_gemm_silu_mul(const void* x, const int32_t* packed, const void* sca
   // the activation needs whole sums: one split, whatever the planner would pick
   wp.stages_per_split = K / Wide::kStageK;
   wp.splits = 1;
+  if (M <= AwqRows16::kRows)
+    return launch_awq_rows16(wp, x, packed, scales, qzeros, nullptr, out, nullptr, nullptr, M, N, K, x_stride, out_stride,
+                             dtype, 0, (hipStream_t)stream, 1, xsum_out, xs_out_stride);
   return launch_awq_wide(wp, x, packed, scales, qzeros, nullptr, out, nullptr, nullptr, M, N, K, x_stride, out_stride,
                          dtype, xsum, xs_stride, 0, (hipStream_t)stream, 1, xsum_out, xs_out_stride);
 }
@@ -1788,6 +1836,13 @@ int sglk_awq_gemm_xs(const void* x, const int32_t* packed, const void* scales, c
   int* tickets = reinterpret_cast<int*>(workspace);
   float* partial = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + (int64_t)kMaxTiles * 4);
   const WidePlan wp = plan_awq_wide(M, N, K, group_size);
+  // few rows: also where a split is a single stage, as long as the slabs (a quarter of the wide kernel's) fit the workspace
+  // that sglk_awq_gemm_workspace_bytes names
+  if (M <= AwqRows16::kRows && wp.splits > 0 && wp.tiles <= kMaxTiles &&
+      (wp.splits == 1 || (int64_t)wp.tiles * wp.splits * (AwqRows16::kRows * 128 * 4) + (int64_t)kMaxTiles * 4 <=
+                             sglk_awq_gemm_workspace_bytes(M, N, K)))
+    return launch_awq_rows16(wp, x, packed, scales, qzeros, bias, out, partial, tickets, M, N, K, x_stride, out_stride, dtype,
+                             0, s);
   if (wp.ok && wp.tiles <= kMaxTiles && aligned16(out) && out_stride % 8 == 0)
     return launch_awq_wide(wp, x, packed, scales, qzeros, bias, out, partial, tickets, M, N, K, x_stride, out_stride,
                            dtype, xsum, xs_stride, 0, s);

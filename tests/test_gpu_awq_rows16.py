@@ -1,0 +1,74 @@
+"""int4 products of at most 16 rows (awq_rows16.h) at the edges of its rule: one row, the last rows of either form, one row
+beyond; splits of one stage (a group a wave), two, and many with a remainder; each way out of the kernel."""
+import pytest
+import torch
+
+from test_gpu_ops import _awq_case, _gemm_close
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+# (K, N): one group a wave / two / a split of 13 groups in turns of 8, last split shorter / one split of 28 groups
+SHAPES = [(512, 128), (4096, 4096), (4096, 6144), (14336, 4096), (3584, 32768)]
+
+
+def _case(M, K, N, dtype, interleave=False):
+    import oracle
+    from sglang_security_amd import ops
+
+    x, qw, sc, qz = _awq_case(M, K, N, 128, dtype, seed=M + K + N)
+    w = [t.to(DEV) for t in (qw, sc, qz)]
+    if interleave:
+        w = ops.awq_interleave_gate_up(*w)
+    return ops, x.to(DEV), (ops.awq_repack(w[0]), w[1], w[2]), oracle.awq_gemm(x, qw, sc, qz)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17])
+@pytest.mark.parametrize("K,N", SHAPES[:4])
+def test_products_and_split_sums(M, K, N, dtype):
+    ops, x, w, want = _case(M, K, N, dtype)
+    wide = torch.randn(M, K + 64, device=DEV).to(dtype)       # rows with something behind them
+    wide[:, :K] = x
+    part = torch.full((ops.awq_gemm_partial_splits(M, N, K), M, N), float("nan"), device=DEV)
+    ops.awq_gemm_partial(wide[:, :K], *w, part)
+    _gemm_close(part.sum(0).to(dtype).cpu(), want, dtype)
+    bias = torch.randn(N, device=DEV).to(dtype)
+    work = torch.zeros(max(ops.awq_gemm_workspace_bytes(M, N, K), 256), dtype=torch.uint8, device=DEV)
+    out = torch.full((M + 1, N + 8), 7.0, dtype=dtype, device=DEV)
+    for _ in range(2):                                          # the tickets are back at zero
+        ops.awq_gemm(x, *w, bias=bias, out=out[:M, :N], workspace=work)
+        _gemm_close(out[:M, :N].cpu(), (want.float() + bias.float().cpu()).to(dtype), dtype)
+    assert (out[M:] == 7).all() and (out[:, N:] == 7).all()
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+@pytest.mark.parametrize("K,N", [(512, 256), (3584, 32768)])
+def test_gated_activation(M, K, N):
+    ops, x, w, want = _case(M, K, N, torch.bfloat16, interleave=True)
+    out = torch.full((M, N // 2), float("nan"), dtype=torch.bfloat16, device=DEV)
+    xs = torch.zeros(N // 256, M + 2, device=DEV)
+    ops.awq_gemm_silu_mul(x, *w, out, None, xs)
+    gate, up = want.float().chunk(2, 1)
+    act = torch.nn.functional.silu(gate).to(torch.bfloat16).float() * up
+    _gemm_close(out.cpu(), act, torch.bfloat16)
+    sums = out.double().view(M, -1, 128).sum(2).t()
+    # 64 additions of fp32 in either addend, values below 4
+    torch.testing.assert_close(xs[:, :M].double(), sums, rtol=0, atol=128 * 4 * 2 ** -23 * 8)
+    assert (xs[:, M:] == 0).all()
+
+
+@pytest.mark.parametrize("M", [1, 16])
+def test_zero_scales_and_rows_that_are_not_numbers(M):
+    """A column whose scales are zero is zero; a row of x that is not a number stays with itself."""
+    ops, x, (packed, sc, qz), _ = _case(M, 4096, 6144, torch.bfloat16)
+    sc = sc.clone()
+    sc[:, 5] = 0
+    x = x.clone()
+    clean = torch.empty(M, 6144, dtype=torch.bfloat16, device=DEV)
+    part = torch.empty(ops.awq_gemm_partial_splits(M, 6144, 4096), M, 6144, device=DEV)
+    ops.awq_gemm_partial(x, packed, sc, qz, part)
+    clean = part.sum(0)
+    assert (clean[:, 5] == 0).all() and (clean[:, 6] != 0).any()
+    x[M - 1, 100] = float("nan")
+    ops.awq_gemm_partial(x, packed, sc, qz, part)
+    assert torch.equal(part.sum(0)[: M - 1], clean[: M - 1]) and part.sum(0)[M - 1].isnan().all()
