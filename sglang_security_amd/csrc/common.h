@@ -225,15 +225,31 @@ __device__ __forceinline__ float scaled_sum(float acc, float row_scale, float co
 }
 
 // ---- wave (64 lanes) reductions ----------------------------------------------------------------
+// Sums and maxima over a wave in the order of a butterfly (lanes 32, 16, 8, 4, 2, 1 apart), on the vector unit: halves and
+// rows are exchanged by permlane swaps, lanes of a row by DPP operands.  Through __shfl_xor every step is a trip to LDS and
+// back, some 60 cycles that nothing hides in a kernel of one reduction; the bits are the same.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, false);
+}
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E;         // quad_perm 1 0 3 2 and 2 3 0 1
+constexpr int kDppRor4 = 0x124, kDppRor8 = 0x128;       // rotation inside rows of 16
+template <typename F>
+__device__ __forceinline__ float wave_fold(float v, F f) {
+  const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(h[0]), __uint_as_float(h[1]));
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  v = f(v, __uint_as_float(dpp<kDppRor8>(__float_as_uint(v))));
+  v = f(v, __uint_as_float(dpp<kDppRor4>(__float_as_uint(v))));  // (equal eight lanes apart: a rotation by 4 is the lane 4 apart)
+  v = f(v, __uint_as_float(dpp<kDppXor2>(__float_as_uint(v))));
+  return f(v, __uint_as_float(dpp<kDppXor1>(__float_as_uint(v))));
+}
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  return wave_fold(v, [](float a, float b) { return a + b; });
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
+  return wave_fold(v, [](float a, float b) { return fmaxf(a, b); });
 }
 
 // One rotary pair in fp32 with a fixed operation order (two roundings per output), so that every kernel that rotates
