@@ -5,6 +5,7 @@
 
 #include <cstdarg>
 #include <cstdio>
+#include <type_traits>
 
 #include "sglk.h"
 
@@ -250,6 +251,22 @@ __device__ __forceinline__ float wave_sum(float v) {
 }
 __device__ __forceinline__ float wave_max(float v) {
   return wave_fold(v, [](float a, float b) { return fmaxf(a, b); });
+}
+// the sum over this lane and the lanes in front of it (whole numbers: in any order)
+__device__ __forceinline__ uint64_t wave_scan(uint64_t v) {
+  auto step = [&](auto ctrl, auto rows) {
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), decltype(ctrl)::value, decltype(rows)::value, 0xF, false);
+    v += ((uint64_t)hi << 32) | lo;
+  };
+  using std::integral_constant;
+  step(integral_constant<int, 0x111>(), integral_constant<int, 0xF>());  // row_shr 1, 2, 4, 8: nothing enters a row
+  step(integral_constant<int, 0x112>(), integral_constant<int, 0xF>());
+  step(integral_constant<int, 0x114>(), integral_constant<int, 0xF>());
+  step(integral_constant<int, 0x118>(), integral_constant<int, 0xF>());
+  step(integral_constant<int, 0x142>(), integral_constant<int, 0xA>());  // a row's last lane to the next row: rows 1 and 3
+  step(integral_constant<int, 0x143>(), integral_constant<int, 0xC>());  // lane 31 to rows 2 and 3
+  return v;
 }
 
 // One rotary pair in fp32 with a fixed operation order (two roundings per output), so that every kernel that rotates

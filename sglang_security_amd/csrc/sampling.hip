@@ -10,13 +10,18 @@
 // is wide enough (sixteen bins an octave) that the chosen bins fit an LDS list, and the other digits are taken from
 // there; rows are read in 16-byte pieces, eight in flight a thread.
 //
-// Measured, 64 rows of 128256, top-k and top-p together: sampling 555 us (256 bins for four 8-bit digits each, a float
-// atomic on a handful of exponents for every element, a thread's elements 500 bytes from the next thread's) -> 81 us with
-// a block a row, 45 us with its rows spread over four blocks; top-p renormalisation 390 -> 66 -> 44 us.  Rows that the guess
-// does not hold for are done over by one block behind the spread launches: sampling from 64 rows of one certain token each
-// (fewer than k above the mean) 615 us at first, 99 unspread, 118 spread; of nearly equal values (bins beyond the lists) 674,
-// 148, 175; one certain row among 64 574, 92, 124.
+// Measured, 64 rows of 128256 out of memory, top-k and top-p together: sampling 555 us (256 bins for four 8-bit digits each, a
+// float atomic on a handful of exponents for every element, a thread's elements 500 bytes from the next thread's) -> 81 us
+// with a block a row, 46.5 with its rows spread over four blocks in four launches, 36 in three; top-p renormalisation 390 -> 66 ->
+// 41.6 -> 37.  (One row of 32000: 28.5 -> 24 and 21.4 -> 19.)  The last step: an element's bin word is bits that it has, where
+// its fixed-point mass took fifteen instructions; the slice is asked for before the cuts are looked for; lists of candidates
+// are counted by the whole block, not walked by a wave (two thousand of them: 6 us); scans run on DPP operands, not through
+// LDS; the chunks' masses are added up beside the search for candidates, a launch less.
+// Rows that the guess does not hold for are done over by one block behind the spread launches: sampling from 64 rows of one certain
+// token each (fewer than k above the mean) 615 us at first, 99 unspread, 118 spread; of nearly equal values (bins beyond the
+// lists) 674, 148, 175; one certain row among 64 574, 92, 124.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
@@ -82,10 +87,14 @@ __device__ __forceinline__ float bmax(float v, float* red) {
 template <typename V>
 __device__ __forceinline__ V bscan(V v, V* red, V& total) {
   V incl = v;
+  if constexpr (std::is_same_v<V, u64>) {
+    incl = wave_scan(v);
+  } else {
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const V u = __shfl_up(incl, o, 64);
-    if ((int)(threadIdx.x & 63) >= o) incl += u;
+    for (int o = 1; o < 64; o <<= 1) {
+      const V u = __shfl_up(incl, o, 64);
+      if ((int)(threadIdx.x & 63) >= o) incl += u;
+    }
   }
   if ((threadIdx.x & 63) == 63) red[threadIdx.x >> 6] = incl;
   __syncthreads();
@@ -222,60 +231,39 @@ __device__ uint32_t refine(const float* __restrict__ x, int n, SampShared& sh, c
   return prefix;
 }
 
-// The same from a list, by one wave: digits of 6, 6 and 7 bits, two bins a lane, no block barrier.
+// One digit of the same, by one wave from 64 or 128 bins, two a lane, which it leaves at zero.  Returns the digit; rank and
+// below go on into it.
 template <bool COUNT>
-__device__ uint32_t refine_list(u64* bins, const Fixed& fx, const uint32_t* list, int listed, int bin, uint32_t rank, u64 below, u64 target,
-                                uint32_t lo) {
+__device__ __forceinline__ int pick_digit(u64* bins, const Fixed& fx, uint32_t& rank, u64& below, u64 target) {
   const int lane = threadIdx.x & 63;
-  uint32_t prefix = (uint32_t)bin << 19;
-  int bits = 19;
-  if (!COUNT && target == 0) target = 1;
-#pragma unroll
-  for (int digit = 0; digit < 3; ++digit) {
-    const int take = digit < 2 ? 6 : 7, shift = bits - take;
-    bins[2 * lane] = bins[2 * lane + 1] = 0;
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // one wave: its LDS accesses are done in order
-    for (int i = lane; i < listed; i += 64) {
-      const uint32_t b = list[i];
-      if ((b >> bits) == (prefix >> bits) && b >= lo) atomicAdd(&bins[(b >> shift) & ((1u << take) - 1)], (1ull << fx.bits) + fx.of(b));
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    const u64 w0 = bins[2 * lane], w1 = bins[2 * lane + 1];
-    u64 incl = w0 + w1;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const u64 v = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += v;
-    }
-    const u64 total = __shfl(incl, 63, 64), before = incl - (w0 + w1);
-    int d = -1;
-    if (COUNT) {
-      const uint32_t c0 = fx.count(w0), c1 = fx.count(w1);
-      uint32_t above = fx.count(total) - fx.count(before) - c0 - c1;
-      uint32_t need = 0;
-      if (above < rank && rank <= above + c1) d = 2 * lane + 1, need = rank - above;
-      above += c1;
-      if (above < rank && rank <= above + c0) d = 2 * lane, need = rank - above;
-      const u64 who = __ballot(d >= 0);
-      const int src = who ? __ffsll(who) - 1 : 0;
-      d = max(__shfl(d, src, 64), 0);
-      rank = __shfl(need, src, 64);
-    } else {
-      const u64 m0 = fx.mass(w0), m1 = fx.mass(w1);
-      const bool reach = below + fx.mass(total) >= target;  // else: the last bin with mass
-      u64 at = below + fx.mass(before), run = at;
-      if (m0 > 0 && (reach ? run + m0 >= target : true)) d = 2 * lane, at = run;
-      run += m0;
-      if (m1 > 0 && (reach ? d < 0 && run + m1 >= target : true)) d = 2 * lane + 1, at = run;
-      const u64 who = __ballot(d >= 0);
-      const int src = !who ? 0 : reach ? __ffsll(who) - 1 : 63 - __clzll(who);
-      d = max(__shfl(d, src, 64), 0);
-      if (who) below = __shfl(at, src, 64);
-    }
-    prefix |= (uint32_t)d << shift;
-    bits = shift;
+  const u64 w0 = bins[2 * lane], w1 = bins[2 * lane + 1];
+  bins[2 * lane] = bins[2 * lane + 1] = 0;
+  const u64 incl = wave_scan(w0 + w1), total = __shfl(incl, 63, 64), before = incl - (w0 + w1);
+  int d = -1;
+  if (COUNT) {
+    const uint32_t c0 = fx.count(w0), c1 = fx.count(w1);
+    uint32_t above = fx.count(total) - fx.count(before) - c0 - c1;
+    uint32_t need = 0;
+    if (above < rank && rank <= above + c1) d = 2 * lane + 1, need = rank - above;
+    above += c1;
+    if (above < rank && rank <= above + c0) d = 2 * lane, need = rank - above;
+    const u64 who = __ballot(d >= 0);
+    const int src = who ? __ffsll(who) - 1 : 0;
+    d = max(__shfl(d, src, 64), 0);
+    rank = __shfl(need, src, 64);
+  } else {
+    const u64 m0 = fx.mass(w0), m1 = fx.mass(w1);
+    const bool reach = below + fx.mass(total) >= target;  // else: the last bin with mass
+    u64 at = below + fx.mass(before), run = at;
+    if (m0 > 0 && (reach ? run + m0 >= target : true)) d = 2 * lane, at = run;
+    run += m0;
+    if (m1 > 0 && (reach ? d < 0 && run + m1 >= target : true)) d = 2 * lane + 1, at = run;
+    const u64 who = __ballot(d >= 0);
+    const int src = !who ? 0 : reach ? __ffsll(who) - 1 : 63 - __clzll(who);
+    d = max(__shfl(d, src, 64), 0);
+    if (who) below = __shfl(at, src, 64);
   }
-  return prefix;
+  return d;
 }
 
 struct RowParams {
@@ -556,13 +544,10 @@ __device__ void walk_chunk(const float* __restrict__ x, int n, float thr, int64_
           if (r > target) at = min(at, mine);
         }
       }
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        at = min(at, __shfl_xor(at, o, 64));
-        mine = max(mine, __shfl_xor(mine, o, 64));
-      }
-      if (at < (1 << 30)) pick = at;
-      last = max(last, mine);
+      // lanes are in the elements' order: the first lane that has one past the target, the last that has one at all
+      const u64 past = __ballot(at < (1 << 30)), some = __ballot(mine >= 0);
+      if (past) pick = __builtin_amdgcn_readlane(at, __ffsll(past) - 1);
+      if (some) last = __builtin_amdgcn_readlane(mine, 63 - __clzll(some));
       run += __shfl(incl, 63, 64);
     }
     if (pick < 0) pick = last;  // rounding at the chunk's end: its last kept element
@@ -718,8 +703,8 @@ __global__ void __launch_bounds__(256) short_rows_kernel(SampArgs a) {
 // ---- rows spread over several blocks --------------------------------------------------------------------------------
 // A unit streams about 20 bytes a clock of a row that the caches do not hold, and a batch of 64 rows leaves three of four
 // units idle.  The same selection in launches that meet at their ends: bins per slice; every block adds its row's bins up
-// and collects its slice's candidates; every block finishes the threshold and writes (or sums) its slice; one block per
-// row picks.  The first digit has a window of 1024 bins (2^64 of the least value binned).  Rows the guess of mass one does
+// and collects its slice's candidates; every block finishes the threshold and writes its slice, or, sampling, one block per
+// row finishes it and picks.  The first digit has a window of 1024 bins (2^64 of the least value binned).  Rows the guess of mass one does
 // not hold for, or whose candidates overflow a list, are done whole by one block of the last launch.
 constexpr int kWindow = 1024;
 constexpr int kMaxSlices = 16;
@@ -730,18 +715,18 @@ struct RowState {
   u64 below, target, above;
   int valid, kbin, pbin, kcount, pcount;
   uint32_t rank;
-  float vmax, thr;
+  float vmax;
 };
 struct SampWs {  // of one row
   u64* bins;        // [slices][kWindow]
   SliceStat* stat;  // [slices]
   RowState* state;
-  uint32_t* fill;   // [2]
   uint32_t* list;   // [2][kList]
+  uint32_t* place;  // [2][kList]: where in the row (sampling)
   float* chunk;     // [kBins]
 };
 __host__ __device__ inline int64_t samp_ws_row(int slices) {
-  return (int64_t)slices * (kWindow * 8 + 16) + 128 + 16 + 2 * kList * 4 + kBins * 4;
+  return (int64_t)slices * (kWindow * 8 + 16) + 128 + 4 * kList * 4 + kBins * 4;
 }
 __device__ __forceinline__ SampWs samp_ws(const SampArgs& a, int row) {
   char* w = a.ws + (int64_t)row * samp_ws_row(a.slices);
@@ -752,9 +737,9 @@ __device__ __forceinline__ SampWs samp_ws(const SampArgs& a, int row) {
   w += 128;
   r.stat = reinterpret_cast<SliceStat*>(w);
   w += a.slices * 16;
-  r.fill = reinterpret_cast<uint32_t*>(w);
-  w += 16;
   r.list = reinterpret_cast<uint32_t*>(w);
+  w += 2 * kList * 4;
+  r.place = reinterpret_cast<uint32_t*>(w);
   w += 2 * kList * 4;
   r.chunk = reinterpret_cast<float*>(w);
   return r;
@@ -780,198 +765,419 @@ __device__ __forceinline__ Guess guess_of(const RowParams& rp, int n) {
   return g;
 }
 
+// A slice in pieces of four elements, piece u of a thread the (threadIdx.x + 1024 u)-th: a wave's piece is a chunk of 256.
+// The first eight are asked for by hold(), before whatever the block has to find out first, and are there when it has; longer
+// slices go on from memory.
+constexpr int kHeld = 8;
 template <bool VEC>
-__global__ void __launch_bounds__(kSampThreads) slice_bins_kernel(SampArgs a) {
-  __shared__ SampShared sh;
-  const int slice = blockIdx.x, row = blockIdx.y, lo = slice * a.slice, n = min(a.slice, a.n - lo);
-  const float* x = a.probs + (int64_t)row * a.in_stride + lo;
-  const RowParams rp = load_params(a, row);
-  const Guess g = guess_of(rp, a.n);
-  const SampWs w = samp_ws(a, row);
-  clear_bins(sh, kWindow);
-  float s = 0.f, o = 0.f, mx = 0.f;
-  const bool bin = g.use_k || g.use_p;
-  each<VEC, 4>(x, n, [&](float raw) {
-    const float v = fmaxf(raw, 0.f);
-    const uint32_t b = __float_as_uint(v);
-    const bool in = bin && v >= g.least;
-    mx = fmaxf(mx, v);
-    s += in ? 0.f : v;
-    o += in ? v : 0.f;
-    if (in) atomicAdd(&sh.bin[min((int)(b >> 19) - g.base, kWindow - 1)], (1ull << g.fx.bits) + g.fx.of(b));
-  });
-  mx = bmax(mx, sh.red);
-  s = bsum(s, sh.red);
-  o = bsum(o, sh.red);
-  if (threadIdx.x == 0) w.stat[slice] = SliceStat{s, o, mx, 0.f};
-  if (slice == 0 && threadIdx.x < 2) w.fill[threadIdx.x] = 0;
-  if (bin) w.bins[slice * kWindow + threadIdx.x] = sh.bin[threadIdx.x];
+__device__ __forceinline__ float4v slice_piece(const float* __restrict__ x, int n, int i) {
+  float4v v = {0.f, 0.f, 0.f, 0.f};
+  if (VEC && 4 * i + 4 <= n) {
+    v = *reinterpret_cast<const float4v*>(x + 4 * i);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (4 * i + e < n) v[e] = x[4 * i + e];
+  }
+  return v;
+}
+// (A slice has 8192 - 15 x 255 elements at least, the last one too.  What does not lie in a whole wave of pieces is read again below.  No branch, so
+// that what was asked for before can be waited for without these.)
+template <bool VEC>
+__device__ __forceinline__ void hold(const float* __restrict__ x, int n, float4v (&r)[kHeld]) {
+#pragma unroll
+  for (int u = 0; u < kHeld; ++u)
+    if constexpr (VEC)
+      r[u] = *reinterpret_cast<const float4v*>(x + 4 * min((int)threadIdx.x + u * kSampThreads, (n >> 2) - 1));
+  __builtin_amdgcn_sched_barrier(0);
+}
+// f(piece, its place, elements of it): whole waves, with pieces of no elements behind the slice's end.  Where a wave's pieces are
+// whole (a scalar question) they are not asked again element by element: these loops are bound by their instructions, and
+// 25 an element instead of ten cost as much as the trip to memory.
+template <bool VEC, typename F>
+__device__ __forceinline__ void each_piece(const float* __restrict__ x, int n, float4v (&r)[kHeld], F f) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x) & ~63, lane = threadIdx.x & 63;
+  int first = wave;
+  if constexpr (VEC) {
+#pragma unroll
+    for (int u = 0; u < kHeld; ++u) {
+      const int at = wave + u * kSampThreads;
+      if (4 * at + 256 <= n) {
+        f(r[u], at + lane, 4);
+        first = at + kSampThreads;
+      }
+    }
+  }
+#pragma unroll 1
+  for (; 4 * first < n; first += 4 * kSampThreads) {
+    float4v v[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) v[u] = slice_piece<VEC>(x, n, first + lane + u * kSampThreads);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int at = first + u * kSampThreads, i = at + lane;
+      if (4 * at < n) f(v[u], i, max(min(n - 4 * i, 4), 0));
+    }
+  }
+}
+
+// A bin's word: count << 40 | the sum of the 19 bits below its digit.  All its elements share the bits above, so that is their
+// exact mass, and adding an element is one 64-bit add of bits that it has already.
+constexpr int kCountAt = 40;
+__device__ __forceinline__ u64 word_sum(u64 w, int digit) {  // in units of 2^(max(digit / 16, 1) - 150)
+  return (w >> kCountAt) * (u64)((digit >> 4 ? 0x800000u : 0u) | ((uint32_t)(digit & 15) << 19)) + (w & ((1ull << kCountAt) - 1));
 }
 
 template <bool VEC>
+__global__ void __launch_bounds__(kSampThreads) slice_bins_kernel(SampArgs a) {
+  __shared__ u64 bins[kWindow];
+  __shared__ float red[3][16];
+  const int slice = blockIdx.x, row = blockIdx.y, lo = slice * a.slice, n = min(a.slice, a.n - lo);
+  const float* x = a.probs + (int64_t)row * a.in_stride + lo;
+  float4v held[kHeld];
+  hold<VEC>(x, n, held);
+  const RowParams rp = load_params(a, row);
+  const Guess g = guess_of(rp, a.n);
+  const SampWs w = samp_ws(a, row);
+  bins[threadIdx.x] = 0;
+  __syncthreads();
+  float s = 0.f, mx = 0.f;
+  const float least = g.use_k || g.use_p ? g.least : __uint_as_float(0x7FC00000u);  // without a filter nothing is binned
+  each_piece<VEC>(x, n, held, [&](const float4v& piece, int, int have) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float raw = e < have ? piece[e] : -1.f, v = fmaxf(raw, 0.f);
+      const bool in = raw >= least;
+      mx = fmaxf(mx, v);
+      s += in ? 0.f : v;
+      if (in) {
+        const uint32_t b = __float_as_uint(raw);
+        atomicAdd(&bins[min((int)(b >> 19) - g.base, kWindow - 1)], (1ull << kCountAt) | (b & 0x7FFFFu));
+      }
+    }
+  });
+  __syncthreads();
+  const u64 word = bins[threadIdx.x];
+  // the window's last bin takes what lies beyond it: no mass of such a row is known
+  float o = threadIdx.x < kWindow - 1 ? ldexpf((float)word_sum(word, g.base + threadIdx.x), max((g.base + (int)threadIdx.x) >> 4, 1) - 150) : word ? __uint_as_float(0x7F800000u) : 0.f;
+  s = wave_sum(s), o = wave_sum(o), mx = wave_max(mx);
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  if (lane == 0) red[0][wid] = s, red[1][wid] = o, red[2][wid] = mx;
+  if (g.use_k || g.use_p) w.bins[slice * kWindow + threadIdx.x] = word;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    SliceStat st{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < 16; ++t) st.under += red[0][t], st.over += red[1][t], st.vmax = fmaxf(st.vmax, red[2][t]);
+    w.stat[slice] = st;
+  }
+}
+
+// SUM (sampling): also the masses of the chunks, of what is kept whatever the cut inside its bin turns out to be; the
+// bin's own elements are listed with their places and added by the last launch.
+template <bool VEC, bool SUM>
 __global__ void __launch_bounds__(kSampThreads) slice_collect_kernel(SampArgs a) {
-  __shared__ SampShared sh;
+  __shared__ u64 bins[kWindow];
+  __shared__ u64 ured[16];
+  __shared__ uint32_t list[2][kList], place[SUM ? 2 : 1][SUM ? kList : 1];
+  __shared__ uint32_t cut[2], fill[2], start[2], need;
+  __shared__ u64 below;
   const int slice = blockIdx.x, row = blockIdx.y, lo = slice * a.slice, n = min(a.slice, a.n - lo);
   const float* x = a.probs + (int64_t)row * a.in_stride + lo;
   const RowParams rp = load_params(a, row);
   const SampWs w = samp_ws(a, row);
   const Guess g = guess_of(rp, a.n);
   const bool bin = g.use_k || g.use_p;
-  // everything the slices left is asked for at once: one trip to memory
-  u64 word[kMaxSlices];
-  float4v stat[kMaxSlices];
+  // what the slices left (a lane a slice for the sums), then the slice itself: it arrives while the cuts are found
+  const int lane = threadIdx.x & 63;
+  float4v stat, held[kHeld];
+  u64 word = 0;
+  uint32_t ahead = 0;  // elements of this thread's bin in the slices in front
+  auto ask = [&](auto most) {
+    u64 part[decltype(most)::value];
+    stat = *reinterpret_cast<const float4v*>(w.stat + min(lane, a.slices - 1));
 #pragma unroll
-  for (int t = 0; t < kMaxSlices; ++t) {
-    if (t < a.slices) {
-      stat[t] = *reinterpret_cast<const float4v*>(w.stat + t);
-      if (bin) word[t] = w.bins[t * kWindow + threadIdx.x];
+    for (int t = 0; t < most; ++t) part[t] = w.bins[min(t, a.slices - 1) * kWindow + threadIdx.x];  // (not written without a filter)
+    __builtin_amdgcn_sched_barrier(0);
+    hold<VEC>(x, n, held);
+#pragma unroll
+    for (int t = 0; t < most; ++t) {
+      word += t < a.slices ? part[t] : 0;
+      ahead += t < slice ? (uint32_t)(part[t] >> kCountAt) : 0;
     }
-  }
+  };
+  if (a.slices <= 4)
+    ask(std::integral_constant<int, 4>());
+  else
+    ask(std::integral_constant<int, kMaxSlices>());
+  if (lane >= a.slices) stat = float4v{0.f, 0.f, 0.f, 0.f};
   RowState st{};
-  double under = 0.0, total = 0.0;
-#pragma unroll
-  for (int t = 0; t < kMaxSlices; ++t)
-    if (t < a.slices) {
-      under += stat[t][0];
-      total += (double)stat[t][0] + (double)stat[t][1];
-      st.vmax = fmaxf(st.vmax, stat[t][2]);
-    }
+  double under = stat[0], total = (double)stat[0] + (double)stat[1];  // the first row of lanes has them all
+  auto ror = [](double v, auto ctrl) {
+    const u64 b = __builtin_bit_cast(u64, v);
+    return __builtin_bit_cast(double, ((u64)dpp<decltype(ctrl)::value>((uint32_t)(b >> 32)) << 32) | dpp<decltype(ctrl)::value>((uint32_t)b));
+  };
+  auto turn = [&](auto ctrl) {
+    under += ror(under, ctrl);
+    total += ror(total, ctrl);
+    st.vmax = fmaxf(st.vmax, __uint_as_float(dpp<decltype(ctrl)::value>(__float_as_uint(st.vmax))));
+  };
+  st.vmax = stat[2];
+  turn(std::integral_constant<int, kDppRor8>());
+  turn(std::integral_constant<int, kDppRor4>());
+  turn(std::integral_constant<int, kDppXor2>());
+  turn(std::integral_constant<int, kDppXor1>());
+  auto first_lane = [](double v) {
+    const u64 b = __builtin_bit_cast(u64, v);
+    return __builtin_bit_cast(double, ((u64)(uint32_t)__builtin_amdgcn_readfirstlane((int)(b >> 32)) << 32) |
+                                          (uint32_t)__builtin_amdgcn_readfirstlane((int)b));
+  };
+  under = first_lane(under), total = first_lane(total);
+  st.vmax = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(st.vmax)));
   st.valid = 1;
   st.kbin = st.pbin = -1;
   if (bin) {
-    u64 sum = 0;
-#pragma unroll
-    for (int t = 0; t < kMaxSlices; ++t) sum += t < a.slices ? word[t] : 0;
-    sh.bin[threadIdx.x] = sum;
-    __syncthreads();
-    // counts and masses in front of this thread's bin in one scan of the packed words
+    // counts and masses in front of this thread's bin in one scan of packed words (masses that do not fit are no valid row's)
+    const int digit = g.base + threadIdx.x, up = max(digit >> 4, 1) - 150 + g.fx.scale;
+    const u64 whole = word_sum(word, digit), mass = up >= 0 ? whole << (up & 63) : up > -64 ? whole >> (-up & 63) : 0;
+    const u64 sum = ((word >> kCountAt) << g.fx.bits) + mass;
+    bins[threadIdx.x] = sum;
     u64 words;
-    const u64 before = bscan<u64>(sum, sh.ured, words);
+    const u64 before = bscan<u64>(sum, ured, words);
     const uint32_t all = g.fx.count(words), c = g.fx.count(sum), behind = all - g.fx.count(before) - c;
     const u64 low = (u64)ldexp(under, g.fx.scale), m = g.fx.mass(sum), run = low + g.fx.mass(before);
     st.target = max((u64)fmin(ceil((double)(1.0f - rp.top_p) * (double)(low + g.fx.mass(words))), 4e18), (u64)1);
     // the whole-row form's checks, and the window's
-    st.valid = total > 0.2 && total < 1.99 && st.vmax < 2.f && all > 0 && (!g.use_k || (int)all >= rp.top_k) &&
+    st.valid = total > 0.2 && total < 1.99 && all > 0 && (!g.use_k || (int)all >= rp.top_k) &&
                (!g.use_p || (under < (double)(1.0f - rp.top_p) * total && low + g.fx.mass(words) >= st.target && low < st.target));
     if (st.valid && g.use_k && behind < (uint32_t)rp.top_k && (uint32_t)rp.top_k <= behind + c) {
-      sh.cut[0] = threadIdx.x;
-      sh.need = rp.top_k - behind;
+      cut[0] = threadIdx.x;
+      start[0] = ahead;
+      need = rp.top_k - behind;
     }
     if (st.valid && g.use_p && m > 0 && run < st.target && run + m >= st.target) {
-      sh.cut[1] = threadIdx.x;
-      sh.below = run;
+      cut[1] = threadIdx.x;
+      start[1] = ahead;
+      below = run;
     }
     __syncthreads();
     if (st.valid && g.use_k) {
-      st.kbin = sh.cut[0];
-      st.rank = sh.need;
-      st.kcount = (int)g.fx.count(sh.bin[st.kbin]);
+      st.kbin = cut[0];
+      st.rank = need;
+      st.kcount = (int)g.fx.count(bins[st.kbin]);
     }
     if (st.valid && g.use_p) {
-      st.pbin = sh.cut[1];
-      st.below = sh.below;
-      st.pcount = (int)g.fx.count(sh.bin[st.pbin]);
+      st.pbin = cut[1];
+      st.below = below;
+      st.pcount = (int)g.fx.count(bins[st.pbin]);
     }
     if (st.kcount > kList || st.pcount > kList) st.valid = 0;
     // for the kept mass: of the bins behind the cut
-    if (st.valid && (int)threadIdx.x == (g.use_k ? st.kbin : st.pbin)) sh.ured[0] = g.fx.mass(words) - g.fx.mass(before) - m;
+    if (st.valid && (int)threadIdx.x == (g.use_k ? st.kbin : st.pbin)) ured[0] = g.fx.mass(words) - g.fx.mass(before) - m;
+    if (threadIdx.x < 2) fill[threadIdx.x] = 0;
     __syncthreads();
-    st.above = sh.ured[0];
+    st.above = ured[0];
   }
   if (slice == 0 && threadIdx.x == 0) *w.state = st;
-  if (!bin || !st.valid) return;  // block-uniform, the same in every block of the row (no fill is read then)
-  if (threadIdx.x < 2) sh.fill[threadIdx.x] = 0;
-  __syncthreads();
+  if ((!bin && !SUM) || !st.valid) return;  // block-uniform, the same in every block of the row
+  // the elements of a bin: bit patterns of one range (negative values and what is no number lie outside), from `least` on
   const uint32_t from = __float_as_uint(g.least);
-  each<VEC, 4>(x, n, [&](float raw) {
-    const uint32_t bits = value_bits(raw);
-    const int d = bits >= from ? min((int)(bits >> 19) - g.base, kWindow - 1) : -2;
-    if (d == st.kbin) sh.list[0][atomicAdd(&sh.fill[0], 1u)] = bits;
-    if (d == st.pbin) sh.list[1][atomicAdd(&sh.fill[1], 1u)] = bits;
+  auto range = [&](int d, uint32_t& lo_bits, uint32_t& span) {
+    const uint32_t first = (uint32_t)(d + g.base) << 19;
+    lo_bits = max(first, from);
+    span = d < 0 ? 0u : first + (1u << 19) - lo_bits;
+  };
+  uint32_t klo, kspan, plo, pspan;
+  range(st.kbin, klo, kspan);
+  range(st.pbin, plo, pspan);
+  // kept for certain: what lies behind the bins, and from the min-p threshold on
+  const int last = max(st.kbin, st.pbin);
+  const float sure = fmaxf(bin ? __uint_as_float((uint32_t)(last + 1 + g.base) << 19) : 0.f, rp.min_p > 0.f ? rp.min_p * st.vmax : 0.f);
+  each_piece<VEC>(x, n, held, [&](const float4v& piece, int at, int have) {
+    float sums[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float raw = e < have ? piece[e] : -1.f;
+      const uint32_t b = __float_as_uint(raw);
+      if (b - klo < kspan) {
+        const uint32_t to = atomicAdd(&fill[0], 1u);
+        list[0][to] = b;
+        if (SUM) place[0][to] = lo + 4 * at + e;
+      }
+      if (b - plo < pspan) {
+        const uint32_t to = atomicAdd(&fill[1], 1u);
+        list[1][to] = b;
+        if (SUM) place[SUM][to] = lo + 4 * at + e;
+      }
+      sums[e] = raw >= sure ? raw : 0.f;
+    }
+    if (SUM) {
+      const float mass = wave_sum((sums[0] + sums[1]) + (sums[2] + sums[3]));
+      if (lane == 0) w.chunk[(lo >> 8) + (at >> 6)] = mass;
+    }
   });
+  if (!bin) return;
   __syncthreads();
-  // a place in the row's lists (in any order: what is taken from them does not depend on it)
-  if (threadIdx.x < 2) sh.cut[threadIdx.x] = sh.fill[threadIdx.x] ? atomicAdd(&w.fill[threadIdx.x], sh.fill[threadIdx.x]) : 0u;
-  __syncthreads();
+  // behind what the slices in front have in the bins (in any order: what is taken from the lists does not depend on it)
 #pragma unroll
   for (int t = 0; t < 2; ++t)
-    for (int i = threadIdx.x; i < (int)sh.fill[t]; i += kSampThreads) w.list[t * kList + sh.cut[t] + i] = sh.list[t][i];
+    for (int i = threadIdx.x; i < (int)fill[t]; i += kSampThreads) {
+      w.list[t * kList + start[t] + i] = list[t][i];
+      if (SUM) w.place[t * kList + start[t] + i] = place[SUM ? t : 0][i];
+    }
+}
+
+struct HeldLists {
+  uint32_t got[2][kList / kSampThreads];
+  __device__ __forceinline__ void load(const uint32_t* from) {  // whatever stands behind the lists' ends is not looked at
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int j = 0; j < kList / kSampThreads; ++j) got[t][j] = from[t * kList + threadIdx.x + j * kSampThreads];
+  }
+};
+
+// The row's threshold from its candidates, which lie two a thread and list in registers: digits of 6, 6 and 7 bits, counted by the
+// whole block and picked by a wave a list (a wave that walks a list of two thousand by itself takes 6 us).  Block-uniform.
+__device__ __forceinline__ float finish_threshold(SampShared& sh, const HeldLists& lists, const RowParams& rp, const Guess& g,
+                                                  const RowState& st) {
+  float thr = 0.f;
+  if (g.use_k || g.use_p) {
+    const int wid = threadIdx.x >> 6;
+    constexpr int kOwn = kList / kSampThreads;
+    if (wid < 2) sh.digit[wid][threadIdx.x & 63] = sh.digit[wid][64 + (threadIdx.x & 63)] = 0;
+    uint32_t prefix[2] = {(uint32_t)(st.kbin + g.base) << 19, (uint32_t)(st.pbin + g.base) << 19};
+    const int listed[2] = {g.use_k ? st.kcount : 0, g.use_p ? st.pcount : 0};
+    u64 word[2][kOwn];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int j = 0; j < kOwn; ++j) word[t][j] = (1ull << g.fx.bits) + g.fx.of(lists.got[t][j]);
+    uint32_t rank = st.rank;
+    u64 below = st.below;
+    int bits = 19;
+    __syncthreads();
+#pragma unroll
+    for (int digit = 0; digit < 3; ++digit) {
+      const int take = digit < 2 ? 6 : 7, shift = bits - take;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int j = 0; j < kOwn; ++j) {
+          const uint32_t b = lists.got[t][j];
+          if ((int)threadIdx.x + j * kSampThreads < listed[t] && (b >> bits) == (prefix[t] >> bits))
+            atomicAdd(&sh.digit[t][(b >> shift) & ((1u << take) - 1)], word[t][j]);
+        }
+      __syncthreads();
+      if (wid < 2) {
+        u64 unused = 0;
+        const int d = wid ? pick_digit<false>(sh.digit[1], g.fx, rank, below, max(st.target, (u64)1))
+                          : pick_digit<true>(sh.digit[0], g.fx, rank, unused, 0);
+        sh.cut[wid] = d;
+      }
+      __syncthreads();
+      prefix[0] |= sh.cut[0] << shift, prefix[1] |= sh.cut[1] << shift;
+      bits = shift;
+    }
+    thr = fmaxf(g.use_k ? __uint_as_float(prefix[0]) : 0.f, g.use_p ? __uint_as_float(prefix[1]) : 0.f);
+  }
+  return rp.min_p > 0.f ? fmaxf(thr, rp.min_p * st.vmax) : thr;
 }
 
 template <bool VEC>
 __global__ void __launch_bounds__(kSampThreads) slice_apply_kernel(SampArgs a) {
   __shared__ SampShared sh;
   const int slice = blockIdx.x, row = blockIdx.y, lo = slice * a.slice, n = min(a.slice, a.n - lo);
-  const float* x = a.probs + (int64_t)row * a.in_stride;
+  const float* x = a.probs + (int64_t)row * a.in_stride + lo;
   const SampWs w = samp_ws(a, row);
-  uint32_t got[2][kList / kSampThreads];  // (whatever stands behind the lists' ends is not looked at)
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int j = 0; j < kList / kSampThreads; ++j) got[t][j] = w.list[t * kList + threadIdx.x + j * kSampThreads];
+  const RowState st = *w.state;
+  HeldLists lists;
+  lists.load(w.list);
+  float4v held[kHeld];
+  hold<VEC>(x, n, held);
   const RowParams rp = load_params(a, row);
   const Guess g = guess_of(rp, a.n);
-  const RowState st = *w.state;
   if (!st.valid) return;  // block-uniform
-  float thr = 0.f, kept = -1.f;
-  if (g.use_k || g.use_p) {
+  const float thr = finish_threshold(sh, lists, rp, g, st);
+  float kept = -1.f;
+  if (g.use_k != g.use_p) {
+    u64 part = 0, all;
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int j = 0; j < kList / kSampThreads; ++j) {
+      const uint32_t b = g.use_k ? lists.got[0][j] : lists.got[1][j];
+      if ((int)threadIdx.x + j * kSampThreads < (g.use_k ? st.kcount : st.pcount) && __uint_as_float(b) >= thr) part += g.fx.of(b);
+    }
+    bscan<u64>(part, sh.ured, all);
+    kept = (float)ldexp((double)(st.above + all), -g.fx.scale);
+  }
+  if (!(kept > 0.f)) {  // no filter: the whole row's mass
+    kept = 0.f;
+    for (int t = 0; t < a.slices; ++t) kept += w.stat[t].under + w.stat[t].over;
+  }
+  const float inv = 1.0f / kept;
+  float* o = a.out + (int64_t)row * a.out_stride + lo;
+  each_piece<VEC>(x, n, held, [&](const float4v& piece, int at, int have) {
+    float4v v;
 #pragma unroll
-      for (int j = 0; j < kList / kSampThreads; ++j) sh.list[t][threadIdx.x + j * kSampThreads] = got[t][j];
-    __syncthreads();
-    const uint32_t from = __float_as_uint(g.least);
-    if (threadIdx.x < 2) sh.cut[threadIdx.x] = 0;
-    __syncthreads();
-    const int wid = threadIdx.x >> 6;
-    if (wid == 0 && g.use_k)
-      sh.cut[0] = refine_list<true>(sh.digit[0], g.fx, sh.list[0], st.kcount, st.kbin + g.base, st.rank, 0, 0, from);
-    if (wid == 1 && g.use_p)
-      sh.cut[1] = refine_list<false>(sh.digit[1], g.fx, sh.list[1], st.pcount, st.pbin + g.base, 0u, st.below, st.target, from);
-    __syncthreads();
-    thr = fmaxf(__uint_as_float(sh.cut[0]), __uint_as_float(sh.cut[1]));
-    if (g.use_k != g.use_p) {
-      u64 part = 0, all;
-      for (int i = threadIdx.x; i < (g.use_k ? st.kcount : st.pcount); i += kSampThreads) {
-        const uint32_t b = sh.list[g.use_k ? 0 : 1][i];
-        if (__uint_as_float(b) >= thr) part += g.fx.of(b);
-      }
-      bscan<u64>(part, sh.ured, all);
-      kept = (float)ldexp((double)(st.above + all), -g.fx.scale);
+    for (int e = 0; e < 4; ++e) v[e] = piece[e] >= thr ? piece[e] * inv : 0.f;
+    if (VEC && have == 4) {
+      *reinterpret_cast<float4v*>(o + 4 * at) = v;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (e < have) o[4 * at + e] = v[e];
     }
-  }
-  if (rp.min_p > 0.f) thr = fmaxf(thr, rp.min_p * st.vmax);
-  if (a.out) {
-    if (!(kept > 0.f)) {  // no filter: the whole row's mass
-      kept = 0.f;
-      for (int t = 0; t < a.slices; ++t) kept += w.stat[t].under + w.stat[t].over;
-    }
-    write_renormed<VEC>(x + lo, a.out + (int64_t)row * a.out_stride + lo, n, thr, 1.0f / kept);
-    return;
-  }
-  if (slice == 0 && threadIdx.x == 0) w.state->thr = thr;
-  sum_chunks<VEC>(x, a.n, thr, 256, lo / 256, (lo + n + 255) / 256, w.chunk);
+  });
 }
 
+// A block a row: the choice where it is sampled from, and the rows that the guess did not hold for.
 template <bool VEC>
 __global__ void __launch_bounds__(kSampThreads) slice_choose_kernel(SampArgs a) {
   __shared__ SampShared sh;
   const int row = blockIdx.x;
   const float* x = a.probs + (int64_t)row * a.in_stride;
   const SampWs w = samp_ws(a, row);
-  if (!w.state->valid) {
-    const RowParams rp = load_params(a, row);
-    if (a.out)
-      renorm_row<VEC, true>(x, a.out + (int64_t)row * a.out_stride, a.n, rp, sh);
-    else
-      sample_row<VEC, true>(x, a.n, rp, a.uniform[row], a.ids + row, sh);
+  const RowParams rp = load_params(a, row);
+  if (a.out) {
+    if (!w.state->valid) renorm_row<VEC, true>(x, a.out + (int64_t)row * a.out_stride, a.n, rp, sh);
     return;
   }
-  if (a.out) return;
+  constexpr int PER = kBins / kSampThreads;
   const int chunks = (a.n + 255) / 256;
-  for (int i = threadIdx.x; i < kBins; i += kSampThreads) sh.chunk[i] = i < chunks ? w.chunk[i] : 0.f;
+  HeldLists lists, places;
+  lists.load(w.list);
+  places.load(w.place);
+  float mass[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) mass[j] = w.chunk[min((int)threadIdx.x + j * kSampThreads, chunks - 1)];
+  const RowState st = *w.state;
+  if (!st.valid) {
+    sample_row<VEC, true>(x, a.n, rp, a.uniform[row], a.ids + row, sh);
+    return;
+  }
+  const Guess g = guess_of(rp, a.n);
+  for (int i = threadIdx.x; i < min(chunks, kBins); i += kSampThreads) sh.bin[i] = 0;
+  const float thr = finish_threshold(sh, lists, rp, g, st);  // a block barrier, or no elements to add
+  // the cut bin's kept elements, in whole numbers: the same in any order
+  const int which = st.kbin >= st.pbin ? 0 : 1, listed = which ? st.pcount : st.kcount;
+  if (g.use_k || g.use_p) {
+#pragma unroll
+    for (int j = 0; j < kList / kSampThreads; ++j) {
+      const uint32_t b = which ? lists.got[1][j] : lists.got[0][j], at = which ? places.got[1][j] : places.got[0][j];
+      if ((int)threadIdx.x + j * kSampThreads < listed && __uint_as_float(b) >= thr) atomicAdd(&sh.bin[at >> 8], g.fx.of(b));
+    }
+  }
   __syncthreads();
-  choose<VEC>(x, a.n, w.state->thr, 256, a.uniform[row], a.ids + row, sh);
+#pragma unroll
+  for (int j = 0; j < PER; ++j) {
+    const int i = threadIdx.x + j * kSampThreads;
+    mass[j] = i < chunks ? mass[j] + (float)ldexp((double)sh.bin[i], -g.fx.scale) : 0.f;
+  }
+  __syncthreads();  // the masses take the place of the sums
+#pragma unroll
+  for (int j = 0; j < PER; ++j) sh.chunk[threadIdx.x + j * kSampThreads] = mass[j];
+  __syncthreads();
+  choose<VEC>(x, a.n, thr, 256, a.uniform[row], a.ids + row, sh);
 }
 
 // Blocks a row is spread over: at least 8192 elements each, and one block a unit at most (what a block scans and waits for
@@ -1010,8 +1216,12 @@ static int launch_filters(SampArgs a, int batch, void* workspace, int64_t worksp
   a.ws = (char*)workspace;
   const dim3 grid(a.slices, batch), block(kSampThreads);
   hipLaunchKernelGGL(vec ? slice_bins_kernel<true> : slice_bins_kernel<false>, grid, block, 0, s, a);
-  hipLaunchKernelGGL(vec ? slice_collect_kernel<true> : slice_collect_kernel<false>, grid, block, 0, s, a);
-  hipLaunchKernelGGL(vec ? slice_apply_kernel<true> : slice_apply_kernel<false>, grid, block, 0, s, a);
+  if (a.out) {
+    hipLaunchKernelGGL((vec ? slice_collect_kernel<true, false> : slice_collect_kernel<false, false>), grid, block, 0, s, a);
+    hipLaunchKernelGGL(vec ? slice_apply_kernel<true> : slice_apply_kernel<false>, grid, block, 0, s, a);
+  } else {
+    hipLaunchKernelGGL((vec ? slice_collect_kernel<true, true> : slice_collect_kernel<false, true>), grid, block, 0, s, a);
+  }
   hipLaunchKernelGGL(vec ? slice_choose_kernel<true> : slice_choose_kernel<false>, dim3(batch), block, 0, s, a);
   SGLK_LAUNCH_CHECK();
   return SGLK_OK;

@@ -167,3 +167,32 @@ def test_one_block_and_several_agree():
         assert torch.equal(ids[:50], torch.cat([ops.sampling_from_probs(x, u[i: i + 1], **kw) for i in range(50)]))
     assert torch.equal(sk.top_p_renorm_probs(many, 0.9)[7:8], sk.top_p_renorm_probs(x, 0.9))
     assert torch.equal(sk.top_k_renorm_probs(many, 77)[7:8], sk.top_k_renorm_probs(x, 77))
+
+
+@pytest.mark.parametrize("B,n", [(6, 40000), (6, 128259), (64, 163843)])
+def test_spread_rows_with_all_filters(B, n):
+    """Rows of different filters in one call over several slices: none, one, two, with a min-p below and above their cut."""
+    from sglang_security_amd import ops
+
+    g = torch.Generator().manual_seed(n)
+    x = _rows("peaked", n, g)
+    x = x * 2.0 ** -math.ceil(math.log2(x.sum().item()))
+    rows = [(0, 1.0, 0.25), (50, 1.0, 0.0), (0, 0.875, 0.0), (50, 0.75, 0.125), (1000, 0.875, 2.0 ** -12), (n, 0.5, 0.0)]
+    rows = [rows[b % 6] for b in range(B)]
+    kt = torch.tensor([r[0] for r in rows], dtype=torch.int32, device=DEV)
+    pt, mt = (torch.tensor([r[i] for r in rows], device=DEV) for i in (1, 2))
+    wide = torch.zeros(B, n + 5, device=DEV)
+    wide[:, 1: n + 1] = x.float().to(DEV)
+    aligned = torch.zeros(B, (n + 3) // 4 * 4, device=DEV)
+    aligned[:, :n] = x.float().to(DEV)
+    for rows_of in (wide[:, 1: n + 1], aligned[:, :n]):
+        for u in (0.0, 0.3, 0.7, 0.999999):
+            ids = ops.sampling_from_probs(rows_of, torch.full((B,), u, device=DEV), kt, pt, mt, True).cpu().long()
+            again = ops.sampling_from_probs(rows_of, torch.full((B,), u, device=DEV), kt, pt, mt, True).cpu().long()
+            assert torch.equal(ids, again)
+            for b in range(6):
+                k, p, m = rows[b]
+                kept = torch.where(x >= max(_threshold(x, k, p, True), m * x.max().item()), x, 0.0)
+                cum = kept.cumsum(0) / kept.sum()
+                for i in ids[b::6].tolist():
+                    assert kept[i] > 0 and cum[i] >= u - 1e-5 and (i == 0 or cum[i - 1] <= u + 1e-5)
