@@ -13,6 +13,7 @@
 #include <cstdlib>
 
 #include "common.h"
+#include "fp8_direct.h"
 #include "fp8_tile.h"
 
 namespace sglk {
@@ -927,6 +928,63 @@ static int fp8_stream_splits(int M, int N, int K) {
   return std::max(1, std::min({(512 + blocks - 1) / blocks, std::max(K / 1024, 1), 8}));
 }
 
+// Splits of K, and whether a call goes to the kernels of fp8_direct.h at all (up to 64 rows).  A split costs its reduction
+// launch, some 2 us: worth it from nine rows on where x is most of what a narrow output's blocks read (32 rows, 14336 x 4096 unsplit
+// 18.8, two splits 13.9 + 2; 4096 x 4096 7.0 and 5.5 + 2), and for the staged form until 256 blocks (64 rows, 4096 x 4096
+// unsplit 9.4, two splits 7.2 + 2; 14336 x 4096 24.4 and 16.0 + 2; 8192 x 1280 14.0 and, four ways, 6.6 + 2).
+struct Fp8Direct {
+  bool ok;
+  int splits, per;  // k-blocks a split
+};
+static Fp8Direct fp8_direct_plan(int M, int N, int K) {
+  const int kblocks = K / 128, strips = N / 16;
+  int splits = 1;
+  if (M > 64) {
+    splits = fp8_stream_splits(M, N, K);
+  } else if (const char* env = getenv("SGLK_FP8_STREAM_SPLITS"); env && atoi(env) > 0) {
+    splits = std::min(atoi(env), kblocks);
+  } else if (N % 4 != 0) {
+    splits = 1;
+  } else if (M > 32) {
+    const int blocks = strips >= 1024 ? (strips + 3) / 4 : (strips + 1) / 2;
+    if (blocks < 192) splits = std::max(1, std::min({(255 + blocks) / blocks, 4, K / 1024}));
+  } else if (M > 8 && strips <= 256 && K >= 8192) {
+    splits = 2;
+  }
+  const int per = (kblocks + splits - 1) / splits;
+  return Fp8Direct{M <= 64, (kblocks + per - 1) / per, per};
+}
+
+// Which tile: 64 columns a block where there are blocks enough, so that x is read least; one strip where there are too few strips
+// to give every unit more.
+template <typename TO>
+int launch_fp8_direct(const Fp8DirectArgs& a, int splits, hipStream_t s) {
+  const int strips = a.N / 16;
+#define SGLK_FP8_DIRECT(MT, CS, WAYS, R)                                                                                        \
+  {                                                                                                                             \
+    constexpr int lds = fp8_direct_lds<MT, CS, WAYS>();                                                                         \
+    if (int rc = ensure_lds<&fp8_direct_kernel<TO, MT, CS, WAYS, R>>(lds)) return rc;                                           \
+    hipLaunchKernelGGL((fp8_direct_kernel<TO, MT, CS, WAYS, R>), dim3((strips + CS - 1) / CS, splits), dim3(64 * WAYS), lds, s, a); \
+  }
+#define SGLK_FP8_STAGED(SB, PW)                                                                                                 \
+  {                                                                                                                             \
+    if (int rc = ensure_lds<&fp8_staged_kernel<TO, SB, PW>>(fp8_staged_lds<SB>())) return rc;                                   \
+    hipLaunchKernelGGL((fp8_staged_kernel<TO, SB, PW>), dim3((strips + SB - 1) / SB, splits), dim3(512), fp8_staged_lds<SB>(), s, a); \
+  }
+  const bool pairs = strips > 256 || (splits > 1 && strips == 256);
+  if (a.M > 32) {
+    if (strips >= 1024) SGLK_FP8_STAGED(4, 2) else SGLK_FP8_STAGED(2, 4)
+  } else if (a.M > 16) {
+    if (strips >= 1024) SGLK_FP8_DIRECT(2, 4, 8, 1) else if (pairs) SGLK_FP8_DIRECT(2, 2, 8, 1) else SGLK_FP8_DIRECT(2, 1, 16, 1)
+  } else {
+    if (strips >= 1024) SGLK_FP8_DIRECT(1, 4, 8, 1) else if (pairs) SGLK_FP8_DIRECT(1, 2, 8, 1) else SGLK_FP8_DIRECT(1, 1, 16, 1)
+  }
+#undef SGLK_FP8_STAGED
+#undef SGLK_FP8_DIRECT
+  SGLK_LAUNCH_CHECK();
+  return SGLK_OK;
+}
+
 }  // namespace
 }  // namespace sglk
 
@@ -1176,7 +1234,7 @@ int sglk_fp8_repack(const void* w_nk, void* packed, int N, int K, int64_t w_stri
 
 int64_t sglk_fp8_mm_packed_workspace_bytes(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 128 != 0 || N % 16 != 0) return 0;
-  const int splits = fp8_stream_splits(M, N, K);
+  const int splits = std::max(fp8_stream_splits(M, N, K), fp8_direct_plan(M, N, K).splits);  // the block-scaled form's, too
   return splits > 1 ? (int64_t)splits * M * N * (int64_t)sizeof(float) : 0;
 }
 
@@ -1188,27 +1246,23 @@ int sglk_fp8_scaled_mm_packed(const void* a, const void* packed, const float* sc
              "fp8_scaled_mm_packed: N=%d must be a multiple of 16, K=%d of 128", N, K);
   SGLK_CHECK(aligned16(a) && aligned16(packed) && a_stride % 16 == 0 && a_stride >= K && out_stride >= N,
              "fp8_scaled_mm_packed: rows must be 16-byte aligned");
-  int splits = fp8_stream_splits(M, N, K);
-  const int kblocks = K / 128;
-  if (splits > 1 && (!workspace || workspace_bytes < (int64_t)splits * M * N * (int64_t)sizeof(float) ||
-                     !aligned16(workspace)))
-    splits = 1;
-  const int per = (kblocks + splits - 1) / splits;
-  const int used = (kblocks + per - 1) / per;
-  const int mblocks = (M + 63) / 64;
+  const Fp8Direct plan = fp8_direct_plan(M, N, K);
+  int used = plan.splits, per = plan.per;
+  if (used > 1 && (!workspace || workspace_bytes < (int64_t)used * M * N * (int64_t)sizeof(float) || !aligned16(workspace)))
+    used = 1, per = K / 128;
   float* partial = used > 1 ? (float*)workspace : nullptr;
-  static const int env_ns = getenv("SGLK_FP8_STREAM_NS") ? atoi(getenv("SGLK_FP8_STREAM_NS")) : 0;
-  const bool two = env_ns == 2;  // two strips per wave measured slower than one on every decode shape of the 8B model
   hipStream_t s = (hipStream_t)stream;
   SGLK_DISPATCH_HALF(out_dtype, TO, {
-    if (two)
-      hipLaunchKernelGGL((fp8_stream_kernel<TO, 2, 4>), dim3((N + 127) / 128, used, mblocks), dim3(256), 0, s,
+    if (plan.ok) {
+      const Fp8DirectArgs d{(const uint8_t*)a, (const uint8_t*)packed, scales_a, scales_b, bias, out, partial,
+                            M,                 N,                      K,        per,      a_stride, out_stride};
+      const int rc = launch_fp8_direct<TO>(d, used, s);
+      if (rc != SGLK_OK) return rc;
+    } else {
+      hipLaunchKernelGGL((fp8_stream_kernel<TO, 1, 4>), dim3((N + 63) / 64, used, (M + 63) / 64), dim3(256), 0, s,
                          (const uint8_t*)a, (const uint8_t*)packed, scales_a, scales_b, bias, out, partial, M, N, K, per,
                          a_stride, out_stride);
-    else
-      hipLaunchKernelGGL((fp8_stream_kernel<TO, 1, 4>), dim3((N + 63) / 64, used, mblocks), dim3(256), 0, s,
-                         (const uint8_t*)a, (const uint8_t*)packed, scales_a, scales_b, bias, out, partial, M, N, K, per,
-                         a_stride, out_stride);
+    }
     if (used > 1) {
       const int64_t vecs = (int64_t)M * (N / 4);
       hipLaunchKernelGGL((fp8_splitk_reduce_kernel<TO>), dim3((unsigned)((vecs + 255) / 256)), dim3(256), 0, s,
@@ -1254,9 +1308,7 @@ int sglk_fp8_blockwise_scaled_mm_packed(const void* a, const void* packed, const
 
 int sglk_fp8_mm_packed_partial_splits(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 128 != 0 || N % 16 != 0) return 0;
-  const int splits = fp8_stream_splits(M, N, K), kblocks = K / 128;
-  const int per = (kblocks + splits - 1) / splits;
-  return (kblocks + per - 1) / per;
+  return fp8_direct_plan(M, N, K).splits;
 }
 
 int sglk_fp8_mm_packed_partial(const void* a, const void* packed, float* partial, int M, int N, int K, int64_t a_stride,
@@ -1266,12 +1318,14 @@ int sglk_fp8_mm_packed_partial(const void* a, const void* packed, float* partial
              "fp8_mm_packed_partial: N=%d must be a multiple of 16, K=%d of 128", N, K);
   SGLK_CHECK(aligned16(a) && aligned16(packed) && aligned16(partial) && a_stride % 16 == 0 && a_stride >= K,
              "fp8_mm_packed_partial: rows must be 16-byte aligned");
-  const int splits = fp8_stream_splits(M, N, K), kblocks = K / 128;
-  const int per = (kblocks + splits - 1) / splits;
-  const int used = (kblocks + per - 1) / per;
-  hipLaunchKernelGGL((fp8_stream_kernel<bf16_t, 1, 4>), dim3((N + 63) / 64, used, (M + 63) / 64), dim3(256), 0,
+  const Fp8Direct plan = fp8_direct_plan(M, N, K);
+  if (plan.ok) {
+    const Fp8DirectArgs d{(const uint8_t*)a, (const uint8_t*)packed, nullptr, nullptr, nullptr, nullptr, partial, M, N, K, plan.per, a_stride, 0};
+    return launch_fp8_direct<bf16_t>(d, plan.splits, (hipStream_t)stream);
+  }
+  hipLaunchKernelGGL((fp8_stream_kernel<bf16_t, 1, 4>), dim3((N + 63) / 64, plan.splits, (M + 63) / 64), dim3(256), 0,
                      (hipStream_t)stream, (const uint8_t*)a, (const uint8_t*)packed, (const float*)nullptr,
-                     (const float*)nullptr, (const void*)nullptr, (void*)nullptr, partial, M, N, K, per, a_stride,
+                     (const float*)nullptr, (const void*)nullptr, (void*)nullptr, partial, M, N, K, plan.per, a_stride,
                      (int64_t)0);
   SGLK_LAUNCH_CHECK();
   return SGLK_OK;

@@ -6,7 +6,8 @@ the same `apply` contract (apply_fp8_linear, layers/quantization/fp8_utils.py:45
 activations, scaled product, bias, output in the activation type).  A checkpoint that is not fp8-serialised is
 quantised per output channel at load time, as the reference does when its scaled product takes per-channel scales
 (:118-127).  `process_weights_after_loading` additionally builds the sequential-streaming copy the decode-size product
-reads (same byte count; inner dimensions of 4096 and more, where that kernel is the faster one).
+reads (same byte count).  Up to 64 rows that product is the faster one from inner dimensions of 512 on (us, one row and
+64: 3584 x 8192 7.1 against 10.8 row-major and 10.6 against 13.0, 896 x 4864 3.0 and 4.3, 5.4 and 6.0), beyond from 4096 on.
 """
 from __future__ import annotations
 
@@ -93,6 +94,8 @@ class W8A8Fp8LinearMethod:
         layer.weight_scale = torch.nn.Parameter(scale, requires_grad=False)
         layer.sglk_shape = (k, n)
         layer.sglk_packed = ops.fp8_repack(qweight) if (n % 16 == 0 and k % 128 == 0 and k >= 4096) else None
+        # shorter inner dimensions: for calls of up to 64 rows, beyond them the row-major kernels are the faster ones
+        layer.sglk_packed_short = ops.fp8_repack(qweight) if (n % 16 == 0 and k % 128 == 0 and 512 <= k < 4096) else None
         layer.sglk_workspace = None
 
     def _workspace(self, layer, m: int, device) -> torch.Tensor:
@@ -115,8 +118,9 @@ class W8A8Fp8LinearMethod:
         xs = torch.empty(m, dtype=torch.float32, device=x.device)
         ops.per_token_quant_fp8(x2, xq, xs)
         ws = self._workspace(layer, m, x.device)
-        if layer.sglk_packed is not None and m <= self.streaming_max_tokens and not ops.fp8_tiled(m, n, k):
-            out = ops.fp8_scaled_mm_packed(xq, layer.sglk_packed, xs, layer.weight_scale, x.dtype, bias, None, ws)
+        packed = layer.sglk_packed_short if m <= 64 and layer.sglk_packed is None else layer.sglk_packed
+        if packed is not None and m <= self.streaming_max_tokens and not ops.fp8_tiled(m, n, k):
+            out = ops.fp8_scaled_mm_packed(xq, packed, xs, layer.weight_scale, x.dtype, bias, None, ws)
         else:
             out = ops.fp8_scaled_mm(xq, layer.weight, xs, layer.weight_scale, x.dtype, bias, None, ws)
         return out.reshape(out_shape)
