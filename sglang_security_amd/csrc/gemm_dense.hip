@@ -34,6 +34,10 @@ struct DenseMma<f16_t> {
   }
 };
 
+}  // namespace sglk
+#include "dense_direct.h"
+namespace sglk {
+
 static constexpr int kDenseXTile = 64 * 256;
 __device__ __forceinline__ int dx_off(int r, int c) { return r * 256 + ((c ^ (r & 15)) << 4); }
 
@@ -278,6 +282,48 @@ static int dense_splits(int M, int N, int K) {
   return std::max(std::min(splits, 8), 1);  // measured on the 8B shapes: 8 x 1792 k beats 16 x 896 k on the down projection
 }
 
+// Splits of the packed product, and whether dense_direct.h takes it: up to 16 rows, to 32 while its inner dimension is
+// short of 8192 (32 rows, 14336 x 4096: 27.0 in eight splits of the staged kernel, 27.9 in two).  Outputs narrower than 512 stay
+// with the order of sums, and the bits, of the row-major product.  A direct block is 32 columns wide, or 64 where that
+// leaves 128 blocks: as many splits as whole blocks fit the units, each of 512 of k at least.
+struct DensePlan {
+  bool direct;
+  int splits, per;  // k-blocks a split
+};
+static DensePlan dense_packed_plan(int M, int N, int K) {
+  const int kblocks = K / 128, strips = N / 16;
+  const bool direct = N >= 512 && (M <= 16 || (M <= 32 && K < 8192)) && !getenv("SGLK_DENSE_SPLITS") && !getenv("SGLK_DENSE_NS");
+  int splits = dense_splits(M, N, K);
+  if (direct) splits = strips >= 512 ? 1 : std::max(1, std::min(256 / ((strips + 1) / 2), kblocks / 4));
+  const int per = (kblocks + splits - 1) / splits;
+  return DensePlan{direct, (kblocks + per - 1) / per, per};
+}
+
+template <typename T, int MT, int CS, int WAYS, bool PACKED>
+static int launch_dense_tile(const DenseDirectArgs& a, int splits, hipStream_t s) {
+  constexpr int lds = dense_direct_lds<MT, CS, WAYS>();
+  if (int rc = ensure_lds<&dense_direct_kernel<T, MT, CS, WAYS, PACKED>>(lds)) return rc;
+  hipLaunchKernelGGL((dense_direct_kernel<T, MT, CS, WAYS, PACKED>), dim3((a.N / 16 + CS - 1) / CS, splits), dim3(64 * WAYS), lds,
+                     s, a);
+  SGLK_LAUNCH_CHECK();
+  return SGLK_OK;
+}
+// the products that dense_packed_plan names
+template <typename T, bool PACKED>
+static int launch_dense_direct(const DenseDirectArgs& a, int splits, hipStream_t s) {
+  if (a.N >= 8192) return a.M <= 16 ? launch_dense_tile<T, 1, 4, 4, PACKED>(a, splits, s) : launch_dense_tile<T, 2, 4, 4, PACKED>(a, splits, s);
+  return a.M <= 16 ? launch_dense_tile<T, 1, 2, 8, PACKED>(a, splits, s) : launch_dense_tile<T, 2, 2, 8, PACKED>(a, splits, s);
+}
+// Calls without a workspace, unsplit, up to 16 rows.  A strip a block and sixteen waves while x is small (four rows, 65536 x 2560:
+// 53.7 us; 64 columns and eight waves 56.7) or the output narrow; from nine rows on, for outputs that fill the units so, 64
+// columns (16 rows: 57.5 and 62; 128256 x 4096 164 and 177).
+static bool dense_direct_whole(int M, int N) { return M <= 16 && N >= 512 && N % 16 == 0 && !getenv("SGLK_DENSE_NS"); }
+template <typename T, bool PACKED>
+static int launch_dense_whole(const DenseDirectArgs& a, hipStream_t s) {
+  if (a.N < 8192 || (a.M <= 8 && a.N >= 16384)) return launch_dense_tile<T, 1, 1, 16, PACKED>(a, 1, s);
+  return a.N < 16384 ? launch_dense_tile<T, 1, 4, 4, PACKED>(a, 1, s) : launch_dense_tile<T, 1, 4, 8, PACKED>(a, 1, s);
+}
+
 }  // namespace sglk
 
 using namespace sglk;
@@ -299,6 +345,24 @@ int sglk_dense_gemm_nt_ws(const void* x, const void* w, const void* bias, void* 
   SGLK_CHECK(x && w && out, "dense_gemm_nt: null pointer");
   SGLK_CHECK(M > 0 && N > 0 && K > 0, "dense_gemm_nt: bad shape");
   SGLK_CHECK(K % 128 == 0, "dense_gemm_nt: K=%d must be a multiple of 128", K);
+  const DensePlan plan = dense_packed_plan(M, N, K);
+  if (plan.direct && N % 16 == 0 && aligned16(x) && aligned16(w) && x_stride % 8 == 0 && w_stride % 8 == 0 &&
+      (plan.splits == 1 || (workspace && workspace_bytes >= (int64_t)plan.splits * M * N * (int64_t)sizeof(float) &&
+                            aligned16(workspace) && aligned16(out) && out_stride % 8 == 0))) {
+    float* partial = plan.splits > 1 ? (float*)workspace : nullptr;
+    const DenseDirectArgs a{(const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, (uint16_t*)out, partial, M, M, N, K,
+                            plan.per,           x_stride,           w_stride,              out_stride};
+    SGLK_DISPATCH_HALF(dtype, T, {
+      if (int rc = launch_dense_direct<T, false>(a, plan.splits, (hipStream_t)stream)) return rc;
+      if (partial) {
+        const int64_t vecs = (int64_t)M * (N / 8);
+        hipLaunchKernelGGL((dense_reduce_kernel<T>), dim3((unsigned)((vecs + 255) / 256)), dim3(256), 0, (hipStream_t)stream, partial,
+                           (const uint16_t*)bias, (uint16_t*)out, M, M, N, plan.splits, out_stride);
+      }
+    });
+    SGLK_LAUNCH_CHECK();
+    return SGLK_OK;
+  }
   const int splits = dense_splits(M, N, K);
   const int64_t need = sglk_dense_gemm_workspace_bytes(M, N, K);
   if (splits <= 1 || !workspace || workspace_bytes < need || !aligned16(workspace) || !aligned16(out) ||
@@ -342,6 +406,11 @@ int sglk_dense_gemm_packed(const void* x, const void* packed, const void* bias, 
   SGLK_CHECK(N % 16 == 0 && K % 128 == 0, "dense_gemm_packed: N=%d must be a multiple of 16, K=%d of 128", N, K);
   SGLK_CHECK(aligned16(x) && aligned16(packed) && x_stride % 8 == 0, "dense_gemm_packed: rows must be 16-byte aligned");
   const int mblocks = (M + 63) / 64;
+  if (dense_direct_whole(M, N)) {
+    const DenseDirectArgs a{(const uint16_t*)x, (const uint16_t*)packed, (const uint16_t*)bias, (uint16_t*)out, nullptr, M, M, N, K,
+                            K / 128,            x_stride,                0,                     out_stride};
+    SGLK_DISPATCH_HALF(dtype, T, { return launch_dense_whole<T, true>(a, (hipStream_t)stream); });
+  }
   if (N >= 16 * 1024) {
     dim3 grid((N + 127) / 128, 1, mblocks);
     SGLK_DISPATCH_HALF(dtype, T,
@@ -367,16 +436,19 @@ int sglk_dense_gemm_packed(const void* x, const void* packed, const void* bias, 
 // sglk_rope_and_store_kv_partial add the splits up in split order and round once, as the int4 path's layer fusion does).
 int sglk_dense_gemm_partial_splits(int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 128 != 0 || N % 16 != 0) return 0;
-  const int splits = dense_splits(M, N, K), kblocks = K / 128;
-  const int per = (kblocks + splits - 1) / splits;
-  return (kblocks + per - 1) / per;  // every split non-empty
+  return dense_packed_plan(M, N, K).splits;  // every split non-empty
 }
 
 static int dense_packed_split_launch(const void* x, const void* packed, float* partial, int M, int Mpad, int N, int K,
                                      int64_t x_stride, int dtype, hipStream_t s) {
-  const int splits = dense_splits(M, N, K), kblocks = K / 128;
-  const int per = (kblocks + splits - 1) / splits;
-  const int used = (kblocks + per - 1) / per;
+  const DensePlan plan = dense_packed_plan(M, N, K);
+  const int used = plan.splits, per = plan.per;
+  if (plan.direct) {
+    const DenseDirectArgs a{(const uint16_t*)x, (const uint16_t*)packed, nullptr, nullptr, partial, M, Mpad, N, K, per, x_stride, 0, 0};
+    int rc = SGLK_OK;
+    SGLK_DISPATCH_HALF(dtype, T, { rc = launch_dense_direct<T, true>(a, used, s); });
+    return rc == SGLK_OK ? used : rc;
+  }
   static const int env_ns = getenv("SGLK_DENSE_NS") ? atoi(getenv("SGLK_DENSE_NS")) : 0;
   // two strips per wave (128 columns per block) halve the activation re-reads; not where that leaves a fractional
   // round of blocks on the 256 CUs below two full rounds (measured on the 8B shapes: o and down 256 blocks, gate_up
@@ -418,6 +490,12 @@ int sglk_dense_gemm_packed_ws(const void* x, const void* packed, const void* bia
   SGLK_CHECK(M > 0 && N > 0 && K > 0, "dense_gemm_packed: bad shape");
   const int splits = (N % 16 == 0 && K % 128 == 0) ? sglk_dense_gemm_partial_splits(M, N, K) : 1;
   const int64_t need = (int64_t)splits * M * N * (int64_t)sizeof(float);
+  if (splits == 1 && N % 16 == 0 && K % 128 == 0 && aligned16(x) && aligned16(packed) && x_stride % 8 == 0 &&
+      dense_packed_plan(M, N, K).direct) {  // the sums of _partial, finished here
+    const DenseDirectArgs a{(const uint16_t*)x, (const uint16_t*)packed, (const uint16_t*)bias, (uint16_t*)out, nullptr, M, M, N, K,
+                            K / 128,            x_stride,                0,                     out_stride};
+    SGLK_DISPATCH_HALF(dtype, T, { return launch_dense_direct<T, true>(a, 1, (hipStream_t)stream); });
+  }
   if (splits <= 1 || !workspace || workspace_bytes < need || !aligned16(workspace) || !aligned16(out) || N % 8 != 0 ||
       out_stride % 8 != 0)
     return sglk_dense_gemm_packed(x, packed, bias, out, M, N, K, x_stride, out_stride, dtype, stream);
@@ -479,6 +557,11 @@ int sglk_dense_gemm_nt(const void* x, const void* w, const void* bias, void* out
   const int mblocks = (M + 63) / 64;
   // two strips per wave halve the activation re-reads; kept for wide outputs only, where the grid still
   // fills the chip several times over
+  if (dense_direct_whole(M, N)) {
+    const DenseDirectArgs a{(const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, (uint16_t*)out, nullptr, M, M, N, K,
+                            K / 128,            x_stride,           w_stride,              out_stride};
+    SGLK_DISPATCH_HALF(dtype, T, { return launch_dense_whole<T, false>(a, (hipStream_t)stream); });
+  }
   const char* env = getenv("SGLK_DENSE_NS");  // 1 / 2 forces the strips per wave (tests)
   const int force = env ? atoi(env) : 0;
   const bool two = force ? force == 2 : N >= 64 * 1024;

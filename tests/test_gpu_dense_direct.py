@@ -1,0 +1,64 @@
+"""16-bit products of at most 32 rows (dense_direct.h): the first and last rows of each form and one beyond; column counts on
+either side of each tile rule, with strips that do not fill a block; k-blocks that do not fill a turn or a split."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32, 33])
+@pytest.mark.parametrize("N,K", [(512, 128), (528, 1152), (2560, 2688), (4112, 640), (8192 - 16, 384), (8192 + 16, 384), (16384 - 16, 256),
+                                 (16384 + 16, 256), (1024, 8320)])
+def test_products(M, N, K, dtype):
+    from sglang_security_amd import ops
+
+    g = torch.Generator(device=DEV).manual_seed(M * N + K)
+    wide = torch.randn(M, K + 64, generator=g, device=DEV).to(dtype)    # rows with something behind them
+    x, w = wide[:, :K], torch.randn(N, K, generator=g, device=DEV).to(dtype)
+    bias = torch.randn(N, generator=g, device=DEV).to(dtype)
+    packed = ops.dense_repack(w)
+    exact = x.double() @ w.double().t()
+    bound = (x.double().abs() @ w.double().abs().t()) * 2.0 ** -21      # fp32 sums of K products
+    splits = ops.dense_gemm_partial_splits(M, N, K)
+    part = torch.full((splits, M, N), float("nan"), device=DEV)
+    assert ops.dense_gemm_packed_partial(x, packed, part) == splits
+    assert ((part.double().sum(0) - exact).abs() <= bound).all()
+    ulp = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    for b in (None, bias):
+        want = exact if b is None else exact + b.double()
+        tol = want.abs() * ulp + bound * 2
+        out = torch.full((M + 1, N + 8), 7.0, dtype=dtype, device=DEV)
+        ops.dense_gemm_packed(x, packed, b, out[:M, :N])
+        assert ((out[:M, :N].double() - want).abs() <= tol).all()
+        assert (out[M:] == 7).all() and (out[:, N:] == 7).all()
+        ws = torch.empty(max(splits * M * N, 4), device=DEV)
+        out = torch.full((M, N), float("nan"), dtype=dtype, device=DEV)
+        ops.dense_gemm_packed_ws(x, packed, b, out, ws)
+        assert ((out.double() - want).abs() <= tol).all()
+        # the row-major weight, with the same bits up to 16 rows
+        rows = torch.empty(M, N, dtype=dtype, device=DEV)
+        ops.dense_gemm_nt(x, w, b, rows, torch.empty(max(ops.dense_gemm_workspace_bytes(M, N, K), 16), dtype=torch.uint8, device=DEV))
+        assert ((rows.double() - want).abs() <= tol).all() and (M > 16 or torch.equal(rows, out))
+        assert ((ops.dense_gemm_nt(x, w, b).double() - want).abs() <= tol).all()
+        assert M > 16 or torch.equal(ops.dense_gemm_nt(x, w, b), ops.dense_gemm_packed(x, packed, b))
+
+
+@pytest.mark.parametrize("M", [1, 16])
+@pytest.mark.parametrize("N", [2560, 16384])
+def test_rows_and_columns_that_are_not_numbers(M, N):
+    from sglang_security_amd import ops
+
+    g = torch.Generator(device=DEV).manual_seed(N)
+    x = torch.randn(M, 1280, generator=g, device=DEV).bfloat16()
+    w = torch.randn(N, 1280, generator=g, device=DEV).bfloat16()
+    clean = ops.dense_gemm_packed(x, ops.dense_repack(w))
+    x[M - 1, 7] = float("inf")
+    w[100, 5] = float("nan")
+    got = ops.dense_gemm_packed(x, ops.dense_repack(w))
+    assert not got[M - 1].isfinite().any() and got[:, 100].isnan().all()
+    keep = torch.ones_like(got, dtype=torch.bool)
+    keep[M - 1] = False
+    keep[:, 100] = False
+    assert torch.equal(got[keep], clean[keep])
