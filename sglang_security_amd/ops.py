@@ -19,8 +19,12 @@ def _ptr(t: Optional[torch.Tensor]) -> int:
     return 0 if t is None else t.data_ptr()
 
 
+# the current stream's handle without a Stream object around it (3 us of a call's 13): what torch's own launchers use
+_raw_stream = torch._C._cuda_getCurrentRawStream
+
+
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.device.index)
 
 
 def _need_gpu(*ts):
@@ -503,8 +507,9 @@ def set_kv_buffer(k_buffer, v_buffer, loc, cache_k, cache_v, k_scale=None, v_sca
     cv = cache_v.reshape(T, -1)
     if ck.stride(1) != 1 or cv.stride(1) != 1:
         raise SglkError("set_kv_buffer: cache_k/cache_v rows must be contiguous")
-    kb = k_buffer.view(k_buffer.shape[0], -1)
-    vb = v_buffer.view(v_buffer.shape[0], -1)
+    # (rows of a pool that is not contiguous have to view as rows of two dimensions, or they are refused)
+    kb = k_buffer if k_buffer.is_contiguous() else k_buffer.view(k_buffer.shape[0], -1)
+    vb = v_buffer if v_buffer.is_contiguous() else v_buffer.view(v_buffer.shape[0], -1)
     check(lib().sglk_set_kv_buffer(_ptr(kb), _ptr(vb), _ptr(ck), _ptr(cv), _ptr(loc), _is64(loc), T, ck.shape[1],
                                    cv.shape[1], kb.stride(0), vb.stride(0), ck.stride(0), cv.stride(0),
                                    k_buffer.element_size(), _stream(k_buffer)), "set_kv_buffer")
