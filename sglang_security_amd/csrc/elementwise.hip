@@ -581,79 +581,89 @@ __global__ void __launch_bounds__(256) act_and_mul_xs_kernel(void* __restrict__ 
   }
 }
 
-// Greedy token: index of the first maximum of every row (torch.argmax, sampler.py greedy path).  One block per row,
-// eight elements per load for 16-bit rows.  The scan is bound by vector instructions, so a thread's own elements (which
-// it visits in ascending order) take one strict comparison each and NaNs are only noted; a row that holds one (a NaN
-// wins, as in torch) is scanned again with the full rule.
-template <typename T>
+// Greedy token: index of the first maximum of every row (torch.argmax, sampler.py greedy path), one block per row.  A 16-bit
+// row is read eight elements a load, U loads of a thread in flight: a large vocabulary's row is one trip to memory.  What
+// is left are vector instructions, so a load's maximum comes from v_maximum3 (which keeps a NaN), is compared with the
+// thread's own once, and the load that held it is kept; the place inside it is looked for at the end.  A row that holds a
+// NaN (it wins, as in torch) is read again for the first one.
+// One row of 128256 bf16 elements: 12.8 us with a comparison an element -> 6.1; 64 rows 14.5 -> 7.2; one fp32 row 23.5 -> 9.3.
+__device__ __forceinline__ float maximum3(float a, float b, float c) {  // (builtins are regrouped into two-operand forms)
+  float r;
+  asm("v_maximum3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  return r;
+}
+
+template <typename T, int U>
 __global__ void __launch_bounds__(1024) argmax_rows_kernel(const void* __restrict__ x, int64_t* __restrict__ out, int cols,
                                                            int64_t row_stride) {
+  constexpr int kNone = 0x7fffffff;
   __shared__ float bv[16];
   __shared__ int bi[16];
   const int64_t row = blockIdx.x;
   float best = -INFINITY;
-  int idx = 0x7fffffff;
-  bool any_nan = false;
-  auto take = [&](float v, int i) {  // a NaN wins, as in torch; among equals (and among NaNs) the lowest index
-    const bool vn = v != v, bn = best != best;
-    if (vn ? (!bn || i < idx) : (!bn && (v > best || (v == best && i < idx)))) {
-      best = v;
-      idx = i;
-    }
-  };
-  auto scan = [&](auto&& visit) {
-    if constexpr (sizeof(typename Raw<T>::type) == 2) {
-      const uint16_t* r = reinterpret_cast<const uint16_t*>(x) + row * row_stride;
-      const int nv = ((row_stride % 8) == 0 && aligned16(x)) ? cols / 8 : 0;
-      // four loads in flight per thread: a row of a large vocabulary is a few trips to memory instead of sixteen
-      int v = threadIdx.x;
-      for (; v + 3 * 1024 < nv; v += 4 * 1024) {
-        short8 q[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) q[u] = reinterpret_cast<const short8*>(r)[v + 1024 * u];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-          for (int j = 0; j < 8; ++j) visit(Conv<T>::to_f32((uint16_t)q[u][j]), 8 * (v + 1024 * u) + j);
-      }
-      for (; v < nv; v += 1024) {
-        const short8 q = reinterpret_cast<const short8*>(r)[v];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) visit(Conv<T>::to_f32((uint16_t)q[j]), 8 * v + j);
-      }
-      for (int i = nv * 8 + threadIdx.x; i < cols; i += 1024) visit(Conv<T>::to_f32(r[i]), i);
-    } else {
-      for (int i = threadIdx.x; i < cols; i += 1024) visit(ld<T>(x, row * row_stride + i), i);
-    }
-  };
+  int idx = kNone;
   // ascending indices within a thread: the first of equal values stays with a strict comparison (a row of nothing
   // but -inf keeps the sentinel and ends at index 0)
-  scan([&](float v, int i) {
-    any_nan |= v != v;
-    if (v > best) {
-      best = v;
-      idx = i;
-    }
-  });
-  if (__syncthreads_or(any_nan)) {  // block-uniform
-    best = -INFINITY;
-    idx = 0x7fffffff;
-    scan(take);
-  }
+  auto one = [&](float v, int i) {
+    if (v > best) idx = i;
+    best = __builtin_elementwise_maximum(best, v);
+  };
+  int done = 0;  // elements in front of the part that is read one by one
+  if constexpr (sizeof(typename Raw<T>::type) == 2) {
+    const uint16_t* r = reinterpret_cast<const uint16_t*>(x) + row * row_stride;
+    const int nv = ((row_stride % 8) == 0 && aligned16(x)) ? cols / 8 : 0;
+    int at = -1;
+    short8 held = short8{};
+    for (int first = threadIdx.x; first - (int)threadIdx.x < nv; first += U * 1024) {
+      short8 q[U];  // behind the last whole piece that piece again: it changes nothing
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(best, o, 64);
-    const int oi = __shfl_xor(idx, o, 64);
-    take(ov, oi);
+      for (int u = 0; u < U; ++u) q[u] = reinterpret_cast<const short8*>(r)[min(first + 1024 * u, nv - 1)];
+      __builtin_amdgcn_sched_barrier(0);  // (the loads would be moved down to where they are used)
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        float m = best;
+#pragma unroll
+        for (int j = 0; j < 8; j += 2)
+          m = maximum3(m, Conv<T>::to_f32((uint16_t)q[u][j]), Conv<T>::to_f32((uint16_t)q[u][j + 1]));
+        if (m > best) {
+          held = q[u];
+          at = min(first + 1024 * u, nv - 1);
+        }
+        best = m;
+      }
+    }
+    if (at >= 0) {
+#pragma unroll
+      for (int j = 7; j >= 0; --j)
+        if (Conv<T>::to_f32((uint16_t)held[j]) == best) idx = 8 * at + j;
+    }
+    done = nv * 8;
   }
+#pragma unroll 4
+  for (int i = done + threadIdx.x; i < cols; i += 1024) one(ld<T>(x, row * row_stride + i), i);
+  const bool nan = __syncthreads_or(best != best);  // block-uniform
+  if (nan) {
+    idx = kNone;
+    for (int i = threadIdx.x; i < cols && idx == kNone; i += 1024) {
+      const float v = ld<T>(x, row * row_stride + i);
+      if (v != v) idx = i;
+    }
+  }
+  auto lowest = [](float a, float b) { return __int_as_float(min(__float_as_int(a), __float_as_int(b))); };
+  auto fold = [&](float v, int i) {  // every lane: the lowest index among the lanes that hold the maximum (or a NaN)
+    const float m = wave_max(v);
+    best = m;
+    idx = __float_as_int(wave_fold(__int_as_float(nan || v == m ? i : kNone), lowest));
+  };
+  fold(best, idx);
   if ((threadIdx.x & 63) == 0) {
     bv[threadIdx.x >> 6] = best;
     bi[threadIdx.x >> 6] = idx;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < 16; ++w) take(bv[w], bi[w]);
-    out[row] = idx == 0x7fffffff ? 0 : idx;
+  if (threadIdx.x < 64) {
+    fold(bv[threadIdx.x & 15], bi[threadIdx.x & 15]);
+    if (threadIdx.x == 0) out[row] = idx == kNone ? 0 : idx;
   }
 }
 
@@ -1030,9 +1040,19 @@ int sglk_argmax(const void* x, int64_t* out, int64_t rows, int cols, int64_t row
   SGLK_CHECK(rows >= 0 && cols > 0 && row_stride >= cols, "argmax: bad shape");
   if (rows == 0) return SGLK_OK;
   SGLK_CHECK(x && out, "argmax: null pointer");
-  SGLK_DISPATCH_FLOAT(dtype, T,
-                      hipLaunchKernelGGL((argmax_rows_kernel<T>), dim3((unsigned)rows), dim3(1024), 0, (hipStream_t)stream,
-                                         x, out, cols, row_stride));
+  // as many loads in flight as the row needs: one that a short row has no use for reads its last piece again
+#define SGLK_AM(U) \
+  hipLaunchKernelGGL((argmax_rows_kernel<T, U>), dim3((unsigned)rows), dim3(1024), 0, (hipStream_t)stream, x, out, cols, row_stride)
+  SGLK_DISPATCH_FLOAT(dtype, T, {
+    constexpr int kMost = sizeof(typename Raw<T>::type) == 2 ? 16 : 2;  // (fp32 rows are read one by one)
+    if (cols > 8 * 8 * 1024)
+      SGLK_AM(kMost);
+    else if (cols > 8 * 2 * 1024)
+      SGLK_AM(std::min(kMost, 8));
+    else
+      SGLK_AM(2);
+  });
+#undef SGLK_AM
   SGLK_LAUNCH_CHECK();
   return SGLK_OK;
 }

@@ -153,6 +153,27 @@ def test_argmax_rows_special_values(dtype):
     assert torch.equal(out[6:], torch.argmax(x[6:], dim=-1))
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("cols", [7, 16384, 16392, 65536, 65541, 131072, 131080, 270000])
+def test_argmax_rows_of_every_length_class(dtype, cols):
+    """Rows of two, eight and sixteen loads a thread, with and without a second round and a remainder: the maximum at the
+    first and the last element, at the seams of the loads, twice in one load, and one NaN behind a larger infinity."""
+    ops = _ops()
+    g = torch.Generator().manual_seed(cols)
+    places = sorted({0, 7 % cols, cols - 1, min(8 * 1024, cols - 1), min(8 * 1024 - 1, cols - 1), (cols - 1) // 8 * 8})
+    x = torch.randn(len(places) + 2, cols, generator=g).clamp(-3, 3)
+    for r, c in enumerate(places):
+        x[r, c] = 9.0
+        x[r, min(c + 1, cols - 1)] = 9.0
+    x[-2, cols // 2] = float("nan")
+    x[-2, 0] = float("inf")
+    x[-1] = float("-inf")
+    x = x.to(dtype).to(DEV)
+    out = torch.empty(len(x), dtype=torch.int64, device=DEV)
+    ops.argmax(x, out)
+    assert out.tolist() == places + [cols // 2, 0]
+
+
 def _run_decode(ops, g, dtype, max_splits=8, splits=None):
     q = g["q"].to(dtype).to(DEV)
     kb, vb = g["k_buffer"].to(dtype).to(DEV), g["v_buffer"].to(dtype).to(DEV)
