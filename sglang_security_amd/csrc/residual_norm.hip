@@ -12,12 +12,15 @@
 
 namespace sglk {
 
-__device__ __forceinline__ float block_sum256(float v, float* red) {
+template <int NW>
+__device__ __forceinline__ float waves_sum(float v, float* red) {
   v = wave_sum(v);
-  __syncthreads();  // red may still be read from an earlier call
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
-  return red[0] + red[1] + red[2] + red[3];
+  float sum = red[0];
+#pragma unroll
+  for (int i = 1; i < NW; ++i) sum += red[i];
+  return sum;
 }
 
 struct ResidualNorm {
@@ -40,17 +43,32 @@ struct ResidualNorm {
   float eps;
 };
 
-template <typename T, int VPT>
-__global__ void __launch_bounds__(256) residual_norm_kernel(ResidualNorm a) {
-  __shared__ float red[4];
+// One block of BT threads a row, VPT pieces of eight elements a thread.  PRE, for few rows: a launch is then a chain of trips
+// to memory and two block sums, so the weights of both norms and what is added on the way are asked for before the first
+// sum, not behind it (16 rows of 2560, two split sums a piece on 256 threads -> a piece a thread and PRE: 5.4 us -> 4.5).
+template <typename T, int BT, int VPT, bool PRE>
+__global__ void __launch_bounds__(BT) residual_norm_kernel(ResidualNorm a) {
+  constexpr int PV = PRE ? VPT : 1;
+  __shared__ float red[2][BT / 64];
   const int out_row = blockIdx.x;
   const int row = a.rows ? a.rows[out_row] : out_row;
   const int nv = a.pitch / 8;
-  float x[VPT][8], s[VPT][8];
+  float x[VPT][8], s[VPT][8], wp[PV][8], wn[PV][8], t0[PV][8], ts[PV][8];
   float ss = 0.f;
+  if constexpr (PRE) {
+#pragma unroll
+    for (int i = 0; i < VPT; ++i) {
+      const int v = threadIdx.x + BT * i;
+      if (v >= nv) continue;
+      if (a.src.p && a.w_post) ld8<float>(a.w_post, 8 * v, wp[i]);
+      if (a.w_next) ld8<float>(a.w_next, 8 * v, wn[i]);
+      if (a.add_x0) ld8<float>(a.x0, (int64_t)row * a.pitch + 8 * v, t0[i]);
+      if (a.step) ld8<float>(a.step, 8 * v, ts[i]);
+    }
+  }
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
-    const int v = threadIdx.x + 256 * i;
+    const int v = threadIdx.x + BT * i;
 #pragma unroll
     for (int j = 0; j < 8; ++j) x[i][j] = s[i][j] = 0.f;
     if (v >= nv) continue;
@@ -71,14 +89,14 @@ __global__ void __launch_bounds__(256) residual_norm_kernel(ResidualNorm a) {
   }
   if (a.src.p) {
     float inv = 1.f;
-    if (a.w_post) inv = 1.0f / sqrtf(block_sum256(ss, red) / (float)a.width + a.eps);
+    if (a.w_post) inv = 1.0f / sqrtf(waves_sum<BT / 64>(ss, red[0]) / (float)a.width + a.eps);
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-      const int v = threadIdx.x + 256 * i;
+      const int v = threadIdx.x + BT * i;
       if (v >= nv) continue;
-      float w[8];
       if (a.w_post) {
-        ld8<float>(a.w_post, 8 * v, w);
+        float(&w)[8] = wp[PRE ? i : 0];
+        if constexpr (!PRE) ld8<float>(a.w_post, 8 * v, w);
 #pragma unroll
         for (int j = 0; j < 8; ++j) x[i][j] += s[i][j] * inv * w[j];
       } else {
@@ -90,16 +108,17 @@ __global__ void __launch_bounds__(256) residual_norm_kernel(ResidualNorm a) {
   float xx = 0.f;
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
-    const int v = threadIdx.x + 256 * i;
+    const int v = threadIdx.x + BT * i;
     if (v >= nv) continue;
-    float t[8];
     if (a.add_x0) {
-      ld8<float>(a.x0, (int64_t)row * a.pitch + 8 * v, t);
+      float(&t)[8] = t0[PRE ? i : 0];
+      if constexpr (!PRE) ld8<float>(a.x0, (int64_t)row * a.pitch + 8 * v, t);
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[i][j] += t[j];
     }
     if (a.step) {
-      ld8<float>(a.step, 8 * v, t);
+      float(&t)[8] = ts[PRE ? i : 0];
+      if constexpr (!PRE) ld8<float>(a.step, 8 * v, t);
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[i][j] += t[j];
     }
@@ -108,13 +127,13 @@ __global__ void __launch_bounds__(256) residual_norm_kernel(ResidualNorm a) {
     for (int j = 0; j < 8; ++j) xx += x[i][j] * x[i][j];
   }
   if (a.w_next) {
-    const float inv = 1.0f / sqrtf(block_sum256(xx, red) / (float)a.width + a.eps);
+    const float inv = 1.0f / sqrtf(waves_sum<BT / 64>(xx, red[1]) / (float)a.width + a.eps);
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-      const int v = threadIdx.x + 256 * i;
+      const int v = threadIdx.x + BT * i;
       if (v >= nv) continue;
-      float w[8];
-      ld8<float>(a.w_next, 8 * v, w);
+      float(&w)[8] = wn[PRE ? i : 0];
+      if constexpr (!PRE) ld8<float>(a.w_next, 8 * v, w);
 #pragma unroll
       for (int j = 0; j < 8; ++j) w[j] *= x[i][j] * inv;
       st8<T>(a.h, (int64_t)out_row * a.h_stride + 8 * v, w);
@@ -217,17 +236,25 @@ int sglk_residual_norm(float* x, const void* embed, const int32_t* ids, int64_t 
   ResidualNorm a{x, embed, ids, embed_stride, embed_scale, RowSource{src, src_f32, splits, part_stride, src_stride}, w_post, x0,
                  add_x0, step, w_next, h, h_stride, rows, store_x, width, pitch, eps};
   const int vecs = pitch / 8;
-#define SGLK_RN(V) hipLaunchKernelGGL((residual_norm_kernel<T, V>), dim3(M), dim3(256), 0, (hipStream_t)stream, a)
+  // up to two rows a CU, every piece is on a thread of its own; more of them fill the chip at any block size, and there
+  // the registers that PRE holds cost more than its earlier requests give (7921 rows of 2560: 47 us -> 54)
+  const bool few = M <= 512;
+#define SGLK_RN(BT, V, P) hipLaunchKernelGGL((residual_norm_kernel<T, BT, V, P>), dim3(M), dim3(BT), 0, (hipStream_t)stream, a)
   SGLK_DISPATCH_FLOAT(dtype, T, {
-    if (vecs <= 256) {
-      SGLK_RN(1);
-    } else if (vecs <= 512) {
-      SGLK_RN(2);
-    } else if (vecs <= 1024) {
-      SGLK_RN(4);
-    } else {
-      SGLK_RN(8);
-    }
+    if (few && vecs <= 256)
+      SGLK_RN(256, 1, true);
+    else if (few && vecs <= 512)
+      SGLK_RN(512, 1, true);
+    else if (few && vecs <= 1024)
+      SGLK_RN(1024, 1, true);
+    else if (vecs <= 256)
+      SGLK_RN(256, 1, false);
+    else if (vecs <= 512)
+      SGLK_RN(256, 2, false);
+    else if (vecs <= 1024)
+      SGLK_RN(256, 4, false);
+    else
+      SGLK_RN(256, 8, false);
   });
 #undef SGLK_RN
   SGLK_LAUNCH_CHECK();

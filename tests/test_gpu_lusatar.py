@@ -79,6 +79,24 @@ def test_residual_norm(width, pitch, dtype, splits):
     assert torch.equal(before, xd)
 
 
+@pytest.mark.parametrize("pitch", [128, 2056, 4096, 4104, 8192])
+@pytest.mark.parametrize("dtype", [BF16, F32])
+def test_residual_norm_of_few_and_many_rows(pitch, dtype):
+    """512 rows take a thread a piece, 513 take 256 threads a row: the same sums in another grouping."""
+    from sglang_security_amd import ops_hybrid as H
+
+    g, eps = gen(pitch), 1e-5
+    d = lambda t: t.clone().to(DEV)
+    x, s, x0, wp, wn, step = rnd(g, 513, pitch), rnd(g, 513, pitch), rnd(g, 513, pitch), rnd(g, pitch), rnd(g, pitch), rnd(g, pitch)
+    for rows in (512, 513):
+        src, sv = source(s[:rows], 2, dtype)
+        xd, h = d(x[:rows]), torch.empty(rows, pitch, dtype=dtype, device=DEV)
+        H.residual_norm(xd, pitch, eps, h, d(wn), src, d(wp), x0=d(x0[:rows]), add_x0=True, step=d(step), dtype=dtype)
+        want = x[:rows].double() + O.rms_norm(sv, wp.double(), eps) + x0[:rows].double() + step.double()
+        close(xd, want, 2e-6, "x")
+        close(h, O.rms_norm(want, wn.double(), eps), 2 * TOL[dtype], "h")
+
+
 @pytest.mark.parametrize("dtype,splits", [(BF16, 0), (BF16, 5), (F32, 1)])
 def test_activations_and_capped_logits(dtype, splits):
     from sglang_security_amd import ops_hybrid as H
