@@ -10,6 +10,11 @@
 // [16 bytes], i.e. every instruction of a wave reads 1 KiB of consecutive memory and a wave walks its strip as one
 // sequential stream -- the row-major form leaves a fifth of the HBM bandwidth unused on the lm_head (rows 8 KiB
 // apart fall on few channels at a time).
+//
+// The loop waits for nothing but what it needs next (64 rows, weights from memory, packed: 4096 x 4096 32.3 us with a wait for
+// everything at each k-block's barrier -> 24.3; 14336 x 4096 110 -> 76; 28672 x 4096 57 -> 45; 16384 x 2560, with one
+// strip a wave as well, 33 -> 22; 128256 x 4096, where many blocks a unit had covered those waits, 190 -> 192, 5.5 TB/s:
+// neither deeper rings, 256 columns a block nor k-blocks begun at different places changed that one).
 #include <algorithm>
 #include <cstdlib>
 
@@ -60,10 +65,9 @@ __global__ void __launch_bounds__(256, 2) dense_gemm_nt_kernel(const uint16_t* _
   const int xr = threadIdx.x >> 2, xq = threadIdx.x & 3;
   // rows past M re-read row M - 1 (their products land in rows nobody reads): no exec-masked branch in the loop
   const uint16_t* xsrc = x + (int64_t)min(m0 + xr, M - 1) * x_stride + 32 * xq;
-  // Activations are requested two k-blocks ahead: loads return in order, so the wait before a tile is
-  // parked leaves only the weight loads issued after its request in flight, and that has to be the
-  // whole weight prefetch depth.
-  int4v xreg[2][4];
+  // Activations and weights are requested PF k-blocks ahead, in turn: loads return in order, so the wait for a tile that is
+  // to be parked leaves the weights of the blocks behind it on their way.
+  int4v xreg[PF][4];
   auto x_fetch = [&](int4v(&xr4)[4], int kb) {
 #pragma unroll
     for (int c = 0; c < 4; ++c)
@@ -94,15 +98,12 @@ __global__ void __launch_bounds__(256, 2) dense_gemm_nt_kernel(const uint16_t* _
     return PACKED ? __builtin_nontemporal_load(reinterpret_cast<const int4v*>(p)) : *reinterpret_cast<const int4v*>(p);
   };
   int4v wq[PF][NS][4];
+  auto w_fetch = [&](int p, int j) {
 #pragma unroll
-  for (int p = 0; p < PF; ++p)
-    if (p < nkb) {
+    for (int s = 0; s < NS; ++s)
 #pragma unroll
-      for (int s = 0; s < NS; ++s)
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-          wq[p][s][c] = wload(wsrc[s] + kbs * p + cs * c);
-    }
+      for (int c = 0; c < 4; ++c) wq[p][s][c] = wload(wsrc[s] + kbs * (int64_t)j + cs * c);
+  };
 
   float4v oacc[NS][4];
 #pragma unroll
@@ -110,62 +111,99 @@ __global__ void __launch_bounds__(256, 2) dense_gemm_nt_kernel(const uint16_t* _
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) oacc[s][mt] = float4v{0.f, 0.f, 0.f, 0.f};
 
-  static_assert(PF % 2 == 0, "the activation registers alternate with the parity of the k-block");
-  x_fetch(xreg[0], kb0);
-  if (nkb > 1) x_fetch(xreg[1], kb0 + 1);
+  static_assert(PF % 2 == 0, "the halves of LDS go by the parity of the k-block");
+#pragma unroll
+  for (int p = 0; p < PF; ++p) {
+    x_fetch(xreg[p], kb0 + min(p, nkb - 1));
+    w_fetch(p, min(p, nkb - 1));
+    __builtin_amdgcn_sched_barrier(0);
+  }
   x_park(xreg[0], 0);
-  __syncthreads();
+  auto meet = [] {  // not for what is on its way from memory
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  meet();
 
-  for (int base = 0; base < nkb; base += PF) {
+  // Whole rounds hold no branch: behind one the compiler would wait for everything that may be on its way.
+  auto step = [&](int j, int p, auto whole) {
+    constexpr bool kWhole = decltype(whole)::value;
+    const int buf = p & 1;
 #pragma unroll
-    for (int p = 0; p < PF; ++p) {
-      const int j = base + p;
-      if (j < nkb) {
-        const int buf = j & 1;
-        if (j + 2 < nkb) x_fetch(xreg[p & 1], kb0 + j + 2);  // block j's own registers were parked a step ago
+    for (int ks = 0; ks < 4; ++ks) {
+      // k-slots of step ks: k = 128*kb + 32*ks + 8*g + e  <->  activation chunk 4*ks + g
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-          // k-slots of step ks: k = 128*kb + 32*ks + 8*g + e  <->  activation chunk 4*ks + g
+      for (int mt = 0; mt < 4; ++mt) {
+        const int4v af = *reinterpret_cast<const int4v*>(xs + buf * kDenseXTile + dx_off(16 * mt + i16, 4 * ks + g));
 #pragma unroll
-          for (int mt = 0; mt < 4; ++mt) {
-            const int4v af = *reinterpret_cast<const int4v*>(xs + buf * kDenseXTile + dx_off(16 * mt + i16, 4 * ks + g));
-#pragma unroll
-            for (int s = 0; s < NS; ++s) oacc[s][mt] = DenseMma<T>::mma(af, wq[p][s][ks], oacc[s][mt]);
-          }
-        }
-        if (j + PF < nkb) {
-#pragma unroll
-          for (int s = 0; s < NS; ++s)
-#pragma unroll
-            for (int c = 0; c < 4; ++c)
-              wq[p][s][c] = wload(wsrc[s] + kbs * (int64_t)(j + PF) + cs * c);
-        }
-        if (j + 1 < nkb) x_park(xreg[(p + 1) & 1], buf ^ 1);
-        __syncthreads();
+        for (int s = 0; s < NS; ++s) oacc[s][mt] = DenseMma<T>::mma(af, wq[p][s][ks], oacc[s][mt]);
       }
     }
+    if (kWhole || j + PF < nkb) {
+      x_fetch(xreg[p], kb0 + j + PF);  // block j was parked a step ago
+      w_fetch(p, j + PF);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (kWhole || j + 1 < nkb) {
+      x_park(xreg[(p + 1) % PF], buf ^ 1);  // its readers met at the end of the step before
+      meet();
+    }
+  };
+  int base = 0;
+  for (; base + 2 * PF <= nkb; base += PF) {
+#pragma unroll
+    for (int p = 0; p < PF; ++p) step(base + p, p, std::true_type());
   }
+#pragma unroll
+  for (int p = 0; p < 2 * PF - 1; ++p)
+    if (base + p < nkb) step(base + p, p % PF, std::false_type());
 
-  const bool direct = partial == nullptr;
+  if (partial) {
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const int n = n0 + 16 * s;
+      if (n >= N) continue;
+#pragma unroll
+      for (int mt = 0; mt < 4; ++mt)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int m = m0 + 16 * mt + 4 * g + r;
+          // written through (agent scope): megabytes of partials left dirty in the L2s would be written back at the
+          // kernel's end, inside its duration (see the wide int4 GEMM)
+          if (m < Mpad)
+            __hip_atomic_store(&partial[((int64_t)blockIdx.y * Mpad + m) * N + n], oacc[s][mt][r], __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    return;
+  }
+  // finished rows leave through LDS, sixteen bytes a thread: a lane of the accumulators holds single elements of four rows
+  constexpr int kCols = 64 * NS, kPitch = kCols + 8;
+  static_assert(64 * kPitch * 2 <= 2 * kDenseXTile, "the block's outputs fit the activations' tiles");
+  uint16_t* ys = reinterpret_cast<uint16_t*>(xs);
+  meet();
 #pragma unroll
   for (int s = 0; s < NS; ++s) {
-    const int n = n0 + 16 * s;
-    if (n >= N) continue;
-    const float bv = (direct && bias) ? Conv<T>::to_f32(bias[n]) : 0.f;
+    const float bv = bias && n0 + 16 * s < N ? Conv<T>::to_f32(bias[n0 + 16 * s]) : 0.f;
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = m0 + 16 * mt + 4 * g + r;
-        if (direct) {
-          if (m < M) out[(int64_t)m * out_stride + n] = Conv<T>::from_f32(oacc[s][mt][r] + bv);
-        } else if (m < Mpad) {
-          // written through (agent scope): megabytes of partials left dirty in the L2s would be written back at the
-          // kernel's end, inside its duration (see the wide int4 GEMM)
-          __hip_atomic_store(&partial[((int64_t)blockIdx.y * Mpad + m) * N + n], oacc[s][mt][r], __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_AGENT);
-        }
-      }
+      for (int r = 0; r < 4; ++r)
+        ys[(16 * mt + 4 * g + r) * kPitch + 16 * (NS * wid + s) + i16] = Conv<T>::from_f32(oacc[s][mt][r] + bv);
+  }
+  meet();
+  const bool wide = out_stride % 8 == 0 && aligned16(out);
+  for (int e = threadIdx.x; e < 64 * (kCols / 8); e += 256) {
+    const int r = e / (kCols / 8), c = e % (kCols / 8) * 8, n = blockIdx.x * kCols + c;
+    if (m0 + r >= M) break;
+    uint16_t* o = out + (int64_t)(m0 + r) * out_stride + n;
+    const uint16_t* y = ys + r * kPitch + c;
+    if (wide && n + 8 <= N) {
+      *reinterpret_cast<int4v*>(o) = *reinterpret_cast<const int4v*>(y);
+    } else {
+      for (int j = 0; j < 8 && n + j < N; ++j) o[j] = y[j];
+    }
   }
 }
 
@@ -411,7 +449,9 @@ int sglk_dense_gemm_packed(const void* x, const void* packed, const void* bias, 
                             K / 128,            x_stride,                0,                     out_stride};
     SGLK_DISPATCH_HALF(dtype, T, { return launch_dense_whole<T, true>(a, (hipStream_t)stream); });
   }
-  if (N >= 16 * 1024) {
+  // two strips a wave halve what is read of x; one, where 128 columns a block would leave units without a block (64 rows:
+  // 16384 x 2560 28.0 us and 21.5, 28672 x 4096 44.6 and 54.3)
+  if ((N + 127) / 128 * mblocks >= 192) {
     dim3 grid((N + 127) / 128, 1, mblocks);
     SGLK_DISPATCH_HALF(dtype, T,
                        hipLaunchKernelGGL((dense_gemm_nt_kernel<T, 2, 2, true>), grid, dim3(256), 0, (hipStream_t)stream,

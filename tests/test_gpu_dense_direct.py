@@ -1,4 +1,4 @@
-"""16-bit products of at most 32 rows (dense_direct.h): the first and last rows of each form and one beyond; column counts on
+"""16-bit products, of at most 32 rows (dense_direct.h) and of more: the first and last rows of each form and one beyond; column counts on
 either side of each tile rule, with strips that do not fill a block; k-blocks that do not fill a turn or a split."""
 import pytest
 import torch
@@ -43,6 +43,32 @@ def test_products(M, N, K, dtype):
         assert ((rows.double() - want).abs() <= tol).all() and (M > 16 or torch.equal(rows, out))
         assert ((ops.dense_gemm_nt(x, w, b).double() - want).abs() <= tol).all()
         assert M > 16 or torch.equal(ops.dense_gemm_nt(x, w, b), ops.dense_gemm_packed(x, packed, b))
+
+
+@pytest.mark.parametrize("kblocks", [1, 2, 3, 4, 5, 7, 8, 9, 11])
+@pytest.mark.parametrize("M,N", [(33, 80), (64, 24448), (64, 24464), (65, 12176), (130, 8208)])
+def test_staged_products(M, N, kblocks):
+    """The staged kernel: rounds of two and of four k-blocks that are whole, short and ragged, one and two strips a wave on
+    either side of the rule, column counts and row lengths that sixteen-byte stores cannot take, the last strip of a block."""
+    from sglang_security_amd import ops
+
+    K, dtype = 128 * kblocks, torch.bfloat16
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x, w = (torch.randn(r, K, generator=g, device=DEV).to(dtype) for r in (M, N))
+    bias = torch.randn(N, generator=g, device=DEV).to(dtype)
+    want = x.double() @ w.double().t() + bias.double()
+    tol = want.abs() * 2.0 ** -8 + (x.double().abs() @ w.double().abs().t()) * 2.0 ** -20
+    packed = torch.full((M + 1, N + 8), 7.0, dtype=dtype, device=DEV)
+    ops.dense_gemm_packed(x, ops.dense_repack(w), bias, packed[:M, :N])
+    assert ((packed[:M, :N].double() - want).abs() <= tol).all()
+    assert (packed[M:] == 7).all() and (packed[:, N:] == 7).all()
+    rows = torch.full((M + 1, N + 5), 7.0, dtype=dtype, device=DEV)     # single elements
+    ops.dense_gemm_nt(x, w, bias, rows[:M, :N])
+    assert torch.equal(rows[:M, :N], packed[:M, :N]) and (rows[M:] == 7).all() and (rows[:, N:] == 7).all()
+    n = N - 3                                                           # the last piece is not whole
+    some = torch.full((M, N), 7.0, dtype=dtype, device=DEV)
+    ops.dense_gemm_nt(x, w[:n], bias[:n], some[:, :n])
+    assert torch.equal(some[:, :n], packed[:M, :n]) and (some[:, n:] == 7).all()
 
 
 @pytest.mark.parametrize("M", [1, 16])
