@@ -102,11 +102,11 @@ __global__ __launch_bounds__(256) void per_token_quant_kernel(const void* __rest
 
 // Rows of up to 16384 elements: a thread holds its NV vectors between the maximum and the codes, all requested at once (the loop
 // above reads a row twice, a trip to memory per vector).  Three launches of 4096 elements and one of 14336: 2048 rows 53.1 -> 49.6 us,
-// 64 rows 16.9 -> 15.2.
-template <typename T, int NV>
-__global__ __launch_bounds__(256) void per_token_quant_held_kernel(const void* __restrict__ x, uint8_t* __restrict__ q,
-                                                                   float* __restrict__ scales, int hidden) {
-  __shared__ float red[4];
+// 64 rows 16.9 -> 15.2.  BT threads: the wide blocks are for few rows, where a row is a chain and not a share of the chip.
+template <typename T, int BT, int NV>
+__global__ __launch_bounds__(BT) void per_token_quant_held_kernel(const void* __restrict__ x, uint8_t* __restrict__ q,
+                                                                  float* __restrict__ scales, int hidden) {
+  __shared__ float red[BT / 64];
   const int64_t row = blockIdx.x;
   const int64_t base = row * hidden;
   float v[NV][8];
@@ -115,20 +115,24 @@ __global__ __launch_bounds__(256) void per_token_quant_held_kernel(const void* _
   for (int k = 0; k < NV; ++k) {
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[k][j] = 0.f;
-    const int i = (threadIdx.x + 256 * k) * 8;
+    const int i = (threadIdx.x + BT * k) * 8;
     if (i < hidden) load8<T>(x, base + i, v[k]);
   }
 #pragma unroll
   for (int k = 0; k < NV; ++k)
 #pragma unroll
     for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[k][j]));
-  amax = block_max_256(amax, red);
+  amax = wave_max(amax);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < BT / 64; ++w) amax = fmaxf(amax, red[w]);
   const float scale = amax / kFp8Max;
   if (threadIdx.x == 0) scales[row] = scale;
   const float inv = 1.0f / scale;
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
-    const int i = (threadIdx.x + 256 * k) * 8;
+    const int i = (threadIdx.x + BT * k) * 8;
     if (i >= hidden) break;
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[k][j] = clamp_sym(v[k][j] * inv, -kFp8Max, kFp8Max);
@@ -999,16 +1003,25 @@ int sglk_per_token_quant_fp8(const void* x, void* q, float* scales, int64_t rows
   if (rows == 0) return SGLK_OK;
   const bool vec = hidden % 8 == 0 && aligned16(x) && ((uintptr_t)q & 7) == 0;
   hipStream_t s = (hipStream_t)stream;
-#define SGLK_HELD(NV) hipLaunchKernelGGL((per_token_quant_held_kernel<T, NV>), dim3((unsigned)rows), dim3(256), 0, s, x, (uint8_t*)q, scales, hidden)
+  // up to two rows a CU a block is as wide as the row (64 rows: 14336 elements 4.7 us -> 4.0, the quantisers of a layer 18.0 -> 16.2)
+  const bool few = rows <= 512;
+#define SGLK_HELD(BT, NV) \
+  hipLaunchKernelGGL((per_token_quant_held_kernel<T, BT, NV>), dim3((unsigned)rows), dim3(BT), 0, s, x, (uint8_t*)q, scales, hidden)
   SGLK_DISPATCH_FLOAT(dtype, T, {
     if (vec && hidden <= 2048)
-      SGLK_HELD(1);
+      SGLK_HELD(256, 1);
+    else if (vec && few && hidden <= 4096)
+      SGLK_HELD(512, 1);
+    else if (vec && few && hidden <= 8192)
+      SGLK_HELD(1024, 1);
+    else if (vec && few && hidden <= 16384)
+      SGLK_HELD(1024, 2);
     else if (vec && hidden <= 4096)
-      SGLK_HELD(2);
+      SGLK_HELD(256, 2);
     else if (vec && hidden <= 8192)
-      SGLK_HELD(4);
+      SGLK_HELD(256, 4);
     else if (vec && hidden <= 16384)
-      SGLK_HELD(8);
+      SGLK_HELD(256, 8);
     else if (vec)
       hipLaunchKernelGGL((per_token_quant_kernel<T, true>), dim3((unsigned)rows), dim3(256), 0, s, x, (uint8_t*)q, scales,
                          hidden);

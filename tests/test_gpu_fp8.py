@@ -68,6 +68,21 @@ def test_per_token_quant_held_rows(hidden, dtype):
     assert torch.equal(_u8(q), wq.view(torch.uint8))
 
 
+@pytest.mark.parametrize("hidden", [2056, 4096, 4104, 8192, 8200, 16384])
+@pytest.mark.parametrize("rows", [512, 513])
+def test_per_token_quant_of_few_and_many_rows(rows, hidden):
+    """512 rows have a block as wide as the row, 513 have 256 threads each: the same bytes and scales."""
+    import oracle
+
+    g = torch.Generator(device=DEV).manual_seed(hidden)
+    x = (torch.randn(rows, hidden, generator=g, device=DEV) * 3).bfloat16()
+    x[rows // 2, hidden - 1] = 1000.0
+    q, s = torch.empty(rows, hidden, dtype=F8, device=DEV), torch.empty(rows, 1, device=DEV)
+    _ops().per_token_quant_fp8(x, q, s)
+    wq, ws = oracle.per_token_quant_fp8(x.cpu())
+    assert torch.equal(s.cpu(), ws) and torch.equal(_u8(q), wq.view(torch.uint8))
+
+
 def test_per_token_quant_golden(golden):
     """Fixture minted from the reference formula (sgl-kernel/tests/test_per_token_quant_fp8.py:15-27)."""
     ops = _ops()
