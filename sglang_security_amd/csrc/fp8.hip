@@ -702,7 +702,7 @@ enum class Fp8Other { kRegister, kSplit, kStreaming };  // what a call falls bac
 //   Narrow ones that stay: 1024 x 128 x 14336 split 18.9, streaming 15.8, tiled 30.9; 512 x 256 x 7168 13.8, 11.8, 17.4.
 static int fp8_tile_choice(int64_t M, int64_t N, int64_t K, Fp8Other other) {
   if (M <= 0 || K % 128 != 0 || N % 16 != 0 || getenv("SGLK_FP8_SPLITS") || getenv("SGLK_FP8_WAVES")) return 0;
-  // up to 64 rows the streaming kernel, which leaves the weights out of the caches, is the faster one in a layer's
+  // up to 64 rows the kernels on the streaming layout, which leave the weights out of the caches, are the faster ones in a layer's
   // sequence of products (28672 x 4096 tiled: a pass of four products 106 us against 100); up to 32 the register
   // kernel's smaller tiles keep up with the memory
   if (M <= (other == Fp8Other::kStreaming ? 64 : 32)) return 0;
@@ -748,7 +748,8 @@ int launch_fp8_tiled(int form, const MmArgs& p, hipStream_t s) {
 }
 
 
-// ---- streaming form of the per-token / per-channel scaled product at decode batch sizes --------------------------
+// ---- streaming form of the scaled products: block scales, and per-token / per-channel ones of more than 64 rows (fp8_direct.h
+// takes the others, on the same layout) ----
 // out[M, N] = (x[M, K] . W[N, K]^T) * sa[m] * sb[n] (+ bias) with the weight re-laid-out once at load time
 // (sglk_fp8_repack) so that every wave instruction reads 1 KiB of consecutive memory:
 //   packed = [N / 16 strips][K / 128 k-blocks][2 halves][64 lanes][16 bytes],
