@@ -192,22 +192,20 @@ struct KvElem<Fp8<F>> {
   }
 
 // ---- split-K partial sums handed to a consumer kernel -------------------------------------------
-// acc[0..7] = sum over splits (in split order) of the 8 floats at partials[s][off .. off+7]; up to eight splits'
-// loads are in flight together
-__device__ __forceinline__ void sum_partials(const float* __restrict__ partials, int splits, int64_t part_stride,
-                                             int64_t off, float (&acc)[8]) {
+// acc[0..7] += the 8 floats at partials[s][off .. off+7] of all splits, in split order; N splits' loads are in flight together
+template <int N>
+__device__ __forceinline__ void add_partials(const float* __restrict__ partials, int splits, int64_t part_stride, int64_t off,
+                                             float (&acc)[8]) {
+  for (int s0 = 0; s0 < splits; s0 += N) {
+    float4v a[N], b[N];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) acc[j] = 0.f;
-  for (int s0 = 0; s0 < splits; s0 += 8) {
-    float4v a[8], b[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < N; ++u) {
       const float* pr = partials + (int64_t)min(s0 + u, splits - 1) * part_stride + off;
       a[u] = *reinterpret_cast<const float4v*>(pr);
       b[u] = *reinterpret_cast<const float4v*>(pr + 4);
     }
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < N; ++u) {
       if (s0 + u < splits) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -217,6 +215,20 @@ __device__ __forceinline__ void sum_partials(const float* __restrict__ partials,
       }
     }
   }
+}
+// acc[0..7] = that sum.  FEW, for kernels of few rows, whose launch is a chain: about as many requests as there are splits (one
+// past the last split repeats it; products that fill the chip with one to four splits would pay for eight).  In kernels
+// of many rows the further form costs more than the requests (16 requests of 64 tokens and 8 steps through the engine: 4701 us with
+// eight requests everywhere, 4657 so; its prompts 0.4% slower with both forms in every kernel).
+template <bool FEW = false>
+__device__ __forceinline__ void sum_partials(const float* __restrict__ partials, int splits, int64_t part_stride,
+                                             int64_t off, float (&acc)[8]) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) acc[j] = 0.f;
+  if (FEW && splits <= 4)
+    add_partials<4>(partials, splits, part_stride, off, acc);
+  else
+    add_partials<8>(partials, splits, part_stride, off, acc);
 }
 
 // value an fp8 product's split sum stores: raw sum * scale of the activation row * scale of the weight column + bias,

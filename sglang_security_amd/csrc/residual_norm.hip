@@ -82,7 +82,7 @@ __global__ void __launch_bounds__(BT) residual_norm_kernel(ResidualNorm a) {
       ld8<float>(a.x, (int64_t)row * a.pitch + 8 * v, x[i]);
     }
     if (a.src.p) {
-      source8<T>(a.src, row, 8 * v, s[i]);
+      source8<T, PRE>(a.src, row, 8 * v, s[i]);
 #pragma unroll
       for (int j = 0; j < 8; ++j) ss += s[i][j] * s[i][j];
     }
@@ -163,7 +163,7 @@ __global__ void __launch_bounds__(256) source_act_kernel(RowSource src, const fl
 }
 
 // out[m][n] = act(src[m][n]) * src[m][N + n]: gate columns, then as many others
-template <typename T>
+template <typename T, bool FEW>
 __global__ void __launch_bounds__(256) source_gated_act_kernel(RowSource src, void* __restrict__ out, int M, int N,
                                                                int64_t out_stride, int act) {
   const int nv = N / 8;
@@ -171,8 +171,8 @@ __global__ void __launch_bounds__(256) source_gated_act_kernel(RowSource src, vo
   if (idx >= (int64_t)M * nv) return;
   const int m = (int)(idx / nv), n = (int)(idx - (int64_t)m * nv) * 8;
   float v[8], w[8];
-  source8<T>(src, m, n, v);
-  source8<T>(src, m, N + n, w);
+  source8<T, FEW>(src, m, n, v);
+  source8<T, FEW>(src, m, N + n, w);
 #pragma unroll
   for (int j = 0; j < 8; ++j)
     v[j] = w[j] * (sizeof(typename Raw<T>::type) == 2 && act == 3 ? silu_fast(v[j]) : activate(v[j], act));
@@ -285,10 +285,16 @@ int sglk_source_gated_act(const void* src, int src_f32, int splits, int64_t part
   SGLK_CHECK(src && out && aligned16(out), "source_gated_act: null or unaligned pointer");
   if (int rc = check_source(src, src_f32, splits, part_stride, src_stride, 2 * N, dtype, "source_gated_act")) return rc;
   const int64_t vecs = (int64_t)M * (N / 8);
-  SGLK_DISPATCH_FLOAT(dtype, T,
-                      hipLaunchKernelGGL((source_gated_act_kernel<T>), dim3((unsigned)((vecs + 255) / 256)), dim3(256), 0,
-                                         (hipStream_t)stream, RowSource{src, src_f32, splits, part_stride, src_stride}, out, M,
-                                         N, out_stride, act));
+#define SGLK_GA(F)                                                                                                        \
+  hipLaunchKernelGGL((source_gated_act_kernel<T, F>), dim3((unsigned)((vecs + 255) / 256)), dim3(256), 0, (hipStream_t)stream, \
+                     RowSource{src, src_f32, splits, part_stride, src_stride}, out, M, N, out_stride, act)
+  SGLK_DISPATCH_FLOAT(dtype, T, {
+    if (src_f32 && splits <= 4)
+      SGLK_GA(true);
+    else
+      SGLK_GA(false);
+  });
+#undef SGLK_GA
   SGLK_LAUNCH_CHECK();
   return SGLK_OK;
 }

@@ -50,10 +50,10 @@ struct RowSource {
   int64_t stride;       // elements from one row to the next
 };
 
-template <typename T>
+template <typename T, bool FEW = false>
 __device__ __forceinline__ void source8(const RowSource& s, int64_t row, int col, float (&v)[8]) {
   if (s.f32)
-    sum_partials(reinterpret_cast<const float*>(s.p), s.splits, s.part_stride, row * s.stride + col, v);
+    sum_partials<FEW>(reinterpret_cast<const float*>(s.p), s.splits, s.part_stride, row * s.stride + col, v);
   else
     ld8<T>(s.p, row * s.stride + col, v);
 }

@@ -58,7 +58,7 @@ __global__ void __launch_bounds__(BT) tied_prep_kernel(TiedPrep a) {
     const int v = threadIdx.x + BT * i;
     if (v >= nv) continue;
     float b[8];
-    source8<T>(a.src, m, 8 * v, x[i]);
+    source8<T, BT == 768>(a.src, m, 8 * v, x[i]);
     ld8<float>(a.bias, 8 * v, b);
     if (v < vq) ld8<float>(a.wq, 8 * v, w[i]);
     float ss = 0.f;
