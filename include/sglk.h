@@ -525,7 +525,8 @@ SGLK_API int sglk_awq_gemm_silu_mul(const void* x, const int32_t* packed, const 
  * kind SGLK_CHAIN_SILU_MUL: what sglk_awq_gemm_silu_mul does (out, out_stride, xsum_out, xs_out_stride).
  * Every job takes the block sums of its x from its producer (xsum_in, xs_stride >= M).  M <= 64; at most 8 jobs;
  * shapes as the two entry points require; every job's column tiles x splits must fit the device's CUs.
- * Same bits as the separate launches.  A job may read what an EARLIER job of the chain wrote only if no job before
+ * Same bits as the separate launches, which up to 16 rows take its place: such a batch's products leave no such start
+ * and end to share.  A job may read what an EARLIER job of the chain wrote only if no job before
  * that writer read the same addresses (the L2s of the XCDs are not coherent inside a launch): distinct buffers per
  * hand-over.  sync: sglk_awq_chain_sync_bytes() bytes of device memory, ZERO before the first launch that uses it
  * (every launch leaves it zero); one chain at a time per sync buffer.  A block that waits two seconds for its

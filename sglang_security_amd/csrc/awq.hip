@@ -660,7 +660,7 @@ struct ZpOnMatrixCores<bf16_t> {
 // row-major to partial[split][M][N] and returns; the consumer kernel adds the splits up.
 // MT: 32-row tiles of the 64-row block that are multiplied (batches of up to 32 rows skip the matrix work of the
 // rows they do not have; staging, reduction and stores keep the 64-row shape, the skipped tile is zeros).  Batches of at
-// most 16 rows come here only in a chain; alone they run on awq_rows16.h.
+// most 16 rows run on awq_rows16.h.
 //
 // One projection is a WideJob.  awq_gemm_wide_kernel runs one job, a block per (column tile, split, row block).
 // awq_chain_kernel (CHAIN) runs a list of jobs in ONE launch of persistent blocks, job j + 1 reading what job j wrote:
@@ -1806,6 +1806,19 @@ int sglk_awq_chain(const sglk_chain_job* jobs, int njobs, void* sync, int M, int
   if (grid > cu_count)
     return fail(SGLK_EUNSUP, "awq_chain: %d blocks do not fit the %d CUs of this device at once", grid, cu_count);
   hipStream_t s = (hipStream_t)stream;
+  // up to 16 rows the separate launches are awq_rows16.h's, with sums in an order of their own: the same kernels here, in turn
+  if (M <= AwqRows16::kRows) {
+    for (int i = 0; i < njobs; ++i) {
+      const WideJob& j = cj.job[i];
+      WidePlan wp{};
+      wp.stages_per_split = j.stages_per_split;
+      wp.splits = j.splits;
+      if (int rc = launch_awq_rows16(wp, j.x, j.packed, j.scales, j.qzeros, nullptr, j.out, j.partial, nullptr, M, j.N, j.K,
+                                     j.x_stride, j.out_stride, dtype, j.partial_mode, s, j.act_mode, j.xsum_out, j.xs_out_stride))
+        return rc;
+    }
+    return SGLK_OK;
+  }
 #define SGLK_CHAIN_LAUNCH(MQ)                                                                                       \
   {                                                                                                                 \
     if (int rc = ensure_lds<&awq_chain_kernel<T, MQ>>(Wide::kLds)) return rc;                                       \

@@ -1280,7 +1280,7 @@ def chain_silu_mul(x, packed, scales, qzeros, xsum, out, xsum_out=None):
 
 def awq_chain(jobs, sync):
     """Several projections in one launch of persistent blocks, each multiplying what the one before it wrote (jobs:
-    chain_partial / chain_silu_mul records, in order).  Same bits as the separate launches."""
+    chain_partial / chain_silu_mul records, in order).  Same bits as the separate launches, which it makes up to 16 rows."""
     n = len(jobs)
     arr = (_ChainJob * n)()
     M = jobs[0]["x"].shape[0]

@@ -72,3 +72,20 @@ def test_zero_scales_and_rows_that_are_not_numbers(M):
     x[M - 1, 100] = float("nan")
     ops.awq_gemm_partial(x, packed, sc, qz, part)
     assert torch.equal(part.sum(0)[: M - 1], clean[: M - 1]) and part.sum(0)[M - 1].isnan().all()
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17])
+def test_chain_gives_the_bits_of_the_separate_launches(M):
+    """gate_up (+ activation) and down as one call and as two, with the splits and the block sums of either."""
+    ops, x, gu, _ = _case(M, 1024, 3072, torch.bfloat16, interleave=True)
+    _, _, dn, _ = _case(M, 1536, 1024, torch.bfloat16)
+    xs = x.float().view(M, -1, 128).sum(2).t().contiguous()
+    act = torch.empty(2, M, 1536, dtype=torch.bfloat16, device=DEV)
+    xs_act = torch.zeros(2, 12, M, device=DEV)
+    part = torch.full((2, ops.awq_gemm_partial_splits(M, 1024, 1536), M, 1024), float("nan"), device=DEV)
+    ops.awq_gemm_silu_mul(x, *gu, act[0], xs, xs_act[0])
+    ops.awq_gemm_partial(act[0], *dn, part[0], xs_act[0])
+    sync = ops.awq_chain_sync(DEV)
+    ops.awq_chain([ops.chain_silu_mul(x, *gu, xs, act[1], xs_act[1]), ops.chain_partial(act[1], *dn, xs_act[1], part[1])], sync)
+    assert ops.awq_chain_status(sync) == 0 and int(sync.abs().sum()) == 0
+    assert torch.equal(act[0], act[1]) and torch.equal(xs_act[0], xs_act[1]) and torch.equal(part[0], part[1])
