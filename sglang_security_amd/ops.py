@@ -19,12 +19,10 @@ def _ptr(t: Optional[torch.Tensor]) -> int:
     return 0 if t is None else t.data_ptr()
 
 
-# the current stream's handle without a Stream object around it (3 us of a call's 13): what torch's own launchers use
-_raw_stream = torch._C._cuda_getCurrentRawStream
-
-
+# the current stream's handle without a Stream object around it (3 us of a call's 13): what torch's own launchers use.
+# Looked up by the call: a torch without GPU support has no such name, and this module is imported there, too.
 def _stream(t: torch.Tensor) -> int:
-    return _raw_stream(t.device.index)
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def _need_gpu(*ts):

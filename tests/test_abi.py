@@ -65,3 +65,15 @@ def test_missing_library_fails_loudly(monkeypatch):
     monkeypatch.setattr(_lib, "LIB_PATH", "/nonexistent/libsglk.so")
     with pytest.raises(ImportError, match="no CPU fallback"):
         _lib.lib()
+
+
+def test_modules_import_where_torch_knows_no_gpu():
+    """A torch without GPU support has no stream look-up; nothing below needs one before its first launch."""
+    import subprocess
+    import sys
+
+    code = ("import torch\n"
+            "if hasattr(torch._C, '_cuda_getCurrentRawStream'): del torch._C._cuda_getCurrentRawStream\n"
+            "import sglang_security_amd.ops, sglang_security_amd.mem_cache.memory_pool, sglang_security_amd.attention.backend\n"
+            "import sglang_security_amd.quantization.awq, sglang_security_amd.quantization.w8a8_fp8\n")
+    subprocess.run([sys.executable, "-c", code], cwd=ROOT, check=True, timeout=300)
