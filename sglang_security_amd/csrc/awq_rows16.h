@@ -8,6 +8,9 @@
 // each, and meet once in LDS.  x . (OFF + q) runs on 16x16x32 tiles (32-row tiles would double the matrix work for rows that are
 // not there); the sum of x that the zero point needs is the same product with a column of ones, so the block sums
 // of x are not read.
+// What is left of x . (OFF + q) - (OFF + z) . sum(x) carries the roundings of both sums, a hundredth of their size in fp16 (OFF
+// is 1024): there a group is two halves, whose sums are smaller (16 rows, 4096 x 4096: 1.22e-5 of the result whole, 9.0e-6
+// so, 1.22e-5 in the wide kernel).
 // Rows that a batch does not have repeat its last one: switching their lanes off costs more than it saves (one row, 4096 x 28672:
 // 15.9 against 15.3 us, two halves of a block 29 against 16).  All figures here: weights from memory, us a launch.
 #pragma once
@@ -41,6 +44,7 @@ template <typename T, int S, int R, int NW>
 __global__ void __launch_bounds__(64 * NW, NW / 4) awq_rows16_kernel(const AwqRows16Args<T> a) {
   using P = AwqRows16;
   constexpr int kTurns = NW * S / 8;
+  constexpr int kParts = AwqMagic<T>::kOff == 128.f ? 1 : 2;  // of a group, each with its zero point taken off by itself
   extern __shared__ __attribute__((aligned(16))) float red[];
   __shared__ int last_block;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -84,24 +88,32 @@ __global__ void __launch_bounds__(64 * NW, NW / 4) awq_rows16_kernel(const AwqRo
     int sz[S / 4];
 #pragma unroll
     for (int c = 0; c < S / 4; ++c) sz[c] = (int)((s[slot][c] << 16) | ((z[slot][c] >> zsh) & 0xF));
-    float4v X = float4v{0.f, 0.f, 0.f, 0.f};
+    float4v X[kParts];
 #pragma unroll
-    for (int d = 0; d < 4; ++d) X = AwqMagic<T>::mma(xf[slot][d], ones, X);
+    for (int h = 0; h < kParts; ++h) X[h] = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < 4; ++d) X[d * kParts / 4] = AwqMagic<T>::mma(xf[slot][d], ones, X[d * kParts / 4]);
 #pragma unroll
     for (int t = 0; t < S; ++t) {
       const uint32_t v = (uint32_t)__builtin_amdgcn_ds_bpermute((16 * (t & 3) + i16) * 4, sz[t >> 2]);
-      float4v p = float4v{0.f, 0.f, 0.f, 0.f};
+      float4v p[kParts];
+#pragma unroll
+      for (int h = 0; h < kParts; ++h) p[h] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int d = 0; d < 4; ++d) {
         const uint32_t q = (uint32_t)w[slot][t][d];
         int4v b;
 #pragma unroll
         for (int e = 0; e < 4; ++e) b[e] = (int)(((q >> (4 * e)) & 0x000F000Fu) | AwqMagic<T>::kOr);
-        p = AwqMagic<T>::mma(xf[slot][d], b, p);
+        p[d * kParts / 4] = AwqMagic<T>::mma(xf[slot][d], b, p[d * kParts / 4]);
       }
       const float sc = Conv<T>::to_f32((uint16_t)(v >> 16)), nz = -(AwqMagic<T>::kOff + (float)(v & 0xF));
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc[t][e] = fmaf(sc, fmaf(nz, X[e], p[e]), acc[t][e]);
+      for (int e = 0; e < 4; ++e) {
+        float s = fmaf(nz, X[0][e], p[0][e]);
+        if constexpr (kParts == 2) s += fmaf(nz, X[1][e], p[1][e]);
+        acc[t][e] = fmaf(sc, s, acc[t][e]);
+      }
     }
   };
   if (n > 0) {

@@ -89,3 +89,30 @@ def test_chain_gives_the_bits_of_the_separate_launches(M):
     ops.awq_chain([ops.chain_silu_mul(x, *gu, xs, act[1], xs_act[1]), ops.chain_partial(act[1], *dn, xs_act[1], part[1])], sync)
     assert ops.awq_chain_status(sync) == 0 and int(sync.abs().sum()) == 0
     assert torch.equal(act[0], act[1]) and torch.equal(xs_act[0], xs_act[1]) and torch.equal(part[0], part[1])
+
+
+@pytest.mark.parametrize("dtype,bound", [(torch.float16, 1.1e-5), (torch.bfloat16, 1.1e-6)])
+@pytest.mark.parametrize("M", [1, 16])
+def test_distance_from_64_bits(M, dtype, bound):
+    """Two sums of about (OFF + z) sqrt(n) are taken off one another, n = 64 (fp16, OFF = 1024) or 128 (bf16, 128) of x at a time,
+    each with the roundings of n / 32 steps: 3.5e-4 a half in fp16, 1e-4 a group in bf16, of a group's 74 that is 7e-6 and 1e-6
+    (no more than a product whose roundings are all of the last step's size); with some for what rounds inside an instruction.
+    Whole groups give 1.22e-5 in fp16."""
+    from sglang_security_amd import ops
+
+    K = N = 4096
+    shifts = torch.tensor([0, 4, 1, 5, 2, 6, 3, 7], device=DEV) * 4
+    nib = lambda t: ((t[..., None] >> shifts) & 15).flatten(-2).double()
+    off = of = 0.0
+    for seed in range(4):
+        g = torch.Generator(device=DEV).manual_seed(seed)
+        words = lambda rows: torch.randint(-(2 ** 31), 2 ** 31 - 1, (rows, N // 8), dtype=torch.int32, generator=g, device=DEV)
+        qw, qz = words(K), words(K // 128)
+        sc = (torch.rand(K // 128, N, generator=g, device=DEV) * 0.01 + 0.001).to(dtype)
+        x = torch.randn(M, K, generator=g, device=DEV).to(dtype)
+        part = torch.empty(ops.awq_gemm_partial_splits(M, N, K), M, N, device=DEV)
+        ops.awq_gemm_partial(x, ops.awq_repack(qw), sc, qz, part)
+        want = x.double() @ ((nib(qw) - nib(qz).repeat_interleave(128, 0)) * sc.double().repeat_interleave(128, 0))
+        off += (part.double().sum(0) - want).square().sum().item()
+        of += want.square().sum().item()
+    assert (off / of) ** 0.5 <= bound
