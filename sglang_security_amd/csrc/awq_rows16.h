@@ -8,9 +8,9 @@
 // each, and meet once in LDS.  x . (OFF + q) runs on 16x16x32 tiles (32-row tiles would double the matrix work for rows that are
 // not there); the sum of x that the zero point needs is the same product with a column of ones, so the block sums
 // of x are not read.
-// What is left of x . (OFF + q) - (OFF + z) . sum(x) carries the roundings of both sums, a hundredth of their size in fp16 (OFF
-// is 1024): there a group is two halves, whose sums are smaller (16 rows, 4096 x 4096: 1.22e-5 of the result whole, 9.0e-6
-// so, 1.22e-5 in the wide kernel).
+// x . (OFF + q) - (OFF + z) . sum(x) is in fp16 (OFF is 1024) a hundredth of either term and carries the roundings of both:
+// there a group is two halves, whose sums are smaller (16 rows, 4096 x 4096: 1.23e-5 of the result whole, 9.0e-6 so, 1.22e-5
+// in the wide kernel).
 // Rows that a batch does not have repeat its last one: switching their lanes off costs more than it saves (one row, 4096 x 28672:
 // 15.9 against 15.3 us, two halves of a block 29 against 16).  All figures here: weights from memory, us a launch.
 #pragma once
@@ -193,10 +193,20 @@ __global__ void __launch_bounds__(64 * NW, NW / 4) awq_rows16_kernel(const AwqRo
   }
   __syncthreads();
   if (!last_block) return;
+  // eight splits of a row are asked for at once, in row order: one after the other each is a trip to memory (16 rows, 14336 x 128 in
+  // 28 splits: 18.9 us -> 9.8; 8192 x 1280 in 16: 14.2 -> 8.7)
   for (int row = tid >> 7; row < M; row += NW / 2) {
+    const float* p = slab + row * 128;
     float sum = 0.f;
-    for (int q = 0; q < a.splits; ++q)
-      sum += __hip_atomic_load(&slab[(int64_t)q * (P::kRows * 128) + row * 128], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int q0 = 0; q0 < a.splits; q0 += 8) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        v[u] = __hip_atomic_load(&p[(int64_t)min(q0 + u, a.splits - 1) * (P::kRows * 128)], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (q0 + u < a.splits) sum += v[u];
+    }
     a.out[(int64_t)row * a.out_stride + col] = Conv<T>::from_f32(sum + bv);
   }
 }

@@ -116,3 +116,21 @@ def test_distance_from_64_bits(M, dtype, bound):
         off += (part.double().sum(0) - want).square().sum().item()
         of += want.square().sum().item()
     assert (off / of) ** 0.5 <= bound
+
+
+@pytest.mark.parametrize("M", [1, 9, 16])
+@pytest.mark.parametrize("K,N", [(512, 256), (4096, 128), (4608, 128), (6656, 256), (14336, 128)])
+def test_last_block_adds_every_split_in_order(M, K, N, monkeypatch):
+    """One to 28 splits of one stage each, counts that are and are no multiple of those asked for at once."""
+    ops, x, w, _ = _case(M, K, N, torch.bfloat16)
+    monkeypatch.setenv("SGLK_AWQ_WIDE", "2")
+    monkeypatch.setenv("SGLK_AWQ_WIDE_SPS", "1")
+    part = torch.full((ops.awq_gemm_partial_splits(M, N, K), M, N), float("nan"), device=DEV)
+    assert len(part) == K // 512
+    ops.awq_gemm_partial(x, *w, part)
+    want = part[0].clone()
+    for p in part[1:]:
+        want += p
+    work = torch.zeros(ops.awq_gemm_workspace_bytes(M, N, K), dtype=torch.uint8, device=DEV)
+    for _ in range(2):
+        assert torch.equal(ops.awq_gemm(x, *w, workspace=work), want.bfloat16())
