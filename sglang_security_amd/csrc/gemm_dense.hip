@@ -321,16 +321,18 @@ static int dense_splits(int M, int N, int K) {
 }
 
 // Splits of the packed product, and whether dense_direct.h takes it: up to 16 rows, to 32 while its inner dimension is
-// short of 8192 (32 rows, 14336 x 4096: 27.0 in eight splits of the staged kernel, 27.9 in two).  Outputs narrower than 512 stay
-// with the order of sums, and the bits, of the row-major product.  A direct block is 32 columns wide, or 64 where that
-// leaves 128 blocks: as many splits as whole blocks fit the units, each of 512 of k at least.
+// short of 8192 (32 rows, 14336 x 4096: 27.0 in eight splits of the staged kernel, 27.9 in two), but from 65536 columns on and below
+// 4096 only to 24 (65536 x 2560, 24 and 28 rows: 58.4 and 61.0 us, staged 59.8 and 58.5; 128256 x 4096, 32 rows 176 and 184).
+// Outputs narrower than 512 stay with the order of sums, and the bits, of the row-major product.  A direct block is 32 columns
+// wide, or 64 where that leaves more than 128 blocks: as many splits as whole blocks fit the units, each of 512 of k at least.
 struct DensePlan {
   bool direct;
   int splits, per;  // k-blocks a split
 };
 static DensePlan dense_packed_plan(int M, int N, int K) {
   const int kblocks = K / 128, strips = N / 16;
-  const bool direct = N >= 512 && (M <= 16 || (M <= 32 && K < 8192)) && !getenv("SGLK_DENSE_SPLITS") && !getenv("SGLK_DENSE_NS");
+  const bool few = M <= 16 || (M <= (N >= 65536 && K < 4096 ? 24 : 32) && K < 8192);
+  const bool direct = N >= 512 && few && !getenv("SGLK_DENSE_SPLITS") && !getenv("SGLK_DENSE_NS");
   int splits = dense_splits(M, N, K);
   if (direct) splits = strips >= 512 ? 1 : std::max(1, std::min(256 / ((strips + 1) / 2), kblocks / 4));
   const int per = (kblocks + splits - 1) / splits;
@@ -346,18 +348,21 @@ static int launch_dense_tile(const DenseDirectArgs& a, int splits, hipStream_t s
   SGLK_LAUNCH_CHECK();
   return SGLK_OK;
 }
-// the products that dense_packed_plan names
+// The products that dense_packed_plan names.  32 columns a block as long as that is one block a unit (8192 columns of 28672, 16
+// rows: 79.9 us, 99.7 with 64 columns on half of the units, 77.3 staged in eight splits; 10240 of 8192: 40.6 and 32.0).
 template <typename T, bool PACKED>
 static int launch_dense_direct(const DenseDirectArgs& a, int splits, hipStream_t s) {
-  if (a.N >= 8192) return a.M <= 16 ? launch_dense_tile<T, 1, 4, 4, PACKED>(a, splits, s) : launch_dense_tile<T, 2, 4, 4, PACKED>(a, splits, s);
+  if (a.N > 8192) return a.M <= 16 ? launch_dense_tile<T, 1, 4, 4, PACKED>(a, splits, s) : launch_dense_tile<T, 2, 4, 4, PACKED>(a, splits, s);
   return a.M <= 16 ? launch_dense_tile<T, 1, 2, 8, PACKED>(a, splits, s) : launch_dense_tile<T, 2, 2, 8, PACKED>(a, splits, s);
 }
-// Calls without a workspace, unsplit, up to 16 rows.  A strip a block and sixteen waves while x is small (four rows, 65536 x 2560:
-// 53.7 us; 64 columns and eight waves 56.7) or the output narrow; from nine rows on, for outputs that fill the units so, 64
-// columns (16 rows: 57.5 and 62; 128256 x 4096 164 and 177).
+// Calls without a workspace, unsplit, up to 16 rows.  A strip a block while x is small or the output narrow: with sixteen waves (four
+// rows, 65536 x 2560: 53.4 us; 64 columns and eight waves 56.0), with eight where that leaves waves without a k-block (151936 x
+// 896, one row and eight: 41.4 and 44.4, with sixteen 48.7 and 56.5, staged 45.2 and 45.9).  From nine rows on, for outputs that
+// fill the units so, 64 columns (16 rows: 57.5 and 62; 128256 x 4096 164 and 177).
 static bool dense_direct_whole(int M, int N) { return M <= 16 && N >= 512 && N % 16 == 0 && !getenv("SGLK_DENSE_NS"); }
 template <typename T, bool PACKED>
 static int launch_dense_whole(const DenseDirectArgs& a, hipStream_t s) {
+  if (a.M <= 8 && a.N >= 16384 && a.K < 2048) return launch_dense_tile<T, 1, 1, 8, PACKED>(a, 1, s);
   if (a.N < 8192 || (a.M <= 8 && a.N >= 16384)) return launch_dense_tile<T, 1, 1, 16, PACKED>(a, 1, s);
   return a.N < 16384 ? launch_dense_tile<T, 1, 4, 4, PACKED>(a, 1, s) : launch_dense_tile<T, 1, 4, 8, PACKED>(a, 1, s);
 }
@@ -384,7 +389,9 @@ int sglk_dense_gemm_nt_ws(const void* x, const void* w, const void* bias, void* 
   SGLK_CHECK(M > 0 && N > 0 && K > 0, "dense_gemm_nt: bad shape");
   SGLK_CHECK(K % 128 == 0, "dense_gemm_nt: K=%d must be a multiple of 128", K);
   const DensePlan plan = dense_packed_plan(M, N, K);
-  if (plan.direct && N % 16 == 0 && aligned16(x) && aligned16(w) && x_stride % 8 == 0 && w_stride % 8 == 0 &&
+  // (wide row-major weights of more than 16 rows stay staged: 32 rows, 65536 x 2560 74.0 us, direct 88.9; 128256 x 4096 219 and 249)
+  const bool direct = plan.direct && (M <= 16 || N < 65536);
+  if (direct && N % 16 == 0 && aligned16(x) && aligned16(w) && x_stride % 8 == 0 && w_stride % 8 == 0 &&
       (plan.splits == 1 || (workspace && workspace_bytes >= (int64_t)plan.splits * M * N * (int64_t)sizeof(float) &&
                             aligned16(workspace) && aligned16(out) && out_stride % 8 == 0))) {
     float* partial = plan.splits > 1 ? (float*)workspace : nullptr;
@@ -595,8 +602,6 @@ int sglk_dense_gemm_nt(const void* x, const void* w, const void* bias, void* out
   SGLK_CHECK(aligned16(x) && aligned16(w) && x_stride % 8 == 0 && w_stride % 8 == 0,
              "dense_gemm_nt: rows must be 16-byte aligned");
   const int mblocks = (M + 63) / 64;
-  // two strips per wave halve the activation re-reads; kept for wide outputs only, where the grid still
-  // fills the chip several times over
   if (dense_direct_whole(M, N)) {
     const DenseDirectArgs a{(const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, (uint16_t*)out, nullptr, M, M, N, K,
                             K / 128,            x_stride,           w_stride,              out_stride};
@@ -604,6 +609,8 @@ int sglk_dense_gemm_nt(const void* x, const void* w, const void* bias, void* out
   }
   const char* env = getenv("SGLK_DENSE_NS");  // 1 / 2 forces the strips per wave (tests)
   const int force = env ? atoi(env) : 0;
+  // two strips per wave halve the activation re-reads; kept for wide outputs only, where the grid still
+  // fills the chip several times over
   const bool two = force ? force == 2 : N >= 64 * 1024;
   if (two) {
     dim3 grid((N + 127) / 128, 1, mblocks);

@@ -45,6 +45,20 @@ def test_products(M, N, K, dtype):
         assert M > 16 or torch.equal(ops.dense_gemm_nt(x, w, b), ops.dense_gemm_packed(x, packed, b))
 
 
+@pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32])
+@pytest.mark.parametrize("N,K", [(8192, 2688), (8208, 2688), (16400, 1152), (16400, 2688), (65536 + 16, 1152)])
+def test_wide_products(M, N, K):
+    """Wide outputs with several k-blocks a wave and a last turn that is not full; the last column count of 32 a block and the
+    first of 64, inner dimensions on either side of sixteen waves."""
+    test_products(M, N, K, torch.bfloat16)
+
+
+@pytest.mark.parametrize("M", [24, 25])
+def test_widest_products_around_the_last_rows_of_the_direct_form(M):
+    test_products(M, 65536 + 16, 640, torch.bfloat16)
+    test_products(M, 65536 - 16, 640, torch.bfloat16)
+
+
 @pytest.mark.parametrize("kblocks", [1, 2, 3, 4, 5, 7, 8, 9, 11])
 @pytest.mark.parametrize("M,N", [(33, 80), (64, 24448), (64, 24464), (65, 12176), (130, 8208)])
 def test_staged_products(M, N, kblocks):
