@@ -15,6 +15,8 @@
 // everything at each k-block's barrier -> 24.3; 14336 x 4096 110 -> 76; 28672 x 4096 57 -> 45; 16384 x 2560, with one
 // strip a wave as well, 33 -> 22; 128256 x 4096, where many blocks a unit had covered those waits, 190 -> 192, 5.5 TB/s:
 // neither deeper rings, 256 columns a block nor k-blocks begun at different places changed that one).
+// A k-block that is not there is asked for all the same, so a single one (K = 128) has the shorter ring: 64 rows, 512 and 4096
+// columns, row-major 4.5 -> 3.3 and 4.9 -> 3.7 us.
 #include <algorithm>
 #include <cstdlib>
 
@@ -421,7 +423,7 @@ int sglk_dense_gemm_nt_ws(const void* x, const void* w, const void* bias, void* 
   dim3 grid((N + 63) / 64, used, mblocks);
   hipStream_t s = (hipStream_t)stream;
   SGLK_DISPATCH_HALF(dtype, T, {
-    hipLaunchKernelGGL((dense_gemm_nt_kernel<T, 1, 4>), grid, dim3(256), 0, s, (const uint16_t*)x, (const uint16_t*)w,
+    hipLaunchKernelGGL((K > 128 ? dense_gemm_nt_kernel<T, 1, 4> : dense_gemm_nt_kernel<T, 1, 2>), grid, dim3(256), 0, s, (const uint16_t*)x, (const uint16_t*)w,
                        (const uint16_t*)nullptr, (uint16_t*)nullptr, (float*)workspace, M, mblocks * 64, N, K, per,
                        x_stride, w_stride, out_stride);
     const int64_t vecs = (int64_t)M * (N / 8);
@@ -468,7 +470,7 @@ int sglk_dense_gemm_packed(const void* x, const void* packed, const void* bias, 
   } else {
     dim3 grid((N + 63) / 64, 1, mblocks);
     SGLK_DISPATCH_HALF(dtype, T,
-                       hipLaunchKernelGGL((dense_gemm_nt_kernel<T, 1, 4, true>), grid, dim3(256), 0, (hipStream_t)stream,
+                       hipLaunchKernelGGL((K > 128 ? dense_gemm_nt_kernel<T, 1, 4, true> : dense_gemm_nt_kernel<T, 1, 2, true>), grid, dim3(256), 0, (hipStream_t)stream,
                                           (const uint16_t*)x, (const uint16_t*)packed, (const uint16_t*)bias,
                                           (uint16_t*)out, (float*)nullptr, M, mblocks * 64, N, K, K / 128, x_stride,
                                           (int64_t)0, out_stride));
@@ -511,7 +513,7 @@ static int dense_packed_split_launch(const void* x, const void* packed, float* p
   } else {
     dim3 grid((N + 63) / 64, used, (M + 63) / 64);
     SGLK_DISPATCH_HALF(dtype, T,
-                       hipLaunchKernelGGL((dense_gemm_nt_kernel<T, 1, 4, true>), grid, dim3(256), 0, s, (const uint16_t*)x,
+                       hipLaunchKernelGGL((K > 128 ? dense_gemm_nt_kernel<T, 1, 4, true> : dense_gemm_nt_kernel<T, 1, 2, true>), grid, dim3(256), 0, s, (const uint16_t*)x,
                                           (const uint16_t*)packed, (const uint16_t*)nullptr, (uint16_t*)nullptr, partial,
                                           M, Mpad, N, K, per, x_stride, (int64_t)0, (int64_t)0));
   }
@@ -622,7 +624,7 @@ int sglk_dense_gemm_nt(const void* x, const void* w, const void* bias, void* out
   } else {
     dim3 grid((N + 63) / 64, 1, mblocks);
     SGLK_DISPATCH_HALF(dtype, T,
-                       hipLaunchKernelGGL((dense_gemm_nt_kernel<T, 1, 4>), grid, dim3(256), 0, (hipStream_t)stream,
+                       hipLaunchKernelGGL((K > 128 ? dense_gemm_nt_kernel<T, 1, 4> : dense_gemm_nt_kernel<T, 1, 2>), grid, dim3(256), 0, (hipStream_t)stream,
                                           (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias,
                                           (uint16_t*)out, (float*)nullptr, M, mblocks * 64, N, K, K / 128, x_stride,
                                           w_stride, out_stride));
