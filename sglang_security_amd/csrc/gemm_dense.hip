@@ -458,9 +458,10 @@ int sglk_dense_gemm_packed(const void* x, const void* packed, const void* bias, 
                             K / 128,            x_stride,                0,                     out_stride};
     SGLK_DISPATCH_HALF(dtype, T, { return launch_dense_whole<T, true>(a, (hipStream_t)stream); });
   }
-  // two strips a wave halve what is read of x; one, where 128 columns a block would leave units without a block (64 rows:
-  // 16384 x 2560 28.0 us and 21.5, 28672 x 4096 44.6 and 54.3)
-  if ((N + 127) / 128 * mblocks >= 192) {
+  // two strips a wave halve what is read of x; one as long as 64 columns a block leave no unit a second block (one strip and two,
+  // 64 rows: 16384 x 2560 20.5 us and 25.0, 18432 x 2560 34.6 and 28.8, 28672 x 4096 56.6 and 45.4; 128 rows: 8192 x 2560 17.6 and
+  // 21.8, 8320 x 4096 46.6 and 35.7, 13824 x 2560 33.9 and 28.7; 192 rows: 6144 x 4096 41.6 and 30.9; 320: 28672 x 4096 240 and 206)
+  if ((N + 127) / 128 * mblocks > 128) {
     dim3 grid((N + 127) / 128, 1, mblocks);
     SGLK_DISPATCH_HALF(dtype, T,
                        hipLaunchKernelGGL((dense_gemm_nt_kernel<T, 2, 2, true>), grid, dim3(256), 0, (hipStream_t)stream,

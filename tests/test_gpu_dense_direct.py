@@ -60,7 +60,7 @@ def test_widest_products_around_the_last_rows_of_the_direct_form(M):
 
 
 @pytest.mark.parametrize("kblocks", [1, 2, 3, 4, 5, 7, 8, 9, 11])
-@pytest.mark.parametrize("M,N", [(33, 80), (64, 24448), (64, 24464), (65, 12176), (130, 8208)])
+@pytest.mark.parametrize("M,N", [(33, 80), (64, 16384), (64, 16400), (65, 8192), (65, 8208), (64, 24448), (64, 24464), (65, 12176), (130, 8208)])
 def test_staged_products(M, N, kblocks):
     """The staged kernel: rounds of two and of four k-blocks that are whole, short and ragged, one and two strips a wave on
     either side of the rule, column counts and row lengths that sixteen-byte stores cannot take, the last strip of a block."""
