@@ -582,11 +582,11 @@ __global__ void __launch_bounds__(256) act_and_mul_xs_kernel(void* __restrict__ 
 }
 
 // Greedy token: index of the first maximum of every row (torch.argmax, sampler.py greedy path), one block per row.  A 16-bit
-// row is read eight elements a load, U loads of a thread in flight: a large vocabulary's row is one trip to memory.  What
+// row is read eight elements a load, U loads of a thread in flight: a large vocabulary's row is two trips to memory.  What
 // is left are vector instructions, so a load's maximum comes from v_maximum3 (which keeps a NaN), is compared with the
 // thread's own once, and the load that held it is kept; the place inside it is looked for at the end.  A row that holds a
 // NaN (it wins, as in torch) is read again for the first one.
-// One row of 128256 bf16 elements: 12.8 us with a comparison an element -> 6.1; 64 rows 14.5 -> 7.2; one fp32 row 23.5 -> 9.3.
+// One row of 128256 bf16 elements: 12.8 us with a comparison an element -> 6.1; 64 rows 14.5 -> 6.9; one fp32 row 23.5 -> 9.3.
 __device__ __forceinline__ float maximum3(float a, float b, float c) {  // (builtins are regrouped into two-operand forms)
   float r;
   asm("v_maximum3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
@@ -1040,17 +1040,20 @@ int sglk_argmax(const void* x, int64_t* out, int64_t rows, int cols, int64_t row
   SGLK_CHECK(rows >= 0 && cols > 0 && row_stride >= cols, "argmax: bad shape");
   if (rows == 0) return SGLK_OK;
   SGLK_CHECK(x && out, "argmax: null pointer");
-  // as many loads in flight as the row needs: one that a short row has no use for reads its last piece again
+  // Loads in flight: as many as a short row has, and rounds that a longer one fills (us, four and eight in flight: one row of
+  // 32000 4.1 and 4.6, 128256 6.0 and 6.1, 151936 6.7 and 7.3; 1024 rows of 65536 23.3 and 22.2, of 128256 47.0 and 46.6, of
+  // 262144 96.9 and 109).  Sixteen are no better anywhere (one row of 128256 6.2, of 151936 9.4; 1024 of 262144 116.7).
 #define SGLK_AM(U) \
   hipLaunchKernelGGL((argmax_rows_kernel<T, U>), dim3((unsigned)rows), dim3(1024), 0, (hipStream_t)stream, x, out, cols, row_stride)
   SGLK_DISPATCH_FLOAT(dtype, T, {
-    constexpr int kMost = sizeof(typename Raw<T>::type) == 2 ? 16 : 2;  // (fp32 rows are read one by one)
-    if (cols > 8 * 8 * 1024)
-      SGLK_AM(kMost);
-    else if (cols > 8 * 2 * 1024)
-      SGLK_AM(std::min(kMost, 8));
-    else
+    constexpr bool kTwo = sizeof(typename Raw<T>::type) == 4;  // (fp32 rows are read one by one)
+    const int rounds = (cols + 8 * 1024 - 1) / (8 * 1024);
+    if (kTwo || rounds <= 2)
       SGLK_AM(2);
+    else if (rounds <= 4 || rounds > 16)
+      SGLK_AM(kTwo ? 2 : 4);
+    else
+      SGLK_AM(kTwo ? 2 : 8);
   });
 #undef SGLK_AM
   SGLK_LAUNCH_CHECK();

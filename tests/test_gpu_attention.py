@@ -154,9 +154,9 @@ def test_argmax_rows_special_values(dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("cols", [7, 16384, 16392, 65536, 65541, 131072, 131080, 270000])
+@pytest.mark.parametrize("cols", [7, 16384, 16392, 32768, 32776, 65536, 65541, 131072, 131080, 270000])
 def test_argmax_rows_of_every_length_class(dtype, cols):
-    """Rows of two, eight and sixteen loads a thread, with and without a second round and a remainder: the maximum at the
+    """Rows of two, four and eight loads a thread, with and without a second round and a remainder: the maximum at the
     first and the last element, at the seams of the loads, twice in one load, and one NaN behind a larger infinity."""
     ops = _ops()
     g = torch.Generator().manual_seed(cols)
