@@ -237,8 +237,11 @@ int sglk_residual_norm(float* x, const void* embed, const int32_t* ids, int64_t 
                  add_x0, step, w_next, h, h_stride, rows, store_x, width, pitch, eps};
   const int vecs = pitch / 8;
   // up to two rows a CU, every piece is on a thread of its own; more of them fill the chip at any block size, and there
-  // the registers that PRE holds cost more than its earlier requests give (7921 rows of 2560: 47 us -> 54)
-  const bool few = M <= 512;
+  // the registers that PRE holds cost more than its earlier requests give (7921 rows of 2560: 47 us -> 54).  Blocks of 1024
+  // threads with many split sums a row are at that point from a second row a CU on (256 threads and 1024, eight splits: 256 rows of
+  // 8192 18.4 us and 16.4, 400 rows 23.9 and 25.3, 512 rows 29.1 and 30.9; of 5120 16.8 and 17.5, 20.0 and 20.7; one split, 512
+  // rows of 5120 10.1 and 8.9)
+  const bool few = M <= 256 || (M <= 512 && (vecs <= 512 || !src_f32 || splits <= 2));
 #define SGLK_RN(BT, V, P) hipLaunchKernelGGL((residual_norm_kernel<T, BT, V, P>), dim3(M), dim3(BT), 0, (hipStream_t)stream, a)
   SGLK_DISPATCH_FLOAT(dtype, T, {
     if (few && vecs <= 256)

@@ -97,6 +97,24 @@ def test_residual_norm_of_few_and_many_rows(pitch, dtype):
         close(h, O.rms_norm(want, wn.double(), eps), 2 * TOL[dtype], "h")
 
 
+@pytest.mark.parametrize("splits", [2, 3, 8])
+def test_residual_norm_of_wide_rows_and_many_splits(splits):
+    """From 257 rows on, wide rows of more than two split sums take 256 threads a row."""
+    from sglang_security_amd import ops_hybrid as H
+
+    pitch, eps = 4104, 1e-5
+    g = gen(splits)
+    d = lambda t: t.clone().to(DEV)
+    x, s, wp, wn = rnd(g, 257, pitch), rnd(g, 257, pitch), rnd(g, pitch), rnd(g, pitch)
+    for rows in (256, 257):
+        src, sv = source(s[:rows], splits, BF16)
+        xd, h = d(x[:rows]), torch.empty(rows, pitch, dtype=BF16, device=DEV)
+        H.residual_norm(xd, pitch, eps, h, d(wn), src, d(wp), dtype=BF16)
+        want = x[:rows].double() + O.rms_norm(sv, wp.double(), eps)
+        close(xd, want, 2e-6, "x")
+        close(h, O.rms_norm(want, wn.double(), eps), 2 * TOL[BF16], "h")
+
+
 @pytest.mark.parametrize("dtype,splits", [(BF16, 0), (BF16, 5), (F32, 1)])
 def test_activations_and_capped_logits(dtype, splits):
     from sglang_security_amd import ops_hybrid as H
