@@ -196,3 +196,50 @@ def test_spread_rows_with_all_filters(B, n):
                 cum = kept.cumsum(0) / kept.sum()
                 for i in ids[b::6].tolist():
                     assert kept[i] > 0 and cum[i] >= u - 1e-5 and (i == 0 or cum[i - 1] <= u + 1e-5)
+
+
+@pytest.mark.parametrize("aligned", [True, False])
+def test_spread_rows_of_special_values(aligned, monkeypatch):
+    """Rows that are not all finite and positive, beside one that is, spread over several blocks and done by one block each."""
+    import sglang_security_amd.sgl_kernel as sk
+    from sglang_security_amd import ops
+
+    n, inf, nan = 40003, float("inf"), float("nan")
+    g = torch.Generator().manual_seed(5)
+    x = _rows("peaked", n, g)
+    x = x * 2.0 ** -math.ceil(math.log2(x.sum().item()))
+    rows = x.float().repeat(10, 1)
+    rows[1, ::3] = nan
+    rows[2, ::3] = -rows[2, ::3]
+    rows[3] = 0.0
+    rows[4], rows[4, 31007] = 0.0, 1.0
+    rows[5, 7] = inf
+    rows[6, 39999:] = inf                       # several of infinite mass, in the last slice
+    rows[7, ::2] = -0.0
+    rows[8] = nan
+    rows[8, 20001], rows[8, 20002] = 0.75, -inf
+    rows[9] = rows[9] * 2.0 ** -130             # no mass to speak of: values down to the smallest there are
+    B = len(rows)
+    wide = torch.full((B, n + 5), nan, device=DEV)
+    at = 0 if aligned else 1
+    if aligned:
+        wide = torch.full((B, (n + 3) // 4 * 4), nan, device=DEV)
+    wide[:, at: at + n] = rows.to(DEV)
+    rows = wide[:, at: at + n]
+    kt = torch.tensor([50, 0, 1000, 7, 2, n, 300, 1, 10, 40], dtype=torch.int32, device=DEV)
+    pt = torch.tensor([0.75, 0.875, 1.0, 0.5, 0.875, 0.875, 1.0, 0.9, 0.5, 0.75], device=DEV)
+    mt = torch.tensor([0.0, 0.25, 0.0, 0.125, 0.0, 0.5, 0.0, 0.0, 0.25, 0.0], device=DEV)
+    assert ops._filter_workspace(rows)[1] > 0
+
+    def everything():
+        got = []
+        for u in (0.0, 0.4, 0.999):
+            u = torch.full((B,), u, device=DEV)
+            for kw in (dict(top_k=kt, top_p=pt, min_p=mt), dict(top_k=kt, top_p=pt), dict(top_k=30), dict(top_p=0.75), dict(min_p=0.25)):
+                got.append(ops.sampling_from_probs(rows, u, **kw))
+        return got + [sk.top_k_renorm_probs(rows, kt), sk.top_p_renorm_probs(rows, pt), sk.top_k_renorm_probs(rows, 30)]
+
+    spread = everything()
+    monkeypatch.setattr(ops, "_filter_workspace", lambda *a, **k: (None, 0))
+    for got, want in zip(spread, everything()):
+        torch.testing.assert_close(got, want, rtol=1e-6 if got.is_floating_point() else 0, atol=0, equal_nan=True)
