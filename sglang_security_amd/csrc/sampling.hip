@@ -834,7 +834,8 @@ __device__ __forceinline__ u64 word_sum(u64 w, int digit) {  // in units of 2^(m
   return (w >> kCountAt) * (u64)((digit >> 4 ? 0x800000u : 0u) | ((uint32_t)(digit & 15) << 19)) + (w & ((1ull << kCountAt) - 1));
 }
 
-template <bool VEC>
+// Draws without a top-k or top-p (FILTER: the call may have one) need no bins, and this launch only for a min-p's largest value.
+template <bool VEC, bool FILTER>
 __global__ void __launch_bounds__(kSampThreads) slice_bins_kernel(SampArgs a) {
   __shared__ u64 bins[kWindow];
   __shared__ float red[3][16];
@@ -848,12 +849,13 @@ __global__ void __launch_bounds__(kSampThreads) slice_bins_kernel(SampArgs a) {
   bins[threadIdx.x] = 0;
   __syncthreads();
   float s = 0.f, mx = 0.f;
-  const float least = g.use_k || g.use_p ? g.least : __uint_as_float(0x7FC00000u);  // without a filter nothing is binned
+  const bool bin = FILTER && (g.use_k || g.use_p);
+  const float least = bin ? g.least : __uint_as_float(0x7FC00000u);  // without a filter nothing is binned
   each_piece<VEC>(x, n, held, [&](const float4v& piece, int, int have) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const float raw = e < have ? piece[e] : -1.f, v = fmaxf(raw, 0.f);
-      const bool in = raw >= least;
+      const bool in = FILTER && raw >= least;
       mx = fmaxf(mx, v);
       s += in ? 0.f : v;
       if (in) {
@@ -869,7 +871,7 @@ __global__ void __launch_bounds__(kSampThreads) slice_bins_kernel(SampArgs a) {
   s = wave_sum(s), o = wave_sum(o), mx = wave_max(mx);
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   if (lane == 0) red[0][wid] = s, red[1][wid] = o, red[2][wid] = mx;
-  if (g.use_k || g.use_p) w.bins[slice * kWindow + threadIdx.x] = word;
+  if (bin) w.bins[slice * kWindow + threadIdx.x] = word;
   __syncthreads();
   if (threadIdx.x == 0) {
     SliceStat st{0.f, 0.f, 0.f, 0.f};
@@ -881,7 +883,7 @@ __global__ void __launch_bounds__(kSampThreads) slice_bins_kernel(SampArgs a) {
 
 // SUM (sampling): also the masses of the chunks, of what is kept whatever the cut inside its bin turns out to be; the
 // bin's own elements are listed with their places and added by the last launch.
-template <bool VEC, bool SUM>
+template <bool VEC, bool SUM, bool FILTER>
 __global__ void __launch_bounds__(kSampThreads) slice_collect_kernel(SampArgs a) {
   __shared__ u64 bins[kWindow];
   __shared__ u64 ured[16];
@@ -893,7 +895,7 @@ __global__ void __launch_bounds__(kSampThreads) slice_collect_kernel(SampArgs a)
   const RowParams rp = load_params(a, row);
   const SampWs w = samp_ws(a, row);
   const Guess g = guess_of(rp, a.n);
-  const bool bin = g.use_k || g.use_p;
+  const bool bin = FILTER && (g.use_k || g.use_p);
   // what the slices left (a lane a slice for the sums), then the slice itself: it arrives while the cuts are found
   const int lane = threadIdx.x & 63;
   float4v stat, held[kHeld];
@@ -912,7 +914,10 @@ __global__ void __launch_bounds__(kSampThreads) slice_collect_kernel(SampArgs a)
       ahead += t < slice ? (uint32_t)(part[t] >> kCountAt) : 0;
     }
   };
-  if (a.slices <= 4)
+  if constexpr (!FILTER) {
+    stat = *reinterpret_cast<const float4v*>(w.stat + min(lane, a.slices - 1));  // (not written without a min-p)
+    hold<VEC>(x, n, held);
+  } else if (a.slices <= 4)
     ask(std::integral_constant<int, 4>());
   else
     ask(std::integral_constant<int, kMaxSlices>());
@@ -1137,7 +1142,7 @@ __global__ void __launch_bounds__(kSampThreads) slice_apply_kernel(SampArgs a) {
 }
 
 // A block a row: the choice where it is sampled from, and the rows that the guess did not hold for.
-template <bool VEC>
+template <bool VEC, bool FILTER>
 __global__ void __launch_bounds__(kSampThreads) slice_choose_kernel(SampArgs a) {
   __shared__ SampShared sh;
   const int row = blockIdx.x;
@@ -1151,37 +1156,47 @@ __global__ void __launch_bounds__(kSampThreads) slice_choose_kernel(SampArgs a) 
   constexpr int PER = kBins / kSampThreads;
   const int chunks = (a.n + 255) / 256;
   HeldLists lists, places;
-  lists.load(w.list);
-  places.load(w.place);
+  if constexpr (FILTER) {
+    lists.load(w.list);
+    places.load(w.place);
+  }
   float mass[PER];
 #pragma unroll
   for (int j = 0; j < PER; ++j) mass[j] = w.chunk[min((int)threadIdx.x + j * kSampThreads, chunks - 1)];
   const RowState st = *w.state;
-  if (!st.valid) {
-    sample_row<VEC, true>(x, a.n, rp, a.uniform[row], a.ids + row, sh);
-    return;
-  }
-  const Guess g = guess_of(rp, a.n);
-  for (int i = threadIdx.x; i < min(chunks, kBins); i += kSampThreads) sh.bin[i] = 0;
-  const float thr = finish_threshold(sh, lists, rp, g, st);  // a block barrier, or no elements to add
-  // the cut bin's kept elements, in whole numbers: the same in any order
-  const int which = st.kbin >= st.pbin ? 0 : 1, listed = which ? st.pcount : st.kcount;
-  if (g.use_k || g.use_p) {
-#pragma unroll
-    for (int j = 0; j < kList / kSampThreads; ++j) {
-      const uint32_t b = which ? lists.got[1][j] : lists.got[0][j], at = which ? places.got[1][j] : places.got[0][j];
-      if ((int)threadIdx.x + j * kSampThreads < listed && __uint_as_float(b) >= thr) atomicAdd(&sh.bin[at >> 8], g.fx.of(b));
+  float thr;
+  if constexpr (FILTER) {
+    if (!st.valid) {
+      sample_row<VEC, true>(x, a.n, rp, a.uniform[row], a.ids + row, sh);
+      return;
     }
+    const Guess g = guess_of(rp, a.n);
+    for (int i = threadIdx.x; i < min(chunks, kBins); i += kSampThreads) sh.bin[i] = 0;
+    thr = finish_threshold(sh, lists, rp, g, st);  // a block barrier, or no elements to add
+    // the cut bin's kept elements, in whole numbers: the same in any order
+    const int which = st.kbin >= st.pbin ? 0 : 1, listed = which ? st.pcount : st.kcount;
+    if (g.use_k || g.use_p) {
+#pragma unroll
+      for (int j = 0; j < kList / kSampThreads; ++j) {
+        const uint32_t b = which ? lists.got[1][j] : lists.got[0][j], at = which ? places.got[1][j] : places.got[0][j];
+        if ((int)threadIdx.x + j * kSampThreads < listed && __uint_as_float(b) >= thr) atomicAdd(&sh.bin[at >> 8], g.fx.of(b));
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      const int i = threadIdx.x + j * kSampThreads;
+      if (i < chunks) mass[j] += (float)ldexp((double)sh.bin[i], -g.fx.scale);
+    }
+    __syncthreads();  // the masses take the place of the sums
+  } else {
+    thr = rp.min_p > 0.f ? fmaxf(0.f, rp.min_p * st.vmax) : 0.f;
   }
-  __syncthreads();
 #pragma unroll
   for (int j = 0; j < PER; ++j) {
     const int i = threadIdx.x + j * kSampThreads;
-    mass[j] = i < chunks ? mass[j] + (float)ldexp((double)sh.bin[i], -g.fx.scale) : 0.f;
+    sh.chunk[i] = i < chunks ? mass[j] : 0.f;
   }
-  __syncthreads();  // the masses take the place of the sums
-#pragma unroll
-  for (int j = 0; j < PER; ++j) sh.chunk[threadIdx.x + j * kSampThreads] = mass[j];
   __syncthreads();
   choose<VEC>(x, a.n, thr, 256, a.uniform[row], a.ids + row, sh);
 }
@@ -1221,14 +1236,22 @@ static int launch_filters(SampArgs a, int batch, void* workspace, int64_t worksp
   a.slices = (a.n + a.slice - 1) / a.slice;
   a.ws = (char*)workspace;
   const dim3 grid(a.slices, batch), block(kSampThreads);
-  hipLaunchKernelGGL(vec ? slice_bins_kernel<true> : slice_bins_kernel<false>, grid, block, 0, s, a);
+  if (!filter && !a.out) {
+    if (a.m_arr || a.m_val > 0.f)
+      hipLaunchKernelGGL((vec ? slice_bins_kernel<true, false> : slice_bins_kernel<false, false>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((vec ? slice_collect_kernel<true, true, false> : slice_collect_kernel<false, true, false>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((vec ? slice_choose_kernel<true, false> : slice_choose_kernel<false, false>), dim3(batch), block, 0, s, a);
+    SGLK_LAUNCH_CHECK();
+    return SGLK_OK;
+  }
+  hipLaunchKernelGGL((vec ? slice_bins_kernel<true, true> : slice_bins_kernel<false, true>), grid, block, 0, s, a);
   if (a.out) {
-    hipLaunchKernelGGL((vec ? slice_collect_kernel<true, false> : slice_collect_kernel<false, false>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((vec ? slice_collect_kernel<true, false, true> : slice_collect_kernel<false, false, true>), grid, block, 0, s, a);
     hipLaunchKernelGGL(vec ? slice_apply_kernel<true> : slice_apply_kernel<false>, grid, block, 0, s, a);
   } else {
-    hipLaunchKernelGGL((vec ? slice_collect_kernel<true, true> : slice_collect_kernel<false, true>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((vec ? slice_collect_kernel<true, true, true> : slice_collect_kernel<false, true, true>), grid, block, 0, s, a);
   }
-  hipLaunchKernelGGL(vec ? slice_choose_kernel<true> : slice_choose_kernel<false>, dim3(batch), block, 0, s, a);
+  hipLaunchKernelGGL((vec ? slice_choose_kernel<true, true> : slice_choose_kernel<false, true>), dim3(batch), block, 0, s, a);
   SGLK_LAUNCH_CHECK();
   return SGLK_OK;
 }

@@ -243,3 +243,25 @@ def test_spread_rows_of_special_values(aligned, monkeypatch):
     monkeypatch.setattr(ops, "_filter_workspace", lambda *a, **k: (None, 0))
     for got, want in zip(spread, everything()):
         torch.testing.assert_close(got, want, rtol=1e-6 if got.is_floating_point() else 0, atol=0, equal_nan=True)
+
+
+@pytest.mark.parametrize("B,n", [(1, 65540), (1, 65541), (3, 151936), (64, 128256)])
+def test_spread_draws_without_a_selection(B, n, monkeypatch):
+    """Rows just long enough to be spread without a top-k or top-p, with a min-p for none, all and some of them, against one
+    block a row; and their renormalisation."""
+    import sglang_security_amd.sgl_kernel as sk
+    from sglang_security_amd import ops
+
+    g = torch.Generator().manual_seed(n)
+    rows = torch.stack([_rows("peaked", n, g) for _ in range(min(B, 3))])
+    rows = (rows * 2.0 ** -math.ceil(math.log2(rows.sum(1).max().item()))).float().to(DEV).repeat(-(-B // 3), 1)[:B].contiguous()
+    some = torch.tensor([(0.0, 0.25, 0.5)[b % 3] for b in range(B)], device=DEV)
+
+    def everything():
+        ids = [ops.sampling_from_probs(rows, torch.full((B,), u, device=DEV), min_p=m) for u in (0.0, 0.37, 0.99999) for m in (0.0, 0.25, some)]
+        return ids + [sk.top_p_renorm_probs(rows, 1.0)]
+
+    spread = everything()
+    monkeypatch.setattr(ops, "_filter_workspace", lambda *a, **k: (None, 0))
+    for got, want in zip(spread, everything()):
+        torch.testing.assert_close(got, want, rtol=1e-6 if got.is_floating_point() else 0, atol=0)
