@@ -1216,10 +1216,10 @@ static int launch_filters(SampArgs a, int batch, void* workspace, int64_t worksp
   const bool both_in_turn = !a.joint && (a.k_arr || a.k_val > 0) && (a.p_arr || a.p_val < 1.f);  // top-p over the k largest
   const bool filter = a.k_arr || (a.k_val > 0 && a.k_val < a.n) || a.p_arr || a.p_val < 1.f;
   a.slices = samp_slices(batch, a.n);
-  // Without a selection to share out, one block a row is the faster one up to 65536 elements (sampling, spread and not: 64
-  // rows of 32000 16.5 and 9.7 us, of 65536 19.2 and 14.4, of 128256 23.5 and 25.2; one row 14.5 and 9.1, 15.3 and 12.6,
-  // 15.8 and 20.5).
-  if (a.slices < 2 || (!filter && a.n <= 65536) || both_in_turn || batch > 65535 || !workspace || (reinterpret_cast<uintptr_t>(workspace) & 15) ||
+  // Without a selection to share out, one block a row is the faster one up to 32768 elements (us, a block and spread: 64 rows of
+  // 16384 8.4 and 9.9, of 32000 11.5 and 10.3, with a min-p 12.2 and 13.7; of 50304 14.6 and 11.7, 15.5 and 15.9; of 128256 25.2
+  // and 14.5, 29.0 and 20.0; one row of 50304 10.8 and 9.6, 13.1 and 13.3, of 128256 19.4 and 9.3, 22.7 and 12.7).
+  if (a.slices < 2 || (!filter && a.n <= 32768) || both_in_turn || batch > 65535 || !workspace || (reinterpret_cast<uintptr_t>(workspace) & 15) ||
       workspace_bytes < samp_ws_row(a.slices) * batch) {
     if (!filter && a.n <= kShort) {
       hipLaunchKernelGGL(vec ? short_rows_kernel<true> : short_rows_kernel<false>, dim3(batch), dim3(256), 0, s, a);

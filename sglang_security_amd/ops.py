@@ -1441,7 +1441,7 @@ def _per_row(v, batch, dtype, name):
 
 def _filter_workspace(probs, filtered=True):
     """(tensor or None, bytes): rows spread over several blocks meet there.  Rows that never are do not ask (1 us of 9 a call)."""
-    if probs.shape[1] < 16384 or (not filtered and probs.shape[1] <= 65536):
+    if probs.shape[1] < 16384 or (not filtered and probs.shape[1] <= 32768):
         return None, 0
     need = int(lib().sglk_sampling_workspace_bytes(probs.shape[0], probs.shape[1]))
     return (torch.empty(need, dtype=torch.uint8, device=probs.device) if need else None), need

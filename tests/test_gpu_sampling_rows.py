@@ -245,7 +245,7 @@ def test_spread_rows_of_special_values(aligned, monkeypatch):
         torch.testing.assert_close(got, want, rtol=1e-6 if got.is_floating_point() else 0, atol=0, equal_nan=True)
 
 
-@pytest.mark.parametrize("B,n", [(1, 65540), (1, 65541), (3, 151936), (64, 128256)])
+@pytest.mark.parametrize("B,n", [(1, 32768), (1, 32772), (5, 32773), (3, 151936), (64, 128256)])
 def test_spread_draws_without_a_selection(B, n, monkeypatch):
     """Rows just long enough to be spread without a top-k or top-p, with a min-p for none, all and some of them, against one
     block a row; and their renormalisation."""
