@@ -948,38 +948,48 @@ static int fp8_stream_splits(int M, int N, int K) {
   return std::max(1, std::min({(512 + blocks - 1) / blocks, std::max(K / 1024, 1), 8}));
 }
 
-// Splits of K, and whether a call goes to the kernels of fp8_direct.h at all (up to 64 rows).  A split costs its reduction
-// launch, some 2 us: worth it from nine rows on where x is most of what a narrow output's blocks read (32 rows, 14336 x 4096 unsplit
-// 18.8, two splits 13.9 + 2; 4096 x 4096 7.0 and 5.5 + 2), and for the staged form until 256 blocks (64 rows, 4096 x 4096
-// unsplit 9.4, two splits 7.2 + 2; 14336 x 4096 24.4 and 16.0 + 2; 8192 x 1280 14.0 and, four ways, 6.6 + 2).
+// Whether a call goes to the kernels of fp8_direct.h at all (up to 64 rows), its splits of K, and one strip or two a block.  From 1024
+// strips on blocks are four wide and unsplit.  Up to 8 rows x is small and a split's reduction launch (some 2 us) costs what it gives
+// (8 rows, 14336 x 4096 12.5 us, in two splits 13.9).  Otherwise the least of what a unit's blocks take: rounds of 256
+// blocks, each so many us a 1024 of k and a start and an end, as fitted to 480 calls (within 1 % of the best form on
+// average).  What the rounds give, us with the reduction, 32 rows: 18432 x 3072 26.2 in two splits of one strip (one round and a half), 20.7 in
+// four of two; 18432 x 10240 56.4 in one split, 46.9 in four; 64 rows: 18432 x 3072 25.2 in three splits, 20.1 in two;
+// 14336 x 5120 28.9 in two, 24.5 in three.
 struct Fp8Direct {
   bool ok;
   int splits, per;  // k-blocks a split
+  bool pairs;       // up to 32 rows: two strips a block
 };
-static Fp8Direct fp8_direct_plan(int M, int N, int K) {
+static Fp8Direct fp8_direct_plan(int M, int N, int K, int most = 8) {
   const int kblocks = K / 128, strips = N / 16;
-  int splits = 1;
+  Fp8Direct plan{M <= 64, 1, kblocks, true};
   if (M > 64) {
-    splits = fp8_stream_splits(M, N, K);
-  } else if (const char* env = getenv("SGLK_FP8_STREAM_SPLITS"); env && atoi(env) > 0) {
-    splits = std::min(atoi(env), kblocks);
-  } else if (N % 4 != 0) {
-    splits = 1;
-  } else if (M > 32) {
-    const int blocks = strips >= 1024 ? (strips + 3) / 4 : (strips + 1) / 2;
-    if (blocks < 192) splits = std::max(1, std::min({(255 + blocks) / blocks, 4, K / 1024}));
-  } else if (M > 8 && strips <= 256 && K >= 8192) {
-    splits = 2;
+    plan.splits = fp8_stream_splits(M, N, K);
+  } else if (strips < 1024) {
+    const char* env = getenv("SGLK_FP8_STREAM_SPLITS");
+    const int forced = env && atoi(env) > 0 && most > 1 ? std::min(atoi(env), kblocks) : 0;
+    const bool staged = M > 32;
+    if (M <= 8) most = 1;
+    most = std::max(1, std::min(most, K / (staged ? 1024 : 2048)));
+    double best = 0.0;
+    for (int wide = staged ? 1 : 0; wide < 2; ++wide) {
+      const int blocks = wide ? (strips + 1) / 2 : strips;
+      const double per_k = staged ? 1.55 : (wide ? 1.1 : 0.75) + 0.18 * M / 16, ends = staged ? 2.35 : 0.85;
+      for (int n = forced ? forced : 1; n <= (forced ? forced : most); ++n) {
+        const double t = (blocks * n + 255) / 256 * (per_k * K / 1024 / n + ends) + (n == 1 ? 0.0 : staged ? 1.5 : 2.0);
+        if (best == 0.0 || t < best) best = t, plan.splits = n, plan.pairs = wide;
+      }
+    }
   }
-  const int per = (kblocks + splits - 1) / splits;
-  return Fp8Direct{M <= 64, (kblocks + per - 1) / per, per};
+  plan.per = (kblocks + plan.splits - 1) / plan.splits;
+  plan.splits = (kblocks + plan.per - 1) / plan.per;
+  return plan;
 }
 
-// Which tile: 64 columns a block where there are blocks enough, so that x is read least; one strip where there are too few strips
-// to give every unit more.
 template <typename TO>
-int launch_fp8_direct(const Fp8DirectArgs& a, int splits, hipStream_t s) {
-  const int strips = a.N / 16;
+int launch_fp8_direct(const Fp8DirectArgs& a, const Fp8Direct& plan, hipStream_t s) {
+  const int strips = a.N / 16, splits = plan.splits;
+  const bool pairs = plan.pairs;
 #define SGLK_FP8_DIRECT(MT, CS, WAYS, R)                                                                                        \
   {                                                                                                                             \
     constexpr int lds = fp8_direct_lds<MT, CS, WAYS>();                                                                         \
@@ -991,7 +1001,6 @@ int launch_fp8_direct(const Fp8DirectArgs& a, int splits, hipStream_t s) {
     if (int rc = ensure_lds<&fp8_staged_kernel<TO, SB, PW>>(fp8_staged_lds<SB>())) return rc;                                   \
     hipLaunchKernelGGL((fp8_staged_kernel<TO, SB, PW>), dim3((strips + SB - 1) / SB, splits), dim3(512), fp8_staged_lds<SB>(), s, a); \
   }
-  const bool pairs = strips > 256 || (splits > 1 && strips == 256);
   if (a.M > 32) {
     if (strips >= 1024) SGLK_FP8_STAGED(4, 2) else SGLK_FP8_STAGED(2, 4)
   } else if (a.M > 16) {
@@ -1275,17 +1284,20 @@ int sglk_fp8_scaled_mm_packed(const void* a, const void* packed, const float* sc
              "fp8_scaled_mm_packed: N=%d must be a multiple of 16, K=%d of 128", N, K);
   SGLK_CHECK(aligned16(a) && aligned16(packed) && a_stride % 16 == 0 && a_stride >= K && out_stride >= N,
              "fp8_scaled_mm_packed: rows must be 16-byte aligned");
-  const Fp8Direct plan = fp8_direct_plan(M, N, K);
-  int used = plan.splits, per = plan.per;
-  if (used > 1 && (!workspace || workspace_bytes < (int64_t)used * M * N * (int64_t)sizeof(float) || !aligned16(workspace)))
-    used = 1, per = K / 128;
+  Fp8Direct plan = fp8_direct_plan(M, N, K);
+  if (plan.splits > 1 &&
+      (!workspace || workspace_bytes < (int64_t)plan.splits * M * N * (int64_t)sizeof(float) || !aligned16(workspace))) {
+    plan = fp8_direct_plan(M, N, K, 1);
+    plan.splits = 1, plan.per = K / 128;
+  }
+  const int used = plan.splits, per = plan.per;
   float* partial = used > 1 ? (float*)workspace : nullptr;
   hipStream_t s = (hipStream_t)stream;
   SGLK_DISPATCH_HALF(out_dtype, TO, {
     if (plan.ok) {
       const Fp8DirectArgs d{(const uint8_t*)a, (const uint8_t*)packed, scales_a, scales_b, bias, out, partial,
                             M,                 N,                      K,        per,      a_stride, out_stride};
-      const int rc = launch_fp8_direct<TO>(d, used, s);
+      const int rc = launch_fp8_direct<TO>(d, plan, s);
       if (rc != SGLK_OK) return rc;
     } else {
       hipLaunchKernelGGL((fp8_stream_kernel<TO, 1, 4>), dim3((N + 63) / 64, used, (M + 63) / 64), dim3(256), 0, s,
@@ -1350,7 +1362,7 @@ int sglk_fp8_mm_packed_partial(const void* a, const void* packed, float* partial
   const Fp8Direct plan = fp8_direct_plan(M, N, K);
   if (plan.ok) {
     const Fp8DirectArgs d{(const uint8_t*)a, (const uint8_t*)packed, nullptr, nullptr, nullptr, nullptr, partial, M, N, K, plan.per, a_stride, 0};
-    return launch_fp8_direct<bf16_t>(d, plan.splits, (hipStream_t)stream);
+    return launch_fp8_direct<bf16_t>(d, plan, (hipStream_t)stream);
   }
   hipLaunchKernelGGL((fp8_stream_kernel<bf16_t, 1, 4>), dim3((N + 63) / 64, plan.splits, (M + 63) / 64), dim3(256), 0,
                      (hipStream_t)stream, (const uint8_t*)a, (const uint8_t*)packed, (const float*)nullptr,

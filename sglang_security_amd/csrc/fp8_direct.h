@@ -16,7 +16,7 @@
 //   4096 x 6144     12.4 -> 6.3     12.9 -> 6.7      13.6 -> 8.3      15.4 -> 10.2
 //   4096 x 4096     10.2 -> 4.8     10.5 -> 5.7      11.0 -> 7.0      12.5 -> 7.2 + 2
 //   4096 x 28672    29.5 -> 21.5    29.6 -> 21.6     30.4 -> 23.3     33.8 -> 28.9
-//   14336 x 4096    18.8 -> 11.8    18.9 -> 14.7     19.7 -> 13.9 + 2 23.7 -> 16.0 + 2
+//   14336 x 4096    18.8 -> 11.8    18.9 -> 14.7     19.7 -> 14.7 + 2 23.7 -> 16.0 + 2
 #pragma once
 #include <algorithm>
 #include <type_traits>

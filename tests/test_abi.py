@@ -77,3 +77,16 @@ def test_modules_import_where_torch_knows_no_gpu():
             "import sglang_security_amd.ops, sglang_security_amd.mem_cache.memory_pool, sglang_security_amd.attention.backend\n"
             "import sglang_security_amd.quantization.awq, sglang_security_amd.quantization.w8a8_fp8\n")
     subprocess.run([sys.executable, "-c", code], cwd=ROOT, check=True, timeout=300)
+
+
+@pytest.mark.parametrize("columns", [512, 1280, 3072, 4080, 4096, 5120, 6144, 7168, 10240])
+def test_fp8_splits_fill_the_units(columns):
+    """64 rows of a long inner dimension, where what a unit has to walk is all that counts: at most a third more than with the
+    best number of splits (blocks of two strips, one after the other on 256 units)."""
+    from sglang_security_amd import ops
+
+    def walk(splits):
+        return -(-columns // 32 * splits // 256) / splits
+
+    got = ops.fp8_mm_packed_partial_splits(64, columns, 18432)
+    assert 1 <= got <= 8 and walk(got) <= 1.34 * min(walk(n) for n in range(1, 9))

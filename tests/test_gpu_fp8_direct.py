@@ -13,7 +13,8 @@ def _fp8(shape, g):
 
 
 @pytest.mark.parametrize("M", [1, 8, 9, 16, 17, 32, 33, 64, 65])
-@pytest.mark.parametrize("N,K", [(16, 128), (48, 1152), (4096, 512), (4096, 8320), (4112, 640), (16384 - 16, 384), (16384 + 16, 384)])
+@pytest.mark.parametrize("N,K", [(16, 128), (48, 1152), (4096, 512), (4096, 8320), (4112, 640), (16384 - 16, 384), (16384 + 16, 384),
+                                 (16384 + 16, 2688), (48, 8320), (1280, 18432), (4080, 14336), (10240, 4096)])
 @pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16])
 def test_products(M, N, K, out_dtype):
     from sglang_security_amd import ops
