@@ -1040,6 +1040,15 @@ def fp8_blockwise_scaled_mm_packed(mat_a, packed, scales_a, scales_b, out_dtype,
     return out
 
 
+def fp8_streams(N, K, rows=None) -> bool:
+    """Whether an e4m3 weight [N, K] that multiplies up to `rows` rows (None: any number) is worth a second copy in the
+    streaming layout.  Up to 64 rows it is the faster one from K = 512 on (us, one row and 64, against row-major: 3584 x
+    8192 7.1 and 10.8, 10.6 and 13.0; 896 x 4864 3.0 and 4.3, 5.4 and 6.0), beyond them, on another kernel, from 4096 on
+    (3584 x 8192, that kernel at 64 rows: 19.8 and 15.3).  The row-major weight stays for larger calls, so a weight that has
+    a copy is held twice."""
+    return N % 16 == 0 and K % 128 == 0 and K >= (512 if rows is not None and rows <= 64 else 4096)
+
+
 def fp8_tiled(M, N, K) -> bool:
     """Whether fp8_scaled_mm on a row-major weight is expected to beat fp8_scaled_mm_packed on its streaming copy."""
     return bool(lib().sglk_fp8_tiled(M, N, K))

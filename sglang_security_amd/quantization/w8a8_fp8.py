@@ -6,8 +6,9 @@ the same `apply` contract (apply_fp8_linear, layers/quantization/fp8_utils.py:45
 activations, scaled product, bias, output in the activation type).  A checkpoint that is not fp8-serialised is
 quantised per output channel at load time, as the reference does when its scaled product takes per-channel scales
 (:118-127).  `process_weights_after_loading` additionally builds the sequential-streaming copy the decode-size product
-reads (same byte count).  Up to 64 rows that product is the faster one from inner dimensions of 512 on (us, one row and
-64: 3584 x 8192 7.1 against 10.8 row-major and 10.6 against 13.0, 896 x 4864 3.0 and 4.3, 5.4 and 6.0), beyond from 4096 on.
+reads, where that is the faster one (ops.fp8_streams: inner dimensions of 4096 and more, for calls of up to 64 rows 512 and
+more).  The row-major weight stays for larger calls: a weight with a copy takes twice its bytes.  A caller that would
+rather have the memory of the shorter ones passes streaming_short_k=False.
 """
 from __future__ import annotations
 
@@ -53,9 +54,11 @@ class W8A8Fp8Config:
 
 
 class W8A8Fp8LinearMethod:
-    def __init__(self, quantization_config: W8A8Fp8Config, streaming_max_tokens: int = 256):
+    def __init__(self, quantization_config: W8A8Fp8Config, streaming_max_tokens: int = 256,
+                 streaming_short_k: bool = True):
         self.quantization_config = quantization_config
         self.streaming_max_tokens = streaming_max_tokens
+        self.streaming_short_k = streaming_short_k  # copies of weights with inner dimensions below 4096
 
     def create_weights(self, layer: torch.nn.Module, input_size_per_partition: int, output_partition_sizes: List[int],
                        input_size: int, output_size: int, params_dtype: torch.dtype, **extra_weight_attrs):
@@ -93,9 +96,10 @@ class W8A8Fp8LinearMethod:
         layer.weight = torch.nn.Parameter(qweight.t(), requires_grad=False)
         layer.weight_scale = torch.nn.Parameter(scale, requires_grad=False)
         layer.sglk_shape = (k, n)
-        layer.sglk_packed = ops.fp8_repack(qweight) if (n % 16 == 0 and k % 128 == 0 and k >= 4096) else None
+        layer.sglk_packed = ops.fp8_repack(qweight) if ops.fp8_streams(n, k) else None
         # shorter inner dimensions: for calls of up to 64 rows, beyond them the row-major kernels are the faster ones
-        layer.sglk_packed_short = ops.fp8_repack(qweight) if (n % 16 == 0 and k % 128 == 0 and 512 <= k < 4096) else None
+        short = self.streaming_short_k and layer.sglk_packed is None and ops.fp8_streams(n, k, 64)
+        layer.sglk_packed_short = ops.fp8_repack(qweight) if short else None
         layer.sglk_workspace = None
 
     def _workspace(self, layer, m: int, device) -> torch.Tensor:
