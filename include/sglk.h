@@ -478,7 +478,8 @@ SGLK_API int sglk_awq_gemm_static(const void* x, const int32_t* packed, const vo
  * None of these has a counterpart in the reference, which runs norm / GEMM / rope / activation as separate
  * ops; they are for callers that own the whole decoder layer (the graph-captured decode step).  Two ideas:
  *  (1) block sums: the fused AWQ GEMM needs X[g][m] = sum of x[m, 128g .. 128g+127]; the kernel that produces
- *      x can write them (xsum [K/128][xs_stride] fp32, xs_stride >= M) and the GEMM then skips its own pass;
+ *      x can write them (xsum [K/128][xs_stride] fp32, xs_stride >= M) and the GEMM then skips its own pass
+ *      (sglk_awq_gemm_reads_xsum: not at up to 16 rows, whose kernel forms them beside its products);
  *  (2) split-K partials: the GEMM stores fp32 partial[split][M][N] (row-major, split stride M*N) and the
  *      consumer adds the splits up, rounds once to the activation type (the value the GEMM would have
  *      stored) and carries on -- no last-block reduction inside the GEMM. */
@@ -490,6 +491,8 @@ SGLK_API int sglk_awq_gemm_xs(const void* x, const int32_t* packed, const void* 
 /* Number of splits sglk_awq_gemm_partial writes for this shape; 0: shape not covered by the partial form
  * (needs K % 512 == 0, N % 128 == 0, group size 128). */
 SGLK_API int sglk_awq_gemm_partial_splits(int M, int N, int K, int group_size);
+/* 0 where a product of this shape leaves supplied block sums unread: its producer need not write them. */
+SGLK_API int sglk_awq_gemm_reads_xsum(int M, int N, int K, int group_size);
 SGLK_API int sglk_awq_gemm_partial(const void* x, const int32_t* packed, const void* scales,
                                    const int32_t* qzeros, const float* xsum, int64_t xs_stride,
                                    float* partial, int M, int N, int K, int group_size, int64_t x_stride,

@@ -1693,6 +1693,10 @@ int sglk_awq_gemm_partial_splits(int M, int N, int K, int group_size) {
   return wp.ok ? wp.splits : 0;
 }
 
+int sglk_awq_gemm_reads_xsum(int M, int N, int K, int group_size) {
+  return M > AwqRows16::kRows || plan_awq_wide(M, N, K, group_size, true).splits == 0;
+}
+
 int sglk_awq_gemm_partial(const void* x, const int32_t* packed, const void* scales, const int32_t* qzeros,
                           const float* xsum, int64_t xs_stride, float* partial, int M, int N, int K, int group_size,
                           int64_t x_stride, int dtype, void* stream) {

@@ -361,6 +361,10 @@ class LlamaDecoder:
                     if not self._keep_ref:
                         w.qweight = None
             self.fused_act = all("gate_up_il" in L for L in self.layers)
+        # block sums that the step's products read, from their producers (none at up to 16 rows outside a chain)
+        reads = self.fused and (self.chain or any(
+            ops.awq_gemm_reads_xsum(self.B, n, kk, c.group_size) for kk, n in (*shapes.values(), (c.hidden, 2 * c.inter))))
+        self.block_sums = (self.xs_hidden, self.xs_attn, self.xs_act) if reads else (None, None, None)
         return self.fused
 
     def _timed(self, name, fn):
@@ -407,69 +411,70 @@ class LlamaDecoder:
         o_view = self.attn_out.view(self.B, c.q_heads, c.head_dim)
         P, S = self.partial, self.part_splits
         tp = getattr(self, "tp_group", None)
+        xs_hidden, xs_attn, xs_act = self.block_sums
         for li, L in enumerate(self.layers):
             if li == 0:
                 self.residual.copy_(self.hidden)
-                ops.fused_add_rmsnorm_ex(self.hidden, None, L["ln1"], c.eps, xsum_out=self.xs_hidden)
+                ops.fused_add_rmsnorm_ex(self.hidden, None, L["ln1"], c.eps, xsum_out=xs_hidden)
             elif tp is None:  # consumes the previous layer's down-projection partials
                 ops.fused_add_rmsnorm_ex(self.hidden, self.residual, L["ln1"], c.eps, partials=P, splits=S["down"],
-                                         xsum_out=self.xs_hidden)
+                                         xsum_out=xs_hidden)
             else:
-                ops.fused_add_rmsnorm_ex(self.hidden, self.residual, L["ln1"], c.eps, xsum_out=self.xs_hidden)
+                ops.fused_add_rmsnorm_ex(self.hidden, self.residual, L["ln1"], c.eps, xsum_out=xs_hidden)
             w = L["qkv"]
-            self._timed("qkv", lambda: ops.awq_gemm_partial(self.hidden, w.packed, w.scales, w.qzeros, P, self.xs_hidden))
+            self._timed("qkv", lambda: ops.awq_gemm_partial(self.hidden, w.packed, w.scales, w.qzeros, P, xs_hidden))
             if self.fold_rope and getattr(self, "shared", False):
                 # the attention kernel assembles q and the new K / V rows from the projection's partial sums itself
                 ops.decode_attention_shared_prefix_rope(P, S["qkv"], self.qkv.numel(), L["qkv_bias"], self.cos_sin,
                                                         self.positions, self.out_cache_loc, self.k_pool[li],
                                                         self.v_pool[li], o_view, self.kv_indptr, self.kv_indices,
                                                         self.group_indptr, self.group_prefix, self.shared_ws,
-                                                        self.max_kv_splits, sm_scale, 0.0, self.xs_attn)
+                                                        self.max_kv_splits, sm_scale, 0.0, xs_attn)
             elif self.rope_role and getattr(self, "shared", False) and getattr(self, "shared_plan", None) is not None:
                 # rotation + pool write as the first blocks of the attention launch
                 ops.decode_attention_shared_planned_rope(P, S["qkv"], self.qkv.numel(), L["qkv_bias"], self.cos_sin,
                                                          self.positions, self.out_cache_loc, q_view, self.k_pool[li],
                                                          self.v_pool[li], o_view, self.kv_indptr, self.kv_indices,
                                                          self.shared_plan, li + 1, self.shared_ws, self.max_kv_splits,
-                                                         sm_scale, 0.0, self.xs_attn)
+                                                         sm_scale, 0.0, xs_attn)
             else:
                 ops.rope_and_store_kv_partial(self.qkv, P, S["qkv"], self.cos_sin, self.positions, self.k_pool[li],
                                               self.v_pool[li], self.out_cache_loc, c.q_heads, c.kv_heads, c.head_dim,
                                               bias=L["qkv_bias"])
-                self.attention(li, q_view, o_view, sm_scale, xsum_out=self.xs_attn)
+                self.attention(li, q_view, o_view, sm_scale, xsum_out=xs_attn)
             w = L["o"]
             if tp is None:
-                self._timed("o", lambda: ops.awq_gemm_partial(self.attn_out, w.packed, w.scales, w.qzeros, P, self.xs_attn))
+                self._timed("o", lambda: ops.awq_gemm_partial(self.attn_out, w.packed, w.scales, w.qzeros, P, xs_attn))
                 ops.fused_add_rmsnorm_ex(self.hidden, self.residual, L["ln2"], c.eps, partials=P, splits=S["o"],
-                                         xsum_out=self.xs_hidden, zero_out=self.xs_act if self.fused_act else None)
+                                         xsum_out=xs_hidden, zero_out=xs_act if self.fused_act else None)
             else:  # row-parallel: this rank's product (split-K closed inside the GEMM), the sum over ranks, the consumer
-                self._timed("o", lambda: ops.awq_gemm_xs(self.attn_out, w.packed, w.scales, w.qzeros, self.xs_attn,
+                self._timed("o", lambda: ops.awq_gemm_xs(self.attn_out, w.packed, w.scales, w.qzeros, xs_attn,
                                                          self.tp_buf, self.workspace))
                 self._tp_sum()
-                ops.fused_add_rmsnorm_ex(self.hidden, self.residual, L["ln2"], c.eps, xsum_out=self.xs_hidden,
-                                         zero_out=self.xs_act if self.fused_act else None)
+                ops.fused_add_rmsnorm_ex(self.hidden, self.residual, L["ln2"], c.eps, xsum_out=xs_hidden,
+                                         zero_out=xs_act if self.fused_act else None)
             if self.fused_act and tp is None and self.chain:
                 # gate_up (+ activation) and down in one launch of persistent blocks: the down projection's first
                 # weights are on their way while gate_up's blocks still reduce and store
                 il, w = L["gate_up_il"], L["down"]
                 self._timed("gate_up+down", lambda: ops.awq_chain(
-                    [ops.chain_silu_mul(self.hidden, il[0], il[1], il[2], self.xs_hidden, self.act, self.xs_act),
-                     ops.chain_partial(self.act, w.packed, w.scales, w.qzeros, self.xs_act, P)], self.chain_sync))
+                    [ops.chain_silu_mul(self.hidden, il[0], il[1], il[2], xs_hidden, self.act, xs_act),
+                     ops.chain_partial(self.act, w.packed, w.scales, w.qzeros, xs_act, P)], self.chain_sync))
                 continue
             if self.fused_act:
                 il = L["gate_up_il"]
                 self._timed("gate_up", lambda: ops.awq_gemm_silu_mul(self.hidden, il[0], il[1], il[2], self.act,
-                                                                     self.xs_hidden, self.xs_act))
+                                                                     xs_hidden, xs_act))
             else:
                 w = L["gate_up"]
-                self._timed("gate_up", lambda: ops.awq_gemm_xs(self.hidden, w.packed, w.scales, w.qzeros, self.xs_hidden,
+                self._timed("gate_up", lambda: ops.awq_gemm_xs(self.hidden, w.packed, w.scales, w.qzeros, xs_hidden,
                                                                self.gate_up, self.workspace))
                 ops.act_and_mul_xs(self.act, self.gate_up, 0, self.xs_act)
             w = L["down"]
             if tp is None:
-                self._timed("down", lambda: ops.awq_gemm_partial(self.act, w.packed, w.scales, w.qzeros, P, self.xs_act))
+                self._timed("down", lambda: ops.awq_gemm_partial(self.act, w.packed, w.scales, w.qzeros, P, xs_act))
             else:
-                self._timed("down", lambda: ops.awq_gemm_xs(self.act, w.packed, w.scales, w.qzeros, self.xs_act,
+                self._timed("down", lambda: ops.awq_gemm_xs(self.act, w.packed, w.scales, w.qzeros, xs_act,
                                                             self.tp_buf, self.workspace))
                 self._tp_sum()
         if tp is None:

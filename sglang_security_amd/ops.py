@@ -1202,6 +1202,11 @@ def awq_gemm_partial_splits(M, N, K, group=128) -> int:
     return int(lib().sglk_awq_gemm_partial_splits(M, N, K, group))
 
 
+def awq_gemm_reads_xsum(M, N, K, group=128) -> bool:
+    """Whether a product of this shape reads block sums that its producer supplies (not at up to 16 rows)."""
+    return bool(lib().sglk_awq_gemm_reads_xsum(M, N, K, group))
+
+
 def awq_gemm_partial(x, packed, scales, qzeros, partial, xsum=None):
     """fp32 split-K partials [splits, M, N] of x @ W into `partial`; returns the number of splits written."""
     _need_gpu(x, packed, scales, qzeros, partial)

@@ -236,7 +236,10 @@ class LlamaPrefill:
         T = input_ids.shape[0]
         hidden, residual = self.hidden[:T], self.residual[:T]
         qkv, attn_out, act = self.qkv[:T], self.attn_out[:T], self.act[:T]
-        xs_h, xs_a = self.xs_hidden[:, :T], self.xs_act[:, :T]
+        xs_h, xs_a, xs_clear = self.xs_hidden[:, :T], self.xs_act[:, :T], self.xs_act
+        if not any(ops.awq_gemm_reads_xsum(T, n, kk, c.group_size)
+                   for kk, n in (*self._shapes.values(), (c.hidden, 2 * c.inter))):
+            xs_h = xs_a = xs_clear = None
         P = self.partial
         S = {k: ops.awq_gemm_partial_splits(T, n, kk, c.group_size) for k, (kk, n) in self._shapes.items()}
         torch.index_select(self.dec.embed, 0, input_ids, out=hidden)
@@ -262,7 +265,7 @@ class LlamaPrefill:
             w = L["o"]
             ops.awq_gemm_partial(attn_out, w.packed, w.scales, w.qzeros, P)
             ops.fused_add_rmsnorm_ex(hidden, residual, L["ln2"], c.eps, partials=P, splits=S["o"], xsum_out=xs_h,
-                                     zero_out=self.xs_act)
+                                     zero_out=xs_clear)
             il = L["gate_up_il"]
             ops.awq_gemm_silu_mul(hidden, il[0], il[1], il[2], act, xs_h, xs_a)
             w = L["down"]

@@ -51,6 +51,9 @@ def test_host_only_calls():
     # remainder splits, one split count per request (rounded to 256)
     assert L.sglk_decode_shared_workspace_bytes(64, 32, 128, 8) == ((2 * 64 * 32 + 2) * 4 + 255) // 256 * 256 + \
         64 * 32 * (8 + 8) * 129 * 4 + 256
+    # block sums are read from 17 rows on, and where the kernel of few rows does not take the shape
+    assert [L.sglk_awq_gemm_reads_xsum(m, 4096, 4096, 128) for m in (1, 16, 17, 64)] == [0, 0, 1, 1]
+    assert L.sglk_awq_gemm_reads_xsum(16, 4096 + 64, 4096, 128) == 1 and L.sglk_awq_gemm_reads_xsum(16, 4096, 4096, 256) == 1
     # argument validation happens before any GPU call
     rc = L.sglk_rmsnorm(None, None, None, 1, 128, 128, 128, 1e-6, 0, 2, None)
     assert rc == -1 and b"null" in L.sglk_last_error().lower()

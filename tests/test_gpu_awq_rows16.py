@@ -134,3 +134,27 @@ def test_last_block_adds_every_split_in_order(M, K, N, monkeypatch):
     work = torch.zeros(ops.awq_gemm_workspace_bytes(M, N, K), dtype=torch.uint8, device=DEV)
     for _ in range(2):
         assert torch.equal(ops.awq_gemm(x, *w, workspace=work), want.bfloat16())
+
+
+@pytest.mark.parametrize("batch", [6, 16, 17])
+def test_decode_step_makes_only_block_sums_that_are_read(batch):
+    """Up to 16 rows the products form the sums of x themselves: the step's norms, attention and gated activation leave the
+    block sums alone, and its logits are the bits of a step that makes them."""
+    from sglang_security_amd.decode_runner import LlamaConfig, LlamaDecoder
+
+    logits = []
+    for forced in (False, True):
+        dec = LlamaDecoder(LlamaConfig.tiny(), batch=batch, pool_slots=1 + 64 + batch * 24, max_ctx=96, device=DEV, seed=0)
+        dec.setup_shared_prefix_batch(prefix_len=64, suffix_len=5)
+        dec.enable_shared_prefix(True)
+        assert dec.enable_fusion(True)
+        buffers = (dec.xs_hidden, dec.xs_attn, dec.xs_act)
+        if forced:
+            dec.block_sums = buffers
+        for t in buffers:
+            t.fill_(float("nan"))
+        dec.step()
+        torch.cuda.synchronize()
+        assert all(bool(t.isnan().all()) for t in buffers) == (batch <= 16 and not forced)
+        logits.append(dec.logits.clone())
+    assert torch.isfinite(logits[0].float()).all() and torch.equal(logits[0], logits[1])
