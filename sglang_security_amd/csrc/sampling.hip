@@ -1186,17 +1186,16 @@ __global__ void __launch_bounds__(kSampThreads) slice_choose_kernel(SampArgs a) 
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
       const int i = threadIdx.x + j * kSampThreads;
-      if (i < chunks) mass[j] += (float)ldexp((double)sh.bin[i], -g.fx.scale);
+      mass[j] = i < chunks ? mass[j] + (float)ldexp((double)sh.bin[i], -g.fx.scale) : 0.f;
     }
     __syncthreads();  // the masses take the place of the sums
   } else {
     thr = rp.min_p > 0.f ? fmaxf(0.f, rp.min_p * st.vmax) : 0.f;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) mass[j] = (int)threadIdx.x + j * kSampThreads < chunks ? mass[j] : 0.f;
   }
 #pragma unroll
-  for (int j = 0; j < PER; ++j) {
-    const int i = threadIdx.x + j * kSampThreads;
-    sh.chunk[i] = i < chunks ? mass[j] : 0.f;
-  }
+  for (int j = 0; j < PER; ++j) sh.chunk[threadIdx.x + j * kSampThreads] = mass[j];
   __syncthreads();
   choose<VEC>(x, a.n, thr, 256, a.uniform[row], a.ids + row, sh);
 }
