@@ -766,7 +766,7 @@ __device__ __forceinline__ long hi64(int4v v) { return (long)(uint32_t)v.z | ((l
 // BW: the block-scaled form (DeepSeek): sa[m, kb] (strides sa_m, sa_k) and sb[n / 128, kb] (strides sb_n, sb_k) scale
 // every 128-k block's product before it is added up; the activation scales of a k-block travel with its tile, the
 // weight scale with the weight pieces.
-template <typename TO, int NS, int PF, bool BW = false, int XPF = PF>
+template <typename TO, int PF, bool BW = false, int XPF = PF>
 __global__ void __launch_bounds__(256, 2) fp8_stream_kernel(const uint8_t* __restrict__ x, const uint8_t* __restrict__ wp,
                                                             const float* __restrict__ sa, const float* __restrict__ sb,
                                                             const void* __restrict__ bias, void* __restrict__ out,
@@ -782,7 +782,7 @@ __global__ void __launch_bounds__(256, 2) fp8_stream_kernel(const uint8_t* __res
   const int m0 = blockIdx.z * 64;
   const int kb0 = blockIdx.y * kb_per_split;
   const int nkb = min(kb_per_split, kblocks - kb0);
-  const int n0 = (blockIdx.x * 4 + wid) * 16 * NS + i16;
+  const int n = (blockIdx.x * 4 + wid) * 16 + i16;
 
   // activations: thread (row xr, quarter xq) moves bytes [32 xq, 32 xq + 32) of its row; a k-block's bytes are
   // requested XPF blocks ahead and parked in LDS one block ahead (a step of the loop is shorter than the way to the
@@ -806,36 +806,23 @@ __global__ void __launch_bounds__(256, 2) fp8_stream_kernel(const uint8_t* __res
       if (xq == 0) sas[buf][xr] = sr;
   };
 
-  const uint8_t* wsrc[NS];
-#pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    const int strip = min((n0 + 16 * s) >> 4, (N >> 4) - 1);
-    wsrc[s] = wp + ((int64_t)strip * kblocks + kb0) * 2048 + 16 * lane;
-  }
+  const uint8_t* wsrc = wp + ((int64_t)min(n >> 4, (N >> 4) - 1) * kblocks + kb0) * 2048 + 16 * lane;
   auto wload = [](const uint8_t* p) { return __builtin_nontemporal_load(reinterpret_cast<const int4v*>(p)); };
-  int4v wq[PF][NS][2];
-  [[maybe_unused]] float wsc[PF][NS];
-  [[maybe_unused]] const float* sbrow[NS];
-  if constexpr (BW) {
-#pragma unroll
-    for (int s = 0; s < NS; ++s) sbrow[s] = sb + (int64_t)(min(n0 + 16 * s, N - 1) >> 7) * sb_n + (int64_t)kb0 * sb_k;
-  }
+  int4v wq[PF][2];
+  [[maybe_unused]] float wsc[PF];
+  [[maybe_unused]] const float* sbrow = nullptr;
+  if constexpr (BW) sbrow = sb + (int64_t)(min(n, N - 1) >> 7) * sb_n + (int64_t)kb0 * sb_k;
 #pragma unroll
   for (int p = 0; p < PF; ++p)
     if (p < nkb) {
 #pragma unroll
-      for (int s = 0; s < NS; ++s) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) wq[p % PF][s][h] = wload(wsrc[s] + 2048 * p + 1024 * h);
-        if constexpr (BW) wsc[p % PF][s] = sbrow[s][(int64_t)p * sb_k];
-      }
+      for (int h = 0; h < 2; ++h) wq[p][h] = wload(wsrc + 2048 * p + 1024 * h);
+      if constexpr (BW) wsc[p] = sbrow[(int64_t)p * sb_k];
     }
 
-  f32x4 oacc[NS][4];
+  f32x4 oacc[4];
 #pragma unroll
-  for (int s = 0; s < NS; ++s)
-#pragma unroll
-    for (int mt = 0; mt < 4; ++mt) oacc[s][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int mt = 0; mt < 4; ++mt) oacc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   constexpr int U = PF > XPF ? PF : XPF;  // the loop is unrolled so that register slots are compile-time
   static_assert(PF % 2 == 0 && XPF % 2 == 0 && U % PF == 0 && U % XPF == 0,
@@ -860,16 +847,13 @@ __global__ void __launch_bounds__(256, 2) fp8_stream_kernel(const uint8_t* __res
             const int4v af0 = *reinterpret_cast<const int4v*>(xs + buf * 8192 + fs_off(16 * mt + i16, 2 * g));
             const int4v af1 = *reinterpret_cast<const int4v*>(xs + buf * 8192 + fs_off(16 * mt + i16, 2 * g + 1));
             const f32x4 as4 = *reinterpret_cast<const f32x4*>(&sas[buf][16 * mt + 4 * g]);  // rows 16 mt + 4 g + r
+            f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+            acc = mma_f8<0>(lo64(af0), lo64(wq[p % PF][0]), acc);
+            acc = mma_f8<0>(hi64(af0), hi64(wq[p % PF][0]), acc);
+            acc = mma_f8<0>(lo64(af1), lo64(wq[p % PF][1]), acc);
+            acc = mma_f8<0>(hi64(af1), hi64(wq[p % PF][1]), acc);
 #pragma unroll
-            for (int s = 0; s < NS; ++s) {
-              f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-              acc = mma_f8<0>(lo64(af0), lo64(wq[p % PF][s][0]), acc);
-              acc = mma_f8<0>(hi64(af0), hi64(wq[p % PF][s][0]), acc);
-              acc = mma_f8<0>(lo64(af1), lo64(wq[p % PF][s][1]), acc);
-              acc = mma_f8<0>(hi64(af1), hi64(wq[p % PF][s][1]), acc);
-#pragma unroll
-              for (int r = 0; r < 4; ++r) oacc[s][mt][r] += acc[r] * (as4[r] * wsc[p % PF][s]);
-            }
+            for (int r = 0; r < 4; ++r) oacc[mt][r] += acc[r] * (as4[r] * wsc[p % PF]);
           }
         } else {
 #pragma unroll
@@ -877,20 +861,14 @@ __global__ void __launch_bounds__(256, 2) fp8_stream_kernel(const uint8_t* __res
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt) {
               const int4v af = *reinterpret_cast<const int4v*>(xs + buf * 8192 + fs_off(16 * mt + i16, 2 * g + h));
-#pragma unroll
-              for (int s = 0; s < NS; ++s) {
-                oacc[s][mt] = mma_f8<0>(lo64(af), lo64(wq[p % PF][s][h]), oacc[s][mt]);
-                oacc[s][mt] = mma_f8<0>(hi64(af), hi64(wq[p % PF][s][h]), oacc[s][mt]);
-              }
+              oacc[mt] = mma_f8<0>(lo64(af), lo64(wq[p % PF][h]), oacc[mt]);
+              oacc[mt] = mma_f8<0>(hi64(af), hi64(wq[p % PF][h]), oacc[mt]);
             }
         }
         if (j + PF < nkb) {
 #pragma unroll
-          for (int s = 0; s < NS; ++s) {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) wq[p % PF][s][h] = wload(wsrc[s] + 2048 * (int64_t)(j + PF) + 1024 * h);
-            if constexpr (BW) wsc[p % PF][s] = sbrow[s][(int64_t)(j + PF) * sb_k];
-          }
+          for (int h = 0; h < 2; ++h) wq[p % PF][h] = wload(wsrc + 2048 * (int64_t)(j + PF) + 1024 * h);
+          if constexpr (BW) wsc[p % PF] = sbrow[(int64_t)(j + PF) * sb_k];
         }
         if (j + 1 < nkb) x_park(xreg[(p + 1) % XPF], buf ^ 1, sareg[(p + 1) % XPF]);
         __syncthreads();
@@ -898,28 +876,24 @@ __global__ void __launch_bounds__(256, 2) fp8_stream_kernel(const uint8_t* __res
     }
   }
 
-  // lane (i16, g) holds rows m0 + 16 mt + 4 g + r of column n0 + 16 s
+  // lane (i16, g) holds rows m0 + 16 mt + 4 g + r of column n
+  if (n >= N) return;
+  const float sbn = (partial || BW) ? 1.f : sb[n];
+  const float bn = (!partial && bias) ? ld<TO>(bias, n) : 0.f;
 #pragma unroll
-  for (int s = 0; s < NS; ++s) {
-    const int n = n0 + 16 * s;
-    if (n >= N) continue;
-    const float sbn = (partial || BW) ? 1.f : sb[n];
-    const float bn = (!partial && bias) ? ld<TO>(bias, n) : 0.f;
+  for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = m0 + 16 * mt + 4 * g + r;
-        if (m >= M) continue;
-        if (partial)
-          __hip_atomic_store(&partial[((int64_t)blockIdx.y * M + m) * N + n], oacc[s][mt][r], __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_AGENT);
-        else if constexpr (BW)
-          st<TO>(out, (int64_t)m * out_stride + n, oacc[s][mt][r]);
-        else
-          st<TO>(out, (int64_t)m * out_stride + n, oacc[s][mt][r] * sa[m] * sbn + bn);
-      }
-  }
+    for (int r = 0; r < 4; ++r) {
+      const int m = m0 + 16 * mt + 4 * g + r;
+      if (m >= M) continue;
+      if (partial)
+        __hip_atomic_store(&partial[((int64_t)blockIdx.y * M + m) * N + n], oacc[mt][r], __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+      else if constexpr (BW)
+        st<TO>(out, (int64_t)m * out_stride + n, oacc[mt][r]);
+      else
+        st<TO>(out, (int64_t)m * out_stride + n, oacc[mt][r] * sa[m] * sbn + bn);
+    }
 }
 
 // row-major e4m3 [N, K] -> the streaming layout above
@@ -1300,7 +1274,7 @@ int sglk_fp8_scaled_mm_packed(const void* a, const void* packed, const float* sc
       const int rc = launch_fp8_direct<TO>(d, plan, s);
       if (rc != SGLK_OK) return rc;
     } else {
-      hipLaunchKernelGGL((fp8_stream_kernel<TO, 1, 4>), dim3((N + 63) / 64, used, (M + 63) / 64), dim3(256), 0, s,
+      hipLaunchKernelGGL((fp8_stream_kernel<TO, 4>), dim3((N + 63) / 64, used, (M + 63) / 64), dim3(256), 0, s,
                          (const uint8_t*)a, (const uint8_t*)packed, scales_a, scales_b, bias, out, partial, M, N, K, per,
                          a_stride, out_stride);
     }
@@ -1333,7 +1307,7 @@ int sglk_fp8_blockwise_scaled_mm_packed(const void* a, const void* packed, const
   hipStream_t s = (hipStream_t)stream;
   SGLK_DISPATCH_HALF(out_dtype, TO, {
     // block-scaled: the scaling holds more registers; the deeper activation request does not pay here (measured)
-    hipLaunchKernelGGL((fp8_stream_kernel<TO, 1, 4, true, 2>), dim3((N + 63) / 64, used, (M + 63) / 64), dim3(256), 0, s,
+    hipLaunchKernelGGL((fp8_stream_kernel<TO, 4, true, 2>), dim3((N + 63) / 64, used, (M + 63) / 64), dim3(256), 0, s,
                        (const uint8_t*)a, (const uint8_t*)packed, scales_a, scales_b, (const void*)nullptr, out, partial, M,
                        N, K, per, (int64_t)K, (int64_t)N, sa_stride_m, sa_stride_k, sb_stride_n, sb_stride_k);
     if (used > 1) {
@@ -1364,7 +1338,7 @@ int sglk_fp8_mm_packed_partial(const void* a, const void* packed, float* partial
     const Fp8DirectArgs d{(const uint8_t*)a, (const uint8_t*)packed, nullptr, nullptr, nullptr, nullptr, partial, M, N, K, plan.per, a_stride, 0};
     return launch_fp8_direct<bf16_t>(d, plan, (hipStream_t)stream);
   }
-  hipLaunchKernelGGL((fp8_stream_kernel<bf16_t, 1, 4>), dim3((N + 63) / 64, plan.splits, (M + 63) / 64), dim3(256), 0,
+  hipLaunchKernelGGL((fp8_stream_kernel<bf16_t, 4>), dim3((N + 63) / 64, plan.splits, (M + 63) / 64), dim3(256), 0,
                      (hipStream_t)stream, (const uint8_t*)a, (const uint8_t*)packed, (const float*)nullptr,
                      (const float*)nullptr, (const void*)nullptr, (void*)nullptr, partial, M, N, K, plan.per, a_stride,
                      (int64_t)0);
