@@ -845,8 +845,8 @@ SGLK_API int sglk_sampling_from_probs(const float* probs, const float* uniform, 
                                       int vocab, int64_t in_stride, void* stream);
 /* The same with a caller's workspace (16-byte aligned, contents of no matter before and after;
  * sglk_sampling_workspace_bytes(batch, vocab), 0 where it would not be used): rows are spread over several blocks in
- * four launches.  Without one, or a smaller one, or where no top-k or top-p is given and rows are short, every row is
- * one block's. */
+ * three launches when sampling (two without a top-k, top-p and min-p), four when renormalising.  Without one, or a smaller one,
+ * or where no top-k or top-p is given and rows are short, every row is one block's. */
 SGLK_API int64_t sglk_sampling_workspace_bytes(int batch, int vocab);
 SGLK_API int sglk_top_k_renorm_probs_ws(const float* probs, float* out, const int32_t* top_k_arr,
                                         int top_k_val, int batch, int vocab, int64_t in_stride,

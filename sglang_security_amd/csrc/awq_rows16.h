@@ -11,8 +11,9 @@
 // x . (OFF + q) - (OFF + z) . sum(x) is in fp16 (OFF is 1024) a hundredth of either term and carries the roundings of both:
 // there a group is two halves, whose sums are smaller (16 rows, 4096 x 4096: 1.23e-5 of the result whole, 9.0e-6 so, 1.22e-5
 // in the wide kernel).
-// Rows that a batch does not have repeat its last one: switching their lanes off costs more than it saves (one row, 4096 x 28672:
-// 15.9 against 15.3 us, two halves of a block 29 against 16).  All figures here: weights from memory, us a launch.
+// Rows that a batch does not have repeat its last one: switching their lanes off costs more than it saves (one row, 4096 x 28672,
+// taken before the launches' last shapes: 15.9 against 15.3 us, two halves of a block 29 against 16).  All figures here: weights
+// from memory, us a launch.
 #pragma once
 #include "awq_common.h"
 

@@ -3,7 +3,10 @@
 //
 // Bound by the weights' way from memory, and on a decode step's shapes (16 to 117 MB over 256 units) by how much of it is
 // asked for at once.  Both kernels multiply whole k-blocks: a lane's 32 bytes of a row and of a strip are the operands of one
-// 16x16x128 f8f6f4 instruction as they stand, at twice the rate of the four 16x16x32 ones it replaces and with the same sums.
+// 16x16x128 f8f6f4 instruction as they stand, at twice the rate of the four 16x16x32 ones it replaces.  It aligns and adds 128
+// products at once where those round in between, so last bits differ; the error against 64-bit sums does not (normal values, 512
+// to 14336 of k: 1.2e-5 to 1.5e-5 of the result with either, and the same to 1 % for positive ones, for outliers 300 times the
+// rest, and for values or blocks of 32 spread over 2^12 to 2^18).
 //
 // Up to 32 rows (direct): no staging and no barrier in the loop.  A block's waves take its k-blocks in turn, ask for their bytes
 // of x and of the weights straight into registers and meet once in LDS; x is a fraction of the weights' bytes, or, under a
