@@ -323,22 +323,55 @@ static int dense_splits(int M, int N, int K) {
 }
 
 // Splits of the packed product, and whether dense_direct.h takes it: up to 16 rows, to 32 while its inner dimension is
-// short of 8192 (32 rows, 14336 x 4096: 27.0 in eight splits of the staged kernel, 27.9 in two), but from 65536 columns on and below
-// 4096 only to 24 (65536 x 2560, 24 and 28 rows: 58.4 and 61.0 us, staged 59.8 and 58.5; 128256 x 4096, 32 rows 176 and 184).
-// Outputs narrower than 512 stay with the order of sums, and the bits, of the row-major product.  A direct block is 32 columns
+// short of 8192 (32 rows, 14336 x 4096: 27.0 in eight splits of the staged kernel, 27.9 in two).  Outputs narrower than 512 stay with the order of sums, and the bits, of the row-major product.  A direct block is 32 columns
 // wide, or 64 where that leaves more than 128 blocks: as many splits as whole blocks fit the units, each of 512 of k at least.
+// A direct block reads the x of its split for itself, and a last round that is not full keeps the others waiting; the staged kernel
+// shares x among four times the columns and takes more splits.  Where one split of 32 columns a block leaves units empty, or one of 64
+// its last round, it is the faster one from some 65536 elements of x a block on, and in a short second round earlier (us of the
+// sums, direct and staged: 32 rows, 4608 x 4352 20.6 and 13.1, 6912 x 5120 24.9 and 18.0, 5120 x 20480 52.8 and 42.2; 16 rows,
+// 13824 x 5120 39.4 and 30.4; 3 rows, 11264 x 16512 81.6 and 69.7).  From 25 rows on so much x is too much for full rounds, too (2560 x
+// 65536, 24 and 28 rows: 58.4 and 61.0, staged 59.8 and 58.5; 2048 x 79808, 27 rows 54 and 71).  The lines are the best of 3668 calls up to 32 rows: sums of
+// split products 1.4 times as slow as before this kernel at worst without them, 1.2 with them, on average 1.37 times faster.
 struct DensePlan {
   bool direct;
   int splits, per;  // k-blocks a split
+  int blocks;       // direct blocks
+  int64_t x;        // elements of x that one of them reads
 };
+static bool dense_short_round(int blocks, double share) { return blocks < share * ((blocks + 255) / 256 * 256); }
 static DensePlan dense_packed_plan(int M, int N, int K) {
   const int kblocks = K / 128, strips = N / 16;
-  const bool few = M <= 16 || (M <= (N >= 65536 && K < 4096 ? 24 : 32) && K < 8192);
-  const bool direct = N >= 512 && few && !getenv("SGLK_DENSE_SPLITS") && !getenv("SGLK_DENSE_NS");
-  int splits = dense_splits(M, N, K);
-  if (direct) splits = strips >= 512 ? 1 : std::max(1, std::min(256 / ((strips + 1) / 2), kblocks / 4));
-  const int per = (kblocks + splits - 1) / splits;
-  return DensePlan{direct, (kblocks + per - 1) / per, per};
+  const bool few = M <= 16 || (M <= 32 && K < 8192);
+  DensePlan p{N >= 512 && few && !getenv("SGLK_DENSE_SPLITS") && !getenv("SGLK_DENSE_NS"), 1, kblocks, 0, 0};
+  if (p.direct) {
+    p.splits = strips >= 512 ? 1 : std::max(1, std::min(256 / ((strips + 1) / 2), kblocks / 4));
+    p.per = (kblocks + p.splits - 1) / p.splits;
+    p.blocks = N > 8192 ? (strips + 3) / 4 : (strips + 1) / 2 * p.splits;
+    p.x = (int64_t)M * 128 * p.per;
+    if (N > 8192)
+      p.direct = !(dense_short_round(p.blocks, 0.68) && (p.blocks > 256 ? p.x > 49152 || K > 4096 : p.x > 81920)) && (M <= 24 || p.x <= (N >= 49152 ? 65536 : 131072));
+    else if (p.splits == 1 && p.blocks > 128 && p.blocks < 218)
+      p.direct = p.x <= (p.blocks < 160 ? 65536 : 131072);
+  }
+  if (!p.direct) p.splits = dense_splits(M, N, K);
+  p.per = (kblocks + p.splits - 1) / p.splits;
+  p.splits = (kblocks + p.per - 1) / p.per;
+  return p;
+}
+// Row-major weights, of whose rows a direct block reads 256 bytes at once: with x on top of that the staged kernel is the faster one
+// earlier.  Not where rows lie a power of two apart, which costs the staged kernel more (us, direct and staged): 16 rows,
+// 2560 x 65536 75.9 and 62.4, 5120 x 65536 149 and 116, but 4096 x 65536 112 and 118, one row 91 and 122.  Lines as above: 1.5 times
+// as slow as before at worst without them, 1.15 with them, on average 1.34 times faster; without a workspace 1.25, 1.09 and 2.1.
+// A call that is direct on one layout only has other last bits there.
+static bool dense_rows_direct(const DensePlan& p, int M, int N, int K, int64_t w_stride) {
+  const bool apart = (w_stride & (w_stride - 1)) == 0;
+  if (!p.direct || (N >= 49152 && (M > 16 || (!apart && p.x > 18432)))) return false;
+  if (N > 8192 && dense_short_round(p.blocks, 0.76) && (p.x > 49152 || K > (p.blocks > 256 ? 3072 : 8192))) return false;
+  return !(N > 20480 && !apart && p.x > 65536);
+}
+static bool dense_rows_whole(int M, int N, int K, int64_t w_stride) {  // unsplit, up to 16 rows
+  const int64_t x = (int64_t)M * K;
+  return (w_stride & (w_stride - 1)) == 0 || N < 8192 || x <= (N >= 40960 ? (M >= 8 ? 18432 : 49152) : N >= 24576 ? 65536 : 131072);
 }
 
 template <typename T, int MT, int CS, int WAYS, bool PACKED>
@@ -362,11 +395,42 @@ static int launch_dense_direct(const DenseDirectArgs& a, int splits, hipStream_t
 // 896, one row and eight: 41.4 and 44.4, with sixteen 48.7 and 56.5, staged 45.2 and 45.9).  From nine rows on, for outputs that
 // fill the units so, 64 columns (16 rows: 57.5 and 62; 128256 x 4096 164 and 177).
 static bool dense_direct_whole(int M, int N) { return M <= 16 && N >= 512 && N % 16 == 0 && !getenv("SGLK_DENSE_NS"); }
+// Row-major weights of short rows have two strips a block from five rows on, in the same order (8 rows, 1536 x 65536 39.1 and 44.4).
 template <typename T, bool PACKED>
 static int launch_dense_whole(const DenseDirectArgs& a, hipStream_t s) {
+  if (!PACKED && a.M > 4 && a.M <= 8 && a.N >= 16384 && a.K < 2048) return launch_dense_tile<T, 1, 2, 8, PACKED>(a, 1, s);
   if (a.M <= 8 && a.N >= 16384 && a.K < 2048) return launch_dense_tile<T, 1, 1, 8, PACKED>(a, 1, s);
   if (a.N < 8192 || (a.M <= 8 && a.N >= 16384)) return launch_dense_tile<T, 1, 1, 16, PACKED>(a, 1, s);
   return a.N < 16384 ? launch_dense_tile<T, 1, 4, 4, PACKED>(a, 1, s) : launch_dense_tile<T, 1, 4, 8, PACKED>(a, 1, s);
+}
+
+// Unsplit, staged: the sums that a single split of the split launches leaves.
+template <typename T>
+static void launch_dense_staged_rows(const void* x, const void* w, const void* bias, void* out, int M, int N, int K, int64_t x_stride,
+                                     int64_t w_stride, int64_t out_stride, hipStream_t s) {
+  const int mblocks = (M + 63) / 64;
+  const char* env = getenv("SGLK_DENSE_NS");  // 1 / 2 forces the strips per wave (tests)
+  const int force = env ? atoi(env) : 0;
+  // two strips per wave halve the activation re-reads; kept for wide outputs only, where the grid still
+  // fills the chip several times over
+  const bool two = force ? force == 2 : N >= 64 * 1024;
+  const dim3 grid(two ? (N + 127) / 128 : (N + 63) / 64, 1, mblocks);
+  hipLaunchKernelGGL((two ? dense_gemm_nt_kernel<T, 2, 2> : K > 128 ? dense_gemm_nt_kernel<T, 1, 4> : dense_gemm_nt_kernel<T, 1, 2>), grid,
+                     dim3(256), 0, s, (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, (uint16_t*)out, (float*)nullptr, M,
+                     mblocks * 64, N, K, K / 128, x_stride, w_stride, out_stride);
+}
+template <typename T>
+static void launch_dense_staged_packed(const void* x, const void* packed, const void* bias, void* out, int M, int N, int K,
+                                       int64_t x_stride, int64_t out_stride, hipStream_t s) {
+  const int mblocks = (M + 63) / 64;
+  // two strips a wave halve what is read of x; one as long as 64 columns a block leave no unit a second block (one strip and two,
+  // 64 rows: 16384 x 2560 20.5 us and 25.0, 18432 x 2560 34.6 and 28.8, 28672 x 4096 56.6 and 45.4; 128 rows: 8192 x 2560 17.6 and
+  // 21.8, 8320 x 4096 46.6 and 35.7, 13824 x 2560 33.9 and 28.7; 192 rows: 6144 x 4096 41.6 and 30.9; 320: 28672 x 4096 240 and 206)
+  const bool two = (N + 127) / 128 * mblocks > 128;
+  const dim3 grid(two ? (N + 127) / 128 : (N + 63) / 64, 1, mblocks);
+  hipLaunchKernelGGL((two ? dense_gemm_nt_kernel<T, 2, 2, true> : K > 128 ? dense_gemm_nt_kernel<T, 1, 4, true> : dense_gemm_nt_kernel<T, 1, 2, true>),
+                     grid, dim3(256), 0, s, (const uint16_t*)x, (const uint16_t*)packed, (const uint16_t*)bias, (uint16_t*)out,
+                     (float*)nullptr, M, mblocks * 64, N, K, K / 128, x_stride, (int64_t)0, out_stride);
 }
 
 }  // namespace sglk
@@ -391,8 +455,7 @@ int sglk_dense_gemm_nt_ws(const void* x, const void* w, const void* bias, void* 
   SGLK_CHECK(M > 0 && N > 0 && K > 0, "dense_gemm_nt: bad shape");
   SGLK_CHECK(K % 128 == 0, "dense_gemm_nt: K=%d must be a multiple of 128", K);
   const DensePlan plan = dense_packed_plan(M, N, K);
-  // (wide row-major weights of more than 16 rows stay staged: 32 rows, 65536 x 2560 74.0 us, direct 88.9; 128256 x 4096 219 and 249)
-  const bool direct = plan.direct && (M <= 16 || N < 65536);
+  const bool direct = dense_rows_direct(plan, M, N, K, w_stride);
   if (direct && N % 16 == 0 && aligned16(x) && aligned16(w) && x_stride % 8 == 0 && w_stride % 8 == 0 &&
       (plan.splits == 1 || (workspace && workspace_bytes >= (int64_t)plan.splits * M * N * (int64_t)sizeof(float) &&
                             aligned16(workspace) && aligned16(out) && out_stride % 8 == 0))) {
@@ -412,6 +475,11 @@ int sglk_dense_gemm_nt_ws(const void* x, const void* w, const void* bias, void* 
   }
   const int splits = dense_splits(M, N, K);
   const int64_t need = sglk_dense_gemm_workspace_bytes(M, N, K);
+  if (splits <= 1 && !direct && aligned16(x) && aligned16(w) && x_stride % 8 == 0 && w_stride % 8 == 0) {
+    SGLK_DISPATCH_HALF(dtype, T, launch_dense_staged_rows<T>(x, w, bias, out, M, N, K, x_stride, w_stride, out_stride, (hipStream_t)stream));
+    SGLK_LAUNCH_CHECK();
+    return SGLK_OK;
+  }
   if (splits <= 1 || !workspace || workspace_bytes < need || !aligned16(workspace) || !aligned16(out) ||
       out_stride % 8 != 0)
     return sglk_dense_gemm_nt(x, w, bias, out, M, N, K, x_stride, w_stride, out_stride, dtype, stream);
@@ -452,30 +520,13 @@ int sglk_dense_gemm_packed(const void* x, const void* packed, const void* bias, 
   SGLK_CHECK(M > 0 && N > 0 && K > 0, "dense_gemm_packed: bad shape");
   SGLK_CHECK(N % 16 == 0 && K % 128 == 0, "dense_gemm_packed: N=%d must be a multiple of 16, K=%d of 128", N, K);
   SGLK_CHECK(aligned16(x) && aligned16(packed) && x_stride % 8 == 0, "dense_gemm_packed: rows must be 16-byte aligned");
-  const int mblocks = (M + 63) / 64;
   if (dense_direct_whole(M, N)) {
     const DenseDirectArgs a{(const uint16_t*)x, (const uint16_t*)packed, (const uint16_t*)bias, (uint16_t*)out, nullptr, M, M, N, K,
                             K / 128,            x_stride,                0,                     out_stride};
     SGLK_DISPATCH_HALF(dtype, T, { return launch_dense_whole<T, true>(a, (hipStream_t)stream); });
   }
-  // two strips a wave halve what is read of x; one as long as 64 columns a block leave no unit a second block (one strip and two,
-  // 64 rows: 16384 x 2560 20.5 us and 25.0, 18432 x 2560 34.6 and 28.8, 28672 x 4096 56.6 and 45.4; 128 rows: 8192 x 2560 17.6 and
-  // 21.8, 8320 x 4096 46.6 and 35.7, 13824 x 2560 33.9 and 28.7; 192 rows: 6144 x 4096 41.6 and 30.9; 320: 28672 x 4096 240 and 206)
-  if ((N + 127) / 128 * mblocks > 128) {
-    dim3 grid((N + 127) / 128, 1, mblocks);
-    SGLK_DISPATCH_HALF(dtype, T,
-                       hipLaunchKernelGGL((dense_gemm_nt_kernel<T, 2, 2, true>), grid, dim3(256), 0, (hipStream_t)stream,
-                                          (const uint16_t*)x, (const uint16_t*)packed, (const uint16_t*)bias,
-                                          (uint16_t*)out, (float*)nullptr, M, mblocks * 64, N, K, K / 128, x_stride,
-                                          (int64_t)0, out_stride));
-  } else {
-    dim3 grid((N + 63) / 64, 1, mblocks);
-    SGLK_DISPATCH_HALF(dtype, T,
-                       hipLaunchKernelGGL((K > 128 ? dense_gemm_nt_kernel<T, 1, 4, true> : dense_gemm_nt_kernel<T, 1, 2, true>), grid, dim3(256), 0, (hipStream_t)stream,
-                                          (const uint16_t*)x, (const uint16_t*)packed, (const uint16_t*)bias,
-                                          (uint16_t*)out, (float*)nullptr, M, mblocks * 64, N, K, K / 128, x_stride,
-                                          (int64_t)0, out_stride));
-  }
+  SGLK_DISPATCH_HALF(dtype, T,
+                     launch_dense_staged_packed<T>(x, packed, bias, out, M, N, K, x_stride, out_stride, (hipStream_t)stream));
   SGLK_LAUNCH_CHECK();
   return SGLK_OK;
 }
@@ -546,6 +597,12 @@ int sglk_dense_gemm_packed_ws(const void* x, const void* packed, const void* bia
                             K / 128,            x_stride,                0,                     out_stride};
     SGLK_DISPATCH_HALF(dtype, T, { return launch_dense_direct<T, true>(a, 1, (hipStream_t)stream); });
   }
+  if (splits == 1 && N % 16 == 0 && K % 128 == 0 && aligned16(x) && aligned16(packed) && x_stride % 8 == 0) {  // likewise
+    SGLK_DISPATCH_HALF(dtype, T,
+                       launch_dense_staged_packed<T>(x, packed, bias, out, M, N, K, x_stride, out_stride, (hipStream_t)stream));
+    SGLK_LAUNCH_CHECK();
+    return SGLK_OK;
+  }
   if (splits <= 1 || !workspace || workspace_bytes < need || !aligned16(workspace) || !aligned16(out) || N % 8 != 0 ||
       out_stride % 8 != 0)
     return sglk_dense_gemm_packed(x, packed, bias, out, M, N, K, x_stride, out_stride, dtype, stream);
@@ -604,32 +661,12 @@ int sglk_dense_gemm_nt(const void* x, const void* w, const void* bias, void* out
   SGLK_CHECK(K % 128 == 0, "dense_gemm_nt: K=%d must be a multiple of 128", K);
   SGLK_CHECK(aligned16(x) && aligned16(w) && x_stride % 8 == 0 && w_stride % 8 == 0,
              "dense_gemm_nt: rows must be 16-byte aligned");
-  const int mblocks = (M + 63) / 64;
-  if (dense_direct_whole(M, N)) {
+  if (dense_direct_whole(M, N) && dense_rows_whole(M, N, K, w_stride)) {
     const DenseDirectArgs a{(const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, (uint16_t*)out, nullptr, M, M, N, K,
                             K / 128,            x_stride,           w_stride,              out_stride};
     SGLK_DISPATCH_HALF(dtype, T, { return launch_dense_whole<T, false>(a, (hipStream_t)stream); });
   }
-  const char* env = getenv("SGLK_DENSE_NS");  // 1 / 2 forces the strips per wave (tests)
-  const int force = env ? atoi(env) : 0;
-  // two strips per wave halve the activation re-reads; kept for wide outputs only, where the grid still
-  // fills the chip several times over
-  const bool two = force ? force == 2 : N >= 64 * 1024;
-  if (two) {
-    dim3 grid((N + 127) / 128, 1, mblocks);
-    SGLK_DISPATCH_HALF(dtype, T,
-                       hipLaunchKernelGGL((dense_gemm_nt_kernel<T, 2, 2>), grid, dim3(256), 0, (hipStream_t)stream,
-                                          (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias,
-                                          (uint16_t*)out, (float*)nullptr, M, mblocks * 64, N, K, K / 128, x_stride,
-                                          w_stride, out_stride));
-  } else {
-    dim3 grid((N + 63) / 64, 1, mblocks);
-    SGLK_DISPATCH_HALF(dtype, T,
-                       hipLaunchKernelGGL((K > 128 ? dense_gemm_nt_kernel<T, 1, 4> : dense_gemm_nt_kernel<T, 1, 2>), grid, dim3(256), 0, (hipStream_t)stream,
-                                          (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias,
-                                          (uint16_t*)out, (float*)nullptr, M, mblocks * 64, N, K, K / 128, x_stride,
-                                          w_stride, out_stride));
-  }
+  SGLK_DISPATCH_HALF(dtype, T, launch_dense_staged_rows<T>(x, w, bias, out, M, N, K, x_stride, w_stride, out_stride, (hipStream_t)stream));
   SGLK_LAUNCH_CHECK();
   return SGLK_OK;
 }

@@ -102,3 +102,38 @@ def test_rows_and_columns_that_are_not_numbers(M, N):
     keep[M - 1] = False
     keep[:, 100] = False
     assert torch.equal(got[keep], clean[keep])
+
+
+@pytest.mark.parametrize("M,N,K", [(25, 5104, 2560), (26, 5104, 2560), (24, 5120, 5376), (25, 5120, 5376), (32, 6992, 4224), (16, 16384, 5120), (12, 16416, 4096),
+                                   (13, 16416, 4096), (1, 16416, 3072), (1, 16416, 3200), (1, 16416, 4224), (16, 22272, 2944), (16, 22288, 4224), (16, 11008, 5120),
+                                   (16, 11008, 5248), (1, 11008, 8192), (1, 11008, 8320), (32, 24576, 4096), (32, 24576, 4224), (16, 49136, 1152), (16, 49152, 1152),
+                                   (16, 49152, 1280), (16, 49152, 2048), (17, 49152, 1152), (5, 16400, 1536), (16, 8192, 6144), (16, 8192, 6272), (7, 40960, 2560),
+                                   (8, 40960, 2560), (16, 20480, 4096), (24, 20480, 4096)])
+def test_sides_of_the_rules(M, N, K):
+    """The last and the first calls of the staged and the direct kernel, on both layouts: right sums on each, and finished rows of the
+    streaming layout are the rounded split sums."""
+    from sglang_security_amd import ops
+
+    g = torch.Generator(device=DEV).manual_seed(M * N + K)
+    x = torch.randn(M, K, generator=g, device=DEV).bfloat16()
+    w = torch.randn(N, K, generator=g, device=DEV).bfloat16()
+    bias = torch.randn(N, generator=g, device=DEV).bfloat16()
+    packed = ops.dense_repack(w)
+    want = x.double() @ w.double().t()
+    bound = (x.double().abs() @ w.double().abs().t()) * 2.0 ** -20     # fp32 sums of K products
+    splits = ops.dense_gemm_partial_splits(M, N, K)
+    part = torch.full((splits, M, N), float("nan"), device=DEV)
+    assert ops.dense_gemm_packed_partial(x, packed, part) == splits
+    total = part[0]
+    for p in part[1:]:
+        total = total + p
+    assert ((total.double() - want).abs() <= bound).all()
+    ws = torch.empty(max(splits * M * N, 4), device=DEV)
+    finished = ops.dense_gemm_packed_ws(x, packed, bias, torch.empty(M, N, dtype=torch.bfloat16, device=DEV), ws)
+    assert torch.equal(finished, (total + bias.float()).bfloat16())
+    want += bias.double()
+    tol = want.abs() * 2.0 ** -8 + 2 * bound
+    need = max(ops.dense_gemm_workspace_bytes(M, N, K), 16)
+    for got in (ops.dense_gemm_packed(x, packed, bias), ops.dense_gemm_nt(x, w, bias),
+                ops.dense_gemm_nt(x, w, bias, None, torch.empty(need, dtype=torch.uint8, device=DEV))):
+        assert ((got.double() - want).abs() <= tol).all()
