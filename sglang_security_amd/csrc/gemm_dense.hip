@@ -15,8 +15,7 @@
 // everything at each k-block's barrier -> 24.3; 14336 x 4096 110 -> 76; 28672 x 4096 57 -> 45; 16384 x 2560, with one
 // strip a wave as well, 33 -> 22; 128256 x 4096, where many blocks a unit had covered those waits, 190 -> 192, 5.5 TB/s:
 // neither deeper rings, 256 columns a block nor k-blocks begun at different places changed that one).
-// A k-block that is not there is asked for all the same, so a single one (K = 128) has the shorter ring: 64 rows, 512 and 4096
-// columns, row-major 4.5 -> 3.3 and 4.9 -> 3.7 us.
+// A k-block that is not there is asked for all the same, so the ring is no longer than a block's k-blocks (dense_staged).
 #include <algorithm>
 #include <cstdlib>
 
@@ -113,7 +112,7 @@ __global__ void __launch_bounds__(256, 2) dense_gemm_nt_kernel(const uint16_t* _
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) oacc[s][mt] = float4v{0.f, 0.f, 0.f, 0.f};
 
-  static_assert(PF % 2 == 0, "the halves of LDS go by the parity of the k-block");
+  static_assert(PF == 1 || PF % 2 == 0, "the halves of LDS go by the parity of the k-block (PF 1: there is one)");
 #pragma unroll
   for (int p = 0; p < PF; ++p) {
     x_fetch(xreg[p], kb0 + min(p, nkb - 1));
@@ -404,6 +403,13 @@ static int launch_dense_whole(const DenseDirectArgs& a, hipStream_t s) {
   return a.N < 16384 ? launch_dense_tile<T, 1, 4, 4, PACKED>(a, 1, s) : launch_dense_tile<T, 1, 4, 8, PACKED>(a, 1, s);
 }
 
+// The staged kernel for blocks of `per` k-blocks: its ring asks for no more than there are (us, ring of four and of two, 64 rows: 256 x
+// 17088 8.6 and 6.0; 256 x 46208, split sums 14.8 and 10.0).
+template <typename T, int NS, bool PACKED>
+static auto dense_staged(int per) {
+  auto* kernel = per > 3 && NS == 1 ? dense_gemm_nt_kernel<T, NS, NS == 1 ? 4 : 2, PACKED> : dense_gemm_nt_kernel<T, NS, 2, PACKED>;
+  return per == 1 ? dense_gemm_nt_kernel<T, NS, 1, PACKED> : kernel;
+}
 // Unsplit, staged: the sums that a single split of the split launches leaves.
 template <typename T>
 static void launch_dense_staged_rows(const void* x, const void* w, const void* bias, void* out, int M, int N, int K, int64_t x_stride,
@@ -415,8 +421,7 @@ static void launch_dense_staged_rows(const void* x, const void* w, const void* b
   // fills the chip several times over
   const bool two = force ? force == 2 : N >= 64 * 1024;
   const dim3 grid(two ? (N + 127) / 128 : (N + 63) / 64, 1, mblocks);
-  hipLaunchKernelGGL((two ? dense_gemm_nt_kernel<T, 2, 2> : K > 128 ? dense_gemm_nt_kernel<T, 1, 4> : dense_gemm_nt_kernel<T, 1, 2>), grid,
-                     dim3(256), 0, s, (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, (uint16_t*)out, (float*)nullptr, M,
+  hipLaunchKernelGGL((two ? dense_staged<T, 2, false>(K / 128) : dense_staged<T, 1, false>(K / 128)), grid, dim3(256), 0, s, (const uint16_t*)x, (const uint16_t*)w, (const uint16_t*)bias, (uint16_t*)out, (float*)nullptr, M,
                      mblocks * 64, N, K, K / 128, x_stride, w_stride, out_stride);
 }
 template <typename T>
@@ -428,8 +433,7 @@ static void launch_dense_staged_packed(const void* x, const void* packed, const 
   // 21.8, 8320 x 4096 46.6 and 35.7, 13824 x 2560 33.9 and 28.7; 192 rows: 6144 x 4096 41.6 and 30.9; 320: 28672 x 4096 240 and 206)
   const bool two = (N + 127) / 128 * mblocks > 128;
   const dim3 grid(two ? (N + 127) / 128 : (N + 63) / 64, 1, mblocks);
-  hipLaunchKernelGGL((two ? dense_gemm_nt_kernel<T, 2, 2, true> : K > 128 ? dense_gemm_nt_kernel<T, 1, 4, true> : dense_gemm_nt_kernel<T, 1, 2, true>),
-                     grid, dim3(256), 0, s, (const uint16_t*)x, (const uint16_t*)packed, (const uint16_t*)bias, (uint16_t*)out,
+  hipLaunchKernelGGL((two ? dense_staged<T, 2, true>(K / 128) : dense_staged<T, 1, true>(K / 128)), grid, dim3(256), 0, s, (const uint16_t*)x, (const uint16_t*)packed, (const uint16_t*)bias, (uint16_t*)out,
                      (float*)nullptr, M, mblocks * 64, N, K, K / 128, x_stride, (int64_t)0, out_stride);
 }
 
@@ -491,7 +495,7 @@ int sglk_dense_gemm_nt_ws(const void* x, const void* w, const void* bias, void* 
   dim3 grid((N + 63) / 64, used, mblocks);
   hipStream_t s = (hipStream_t)stream;
   SGLK_DISPATCH_HALF(dtype, T, {
-    hipLaunchKernelGGL((K > 128 ? dense_gemm_nt_kernel<T, 1, 4> : dense_gemm_nt_kernel<T, 1, 2>), grid, dim3(256), 0, s, (const uint16_t*)x, (const uint16_t*)w,
+    hipLaunchKernelGGL((dense_staged<T, 1, false>(per)), grid, dim3(256), 0, s, (const uint16_t*)x, (const uint16_t*)w,
                        (const uint16_t*)nullptr, (uint16_t*)nullptr, (float*)workspace, M, mblocks * 64, N, K, per,
                        x_stride, w_stride, out_stride);
     const int64_t vecs = (int64_t)M * (N / 8);
@@ -559,13 +563,13 @@ static int dense_packed_split_launch(const void* x, const void* packed, float* p
   if (two) {
     dim3 grid((N + 127) / 128, used, (M + 63) / 64);
     SGLK_DISPATCH_HALF(dtype, T,
-                       hipLaunchKernelGGL((dense_gemm_nt_kernel<T, 2, 2, true>), grid, dim3(256), 0, s, (const uint16_t*)x,
+                       hipLaunchKernelGGL((dense_staged<T, 2, true>(per)), grid, dim3(256), 0, s, (const uint16_t*)x,
                                           (const uint16_t*)packed, (const uint16_t*)nullptr, (uint16_t*)nullptr, partial,
                                           M, Mpad, N, K, per, x_stride, (int64_t)0, (int64_t)0));
   } else {
     dim3 grid((N + 63) / 64, used, (M + 63) / 64);
     SGLK_DISPATCH_HALF(dtype, T,
-                       hipLaunchKernelGGL((K > 128 ? dense_gemm_nt_kernel<T, 1, 4, true> : dense_gemm_nt_kernel<T, 1, 2, true>), grid, dim3(256), 0, s, (const uint16_t*)x,
+                       hipLaunchKernelGGL((dense_staged<T, 1, true>(per)), grid, dim3(256), 0, s, (const uint16_t*)x,
                                           (const uint16_t*)packed, (const uint16_t*)nullptr, (uint16_t*)nullptr, partial,
                                           M, Mpad, N, K, per, x_stride, (int64_t)0, (int64_t)0));
   }

@@ -137,3 +137,21 @@ def test_sides_of_the_rules(M, N, K):
     for got in (ops.dense_gemm_packed(x, packed, bias), ops.dense_gemm_nt(x, w, bias),
                 ops.dense_gemm_nt(x, w, bias, None, torch.empty(need, dtype=torch.uint8, device=DEV))):
         assert ((got.double() - want).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("M", [33, 64, 130])
+@pytest.mark.parametrize("N,kblocks", [(1040, 1), (1040, 2), (1040, 3), (16640, 1), (65536, 1), (65536 + 16, 2), (65536, 3)])
+def test_split_sums_of_few_k_blocks(M, N, kblocks):
+    """Rings of one, two and four k-blocks, one and two strips a wave, where the sums stay in 32 bits."""
+    from sglang_security_amd import ops
+
+    K = 128 * kblocks
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x, w = (torch.randn(r, K, generator=g, device=DEV).bfloat16() for r in (M, N))
+    splits = ops.dense_gemm_partial_splits(M, N, K)
+    part = torch.full((splits, M, N), float("nan"), device=DEV)
+    assert ops.dense_gemm_packed_partial(x, ops.dense_repack(w), part) == splits
+    bound = (x.double().abs() @ w.double().abs().t()) * 2.0 ** -21      # fp32 sums of K products
+    assert ((part.double().sum(0) - x.double() @ w.double().t()).abs() <= bound).all()
+    rows = ops.dense_gemm_nt(x, w)
+    assert torch.equal(rows, ops.dense_gemm_packed(x, ops.dense_repack(w)))
