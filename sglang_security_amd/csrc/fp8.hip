@@ -936,8 +936,9 @@ struct Fp8Direct {
 };
 static Fp8Direct fp8_direct_plan(int M, int N, int K, int most = 8) {
   const int kblocks = K / 128, strips = N / 16;
-  Fp8Direct plan{M <= 64, 1, kblocks, true};
-  if (M > 64) {
+  // (a single k-block of more than 32 rows: the staged kernel would ask for four of x; 128 x 26864, 64 rows 4.5 us and 7.1)
+  Fp8Direct plan{M <= 32 || (M <= 64 && kblocks > 1), 1, kblocks, true};
+  if (!plan.ok) {
     plan.splits = fp8_stream_splits(M, N, K);
   } else if (strips < 1024) {
     const char* env = getenv("SGLK_FP8_STREAM_SPLITS");
@@ -976,7 +977,8 @@ int launch_fp8_direct(const Fp8DirectArgs& a, const Fp8Direct& plan, hipStream_t
     hipLaunchKernelGGL((fp8_staged_kernel<TO, SB, PW>), dim3((strips + SB - 1) / SB, splits), dim3(512), fp8_staged_lds<SB>(), s, a); \
   }
   if (a.M > 32) {
-    if (strips >= 1024) SGLK_FP8_STAGED(4, 2) else SGLK_FP8_STAGED(2, 4)
+    // (weights four stages of four k-blocks ahead, where there are more than two)
+    if (strips >= 1024) SGLK_FP8_STAGED(4, 2) else if (plan.per > 8) SGLK_FP8_STAGED(2, 4) else SGLK_FP8_STAGED(2, 2)
   } else if (a.M > 16) {
     if (strips >= 1024) SGLK_FP8_DIRECT(2, 4, 8, 1) else if (pairs) SGLK_FP8_DIRECT(2, 2, 8, 1) else SGLK_FP8_DIRECT(2, 1, 16, 1)
   } else {

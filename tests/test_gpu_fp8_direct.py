@@ -65,3 +65,10 @@ def test_codes_that_are_not_numbers_stay_in_their_rows_and_columns(M):
     keep[M - 1] = False
     keep[:, 100] = False
     assert torch.equal(got[keep], clean[keep])
+
+
+@pytest.mark.parametrize("M", [33, 64])
+@pytest.mark.parametrize("K", [128, 256, 512, 1024, 1152])
+def test_few_stages(M, K):
+    """More than 32 rows of one k-block, of two, of one stage, two and three: the weights' ring is no longer than that."""
+    test_products(M, 1040, K, torch.bfloat16)
