@@ -1,5 +1,5 @@
-// 16-bit products of at most 32 rows, on the streaming weight layout (sglk_dense_repack) and, with the same bits, on row-major
-// weights (included by gemm_dense.hip).
+// 16-bit products of at most 32 rows, those that gemm_dense.hip's rules leave to this kernel, on the streaming weight layout
+// (sglk_dense_repack) and, with the same bits, on row-major weights (included by gemm_dense.hip).
 //
 // Bound by the weights' way from memory.  The staged kernel shares x through LDS and meets at a barrier every 128 of k, two to
 // four k-blocks a wave on their way; with so few rows x is a fraction of the weights, so nothing is staged here: a block's

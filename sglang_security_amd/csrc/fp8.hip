@@ -977,7 +977,8 @@ int launch_fp8_direct(const Fp8DirectArgs& a, const Fp8Direct& plan, hipStream_t
     hipLaunchKernelGGL((fp8_staged_kernel<TO, SB, PW>), dim3((strips + SB - 1) / SB, splits), dim3(512), fp8_staged_lds<SB>(), s, a); \
   }
   if (a.M > 32) {
-    // (weights four stages of four k-blocks ahead, where there are more than two)
+    // (weights four stages of four k-blocks ahead, where there are more than two: 64 rows, 512 x 15328 6.7 us -> 5.8, 640 x 10224 7.3
+    // -> 6.6)
     if (strips >= 1024) SGLK_FP8_STAGED(4, 2) else if (plan.per > 8) SGLK_FP8_STAGED(2, 4) else SGLK_FP8_STAGED(2, 2)
   } else if (a.M > 16) {
     if (strips >= 1024) SGLK_FP8_DIRECT(2, 4, 8, 1) else if (pairs) SGLK_FP8_DIRECT(2, 2, 8, 1) else SGLK_FP8_DIRECT(2, 1, 16, 1)
