@@ -1141,7 +1141,17 @@ __global__ void __launch_bounds__(kSampThreads) slice_apply_kernel(SampArgs a) {
   });
 }
 
-// A block a row: the choice where it is sampled from, and the rows that the guess did not hold for.
+// Renormalised rows that the guess did not hold for, a block a row (48 rows of 256000 nearly equal values 126 us; 132 in the
+// kernel that samples, whose registers it shared).
+template <bool VEC>
+__global__ void __launch_bounds__(kSampThreads) slice_redo_kernel(SampArgs a) {
+  __shared__ SampShared sh;
+  const int row = blockIdx.x;
+  if (samp_ws(a, row).state->valid) return;
+  renorm_row<VEC, true>(a.probs + (int64_t)row * a.in_stride, a.out + (int64_t)row * a.out_stride, a.n, load_params(a, row), sh);
+}
+
+// A block a row that is sampled from: the choice, and all of it where the guess did not hold.
 template <bool VEC, bool FILTER>
 __global__ void __launch_bounds__(kSampThreads) slice_choose_kernel(SampArgs a) {
   __shared__ SampShared sh;
@@ -1149,10 +1159,6 @@ __global__ void __launch_bounds__(kSampThreads) slice_choose_kernel(SampArgs a) 
   const float* x = a.probs + (int64_t)row * a.in_stride;
   const SampWs w = samp_ws(a, row);
   const RowParams rp = load_params(a, row);
-  if (a.out) {
-    if (!w.state->valid) renorm_row<VEC, true>(x, a.out + (int64_t)row * a.out_stride, a.n, rp, sh);
-    return;
-  }
   constexpr int PER = kBins / kSampThreads;
   const int chunks = (a.n + 255) / 256;
   HeldLists lists, places;
@@ -1247,10 +1253,11 @@ static int launch_filters(SampArgs a, int batch, void* workspace, int64_t worksp
   if (a.out) {
     hipLaunchKernelGGL((vec ? slice_collect_kernel<true, false, true> : slice_collect_kernel<false, false, true>), grid, block, 0, s, a);
     hipLaunchKernelGGL(vec ? slice_apply_kernel<true> : slice_apply_kernel<false>, grid, block, 0, s, a);
+    hipLaunchKernelGGL(vec ? slice_redo_kernel<true> : slice_redo_kernel<false>, dim3(batch), block, 0, s, a);
   } else {
     hipLaunchKernelGGL((vec ? slice_collect_kernel<true, true, true> : slice_collect_kernel<false, true, true>), grid, block, 0, s, a);
+    hipLaunchKernelGGL((vec ? slice_choose_kernel<true, true> : slice_choose_kernel<false, true>), dim3(batch), block, 0, s, a);
   }
-  hipLaunchKernelGGL((vec ? slice_choose_kernel<true, true> : slice_choose_kernel<false, true>), dim3(batch), block, 0, s, a);
   SGLK_LAUNCH_CHECK();
   return SGLK_OK;
 }
