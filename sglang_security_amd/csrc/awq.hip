@@ -24,6 +24,7 @@
 
 #include "awq_common.h"
 #include "awq_rows16.h"
+#include "awq_tall.h"
 
 namespace sglk {
 
@@ -1526,7 +1527,7 @@ static int static_prepare_kernels() {
   if (int rc = ensure_lds<&awq_gemm_kernel<T, 4, 1, 4>>(GemmGeom<4, 1, 4>::kLds)) return rc;
   if (int rc = ensure_lds<&awq_gemm_kernel<T, 8, 1, 6>>(GemmGeom<8, 1, 6>::kLds)) return rc;
   if (int rc = ensure_lds<&awq_gemm_kernel<T, 8, 1, 4>>(GemmGeom<8, 1, 4>::kLds)) return rc;
-  return SGLK_OK;
+  return prepare_awq_tall();
 }
 
 
@@ -1724,6 +1725,13 @@ int sglk_awq_gemm_silu_mul(const void* x, const int32_t* packed, const void* sca
   SGLK_CHECK(out_stride >= N / 2, "awq_gemm_silu_mul: out_stride smaller than N/2");
   SGLK_CHECK(!xsum || xs_stride >= M, "awq_gemm_silu_mul: xs_stride smaller than M");
   SGLK_CHECK(!xsum_out || xs_out_stride >= M, "awq_gemm_silu_mul: xs_out_stride smaller than M");
+  // the activation needs whole sums: one split, whatever the planner would pick
+  if (const TallPlan tp = plan_awq_tall(M, N, K, group_size, dtype, true); tp.ok && x_stride < kTallMaxStride)
+    return launch_awq_tall(tp,
+                           AwqTallArgs{(const uint16_t*)x, packed, (const uint16_t*)scales, qzeros, nullptr, (uint16_t*)out,
+                                       nullptr, nullptr, xsum, xsum_out, x_stride, out_stride, xs_stride, xs_out_stride, M, N, K,
+                                       0, 0, 1, 0},
+                           (hipStream_t)stream);
   WidePlan wp = plan_awq_wide(M, N, K, group_size, true);
   if (!wp.ok)
     return fail(SGLK_EUNSUP, "awq_gemm_silu_mul: needs K %% 512 == 0 and group size 128 (K=%d G=%d)", K, group_size);
@@ -1852,6 +1860,16 @@ int sglk_awq_gemm_xs(const void* x, const int32_t* packed, const void* scales, c
   hipStream_t s = (hipStream_t)stream;
   int* tickets = reinterpret_cast<int*>(workspace);
   float* partial = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + (int64_t)kMaxTiles * 4);
+  if (M > kGemmBM) {
+    const TallPlan tp = plan_awq_tall(M, N, K, group_size, dtype, false,
+                                      sglk_awq_gemm_workspace_bytes(M, N, K) - (int64_t)kMaxTiles * 4);
+    if (tp.ok && tp.tiles <= kMaxTiles && x_stride < kTallMaxStride)
+      return launch_awq_tall(tp,
+                             AwqTallArgs{(const uint16_t*)x, packed, (const uint16_t*)scales, qzeros, (const uint16_t*)bias,
+                                         (uint16_t*)out, partial, tickets, xsum, nullptr, x_stride, out_stride, xs_stride, 0, M,
+                                         N, K, 0, 0, 0, 0},
+                             s);
+  }
   const WidePlan wp = plan_awq_wide(M, N, K, group_size);
   // few rows: also where a split is a single stage, as long as the slabs (a quarter of the wide kernel's) fit the workspace
   // that sglk_awq_gemm_workspace_bytes names
