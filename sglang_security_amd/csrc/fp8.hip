@@ -679,7 +679,7 @@ template <typename TO, int BM, int BN, int WM, int WN, int ST>
 int launch_fp8_tile(const MmArgs& p, hipStream_t s) {
   constexpr int lds = ST * (BM + BN) * 128;
   if (int rc = ensure_lds<fp8_tile_kernel<TO, BM, BN, WM, WN, ST>>(lds)) return rc;
-  const Fp8TileArgs t{p.a, p.b, p.sa, p.sb, p.bias, p.out, p.M, p.N, p.K, (p.M + BM - 1) / BM, (p.N + BN - 1) / BN,
+  const Fp8TileArgs t{p.a, p.b, p.sa, p.sb, p.bias, p.out, p.M, p.N, p.K, (p.M + BM - 1) / BM, (p.N + BN - 1) / BN, 0, 0,
                       p.a_stride, p.b_stride, p.out_stride};
   hipLaunchKernelGGL((fp8_tile_kernel<TO, BM, BN, WM, WN, ST>), dim3((unsigned)t.mt * t.nt), dim3(64 * WM * WN), lds, s, t);
   SGLK_LAUNCH_CHECK();
@@ -688,15 +688,44 @@ int launch_fp8_tile(const MmArgs& p, hipStream_t s) {
 
 static int fp8_stream_splits(int M, int N, int K);
 
+// Strips of a product on blocks of 256 rows: 256 columns wide while they fill whole rounds of 256 units; what is left over, if it
+// would fill no more than three quarters of a round, in strips of 192 or 128.
+struct Fp8Strips {
+  int mt, whole, tail, narrow;  // row tiles, strips of 256 columns, strips of `narrow` columns behind them
+};
+static Fp8Strips fp8_strips(int64_t M, int64_t N) {
+  const int64_t mt = (M + 255) / 256, all = (N + 255) / 256, whole = mt * all / 256 * 256 / mt;
+  for (int narrow : {128, 192}) {
+    const int64_t tail = (N - whole * 256 + narrow - 1) / narrow;
+    if (whole < all && mt * tail <= 256) return {(int)mt, (int)whole, (int)tail, narrow};
+  }
+  return {(int)mt, (int)all, 0, 128};
+}
+
+template <typename TO>
+int launch_fp8_tile4(const MmArgs& p, hipStream_t s) {
+  constexpr int lds = (2 * 256 + 3 * 256) * 128;
+  if (int rc = ensure_lds<fp8_tile4_kernel<TO>>(lds)) return rc;
+  const Fp8Strips st = fp8_strips(p.M, p.N);
+  const Fp8TileArgs t{p.a, p.b, p.sa, p.sb, p.bias, p.out, p.M, p.N, p.K, st.mt, st.whole, st.tail, st.narrow,
+                      p.a_stride, p.b_stride, p.out_stride};
+  hipLaunchKernelGGL((fp8_tile4_kernel<TO>), dim3((unsigned)st.mt * (st.whole + st.tail)), dim3(256), lds, s, t);
+  SGLK_LAUNCH_CHECK();
+  return SGLK_OK;
+}
+
 enum class Fp8Other { kRegister, kSplit, kStreaming };  // what a call falls back on; a later one could also take the earlier
 
 // Which tile form multiplies [M, K] x [N, K] fastest (0: none, the call falls back on `other`).  Estimates in
-// microseconds, fitted to launches on weights that come from memory: a tile form needs its time per k-block of 128 for
-// every round of blocks; the others take the lesser of an estimate by work and one by rounds (narrow outputs spread K
-// over idle units, which the tiles do not).  Measured against the register kernel, the split and the streaming one:
+// microseconds, fitted to launches on weights that come from memory: a tile form needs its start and end and its time per
+// k-block of 128 for every round of blocks; the others take the lesser of an estimate by work and one by rounds (narrow outputs
+// spread K over idle units, which the tiles do not).  Measured against the register kernel, the split and the streaming one:
 //   N, K of the 8B model's projections and of the 70B model's on one of eight ranks, M = 1 .. 2048: 2048 x 28672 x 4096
-//   1190 -> 214 (streaming 788); 2048 x 4096 x 14336 593 -> 110 (349); 256 x 4096 x 14336 79 -> 37 (68); 128 x 28672 x
+//   1190 -> 181 (streaming 788); 2048 x 4096 x 14336 593 -> 95 (349); 256 x 4096 x 14336 79 -> 37 (68); 128 x 28672 x
 //   4096 83 -> 33 (57); 128 x 4096 x 4096 14.6 -> 12.9 (16.5); 64 x 28672 x 4096 without the streaming copy 50 -> 30;
+//   between the forms, the same projections at 18 sizes from 65 to 2048 rows: no choice is slower than the fastest form by more
+//   than a tenth.  Four waves against the older forms: 2048 x 6144 x 4096 50 -> 42, 2048 x 4096 x 4096 40 -> 32, 1300 x 7168 x 8192
+//   88 -> 67, 700 x 28672 x 4096 97 -> 79; eight waves stay where a full round has few k-blocks: 2048 x 8192 x 1024 20 and 21.
 //   M = 33 .. 2048, N = 32 .. 8192, K = 512 .. 14336, 1008 sizes: no call on tiles is slower than its fallback by more
 //   than 4 % (33 x 6144 x 14336), none that stays would gain more than 11 % (the same, against the split kernel).
 //   Narrow ones that stay: 1024 x 128 x 14336 split 18.9, streaming 15.8, tiled 30.9; 512 x 256 x 7168 13.8, 11.8, 17.4.
@@ -709,12 +738,17 @@ static int fp8_tile_choice(int64_t M, int64_t N, int64_t K, Fp8Other other) {
   auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   auto rounds = [&](int bm, int bn, int per_round) { return (double)up(up(M, bm) * up(N, bn), per_round); };
   const double small = M <= 64 && N >= 8192 ? 0.35 : 0.28;  // one row of blocks: 128 units ask memory for all the weights
-  const double cost[5] = {1.35 * rounds(256, 256, 256), 1.05 * rounds(128, 128, 512), 0.56 * rounds(128, 128, 256),
-                          0.42 * rounds(64, 128, 256), small * rounds(64, 64, 256)};
+  const double kb = (double)K / 128;
+  const Fp8Strips st = fp8_strips(M, N);
+  const double wide = (double)up((int64_t)st.mt * st.whole, 256) * (13 + 1.18 * kb) +
+                      (st.tail == 0 ? 0.0 : st.narrow == 128 ? 9.5 + 0.79 * kb : 11 + 1.1 * kb);
+  const double cost[6] = {3 + rounds(256, 256, 256) * (7 + 1.4 * kb), rounds(128, 128, 512) * (5.4 + 1.07 * kb),
+                          1.5 + rounds(128, 128, 256) * (3.2 + 0.58 * kb), 1.65 + rounds(64, 128, 256) * (1.5 + 0.42 * kb),
+                          2.5 + rounds(64, 64, 256) * (0.6 + small * kb),  wide};
   int best = 0;
-  for (int i = 1; i < 5; ++i)
+  for (int i = 1; i < 6; ++i)
     if (cost[i] < cost[best]) best = i;
-  const double tiled = cost[best] * (K / 128) + 3.15, passes = (double)up(M, 64), mb = (double)N * K * 1e-6;
+  const double tiled = cost[best], passes = (double)up(M, 64), mb = (double)N * K * 1e-6;
   auto by_rounds = [&](int splits, int bn, double per_block, double partial) {  // partial: us a million sums left by a split
     const double per = (double)up(K / 128, splits), blocks = (double)up(N, bn) * passes * splits;
     return (splits > 1 ? 1.3 + partial * 1e-6 * splits * M * N : 0.0) + per_block * per * std::max(1.0, blocks / 256);
@@ -743,7 +777,8 @@ int launch_fp8_tiled(int form, const MmArgs& p, hipStream_t s) {
     case 2: return launch_fp8_tile<TO, 128, 128, 2, 2, 2>(p, s);  // two
     case 3: return launch_fp8_tile<TO, 128, 128, 2, 2, 4>(p, s);  // one, three stages ahead
     case 4: return launch_fp8_tile<TO, 64, 128, 1, 4, 6>(p, s);
-    default: return launch_fp8_tile<TO, 64, 64, 1, 2, 4>(p, s);
+    case 5: return launch_fp8_tile<TO, 64, 64, 1, 2, 4>(p, s);
+    default: return launch_fp8_tile4<TO>(p, s);
   }
 }
 

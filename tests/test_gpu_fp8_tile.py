@@ -32,6 +32,14 @@ def test_scaled_products_of_many_rows(M, N, K, dtype, bias):
         assert out is None or out._base[:, N:].isnan().all()      # what lies between the rows stays
 
 
+# four waves a block: strips of 192 columns alone, of 128 alone, of 256 alone, of 256 with 128 and with 192 behind them; rows and
+# columns that do not fill them, an odd and an even number of k-blocks
+@pytest.mark.parametrize("M,N,K,bias", [(2048, 6144, 1024, False), (2047, 4112, 1152, True), (700, 6160, 2048, False),
+                                        (1700, 8192, 3584, True), (2048, 8208, 2048, False), (1300, 28688, 4096, True)])
+def test_blocks_of_four_waves(M, N, K, bias):
+    test_scaled_products_of_many_rows(M, N, K, torch.bfloat16, bias)
+
+
 def test_rule_covers_decode_and_prompts():
     """Single rows stay on the kernels that stream; prompts go to the tiles, with and without the streaming copy."""
     from sglang_security_amd import ops
