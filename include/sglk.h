@@ -609,8 +609,8 @@ SGLK_API int sglk_decode_attention_shared_prefix_rope(
 SGLK_API int sglk_dense_gemm_nt(const void* x, const void* w, const void* bias, void* out, int M, int N,
                                 int K, int64_t x_stride, int64_t w_stride, int64_t out_stride,
                                 int dtype, void* stream);
-/* Large-M (extend / prefill) products, out[M, N] = x[M, K] @ W (+ bias) on 256 x 128 output tiles with
- * v_mfma_f32_32x32x16 and two LDS stages.  sglk_awq_gemm_prefill dequantises the packed int4 weight on the way into
+/* Large-M (extend / prefill) products, out[M, N] = x[M, K] @ W (+ bias) on tiles of up to 256 x 256 with
+ * v_mfma_f32_32x32x16.  sglk_awq_gemm_prefill dequantises the packed int4 weight on the way into
  * LDS -- (q - z) * scale rounded to the activation type, i.e. exactly the matrix the reference's
  * awq_dequantize-then-matmul multiplies by (python/sglang/srt/layers/quantization/awq.py:197-215) -- so no
  * dequantised copy is written to memory; sglk_dense_gemm_prefill takes a 16-bit weight [N, K].
@@ -618,6 +618,8 @@ SGLK_API int sglk_dense_gemm_nt(const void* x, const void* w, const void* bias, 
 SGLK_API int sglk_awq_gemm_prefill(const void* x, const int32_t* packed, const void* scales, const int32_t* qzeros,
                                    const void* bias, void* out, int M, int N, int K, int group_size,
                                    int64_t x_stride, int64_t out_stride, int dtype, void* stream);
+/* Whether sglk_awq_gemm_prefill is expected to be faster than a dequantisation to memory and a library product. */
+SGLK_API int sglk_awq_prefill_fused(int M, int N, int K);
 SGLK_API int sglk_dense_gemm_prefill(const void* x, const void* w, const void* bias, void* out, int M, int N, int K,
                                      int64_t x_stride, int64_t w_stride, int64_t out_stride, int dtype,
                                      void* stream);

@@ -3,37 +3,15 @@
 //     ((q - z) * scale rounded to the activation type: the very weights the reference's
 //     awq_dequantize-then-matmul multiplies by, python/sglang/srt/layers/quantization/awq.py:197-215), and
 //   * dense 16-bit weights [N, K] (bf16 / fp16 checkpoints: layers/linear.py UnquantizedLinearMethod).
-//
-// A block of four waves owns a 256 x 128 output tile and walks K in steps of 32 through two LDS stages
-// (A: 256 rows x 64 bytes, B: 128 columns x 64 bytes, k contiguous in both, 16-byte chunks XOR-swizzled by
-// (row >> 2) & 3 so that the eight lanes a 16-byte LDS read serves at a time fall on eight different bank
-// groups).  Wave (wm, wn) multiplies rows [128 wm, +128) by columns [64 wn, +64): 4 x 2 tiles of
-// v_mfma_f32_32x32x16, 128 accumulator registers, six operand reads (6 KiB) per eight matrix instructions.
-// The next stage's rows travel global -> registers while the current one is multiplied, and are parked (the
-// int4 words dequantised first) before the one barrier per stage.  The output tile is transposed through LDS
-// so that it leaves in 16-byte row pieces.
+// prefill_tile.h holds the kernel.  The one below serves rows whose pitch is beyond its 32-bit offsets: a block of four waves owns a
+// 256 x 128 output tile and walks K in steps of 32 through two LDS stages (A: 256 rows x 64 bytes, B: 128 columns x 64 bytes, k
+// contiguous in both, 16-byte chunks XOR-swizzled by (row >> 2) & 3); rows travel global -> registers while the current stage is
+// multiplied, and are parked (the int4 words dequantised first) before the one barrier per stage.
 #include <algorithm>
 
-#include "common.h"
+#include "prefill_tile.h"
 
 namespace sglk {
-
-template <typename T>
-struct Mfma32;
-template <>
-struct Mfma32<bf16_t> {
-  static __device__ __forceinline__ float16v mma(int4v a, int4v b, float16v c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bfloat8, a), __builtin_bit_cast(bfloat8, b), c, 0,
-                                                   0, 0);
-  }
-};
-template <>
-struct Mfma32<f16_t> {
-  static __device__ __forceinline__ float16v mma(int4v a, int4v b, float16v c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0,
-                                                  0);
-  }
-};
 
 static constexpr int kPfBM = 256, kPfBN = 128, kPfBK = 32;
 static constexpr int kPfABytes = kPfBM * 64, kPfBBytes = kPfBN * 64;
@@ -171,7 +149,7 @@ __global__ void __launch_bounds__(256, 2) prefill_gemm_kernel(
 #pragma unroll
       for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt) acc[mt][nt] = Mfma32<T>::mma(af[mt], bf[nt], acc[mt][nt]);
+        for (int nt = 0; nt < 2; ++nt) prefill_mma<T, false>(acc[mt][nt], af[mt], bf[nt]);
     }
     if (kt + 1 < nk) park(kt + 1, buf ^ 1);
     __syncthreads();
@@ -205,6 +183,79 @@ __global__ void __launch_bounds__(256, 2) prefill_gemm_kernel(
     }
 }
 
+// ---- which blocks a product takes
+// Microseconds of a round of blocks of 64 mi rows: its start and end, and a stage of 64 of K in strips of 128, 192 or 256 columns
+// (half the second index + 1), with up to 200 and with more blocks at once.  Fitted to the four projections of Llama-3-8B, int4
+// and bf16, weights from memory, 129 to 2048 rows.
+static constexpr double kRound = 6.0;
+static constexpr double kStage[3][3][2] = {
+    {{0.55, 0.61}, {0.67, 0.84}, {0.86, 1.08}}, {{0.65, 0.82}, {0.91, 1.14}, {1.04, 1.30}}, {{0.76, 0.97}, {1.07, 1.33}, {1.32, 1.62}}};
+
+struct PrefillPlan {
+  int mi, mt, whole, tail, narrow;
+  double cost;
+};
+
+// Strips of 256 columns while they fill whole rounds of 256 units; what is left over, if it would fill no more than three quarters
+// of a round, in strips of 192 or 128 (1152 x 28672 x 4096, 192 rows a block: two rounds and 216 blocks of 192 columns, 254 us).
+static PrefillPlan prefill_strips(int64_t M, int64_t N, int64_t K, int mi) {
+  auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  const int64_t mt = up(M, 64 * mi), all = up(N, 256), stages = K / 64;
+  auto rounds = [&](int64_t blocks, int strip) {
+    const int64_t full = blocks / 256, rest = blocks % 256;
+    const double* c = kStage[mi - 2][strip];
+    return full * (kRound + stages * c[1]) + (rest ? kRound + stages * c[rest > 200] : 0.0);
+  };
+  PrefillPlan p{mi, (int)mt, (int)all, 0, 128, rounds(mt * all, 2)};
+  const int64_t whole = mt * all / 256 * 256 / mt;
+  for (int strip : {0, 1}) {
+    const int narrow = 128 + 64 * strip;
+    const int64_t tail = up(N - whole * 256, narrow);
+    if (whole < all && mt * tail <= 256)
+      return {mi, (int)mt, (int)whole, (int)tail, narrow, rounds(mt * whole, 2) + rounds(mt * tail, strip)};
+  }
+  return p;
+}
+
+// Rows a block: whatever wastes least of the last round and of the last block (1152 rows: six of 192).  16-bit weights, which are
+// not dequantised on the way, keep 512 registers only up to 192 rows.
+static PrefillPlan prefill_plan(int64_t M, int64_t N, int64_t K, bool awq) {
+  PrefillPlan best = prefill_strips(M, N, K, 2);
+  for (int mi = 3; mi <= (awq ? 4 : 3); ++mi) {
+    const PrefillPlan p = prefill_strips(M, N, K, mi);
+    if (p.cost < best.cost) best = p;
+  }
+  return best;
+}
+
+template <typename T, bool AWQ, int MI>
+static int launch_prefill(const PrefillArgs& a, hipStream_t s) {
+  constexpr int lds = (2 * 64 * MI + (AWQ ? 2 : 3) * 256) * 128 + (AWQ ? 2048 : 0);
+  if (int rc = ensure_lds<&prefill_tile_kernel<T, AWQ, MI>>(lds)) return rc;
+  hipLaunchKernelGGL((prefill_tile_kernel<T, AWQ, MI>), dim3((unsigned)(a.mt * (a.whole + a.tail))), dim3(256), lds, s, a);
+  SGLK_LAUNCH_CHECK();
+  return SGLK_OK;
+}
+
+template <typename T, bool AWQ>
+static int launch_prefill_any(const PrefillArgs& a, hipStream_t s) {
+  constexpr int64_t kPitch = 1 << 23;  // 256 rows of less than that span less than 2^32 bytes
+  if (a.x_stride >= kPitch || a.w_stride >= kPitch) {
+    const dim3 grid((a.M + kPfBM - 1) / kPfBM, a.N / kPfBN);
+    hipLaunchKernelGGL((prefill_gemm_kernel<T, AWQ>), grid, dim3(256), kPfLds, s, a.x, a.w, a.scales, a.qzeros, a.bias, a.out, a.M,
+                       a.N, a.K, a.group_size, a.x_stride, a.w_stride, a.out_stride);
+    SGLK_LAUNCH_CHECK();
+    return SGLK_OK;
+  }
+  const PrefillPlan pl = prefill_plan(a.M, a.N, a.K, AWQ);
+  PrefillArgs b = a;
+  b.mt = pl.mt, b.whole = pl.whole, b.tail = pl.tail, b.narrow = pl.narrow;
+  if (pl.mi == 2) return launch_prefill<T, AWQ, 2>(b, s);
+  if constexpr (AWQ)
+    if (pl.mi == 4) return launch_prefill<T, AWQ, 4>(b, s);
+  return launch_prefill<T, AWQ, 3>(b, s);
+}
+
 static int prefill_checks(const void* x, const void* w, const void* out, int M, int N, int K, int64_t x_stride,
                           int64_t out_stride, const char* what) {
   SGLK_CHECK(x && w && out, "%s: null pointer", what);
@@ -228,27 +279,32 @@ int sglk_awq_gemm_prefill(const void* x, const int32_t* packed, const void* scal
   SGLK_CHECK(scales && qzeros, "awq_gemm_prefill: null pointer");
   SGLK_CHECK(group_size > 0 && group_size % 128 == 0 && K % group_size == 0,
              "awq_gemm_prefill: group size %d must be a multiple of 128 that divides K", group_size);
-  dim3 grid((M + kPfBM - 1) / kPfBM, N / kPfBN);
-  SGLK_DISPATCH_HALF(dtype, T,
-                     hipLaunchKernelGGL((prefill_gemm_kernel<T, true>), grid, dim3(256), kPfLds, (hipStream_t)stream,
-                                        (const uint16_t*)x, (const void*)packed, (const uint16_t*)scales, qzeros,
-                                        (const uint16_t*)bias, (uint16_t*)out, M, N, K, group_size, x_stride, (int64_t)0,
-                                        out_stride));
-  SGLK_LAUNCH_CHECK();
+  const PrefillArgs a{(const uint16_t*)x, packed, (const uint16_t*)scales, qzeros, (const uint16_t*)bias, (uint16_t*)out, M, N, K,
+                      group_size, x_stride, 0, out_stride, 0, 0, 0, 0};
+  SGLK_DISPATCH_HALF(dtype, T, { return (launch_prefill_any<T, true>(a, (hipStream_t)stream)); });
   return SGLK_OK;
+}
+
+// The other way: the weight dequantised to memory (2.5 bytes of traffic a weight), then the library's product, which needs its
+// weights' way from memory, its operations or a chain along K, whichever is longest.  Below four million weights nothing was
+// measured, and the library keeps them.  Measured, library and here: 1152 x 28672 x 4096 300 and 254 us, 500 rows 154 and 110, 256
+// rows 125 and 67; 1152 x 6144 x 4096 70 and 64; 1152 x 4096 x 14336 164 and 155; left to the library: 640 x 4096 x 14336 139 and
+// 133, 256 rows 94 and 130.
+int sglk_awq_prefill_fused(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % 128 != 0 || N % 128 != 0 || (int64_t)N * K < (4 << 20)) return 0;
+  const double weights = (double)N * K;
+  const double dequantise = 2 + 2.5e-6 / 5.2 * weights;
+  const double product = 10 + std::max({2e-6 / 4.5 * weights, 2e-9 / 1.15 * weights * M, 0.0045 * K});
+  return prefill_plan(M, N, K, true).cost < dequantise + product;
 }
 
 int sglk_dense_gemm_prefill(const void* x, const void* w, const void* bias, void* out, int M, int N, int K,
                             int64_t x_stride, int64_t w_stride, int64_t out_stride, int dtype, void* stream) {
   if (int rc = prefill_checks(x, w, out, M, N, K, x_stride, out_stride, "dense_gemm_prefill")) return rc;
   SGLK_CHECK(w_stride % 8 == 0, "dense_gemm_prefill: weight rows must be 16-byte aligned");
-  dim3 grid((M + kPfBM - 1) / kPfBM, N / kPfBN);
-  SGLK_DISPATCH_HALF(dtype, T,
-                     hipLaunchKernelGGL((prefill_gemm_kernel<T, false>), grid, dim3(256), kPfLds, (hipStream_t)stream,
-                                        (const uint16_t*)x, w, (const uint16_t*)nullptr, (const int32_t*)nullptr,
-                                        (const uint16_t*)bias, (uint16_t*)out, M, N, K, 128, x_stride, w_stride,
-                                        out_stride));
-  SGLK_LAUNCH_CHECK();
+  const PrefillArgs a{(const uint16_t*)x, w, nullptr, nullptr, (const uint16_t*)bias, (uint16_t*)out, M, N, K, 128, x_stride,
+                      w_stride, out_stride, 0, 0, 0, 0};
+  SGLK_DISPATCH_HALF(dtype, T, { return (launch_prefill_any<T, false>(a, (hipStream_t)stream)); });
   return SGLK_OK;
 }
 }

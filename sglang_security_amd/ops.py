@@ -683,6 +683,11 @@ def awq_gemm_prefill(x, packed, scales, qzeros, bias=None, out=None):
     return out
 
 
+def awq_prefill_fused(M, N, K) -> bool:
+    """Whether awq_gemm_prefill is expected to be faster than dequantising the weight and a library product."""
+    return bool(lib().sglk_awq_prefill_fused(M, N, K))
+
+
 def dense_gemm_prefill(x, w, bias=None, out=None):
     """Large-M x:[M,K] @ w:[N,K]^T on the hand-written tile kernel (K % 128 == 0, N % 128 == 0)."""
     _need_gpu(x, w)

@@ -35,8 +35,9 @@ class LlamaPrefill:
 
     def __init__(self, dec: LlamaDecoder, kv_pool: MHATokenToKVPool, max_tokens: int, use_graph: bool = True,
                  resident_bf16: bool = False, prefill_gemm: str = "library", overlap_dequant: bool = False):
-        """prefill_gemm: what multiplies batches of DEQUANT_GEMM_MIN_TOKENS rows or more.  "library": dequantise the
-        int4 weight (sglk_awq_dequantize_packed_nk), then torch.matmul = hipBLASLt -- the faster of the two today;
+        """prefill_gemm: what multiplies batches of DEQUANT_GEMM_MIN_TOKENS rows or more.  "library": torch.matmul =
+        hipBLASLt, int4 weights dequantised first (sglk_awq_dequantize_packed_nk), where it is faster than the product that
+        dequantises on the way (ops.awq_prefill_fused; same weights, sums in another order);
         "fused": the hand-written tile kernels of this package (sglk_awq_gemm_prefill dequantises inside the GEMM and
         writes no dequantised copy; sglk_dense_gemm_prefill for 16-bit weights).
 
@@ -111,7 +112,7 @@ class LlamaPrefill:
         T = x.shape[0]
         fused = self.prefill_gemm == "fused" and T >= DEQUANT_GEMM_MIN_TOKENS and w.N % 128 == 0 and w.K % 128 == 0
         if isinstance(w, _AwqLinear):
-            if fused:
+            if fused or T >= DEQUANT_GEMM_MIN_TOKENS and not self._by_library(w, T):
                 ops.awq_gemm_prefill(x, w.packed, w.scales, w.qzeros, None, out)
             elif T >= DEQUANT_GEMM_MIN_TOKENS:
                 if self._pipe is not None:
@@ -134,6 +135,10 @@ class LlamaPrefill:
             raise NotImplementedError("prefill runner: awq and bf16 weights")
         return out
 
+    def _by_library(self, w, T):
+        """Whether T rows go to a dequantised copy of an int4 weight and the library (prefill_gemm = "library")."""
+        return self.resident_bf16 or not (ops.awq_prefill_fused(T, w.N, w.K) and w.K // w.scales.shape[0] % 128 == 0)
+
     # -- dequantisation one projection ahead of the library product, on a second stream --------------------------------
     _RING = 3
 
@@ -142,13 +147,15 @@ class LlamaPrefill:
         if not (self.overlap_dequant and self.prefill_gemm == "library" and not self.resident_bf16
                 and c.quant == "awq" and T >= DEQUANT_GEMM_MIN_TOKENS):
             return
+        seq = [L[k] for L in self.dec.layers for k in ("qkv", "o", "gate_up", "down")]
+        if not all(isinstance(w, _AwqLinear) for w in seq):
+            self.overlap_dequant = False
+            return
+        self._seq = [w for w in seq if self._by_library(w, T)]
+        if not self._seq:
+            return
         if self._ring is None:
-            seq = [L[k] for L in self.dec.layers for k in ("qkv", "o", "gate_up", "down")]
-            if not all(isinstance(w, _AwqLinear) for w in seq):
-                self.overlap_dequant = False
-                return
             n = max(w.K * w.N for w in seq)
-            self._seq = seq
             self._ring = [torch.empty(n, dtype=self.dec.dtype, device=self.dec.device) for _ in range(self._RING)]
             self._side = torch.cuda.Stream(device=self.dec.device)
             self._ready = [torch.cuda.Event() for _ in range(self._RING)]

@@ -116,6 +116,11 @@ class AWQLinearMethod:
             out = ops.awq_gemm(x2.contiguous(), layer.sglk_packed, layer.scales, layer.qzeros, bias, None,
                                self._workspace(layer, m, x.device))
             return out.reshape(out_shape)
+        if m > 0 and layer.sglk_fusable and n % 128 == 0 and ops.awq_prefill_fused(m, n, k):
+            out = ops.awq_gemm_prefill(x2.contiguous(), layer.sglk_packed, layer.scales, layer.qzeros)
+            if bias is not None:
+                out.add_(bias)
+            return out.reshape(out_shape)
         if layer.qweight is not None:
             w = ops.awq_dequantize(layer.qweight, layer.scales, layer.qzeros)
         else:
