@@ -257,7 +257,7 @@ __device__ __forceinline__ void fp8_tile4(const Fp8TileArgs& p, char* lds, int m
 #pragma unroll
     for (int d = 0; d < NA; ++d) issue_a(i, i, d);
   }
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SA - 1) * (NA + NB)) : "memory");
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((SA - 1) * (NA + NB)) : "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 #pragma unroll
