@@ -618,6 +618,11 @@ SGLK_API int sglk_dense_gemm_nt(const void* x, const void* w, const void* bias, 
 SGLK_API int sglk_awq_gemm_prefill(const void* x, const int32_t* packed, const void* scales, const int32_t* qzeros,
                                    const void* bias, void* out, int M, int N, int K, int group_size,
                                    int64_t x_stride, int64_t out_stride, int dtype, void* stream);
+/* The same with silu(gate) * up behind it, on a weight interleaved as for sglk_awq_gemm_silu_mul: out [M, N / 2], the values of the
+ * product followed by sglk_act_and_mul.  N % 256 == 0. */
+SGLK_API int sglk_awq_gemm_prefill_silu_mul(const void* x, const int32_t* packed, const void* scales, const int32_t* qzeros,
+                                            void* out, int M, int N, int K, int group_size, int64_t x_stride,
+                                            int64_t out_stride, int dtype, void* stream);
 /* Whether sglk_awq_gemm_prefill is expected to be faster than a dequantisation to memory and a library product. */
 SGLK_API int sglk_awq_prefill_fused(int M, int N, int K);
 SGLK_API int sglk_dense_gemm_prefill(const void* x, const void* w, const void* bias, void* out, int M, int N, int K,

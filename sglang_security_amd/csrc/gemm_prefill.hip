@@ -198,7 +198,7 @@ struct PrefillPlan {
 
 // Strips of 256 columns while they fill whole rounds of 256 units; what is left over, if it would fill no more than three quarters
 // of a round, in strips of 192 or 128 (1152 x 28672 x 4096, 192 rows a block: two rounds and 216 blocks of 192 columns, 254 us).
-static PrefillPlan prefill_strips(int64_t M, int64_t N, int64_t K, int mi) {
+static PrefillPlan prefill_strips(int64_t M, int64_t N, int64_t K, int mi, bool gated) {
   auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   const int64_t mt = up(M, 64 * mi), all = up(N, 256), stages = K / 64;
   auto rounds = [&](int64_t blocks, int strip) {
@@ -208,7 +208,7 @@ static PrefillPlan prefill_strips(int64_t M, int64_t N, int64_t K, int mi) {
   };
   PrefillPlan p{mi, (int)mt, (int)all, 0, 128, rounds(mt * all, 2)};
   const int64_t whole = mt * all / 256 * 256 / mt;
-  for (int strip : {0, 1}) {
+  for (int strip = 0; strip < (gated ? 1 : 2); ++strip) {  // (a gate block and its up block: strips of whole 128s)
     const int narrow = 128 + 64 * strip;
     const int64_t tail = up(N - whole * 256, narrow);
     if (whole < all && mt * tail <= 256)
@@ -219,10 +219,10 @@ static PrefillPlan prefill_strips(int64_t M, int64_t N, int64_t K, int mi) {
 
 // Rows a block: whatever wastes least of the last round and of the last block (1152 rows: six of 192).  16-bit weights, which are
 // not dequantised on the way, keep 512 registers only up to 192 rows.
-static PrefillPlan prefill_plan(int64_t M, int64_t N, int64_t K, bool awq) {
-  PrefillPlan best = prefill_strips(M, N, K, 2);
+static PrefillPlan prefill_plan(int64_t M, int64_t N, int64_t K, bool awq, bool gated = false) {
+  PrefillPlan best = prefill_strips(M, N, K, 2, gated);
   for (int mi = 3; mi <= (awq ? 4 : 3); ++mi) {
-    const PrefillPlan p = prefill_strips(M, N, K, mi);
+    const PrefillPlan p = prefill_strips(M, N, K, mi, gated);
     if (p.cost < best.cost) best = p;
   }
   return best;
@@ -237,17 +237,18 @@ static int launch_prefill(const PrefillArgs& a, hipStream_t s) {
   return SGLK_OK;
 }
 
+static constexpr int64_t kPrefillPitch = 1 << 23;  // 256 rows of less than that span less than 2^32 bytes
+
 template <typename T, bool AWQ>
 static int launch_prefill_any(const PrefillArgs& a, hipStream_t s) {
-  constexpr int64_t kPitch = 1 << 23;  // 256 rows of less than that span less than 2^32 bytes
-  if (a.x_stride >= kPitch || a.w_stride >= kPitch) {
+  if (a.x_stride >= kPrefillPitch || a.w_stride >= kPrefillPitch) {
     const dim3 grid((a.M + kPfBM - 1) / kPfBM, a.N / kPfBN);
     hipLaunchKernelGGL((prefill_gemm_kernel<T, AWQ>), grid, dim3(256), kPfLds, s, a.x, a.w, a.scales, a.qzeros, a.bias, a.out, a.M,
                        a.N, a.K, a.group_size, a.x_stride, a.w_stride, a.out_stride);
     SGLK_LAUNCH_CHECK();
     return SGLK_OK;
   }
-  const PrefillPlan pl = prefill_plan(a.M, a.N, a.K, AWQ);
+  const PrefillPlan pl = prefill_plan(a.M, a.N, a.K, AWQ, a.gated);
   PrefillArgs b = a;
   b.mt = pl.mt, b.whole = pl.whole, b.tail = pl.tail, b.narrow = pl.narrow;
   if (pl.mi == 2) return launch_prefill<T, AWQ, 2>(b, s);
@@ -280,7 +281,22 @@ int sglk_awq_gemm_prefill(const void* x, const int32_t* packed, const void* scal
   SGLK_CHECK(group_size > 0 && group_size % 128 == 0 && K % group_size == 0,
              "awq_gemm_prefill: group size %d must be a multiple of 128 that divides K", group_size);
   const PrefillArgs a{(const uint16_t*)x, packed, (const uint16_t*)scales, qzeros, (const uint16_t*)bias, (uint16_t*)out, M, N, K,
-                      group_size, x_stride, 0, out_stride, 0, 0, 0, 0};
+                      group_size, x_stride, 0, out_stride, 0, 0, 0, 0, 0};
+  SGLK_DISPATCH_HALF(dtype, T, { return (launch_prefill_any<T, true>(a, (hipStream_t)stream)); });
+  return SGLK_OK;
+}
+
+int sglk_awq_gemm_prefill_silu_mul(const void* x, const int32_t* packed, const void* scales, const int32_t* qzeros, void* out,
+                                   int M, int N, int K, int group_size, int64_t x_stride, int64_t out_stride, int dtype,
+                                   void* stream) {
+  if (int rc = prefill_checks(x, packed, out, M, N, K, x_stride, out_stride, "awq_gemm_prefill_silu_mul")) return rc;
+  SGLK_CHECK(scales && qzeros, "awq_gemm_prefill_silu_mul: null pointer");
+  SGLK_CHECK(N % 256 == 0 && out_stride >= N / 2, "awq_gemm_prefill_silu_mul: N=%d must be a multiple of 256, out rows hold N / 2", N);
+  SGLK_CHECK(group_size > 0 && group_size % 128 == 0 && K % group_size == 0,
+             "awq_gemm_prefill_silu_mul: group size %d must be a multiple of 128 that divides K", group_size);
+  SGLK_CHECK(x_stride < kPrefillPitch, "awq_gemm_prefill_silu_mul: rows %lld elements apart", (long long)x_stride);
+  const PrefillArgs a{(const uint16_t*)x, packed, (const uint16_t*)scales, qzeros, nullptr, (uint16_t*)out, M, N, K,
+                      group_size, x_stride, 0, out_stride, 1, 0, 0, 0, 0};
   SGLK_DISPATCH_HALF(dtype, T, { return (launch_prefill_any<T, true>(a, (hipStream_t)stream)); });
   return SGLK_OK;
 }
@@ -303,7 +319,7 @@ int sglk_dense_gemm_prefill(const void* x, const void* w, const void* bias, void
   if (int rc = prefill_checks(x, w, out, M, N, K, x_stride, out_stride, "dense_gemm_prefill")) return rc;
   SGLK_CHECK(w_stride % 8 == 0, "dense_gemm_prefill: weight rows must be 16-byte aligned");
   const PrefillArgs a{(const uint16_t*)x, w, nullptr, nullptr, (const uint16_t*)bias, (uint16_t*)out, M, N, K, 128, x_stride,
-                      w_stride, out_stride, 0, 0, 0, 0};
+                      w_stride, out_stride, 0, 0, 0, 0, 0};
   SGLK_DISPATCH_HALF(dtype, T, { return (launch_prefill_any<T, false>(a, (hipStream_t)stream)); });
   return SGLK_OK;
 }

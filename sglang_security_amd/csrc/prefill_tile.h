@@ -54,6 +54,7 @@ struct PrefillArgs {
   uint16_t* out;
   int M, N, K, group_size;
   int64_t x_stride, w_stride, out_stride;
+  int gated;                    // blocks of 64 columns alternate between gate and up: out = silu(gate) * up, N / 2 columns
   int mt, whole, tail, narrow;  // row tiles, strips of 256 columns, strips of `narrow` columns behind them
 };
 
@@ -255,7 +256,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& p, char* lds, in
 #pragma unroll
       for (int d = 0; d < NA; ++d) issue_a(s, s, d);
     }
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NA + NB) : "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(NA + NB) : "memory");
   }
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
@@ -346,7 +347,8 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& p, char* lds, in
   asm volatile("" : "+v"(tid));  // what depends on the lane is formed again: kept over the loop it would go out to memory
   const int ln = tid & 63, row31 = ln & 31, up = ln >> 5;
   char* ol = lds + (tid >> 6) * 32 * kPitch;
-  auto rows = [&](auto with_bias) {
+  auto rows = [&](auto kind) {  // 0: plain, 1: with a bias, 2: gated
+    constexpr int kKind = decltype(kind)::value;
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
 #pragma unroll
@@ -354,14 +356,44 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& p, char* lds, in
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           short4v v, bias = {0, 0, 0, 0};
-          if constexpr (decltype(with_bias)::value)
+          if constexpr (kKind == 1)
             bias = *reinterpret_cast<const short4v*>(p.bias + min(n0 + wn + 32 * j + 8 * g + 4 * up, p.N - 4));
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            v[r] = (short)Conv<T>::from_f32(
-                acc[i][j][4 * g + r] + (decltype(with_bias)::value ? Conv<T>::to_f32((uint16_t)bias[r]) : 0.f));
+            v[r] = (short)Conv<T>::from_f32(acc[i][j][4 * g + r] + (kKind == 1 ? Conv<T>::to_f32((uint16_t)bias[r]) : 0.f));
           *reinterpret_cast<short4v*>(ol + row31 * kPitch + (32 * j + 8 * g + 4 * up) * 2) = v;
         }
+      if constexpr (kKind == 2) {
+        // the rounding points of the product followed by silu_and_mul; a wave of 128 columns holds a gate block and its up
+        // block, of 64 columns one of them: there the two waves of a row take half the rows each
+        if constexpr (NJ == 2)
+          __syncthreads();
+        else
+          __builtin_amdgcn_wave_barrier();
+        constexpr int kPieces = 32 * 8 / (NJ == 2 ? 2 : 1);
+        const char* gl = NJ == 2 ? lds + ((tid >> 6) & ~1) * 32 * kPitch : ol;
+        const char* ul = NJ == 2 ? gl + 32 * kPitch : ol + 128;
+#pragma unroll
+        for (int t = 0; t < kPieces / 64; ++t) {
+          const int piece = t * 64 + ln + (NJ == 2 ? (tid >> 6 & 1) * kPieces : 0), row = piece >> 3, c = piece & 7;
+          const short8 gate = *reinterpret_cast<const short8*>(gl + row * kPitch + c * 16);
+          const short8 upper = *reinterpret_cast<const short8*>(ul + row * kPitch + c * 16);
+          short8 o;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float x = Conv<T>::to_f32((uint16_t)gate[e]);
+            const float sv = Conv<T>::to_f32(Conv<T>::from_f32(x / (1.0f + __expf(-x))));
+            o[e] = (short)Conv<T>::from_f32(sv * Conv<T>::to_f32((uint16_t)upper[e]));
+          }
+          const int m = m0 + wm + 32 * i + row, n = n0 + (NJ == 2 ? 0 : wn);  // N % 256 == 0
+          if (m < p.M && n < p.N) *reinterpret_cast<short8*>(p.out + (int64_t)m * p.out_stride + n / 2 + 8 * c) = o;
+        }
+        if constexpr (NJ == 2)
+          __syncthreads();
+        else
+          __builtin_amdgcn_wave_barrier();
+        continue;
+      }
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
       for (int t = 0; t < 32 * kPer / 64; ++t) {
@@ -373,10 +405,12 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& p, char* lds, in
       __builtin_amdgcn_wave_barrier();
     }
   };
+  if constexpr (AWQ && NJ != 3)
+    if (p.gated) return rows(std::integral_constant<int, 2>{});
   if (p.bias)
-    rows(std::true_type{});
+    rows(std::integral_constant<int, 1>{});
   else
-    rows(std::false_type{});
+    rows(std::integral_constant<int, 0>{});
 }
 
 template <typename T, bool AWQ, int MI>

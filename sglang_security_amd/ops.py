@@ -683,6 +683,17 @@ def awq_gemm_prefill(x, packed, scales, qzeros, bias=None, out=None):
     return out
 
 
+def awq_gemm_prefill_silu_mul(x, packed, scales, qzeros, out):
+    """out[M, N/2] = silu(x @ W_gate) * (x @ W_up) for many rows, on a weight interleaved by awq_interleave_gate_up."""
+    _need_gpu(x, packed, scales, qzeros, out)
+    M, K = x.shape
+    N = scales.shape[1]
+    check(lib().sglk_awq_gemm_prefill_silu_mul(_ptr(x), _ptr(packed), _ptr(scales), _ptr(qzeros), _ptr(out), M, N, K,
+                                               K // scales.shape[0], x.stride(0), out.stride(0), dtype_code(x.dtype), _stream(x)),
+          "awq_gemm_prefill_silu_mul")
+    return out
+
+
 def awq_prefill_fused(M, N, K) -> bool:
     """Whether awq_gemm_prefill is expected to be faster than dequantising the weight and a library product."""
     return bool(lib().sglk_awq_prefill_fused(M, N, K))

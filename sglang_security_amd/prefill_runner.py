@@ -139,6 +139,12 @@ class LlamaPrefill:
         """Whether T rows go to a dequantised copy of an int4 weight and the library (prefill_gemm = "library")."""
         return self.resident_bf16 or not (ops.awq_prefill_fused(T, w.N, w.K) and w.K // w.scales.shape[0] % 128 == 0)
 
+    def _gated(self, L, T):
+        """Whether gate_up takes the activation along: a product that dequantises on the way, on the decoder's interleaved copy."""
+        w = L["gate_up"]
+        return (T >= DEQUANT_GEMM_MIN_TOKENS and "gate_up_il" in L and w.N % 256 == 0
+                and (self.prefill_gemm == "fused" and w.K % 128 == 0 or not self._by_library(w, T)))
+
     # -- dequantisation one projection ahead of the library product, on a second stream --------------------------------
     _RING = 3
 
@@ -318,8 +324,11 @@ class LlamaPrefill:
                                      sm_scale)
             self._linear(L["o"], attn_out, hidden)
             ops.fused_add_rmsnorm(hidden, residual, L["ln2"], c.eps)
-            self._linear(L["gate_up"], hidden, gate_up)
-            ops.act_and_mul(act, gate_up, 0)
+            if self._gated(L, hidden.shape[0]):
+                ops.awq_gemm_prefill_silu_mul(hidden, *L["gate_up_il"], act)
+            else:
+                self._linear(L["gate_up"], hidden, gate_up)
+                ops.act_and_mul(act, gate_up, 0)
             self._linear(L["down"], act, hidden)
 
     def first_token(self, hidden: torch.Tensor, residual: torch.Tensor, last_row: int) -> torch.Tensor:

@@ -102,3 +102,20 @@ def test_rule_stays_where_it_was_measured():
     assert ops.awq_prefill_fused(1152, 28672, 4096) and ops.awq_prefill_fused(256, 28672, 4096)
     assert not ops.awq_prefill_fused(256, 4096, 14336)          # few blocks along a long inner dimension
     assert not ops.awq_prefill_fused(300, 1024, 512) and not ops.awq_prefill_fused(300, 28672, 4000)
+
+
+@pytest.mark.parametrize("M,K,inter", [(300, 256, 128), (256, 512, 14336), (1152, 256, 14336), (700, 384, 6144), (2048, 128, 14336)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_gated_rows_are_those_of_two_launches(M, K, inter, dtype):
+    """Strips of 256 and of 128 columns: the activation's bits are those of the product followed by act_and_mul."""
+    from sglang_security_amd import ops
+
+    qw, sc, qz, g = _int4(K, 2 * inter, dtype, M + inter)
+    x = torch.randn(M, K, device=DEV, generator=g).to(dtype)
+    want = torch.empty(M, inter, dtype=dtype, device=DEV)
+    ops.act_and_mul(want, ops.awq_gemm_prefill(x, ops.awq_repack(qw), sc, qz), 0)
+    qi, si, zi = ops.awq_interleave_gate_up(qw, sc, qz)
+    buf = torch.full((M + 1, inter + 8), 7.0, dtype=dtype, device=DEV)
+    ops.awq_gemm_prefill_silu_mul(x, ops.awq_repack(qi), si, zi, buf[:M, :inter])
+    assert torch.equal(buf[:M, :inter], want)
+    assert bool((buf[M] == 7).all()) and bool((buf[:, inter:] == 7).all())
