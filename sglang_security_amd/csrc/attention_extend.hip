@@ -324,12 +324,13 @@ static int extend_attention_impl(const void* q_extend, const void* k_extend, con
     // kv heads run fastest: with eight of them the blocks of one head share an XCD's L2
     const int gy = (int)std::min<int64_t>(row_blocks, 65535), gz = kv_splits > 1 ? 1 : (int)((row_blocks + gy - 1) / gy);
     const dim3 grid(Hkv * B, gy, kv_splits > 1 ? kv_splits : gz);
+    const int wide = kv_splits == 1 && aligned16(o_extend) && mult8(o_stride_t) && mult8(o_stride_h);
     auto u16 = [](const void* p) { return reinterpret_cast<const uint16_t*>(p); };
     const ExtendArgs a{u16(q_extend), u16(k_extend), u16(v_extend), u16(k_buffer), u16(v_buffer),
                        reinterpret_cast<uint16_t*>(o_extend), qo_indptr, kv_indptr, kv_indices, Hq, Hkv, q_stride_t, q_stride_h,
                        ke_stride_h, ve_stride_h, o_stride_t, o_stride_h, k_stride_h, v_stride_h, (uint32_t)(2 * ke_stride_t),
                        (uint32_t)(2 * ve_stride_t), (uint32_t)(2 * k_stride_n), (uint32_t)(2 * v_stride_n), sm_scale, logit_cap,
-                       causal, kv_splits, gy * gz - 1, kv_splits > 1 ? 0 : gy, part_o, part_lse};
+                       causal, kv_splits, wide, gy * gz - 1, kv_splits > 1 ? 0 : gy, part_o, part_lse};
 #define SGLK_EXT(DV, PRE)                                                                    \
   SGLK_DISPATCH_HALF(dtype, T, {                                                             \
     if (int rc = ensure_lds<extend_tile_kernel<T, DV, PRE>>(4 * kExtTokens * 2 * DV)) return rc; \

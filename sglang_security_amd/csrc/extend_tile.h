@@ -16,7 +16,7 @@
 // 0.00197 with that on tiles of 32 tokens, which had more probabilities of exactly one).
 //
 // Measured (bf16, launch alone): 8 prompts of 768 to 1152 tokens, 32 / 8 heads of 128: 264 us (one block per 64 rows of
-// one head, 32-token tiles on 16x16x32) -> 124 us, 525 TFLOP/s; one prompt of 1152 tokens: 69 -> 36 us; 128 tokens over
+// one head, 32-token tiles on 16x16x32) -> 119 us, 547 TFLOP/s; one prompt of 1152 tokens: 69 -> 36 us; 128 tokens over
 // 1024 cached, split 8 ways: 20.1 -> 14.6 us; 4 prompts of 667 to 1000 tokens over 683 to 1024 cached, 14 / 2 heads of
 // 64: 3.24 ms (wave per row) -> 0.052 ms.  Operand reads are spelled out ahead of the products that use them: the
 // compiler's own order waits for each (8 prompts: 137.5 -> 134.5 us of a call with its copies, one box).
@@ -70,6 +70,7 @@ struct ExtendArgs {
   uint32_t ke_row, ve_row, kb_row, vb_row;  // bytes from row to row (below 2^32: one 32 x 32 + 64-bit product an address)
   float sm_scale, logit_cap;
   int causal, kv_splits;
+  int wide_rows;  // rows leave whole: not split, and they start at multiples of 16 bytes
   int last_block, z_blocks;  // of rows, over the grid's second dimension and, unsplit, its third (blocks a step of it has, else 0)
   float *part_o, *part_lse;  // kv_splits > 1: [T, Hq, kv_splits, D] and [T, Hq, kv_splits]
 };
@@ -315,7 +316,7 @@ __device__ __forceinline__ bool extend_walk(const ExtendArgs& a, const int tid, 
       for (int k = 0; k < 4; ++k)
 #pragma unroll
         for (int e = 0; e < 8; e += 2) psum = add_pair<T>(pf[k][e], pf[k][e + 1], psum);
-    lsum += psum;
+    if constexpr (!CAREFUL) lsum += psum;
     if constexpr (CAREFUL) {
       // A value that is not finite counts as zero in the product; two more products count those of a row's 16 tokens on
       // either side (a NaN, and an infinity of weight zero, is one on both), and one infinity stands for a side.
@@ -343,7 +344,7 @@ __device__ __forceinline__ bool extend_walk(const ExtendArgs& a, const int tid, 
         }
         if constexpr (!P2)
 #pragma unroll
-          for (int e = 0; e < 8; e += 2) lsum = add_pair<T>(hp[e], hp[e + 1], lsum);
+          for (int e = 0; e < 8; e += 2) psum = add_pair<T>(hp[e], hp[e + 1], psum);  // in the first walk's order
 #pragma unroll
         for (int n = 0; n < NV; ++n) {
           __builtin_amdgcn_sched_barrier(0);
@@ -372,6 +373,7 @@ __device__ __forceinline__ bool extend_walk(const ExtendArgs& a, const int tid, 
           }
         }
       }
+      lsum += psum;
       continue;
     }
 #pragma unroll
@@ -404,7 +406,38 @@ __device__ __forceinline__ bool extend_walk(const ExtendArgs& a, const int tid, 
 #pragma unroll
     for (int r = 0; r < 16; ++r) zero[r & 3] = fmaf(oacc[n][r], 0.f, zero[r & 3]);
   const float nan = (zero[0] + zero[1]) + (zero[2] + zero[3]);
-  const bool odd = nan != 0.f || __shfl_xor(nan, 32, 64) != 0.f;
+  const float nan_other = __shfl_xor(nan, 32, 64);  // by all lanes, whatever their own is
+  const bool odd = nan != 0.f || nan_other != 0.f;
+  if constexpr (!CAREFUL && D == 128) {
+    if (a.wide_rows) {
+      // Whole rows, turned in the stage that the last tile does not use: a lane's own pieces of 8 bytes are 16 requests a wave,
+      // each of 16 bytes of 32 rows.  8 prompts of 512 tokens 41.4 -> 37.5 us, of 1024 108 -> 102, 8 of 768 to 1152 in a call with its
+      // copies 120.3 -> 115.5.  Stored past the caches they are 3 us faster still, and the product that reads them 7 slower.  Head size
+      // 64 has half the bytes a row and gains nothing (52.3 -> 52.9 for 4 prompts over cached prefixes).
+      char* ol = lds + (nt & 1) * 2 * kStage + wid * (64 * D);
+      auto out_off = [&](int r, int piece) { return r * 2 * D + ((piece ^ (r & 15)) << 4); };
+#pragma unroll
+      for (int n = 0; n < NV; ++n)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          short4v v;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = (short)Conv<T>::from_f32(oacc[n][4 * g + r] * inv);
+          *reinterpret_cast<short4v*>(ol + out_off(l31, 4 * n + g) + 8 * hi) = v;
+        }
+      __builtin_amdgcn_wave_barrier();  // the wave's own LDS rows: in order, no block barrier
+      const uint64_t leave = __ballot(mine && !odd);
+      const int64_t off = (int64_t)(q0 + tok) * a.o_st + (int64_t)head * a.o_sh;
+#pragma unroll
+      for (int t = 0; t < 32 * kTpr / 64; ++t) {
+        const int r = t * (64 / kTpr) + lane / kTpr, piece = lane % kTpr;
+        const int4v v = *reinterpret_cast<const int4v*>(ol + out_off(r, piece));
+        const int64_t to = __shfl(off, r, 64);
+        if (leave >> r & 1) *reinterpret_cast<int4v*>(a.o + to + piece * 8) = v;
+      }
+      return mine && odd;
+    }
+  }
   if (!mine || (odd && !CAREFUL)) return mine && odd;
   // lane (row, hi) holds elements 32 n + 8 g + 4 hi + 0 .. 3 of its row
   if (a.kv_splits > 1) {

@@ -256,3 +256,19 @@ def test_a_split_without_a_sum_is_not_lost(D, pool):
         o = torch.zeros_like(q)
         ops.extend_attention_split(q, ke, ve, o, kb, vb, qo, kp, ki, 9, 1.0 / math.sqrt(D), 0.0, True, splits)
         assert o[:7, :2].isnan().all() and o[:7, 2:].isfinite().all() and o[7:].isfinite().all()
+
+
+@pytest.mark.parametrize("pre,ext", [(0, 64), (0, 65), (0, 128), (0, 129), (0, 200), (64, 64), (65, 63), (128, 1), (129, 192), (1, 127)])
+@pytest.mark.parametrize("gap", [0, 4])
+def test_unsplit_rows_of_one_to_six_tiles(pre, ext, gap):
+    """Head size 128, not split: rows leave whole through the stage that the last tile does not use (odd and even numbers of
+    tiles, a last block of few rows) and, starting 8 bytes off, in pieces."""
+    import oracle
+    from sglang_security_amd import ops
+
+    t = _case(8, 2, 128, [pre], [ext], torch.bfloat16, seed=pre + ext)
+    want = oracle.extend_attention(*t, 1 / math.sqrt(128), 0.0, True)
+    g = [x.to(DEV) for x in t]
+    o = torch.full((ext * 8 * 128 + gap,), float("nan"), dtype=torch.bfloat16, device=DEV)[gap:].view(ext, 8, 128)
+    ops.extend_attention_split(*g[:3], o, *g[3:], ext, 1 / math.sqrt(128), 0.0, True, 1)
+    assert (o.float().cpu() - want).abs().max().item() < TOL[torch.bfloat16]
