@@ -41,6 +41,21 @@ __global__ void __launch_bounds__(256) short_conv_kernel(ShortConv a) {
   short_conv_rows<T, R, ACT>(a, (int)(idx / nv) * R, (int)(idx % nv) * 8);
 }
 
+// 4 G rows a thread, the last ones first: those at the ends of sequences, which go four at a time, take longest.
+template <typename T, int G, int ACT>
+__global__ void __launch_bounds__(256) short_conv_run_kernel(ShortConv a) {
+  const uint32_t nv = a.W / 8, runs = (a.M + 4 * G - 1) / (4 * G);
+  const uint32_t idx = blockIdx.x * 256 + threadIdx.x, run = idx / nv;
+  if (run >= runs) return;
+  const int m0 = (int)(runs - 1 - run) * 4 * G, c = (int)(idx - run * nv) * 8;
+  const int s = a.seq.row_seq[m0];
+  if (m0 + 4 * G <= a.M && a.seq.row_seq[m0 + 4 * G - 1] == s && m0 - a.seq.row0[s] >= 3) {
+    short_conv_run<T, G, ACT>(a, m0, c);
+    return;
+  }
+  for (int g = 0; g < G && m0 + 4 * g < a.M; ++g) short_conv_rows<T, 4, ACT>(a, m0 + 4 * g, c);
+}
+
 template <typename T>
 __global__ void __launch_bounds__(256) short_conv_state_kernel(ShortConv a, int seq0) {
   const int c = blockIdx.x * 256 + threadIdx.x;
@@ -701,6 +716,25 @@ int sglk_short_conv(const void* src, int src_f32, int splits, int64_t part_strid
   const int64_t threads = (int64_t)((M + per - 1) / per) * (W / 8);
   const dim3 grid((unsigned)((threads + 255) / 256));
 #define SGLK_SC(R, A) hipLaunchKernelGGL((short_conv_kernel<T, R, A>), grid, dim3(256), 0, (hipStream_t)stream, a)
+  // Eight rows a thread once that leaves four blocks a unit (5120 channels: from 3280 rows on).  A thread's filters and biases are
+  // 160 bytes beside 16 a row, so four rows cost as much in them as in rows: 7921 rows of 5120 channels 59 -> 44 us; 12 rows 44, 16
+  // 48; 2164 rows, fewer blocks than that, 21 -> 22.
+  constexpr int G = 2;
+  const int64_t run_threads = (int64_t)((M + 4 * G - 1) / (4 * G)) * (W / 8);
+  if (taps == 4 && !src_f32 && dtype != SGLK_F32 && run_threads >= 4 * 256 * 256 && run_threads < (1ll << 31)) {
+    const dim3 run_grid((unsigned)((run_threads + 255) / 256));
+    SGLK_DISPATCH_HALF(dtype, T, {
+      if (act == 3)
+        hipLaunchKernelGGL((short_conv_run_kernel<T, G, 3>), run_grid, dim3(256), 0, (hipStream_t)stream, a);
+      else
+        hipLaunchKernelGGL((short_conv_run_kernel<T, G, 0>), run_grid, dim3(256), 0, (hipStream_t)stream, a);
+      if (n_seqs > singles)
+        hipLaunchKernelGGL((short_conv_state_kernel<T>), dim3((W + 255) / 256, n_seqs - singles), dim3(256), 0, (hipStream_t)stream,
+                           a, singles);
+    });
+    SGLK_LAUNCH_CHECK();
+    return SGLK_OK;
+  }
   SGLK_DISPATCH_FLOAT(dtype, T, {
     if (per == 4 && act == 3)
       SGLK_SC(4, 3);
