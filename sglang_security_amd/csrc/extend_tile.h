@@ -16,7 +16,7 @@
 // 0.00197 with that on tiles of 32 tokens, which had more probabilities of exactly one).
 //
 // Measured (bf16, launch alone): 8 prompts of 768 to 1152 tokens, 32 / 8 heads of 128: 264 us (one block per 64 rows of
-// one head, 32-token tiles on 16x16x32) -> 119 us, 547 TFLOP/s; one prompt of 1152 tokens: 69 -> 36 us; 128 tokens over
+// one head, 32-token tiles on 16x16x32) -> 113 us, 576 TFLOP/s; one prompt of 1152 tokens: 69 -> 36 us; 128 tokens over
 // 1024 cached, split 8 ways: 20.1 -> 14.6 us; 4 prompts of 667 to 1000 tokens over 683 to 1024 cached, 14 / 2 heads of
 // 64: 3.24 ms (wave per row) -> 0.052 ms.  Operand reads are spelled out ahead of the products that use them: the
 // compiler's own order waits for each (8 prompts: 137.5 -> 134.5 us of a call with its copies, one box).
