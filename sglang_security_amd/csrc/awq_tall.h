@@ -12,8 +12,10 @@
 //
 // A barrier each half, before its last k-step: by then a wave holds that k-step's operands, so behind the barrier the half's
 // buffer is free for the next stage's and the other half's rows are there, while products are left to issue.  In the last k-step of a
-// stage a row tile's products and its zero-point term are followed by its change to the next group's unit, under the products
-// of the tile after it.
+// stage a row tile's products are followed by its change to the next group's unit, under the products of the tile after it.
+//
+// With the producer's sums a group begins with its zero-point term, as in the wide kernel, and whole sums are that kernel's to the bit,
+// those left for the next product too.  Sums formed here are there only behind the group's last k-step, and so is its term.
 #pragma once
 #include "awq_common.h"
 
@@ -234,6 +236,20 @@ __global__ void __launch_bounds__(512, 2) awq_tall_kernel(AwqTallArgs a) {
       asm volatile("" : "+v"(R[ct][rt]));  // here, not where the next product needs it
     }
   };
+  // R + (a + b + c) bz, X = a + b + c exactly, three values of the operand type
+  auto zero_point = [&](int rt, float X, const uint32_t(&z)[2]) {
+    const uint32_t xa = __float_as_uint(X) & 0xFFFF0000u;
+    const float r1 = X - __uint_as_float(xa);
+    const uint32_t xb = __float_as_uint(r1) & 0xFFFF0000u;
+    const float r2 = r1 - __uint_as_float(xb);
+    const int4v ax = int4v{(int)((xa >> 16) | xb), (int)(__float_as_uint(r2) >> 16), 0, 0};
+#pragma unroll
+    for (int ct = 0; ct < 2; ++ct)
+      R[ct][rt] = AwqMagic<T>::mma32(ax, int4v{(int)(z[ct] * 0x10001u), (int)z[ct], 0, 0}, R[ct][rt]);
+  };
+  auto given_sum = [&](int slot, int rt) {
+    return reinterpret_cast<const float*>(smem + kXsOff + (slot * 8 + wid) * 512)[32 * rt + r32];
+  };
   float xacc[RT];  // this lane's part of the block sums of the group (without XS)
   auto add_sums = [&](const int4v(&af)[RT]) {
     if constexpr (!XS)
@@ -264,6 +280,9 @@ __global__ void __launch_bounds__(512, 2) awq_tall_kernel(AwqTallArgs a) {
   prep(un, false, 0, ratio);
   read_a(0, af[0]);
   dequant(0, 0, bf[0]);
+  if constexpr (XS)
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) zero_point(rt, given_sum(0, rt), bz);
 
   const int npad = (nst + 1) / 2 * 2;
   for (int i0 = 0; i0 < npad; i0 += 2) {
@@ -299,10 +318,9 @@ __global__ void __launch_bounds__(512, 2) awq_tall_kernel(AwqTallArgs a) {
       __builtin_amdgcn_sched_barrier(0);
       add_sums(af[1]);
       float X[RT];
+      if constexpr (!XS)
 #pragma unroll
-      for (int rt = 0; rt < RT; ++rt)
-        X[rt] = XS ? reinterpret_cast<const float*>(smem + kXsOff + (u * 8 + wid) * 512)[32 * rt + r32]
-                   : xacc[rt] + __shfl_xor(xacc[rt], 32, 64);
+        for (int rt = 0; rt < RT; ++rt) X[rt] = xacc[rt] + __shfl_xor(xacc[rt], 32, 64);
       // everything has landed: the next stage's first half, its weights, scales and sums
       asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)"
                    : "+v"(wreg[u ^ 1][0]), "+v"(wreg[u ^ 1][1]), "+v"(wreg[u ^ 1][2]), "+v"(wreg[u ^ 1][3])::"memory");
@@ -310,36 +328,33 @@ __global__ void __launch_bounds__(512, 2) awq_tall_kernel(AwqTallArgs a) {
       issue_x(i + 1, 1);
       issue_rest(i + 2, u);
       read_unit(u ^ 1, un);
+      if constexpr (XS)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) X[rt] = last ? 0.f : given_sum(u ^ 1, rt);
       const uint32_t bzo[2] = {bz[0], bz[1]};
       int4v na[RT], nb[2];
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
 #pragma unroll
         for (int ct = 0; ct < 2; ++ct) R[ct][rt] = AwqMagic<T>::mma32(af[1][rt], bf[1][ct], R[ct][rt]);
-        // X = a + b + c exactly, three values of the operand type
-        const uint32_t xa = __float_as_uint(X[rt]) & 0xFFFF0000u;
-        const float r1 = X[rt] - __uint_as_float(xa);
-        const uint32_t xb = __float_as_uint(r1) & 0xFFFF0000u;
-        const float r2 = r1 - __uint_as_float(xb);
-        const int4v ax = int4v{(int)((xa >> 16) | xb), (int)(__float_as_uint(r2) >> 16), 0, 0};
-#pragma unroll
-        for (int ct = 0; ct < 2; ++ct)
-          R[ct][rt] = AwqMagic<T>::mma32(ax, int4v{(int)(bzo[ct] * 0x10001u), (int)bzo[ct], 0, 0}, R[ct][rt]);
+        if constexpr (!XS) zero_point(rt, X[rt], bzo);
         na[rt] = *reinterpret_cast<const int4v*>(smem + abase + rt * 4096);
         if (rt == 0) {
           prep(un, last, u ^ 1, ratio);
         } else {
           change_unit(rt - 1, ratio);
+          if constexpr (XS) zero_point(rt - 1, X[rt - 1], bz);
         }
         if (rt == RT - 1) dequant(u ^ 1, 0, nb);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x2, 9, 0);
+          __builtin_amdgcn_sched_group_barrier(0x2, XS ? 18 : 9, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
       change_unit(RT - 1, ratio);
+      if constexpr (XS) zero_point(RT - 1, X[RT - 1], bz);
       if (last) goto done;
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) af[0][rt] = na[rt];
@@ -402,28 +417,34 @@ done:
         }
       }
     __syncthreads();
-    // four threads a row: its pieces, and its sum for the next product's zero-point term
-    const int row = tid >> 2, quarter = tid & 3;
+    // Four threads a row, 8 of every 16 columns each: its pieces, and its sum for the next product's zero-point term, in the wide
+    // kernel's order (a column tile's numbers 16, 8, 4, 2 and 1 apart, then the two tiles)
+    const int row = tid >> 2, ctile = tid >> 1 & 1, odd = tid & 1;
     if (row < 32 * RT && m0 + row < a.M) {
-      const char* src = tile + row * kOutPitch + quarter * 32;
-      uint16_t* dst = a.out + (int64_t)(m0 + row) * a.out_stride + blockIdx.x * 64 + quarter * 16;
-      float sum = 0.f;
+      const int at = 32 * ctile + 8 * odd;
+      const char* src = tile + row * kOutPitch + 2 * at;
+      uint16_t* dst = a.out + (int64_t)(m0 + row) * a.out_stride + blockIdx.x * 64 + at;
+      float sum[8];
 #pragma unroll
       for (int c = 0; c < 2; ++c) {
-        const int4v v = *reinterpret_cast<const int4v*>(src + 16 * c);
+        const int4v v = *reinterpret_cast<const int4v*>(src + 32 * c);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sum = AwqMagic<T>::pair_sum((uint32_t)v[e], sum);
-        if (a.wide_out) {
-          *reinterpret_cast<int4v*>(dst + 8 * c) = v;
-        } else {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) dst[8 * c + e] = (uint16_t)((uint32_t)v[e >> 1] >> (16 * (e & 1)));
+        for (int e = 0; e < 8; ++e) {
+          const uint16_t o = (uint16_t)((uint32_t)v[e >> 1] >> (16 * (e & 1)));
+          sum[e] = c ? sum[e] + Conv<T>::to_f32(o) : Conv<T>::to_f32(o);
+          if (!a.wide_out) dst[16 * c + e] = o;
         }
+        if (a.wide_out) *reinterpret_cast<int4v*>(dst + 16 * c) = v;
       }
       if (a.xsum_out) {
-        sum += __shfl_xor(sum, 1, 64);
-        sum += __shfl_xor(sum, 2, 64);
-        if (quarter == 0) atomicAdd(&a.xsum_out[(int64_t)(blockIdx.x >> 1) * a.xs_out_stride + m0 + row], sum);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) sum[e] += __shfl_xor(sum[e], 1, 64);
+#pragma unroll
+        for (int d = 4; d > 0; d >>= 1)
+#pragma unroll
+          for (int e = 0; e < d; ++e) sum[e] += sum[e + d];
+        sum[0] += __shfl_xor(sum[0], 2, 64);
+        if ((tid & 3) == 0) atomicAdd(&a.xsum_out[(int64_t)(blockIdx.x >> 1) * a.xs_out_stride + m0 + row], sum[0]);
       }
     }
     return;

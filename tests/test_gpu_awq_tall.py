@@ -30,7 +30,8 @@ def _wide(monkeypatch, call):
 @pytest.mark.parametrize("K,inter", [(4096, 14336), (1536, 14336)])
 def test_gated_rows_and_their_sums(monkeypatch, M, K, inter):
     """Every output of the gated form, ragged rows among them, with and without the producer's block sums: the unfused sequence's
-    roundings, so half an ulp of bf16 twice (2^-8 each) beside the product's own 1e-6; rows behind M stay as they were."""
+    roundings, so half an ulp of bf16 twice (2^-8 each) beside the product's own 1e-6; rows behind M stay as they were.  With the
+    producer's sums, rows and the sums left for the next product are the wide kernel's bits."""
     from sglang_security_amd import ops
 
     x, qw, sc, qz = (t.to(DEV) for t in _case(M, K, 2 * inter, M + K))
@@ -42,14 +43,22 @@ def test_gated_rows_and_their_sums(monkeypatch, M, K, inter):
     wide = torch.nn.functional.pad(x, (8, 8))[:, 8:-8]  # rows with a pitch of their own
     sums = x.float().view(M, -1, 128).sum(-1).t().contiguous()
     for rows, xs, pitch in ((x, None, inter), (wide, sums, inter), (x, sums, inter + 4)):
-        buf = torch.full((M + 2, pitch), 7.0, dtype=torch.bfloat16, device=DEV)
-        out, left = buf[:M, :inter], torch.zeros(inter // 128, M, device=DEV)
-        ops.awq_gemm_silu_mul(rows, packed, si, zi, out, xs, left)
+        def call():
+            buf = torch.full((M + 2, pitch), 7.0, dtype=torch.bfloat16, device=DEV)
+            left = torch.zeros(inter // 128, M, device=DEV)
+            ops.awq_gemm_silu_mul(rows, packed, si, zi, buf[:M, :inter], xs, left)
+            return buf, left
+
+        buf, left = call()
+        out = buf[:M, :inter]
         # a sum that falls on the other side of a rounding boundary moves gate or up by an ulp
         torch.testing.assert_close(out.double(), want, rtol=4 * 2 ** -8, atol=2 ** -8 * want.abs().mean().item())
         assert (out.double() - want).norm() / want.norm() < 2 ** -8
         torch.testing.assert_close(left, out.float().view(M, -1, 128).sum(-1).t(), rtol=1e-4, atol=2e-2)
         assert bool((buf[M:] == 7).all()) and bool((buf[:, inter:] == 7).all())
+        if xs is not None:
+            for mine, theirs in zip((buf, left), _wide(monkeypatch, call)):
+                assert torch.equal(mine, theirs)
 
 
 @pytest.mark.parametrize("M,K,N", [(65, 4096, 28672), (128, 2048, 28672), (300, 1024, 16384), (96, 1536, 12288)])
