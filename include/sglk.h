@@ -445,11 +445,14 @@ SGLK_API int sglk_awq_dequantize_packed_nk(const int32_t* packed, const void* sc
  * the matrix cores; W in the sglk_awq_repack layout.  Fuses AWQLinearMethod.apply,
  * python/sglang/srt/layers/quantization/awq.py:197-215 (awq_dequantize + torch.matmul).
  * Computes x @ ((q - z) * s) with (q - z) * s never rounded to half precision (fp32 accumulation).
- * K % 128 == 0, N % 64 == 0, group_size a multiple of 128; any M (rows are processed 64 at a time).
+ * K % 128 == 0, N % 64 == 0, group_size a multiple of 128; any M (rows are processed 64, 96 or 128 at a time).
  * workspace: sglk_awq_gemm_workspace_bytes() bytes, always required.  Its first 16 KiB are split-K ticket
  * counters: they must be zero before the first call and every call leaves them zero, so one zero-filled
  * buffer serves any number of consecutive calls on a stream (calls that overlap on two streams need two). */
 SGLK_API int64_t sglk_awq_gemm_workspace_bytes(int M, int N, int K);
+/* Rows a block, 96 or 128, of the kernel that dequantises a weight once for so many, if it is the one to take a product (gated:
+ * sglk_awq_gemm_silu_mul, else sglk_awq_gemm), and the splits along K; else 0.  Host only. */
+SGLK_API int sglk_awq_gemm_tall_rows(int M, int N, int K, int group_size, int dtype, int gated, int* splits);
 SGLK_API int sglk_awq_gemm(const void* x, const int32_t* packed, const void* scales,
                            const int32_t* qzeros, const void* bias, void* out, float* workspace,
                            int M, int N, int K, int group_size, int64_t x_stride, int64_t out_stride,

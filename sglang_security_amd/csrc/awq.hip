@@ -1624,6 +1624,24 @@ int64_t sglk_awq_gemm_workspace_bytes(int M, int N, int K) {
   return bytes + (int64_t)kMaxTiles * 4;
 }
 
+// What awq_tall.h's kernel makes of a product, if it is the one to take it: whole sums if gated, else as many splits as the slabs of
+// sglk_awq_gemm_workspace_bytes hold.
+static TallPlan tall_plan(int M, int N, int K, int group_size, int dtype, bool gated) {
+  if (M <= kGemmBM) return TallPlan{};
+  TallPlan p = plan_awq_tall(M, N, K, group_size, dtype, gated,
+                             gated ? 0 : sglk_awq_gemm_workspace_bytes(M, N, K) - (int64_t)kMaxTiles * 4);
+  p.ok = p.ok && (gated || p.tiles <= kMaxTiles);
+  return p;
+}
+
+int sglk_awq_gemm_tall_rows(int M, int N, int K, int group_size, int dtype, int gated, int* splits) {
+  if (M <= 0 || N <= 0 || K <= 0 || group_size <= 0) return 0;
+  const TallPlan p = tall_plan(M, N, K, group_size, dtype, gated != 0);
+  if (!p.ok) return 0;
+  if (splits) *splits = p.splits;
+  return 32 * p.rt;
+}
+
 static int launch_awq_wide(const WidePlan& wp, const void* x, const int32_t* packed, const void* scales,
                            const int32_t* qzeros, const void* bias, void* out, float* partial, int* tickets, int M, int N,
                            int K, int64_t x_stride, int64_t out_stride, int dtype, const float* xsum, int64_t xs_stride,
@@ -1726,7 +1744,7 @@ int sglk_awq_gemm_silu_mul(const void* x, const int32_t* packed, const void* sca
   SGLK_CHECK(!xsum || xs_stride >= M, "awq_gemm_silu_mul: xs_stride smaller than M");
   SGLK_CHECK(!xsum_out || xs_out_stride >= M, "awq_gemm_silu_mul: xs_out_stride smaller than M");
   // the activation needs whole sums: one split, whatever the planner would pick
-  if (const TallPlan tp = plan_awq_tall(M, N, K, group_size, dtype, true); tp.ok && x_stride < kTallMaxStride)
+  if (const TallPlan tp = tall_plan(M, N, K, group_size, dtype, true); tp.ok && x_stride < kTallMaxStride)
     return launch_awq_tall(tp,
                            AwqTallArgs{(const uint16_t*)x, packed, (const uint16_t*)scales, qzeros, nullptr, (uint16_t*)out,
                                        nullptr, nullptr, xsum, xsum_out, x_stride, out_stride, xs_stride, xs_out_stride, M, N, K,
@@ -1860,16 +1878,12 @@ int sglk_awq_gemm_xs(const void* x, const int32_t* packed, const void* scales, c
   hipStream_t s = (hipStream_t)stream;
   int* tickets = reinterpret_cast<int*>(workspace);
   float* partial = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + (int64_t)kMaxTiles * 4);
-  if (M > kGemmBM) {
-    const TallPlan tp = plan_awq_tall(M, N, K, group_size, dtype, false,
-                                      sglk_awq_gemm_workspace_bytes(M, N, K) - (int64_t)kMaxTiles * 4);
-    if (tp.ok && tp.tiles <= kMaxTiles && x_stride < kTallMaxStride)
-      return launch_awq_tall(tp,
-                             AwqTallArgs{(const uint16_t*)x, packed, (const uint16_t*)scales, qzeros, (const uint16_t*)bias,
-                                         (uint16_t*)out, partial, tickets, xsum, nullptr, x_stride, out_stride, xs_stride, 0, M,
-                                         N, K, 0, 0, 0, 0},
-                             s);
-  }
+  if (const TallPlan tp = tall_plan(M, N, K, group_size, dtype, false); tp.ok && x_stride < kTallMaxStride)
+    return launch_awq_tall(tp,
+                           AwqTallArgs{(const uint16_t*)x, packed, (const uint16_t*)scales, qzeros, (const uint16_t*)bias,
+                                       (uint16_t*)out, partial, tickets, xsum, nullptr, x_stride, out_stride, xs_stride, 0, M,
+                                       N, K, 0, 0, 0, 0},
+                           s);
   const WidePlan wp = plan_awq_wide(M, N, K, group_size);
   // few rows: also where a split is a single stage, as long as the slabs (a quarter of the wide kernel's) fit the workspace
   // that sglk_awq_gemm_workspace_bytes names

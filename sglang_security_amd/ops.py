@@ -648,6 +648,13 @@ def awq_gemm_workspace_bytes(M, N, K) -> int:
     return int(lib().sglk_awq_gemm_workspace_bytes(M, N, K))
 
 
+def awq_gemm_tall_rows(M, N, K, group=128, dtype=torch.bfloat16, gated=False):
+    """(rows a block, splits along K) where awq_gemm (gated: awq_gemm_silu_mul) takes blocks of 96 or 128 rows, else None."""
+    splits = C.c_int(0)
+    rows = lib().sglk_awq_gemm_tall_rows(M, N, K, group, dtype_code(dtype), int(gated), C.byref(splits))
+    return (rows, splits.value) if rows else None
+
+
 def awq_gemm(x, packed, scales, qzeros, bias=None, out=None, workspace=None):
     """x:[M,K] @ W -> [M,N]; packed from awq_repack(qweight)."""
     _need_gpu(x, packed, scales, qzeros)

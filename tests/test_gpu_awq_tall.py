@@ -26,14 +26,23 @@ def _wide(monkeypatch, call):
     return out
 
 
-@pytest.mark.parametrize("M", [65, 96, 97, 128, 192, 200, 255])
-@pytest.mark.parametrize("K,inter", [(4096, 14336), (1536, 14336)])
-def test_gated_rows_and_their_sums(monkeypatch, M, K, inter):
+def _takes(M, N, K, rows, splits=1, gated=False):
+    """The size is one that blocks of so many rows take, K in so many splits."""
+    from sglang_security_amd import ops
+
+    assert ops.awq_gemm_tall_rows(M, N, K, gated=gated) == (rows, splits)
+
+
+@pytest.mark.parametrize("M,K,inter,block", [(65, 4096, 14336, 96), (96, 4096, 14336, 96), (97, 4096, 14336, 128), (128, 4096, 14336, 128),
+                                            (192, 4096, 14336, 96), (200, 4096, 14336, 128), (255, 4096, 14336, 128),
+                                            (65, 1024, 8320, 96), (96, 1536, 14336, 96), (97, 1536, 8320, 128), (128, 2560, 8320, 128)])
+def test_gated_rows_and_their_sums(monkeypatch, M, K, inter, block):
     """Every output of the gated form, ragged rows among them, with and without the producer's block sums: the unfused sequence's
     roundings, so half an ulp of bf16 twice (2^-8 each) beside the product's own 1e-6; rows behind M stay as they were.  With the
     producer's sums, rows and the sums left for the next product are the wide kernel's bits."""
     from sglang_security_amd import ops
 
+    _takes(M, 2 * inter, K, block, gated=True)
     x, qw, sc, qz = (t.to(DEV) for t in _case(M, K, 2 * inter, M + K))
     qi, si, zi = ops.awq_interleave_gate_up(qw, sc, qz)
     packed = ops.awq_repack(qi)
@@ -61,52 +70,74 @@ def test_gated_rows_and_their_sums(monkeypatch, M, K, inter):
                 assert torch.equal(mine, theirs)
 
 
-@pytest.mark.parametrize("M,K,N", [(65, 4096, 28672), (128, 2048, 28672), (300, 1024, 16384), (96, 1536, 12288)])
-def test_finished_rows(monkeypatch, M, K, N):
-    """Finished rows with a bias, twice over one workspace, no further from 64 bits than the wide kernel's: what is left after the
-    rounding to bf16 is that rounding."""
+@pytest.mark.parametrize("M,K,N,rows,splits", [(65, 4096, 28672, 96, 1), (96, 1024, 16640, 96, 1), (97, 1536, 16640, 128, 1),
+                                               (128, 2560, 16640, 128, 1), (80, 5632, 11008, 96, 2), (192, 28672, 8192, 96, 2),
+                                               (128, 8192, 10240, 128, 2), (97, 13824, 8448, 128, 3), (65, 13824, 5120, 96, 4),
+                                               (255, 24576, 3072, 128, 4), (65, 9728, 16640, 96, 5), (96, 18432, 3072, 96, 6)])
+def test_finished_rows(monkeypatch, M, K, N, rows, splits):
+    """Finished rows with a bias, whole and split along K, twice over one workspace of the size that is asked for, no further from 64
+    bits than the wide kernel's: what is left after the rounding to bf16 is that rounding."""
     from sglang_security_amd import ops
 
+    _takes(M, N, K, rows, splits)
     x, qw, sc, qz = (t.to(DEV) for t in _case(M, K, N, K + N))
     bias = torch.randn(N, device=DEV).to(torch.bfloat16)
     packed = ops.awq_repack(qw)
-    want = x.double() @ _weight64(qw, sc, qz) + bias.double()
-    work = torch.zeros(max(ops.awq_gemm_workspace_bytes(M, N, K), 256), dtype=torch.uint8, device=DEV)
-    call = lambda: ops.awq_gemm(x, packed, sc, qz, bias, None, work)
-    got, again = call(), call()
-    assert torch.equal(got, again)
-    err = lambda t: ((t.double() - want).norm() / want.norm()).item()
-    assert err(got) <= 1.01 * err(_wide(monkeypatch, call))
+    want = x.double() @ _weight64(qw, sc, qz)
+    size = ops.awq_gemm_workspace_bytes(M, N, K)
+    work = torch.zeros(size + 4096, dtype=torch.uint8, device=DEV)
+    work[size:] = 7
+    sums = x.float().view(M, -1, 128).sum(-1).t().contiguous()
+    err = lambda t, w: ((t.double() - w).norm() / w.norm()).item()
+    finished = lambda: ops.awq_gemm(x, packed, sc, qz, bias, None, work)
+
+    def with_sums():
+        buf = torch.full((M + 2, N + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+        ops.awq_gemm_xs(x, packed, sc, qz, sums, buf[:M, :N], work)
+        assert bool((buf[M:] == 7).all()) and bool((buf[:, N:] == 7).all())
+        return buf[:M, :N]
+
+    for call, exact in ((finished, want + bias.double()), (with_sums, want)):
+        got, again = call(), call()
+        assert torch.equal(got, again)
+        assert bool((work[size:] == 7).all()) and not bool(work[: 4 * 4096].any())   # tickets are left at zero
+        assert err(got, exact) <= 1.01 * err(_wide(monkeypatch, call), exact)
 
 
-def test_zero_scales_and_few_stages(monkeypatch):
-    """Columns whose scale is zero in the first, a middle, the last or all groups, over one to three stages: nothing from there, the
-    rest as before; a capture replays the same bits."""
+@pytest.mark.parametrize("M,K,rows", [(96, 1024, 96), (80, 1536, 96), (128, 1536, 128), (100, 2560, 128)])
+def test_zero_scales_and_few_stages(monkeypatch, M, K, rows):
+    """Columns whose scale is zero in the first, a middle, the last or all groups, over two, three and five stages: nothing from there,
+    the rest as before; a capture replays the same bits."""
     from sglang_security_amd import ops
 
-    for K in (512, 1024, 1536):
-        M, inter = 128, 14336
-        x, qw, sc, qz = (t.to(DEV) for t in _case(M, K, 2 * inter, K))
-        sc[0, 0::7] = 0
-        sc[K // 256, 1::7] = 0
-        sc[-1, 2::7] = 0
-        sc[:, 3::7] = 0
-        qi, si, zi = ops.awq_interleave_gate_up(qw, sc, qz)
-        packed = ops.awq_repack(qi)
-        gu = (x.double() @ _weight64(qw, sc, qz)).to(torch.bfloat16).double()
-        want = torch.nn.functional.silu(gu[:, :inter]).to(torch.bfloat16).double() * gu[:, inter:]
-        out = torch.empty(M, inter, dtype=torch.bfloat16, device=DEV)
-        stream = torch.cuda.Stream()
-        with torch.cuda.stream(stream):
-            ops.awq_gemm_silu_mul(x, packed, si, zi, out)
+    inter = 8320
+    _takes(M, 2 * inter, K, rows, gated=True)
+    x, qw, sc, qz = (t.to(DEV) for t in _case(M, K, 2 * inter, K))
+    sc[0, 0::7] = 0
+    sc[K // 256, 1::7] = 0
+    sc[-1, 2::7] = 0
+    sc[:, 3::7] = 0
+    qi, si, zi = ops.awq_interleave_gate_up(qw, sc, qz)
+    packed = ops.awq_repack(qi)
+    gu = (x.double() @ _weight64(qw, sc, qz)).to(torch.bfloat16).double()
+    want = torch.nn.functional.silu(gu[:, :inter]).to(torch.bfloat16).double() * gu[:, inter:]
+    sums = x.float().view(M, -1, 128).sum(-1).t().contiguous()
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        for xs in (None, sums):
+            out = torch.empty(M, inter, dtype=torch.bfloat16, device=DEV)
+            ops.awq_gemm_silu_mul(x, packed, si, zi, out, xs)
             eager = out.clone()
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph, stream=stream):
-                ops.awq_gemm_silu_mul(x, packed, si, zi, out)
+                ops.awq_gemm_silu_mul(x, packed, si, zi, out, xs)
             for _ in range(2):
                 out.zero_()
                 graph.replay()
                 stream.synchronize()
                 assert torch.equal(out, eager)
-        assert (eager.double() - want).norm() / want.norm() < 2 ** -8
-        assert bool((eager[:, 3::7] == 0).all())
+            assert (eager.double() - want).norm() / want.norm() < 2 ** -8
+            assert bool((eager[:, 3::7] == 0).all())
+            if xs is not None:
+                assert torch.equal(eager, _wide(monkeypatch, lambda: ops.awq_gemm_silu_mul(x, packed, si, zi, out, xs).clone()))
