@@ -626,6 +626,9 @@ SGLK_API int sglk_awq_gemm_prefill(const void* x, const int32_t* packed, const v
 SGLK_API int sglk_awq_gemm_prefill_silu_mul(const void* x, const int32_t* packed, const void* scales, const int32_t* qzeros,
                                             void* out, int M, int N, int K, int group_size, int64_t x_stride,
                                             int64_t out_stride, int dtype, void* stream);
+/* How the two cut a product: tiles[5] = { rows a block, row tiles, strips of 256 columns, narrower strips behind them, their columns }.
+ * Host only. */
+SGLK_API int sglk_awq_gemm_prefill_tiles(int M, int N, int K, int gated, int* tiles);
 /* Whether sglk_awq_gemm_prefill is expected to be faster than a dequantisation to memory and a library product. */
 SGLK_API int sglk_awq_prefill_fused(int M, int N, int K);
 SGLK_API int sglk_dense_gemm_prefill(const void* x, const void* w, const void* bias, void* out, int M, int N, int K,

@@ -301,6 +301,14 @@ int sglk_awq_gemm_prefill_silu_mul(const void* x, const int32_t* packed, const v
   return SGLK_OK;
 }
 
+int sglk_awq_gemm_prefill_tiles(int M, int N, int K, int gated, int* tiles) {
+  SGLK_CHECK(tiles && M > 0 && N > 0 && K > 0, "awq_gemm_prefill_tiles: bad argument");
+  const PrefillPlan p = prefill_plan(M, N, K, true, gated != 0);
+  const int all[5] = {64 * p.mi, p.mt, p.whole, p.tail, p.narrow};
+  std::copy(all, all + 5, tiles);
+  return SGLK_OK;
+}
+
 // The other way: the weight dequantised to memory (2.5 bytes of traffic a weight), then the library's product, which needs its
 // weights' way from memory, its operations or a chain along K, whichever is longest.  Below four million weights nothing was
 // measured, and the library keeps them.  Measured, library and here: 1152 x 28672 x 4096 300 and 254 us, 500 rows 154 and 110, 256

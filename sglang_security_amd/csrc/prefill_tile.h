@@ -122,12 +122,15 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& p, char* lds, in
     const char* src = reinterpret_cast<const char*>(p.w) + (int64_t)min(kb, nkb - 1) * nstrips * 1024;
     asm volatile("global_load_dwordx4 %0, %1, %2" : "=&v"(wreg[set][t]) : "v"(woff[t]), "s"(src) : "memory");
   };
-  const int col0 = min(first * 16, p.N - 16 * NJ);  // N % 128 == 0: a wave's columns lie inside, or none does
+  // scales and zeros of strip t lie behind those of the wave's first one.  Of 48 columns the last 16 or 32 may lie past N: their
+  // lanes ask for nothing, and what is made of them is never stored.  A wave that has no column takes the last ones.
+  const int col0 = first < nstrips ? first * 16 : p.N - 16 * NJ;
+  const int live = min(NJ, nstrips - col0 / 16);
   auto load_sz = [&](int kb, int slot, int which) {
     const int gq = min(kb, nkb - 1) * 128 / p.group_size;
     const char* src = which == 0 ? reinterpret_cast<const char*>(p.scales + (int64_t)gq * p.N + col0)
                                  : reinterpret_cast<const char*>(p.qzeros + (int64_t)gq * (p.N / 8) + col0 / 8);
-    const uint64_t mask = which == 0 ? (1ull << (8 * NJ)) - 1 : (1ull << (2 * NJ)) - 1;
+    const uint64_t mask = (1ull << (which == 0 ? 8 * live : 2 * live)) - 1;
     uint64_t saved;
     asm volatile(
         "s_mov_b32 m0, %1\n\t"

@@ -701,6 +701,13 @@ def awq_gemm_prefill_silu_mul(x, packed, scales, qzeros, out):
     return out
 
 
+def awq_gemm_prefill_tiles(M, N, K, gated=False):
+    """(rows a block, row tiles, strips of 256 columns, narrower strips behind them, their columns) of such a product."""
+    tiles = (C.c_int * 5)()
+    check(lib().sglk_awq_gemm_prefill_tiles(M, N, K, int(gated), tiles), "awq_gemm_prefill_tiles")
+    return tuple(tiles)
+
+
 def awq_prefill_fused(M, N, K) -> bool:
     """Whether awq_gemm_prefill is expected to be faster than dequantising the weight and a library product."""
     return bool(lib().sglk_awq_prefill_fused(M, N, K))

@@ -46,6 +46,20 @@ def test_int4_gives_the_bits_of_its_dequantised_weights(M, K, N, group, dtype):
     assert ((got.double() - want).abs() <= unit * want.abs() + 1e-5 * want.abs().max()).all()
 
 
+# strips of 192 columns of which the last has 64 or 128: 128, 192 and 256 rows a block, behind whole strips of 256 and without any
+@pytest.mark.parametrize("M,K,N,rows,left", [(627, 128, 6784, 128, 64), (627, 256, 6656, 128, 128), (563, 128, 22016, 128, 128),
+                                             (1600, 384, 4096, 192, 64), (819, 128, 7424, 192, 128), (2355, 128, 7424, 192, 64),
+                                             (2112, 256, 4096, 256, 64), (1100, 256, 7168, 256, 64), (800, 128, 27648, 256, 128),
+                                             (3200, 128, 28672, 256, 128), (3700, 128, 28672, 256, 64)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_a_last_strip_that_is_not_full(M, K, N, rows, left, dtype):
+    from sglang_security_amd import ops
+
+    block, _, whole, _, narrow = ops.awq_gemm_prefill_tiles(M, N, K)
+    assert (block, narrow, (N - 256 * whole) % narrow) == (rows, 192, left)
+    test_int4_gives_the_bits_of_its_dequantised_weights(M, K, N, 128, dtype)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_values_that_are_not_finite(dtype):
     """Infinite and NaN scales and activations reach what they reach through the dequantised weights, and nothing else."""
