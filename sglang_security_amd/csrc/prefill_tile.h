@@ -20,20 +20,15 @@
 namespace sglk {
 
 // acc += a . b.  PINNED: where the text stands.  Left to the compiler, products gather behind the requests and conversions that are
-// to run under them.  (Nobody reads an accumulator before the loop is over, and the same one comes up again half of P products later.)
+// to run under them.  The instruction itself is the compiler's, which knows how long its sums take: written out as text, a copy of an
+// accumulator that it places behind one would read them too early.
 template <typename T, bool PINNED>
 __device__ __forceinline__ void prefill_mma(float16v& acc, int4v a, int4v b) {
-  if constexpr (std::is_same<T, bf16_t>::value) {
-    if constexpr (PINNED)
-      asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
-    else
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bfloat8, a), __builtin_bit_cast(bfloat8, b), acc, 0, 0, 0);
-  } else {
-    if constexpr (PINNED)
-      asm volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+a"(acc) : "v"(a), "v"(b));
-    else
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), acc, 0, 0, 0);
-  }
+  if constexpr (std::is_same<T, bf16_t>::value)
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bfloat8, a), __builtin_bit_cast(bfloat8, b), acc, 0, 0, 0);
+  else
+    acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), acc, 0, 0, 0);
+  if constexpr (PINNED) asm volatile("" : "+a"(acc));
 }
 
 // two numbers, each rounded to nearest
@@ -338,7 +333,7 @@ __device__ __forceinline__ void prefill_tile(const PrefillArgs& p, char* lds, in
   }
   (void)pb;
 
-  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");  // and the last products are through
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
 #pragma unroll
   for (int i = 0; i < SW; ++i) landed(i);
   __builtin_amdgcn_s_barrier();

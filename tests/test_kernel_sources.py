@@ -16,3 +16,11 @@ def test_ring_barriers_wait_for_lds_reads():
             seen += 1
             assert "vmcnt" in m[1] and "lgkmcnt(0)" in m[1], (os.path.basename(path), m[0])
     assert seen >= 2
+
+
+def test_matrix_instructions_are_the_compilers():
+    """A matrix instruction written out as text leaves its sums some cycles later without the compiler knowing: it may place a copy of them
+    right behind.  Only the builtins carry that."""
+    for path in glob.glob(os.path.join(CSRC, "*.h")) + glob.glob(os.path.join(CSRC, "*.hip")):
+        src = re.sub(r"//[^\n]*", "", open(path).read())
+        assert not re.search(r'"[^"]*v_s?mfma', src), os.path.basename(path)
