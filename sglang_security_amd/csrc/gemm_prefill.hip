@@ -3,8 +3,8 @@
 //     ((q - z) * scale rounded to the activation type: the very weights the reference's
 //     awq_dequantize-then-matmul multiplies by, python/sglang/srt/layers/quantization/awq.py:197-215), and
 //   * dense 16-bit weights [N, K] (bf16 / fp16 checkpoints: layers/linear.py UnquantizedLinearMethod).
-// prefill_tile.h holds the kernel.  The one below serves rows whose pitch is beyond its 32-bit offsets: a block of four waves owns a
-// 256 x 128 output tile and walks K in steps of 32 through two LDS stages (A: 256 rows x 64 bytes, B: 128 columns x 64 bytes, k
+// prefill_tile.h holds the kernel.  The one below serves rows whose pitch is beyond its 32-bit offsets, and scales and biases that do not
+// start where it loads them from, at a multiple of 4 and of 8 bytes: a block of four waves owns a 256 x 128 output tile and walks K in steps of 32 through two LDS stages (A: 256 rows x 64 bytes, B: 128 columns x 64 bytes, k
 // contiguous in both, 16-byte chunks XOR-swizzled by (row >> 2) & 3); rows travel global -> registers while the current stage is
 // multiplied, and are parked (the int4 words dequantised first) before the one barrier per stage.
 #include <algorithm>
@@ -238,10 +238,11 @@ static int launch_prefill(const PrefillArgs& a, hipStream_t s) {
 }
 
 static constexpr int64_t kPrefillPitch = 1 << 23;  // 256 rows of less than that span less than 2^32 bytes
+static bool starts_at(const void* p, uintptr_t multiple) { return reinterpret_cast<uintptr_t>(p) % multiple == 0; }
 
 template <typename T, bool AWQ>
 static int launch_prefill_any(const PrefillArgs& a, hipStream_t s) {
-  if (a.x_stride >= kPrefillPitch || a.w_stride >= kPrefillPitch) {
+  if (a.x_stride >= kPrefillPitch || a.w_stride >= kPrefillPitch || !starts_at(a.scales, 4) || !starts_at(a.bias, 8)) {
     const dim3 grid((a.M + kPfBM - 1) / kPfBM, a.N / kPfBN);
     hipLaunchKernelGGL((prefill_gemm_kernel<T, AWQ>), grid, dim3(256), kPfLds, s, a.x, a.w, a.scales, a.qzeros, a.bias, a.out, a.M,
                        a.N, a.K, a.group_size, a.x_stride, a.w_stride, a.out_stride);
@@ -295,6 +296,7 @@ int sglk_awq_gemm_prefill_silu_mul(const void* x, const int32_t* packed, const v
   SGLK_CHECK(group_size > 0 && group_size % 128 == 0 && K % group_size == 0,
              "awq_gemm_prefill_silu_mul: group size %d must be a multiple of 128 that divides K", group_size);
   SGLK_CHECK(x_stride < kPrefillPitch, "awq_gemm_prefill_silu_mul: rows %lld elements apart", (long long)x_stride);
+  SGLK_CHECK(starts_at(scales, 4), "awq_gemm_prefill_silu_mul: scales must be 4-byte aligned");
   const PrefillArgs a{(const uint16_t*)x, packed, (const uint16_t*)scales, qzeros, nullptr, (uint16_t*)out, M, N, K,
                       group_size, x_stride, 0, out_stride, 1, 0, 0, 0, 0};
   SGLK_DISPATCH_HALF(dtype, T, { return (launch_prefill_any<T, true>(a, (hipStream_t)stream)); });

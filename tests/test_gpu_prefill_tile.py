@@ -61,6 +61,28 @@ def test_a_last_strip_that_is_not_full(M, K, N, rows, left, dtype):
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_scales_and_biases_that_start_anywhere(dtype):
+    """Scales off 4 bytes, biases off 8: the same numbers as from aligned copies (the gated form, which asks for whole pairs, refuses)."""
+    from sglang_security_amd import ops
+    from sglang_security_amd._lib import SglkError
+
+    M, K, N = 300, 256, 512
+    qw, sc, qz, g = _int4(K, N, dtype, 11)
+    x = torch.randn(M, K, device=DEV, generator=g).to(dtype)
+    off = lambda t: torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)
+    bias = torch.randn(N, device=DEV, generator=g).to(dtype)
+    packed = ops.awq_repack(qw)
+    w = ops.awq_dequantize_packed_nk(packed, sc, qz)
+    want = x.double() @ w.double().t() + bias.double()
+    unit = 2 ** -8 if dtype == torch.bfloat16 else 2 ** -11   # as above
+    for got in (ops.awq_gemm_prefill(x, packed, off(sc), qz, bias), ops.awq_gemm_prefill(x, packed, sc, qz, off(bias)),
+                ops.dense_gemm_prefill(x, w, off(bias))):
+        assert ((got.double() - want).abs() <= unit * want.abs() + 1e-5 * want.abs().max()).all()
+    with pytest.raises(SglkError):
+        ops.awq_gemm_prefill_silu_mul(x, packed, off(sc), qz, torch.empty(M, N // 2, dtype=dtype, device=DEV))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_values_that_are_not_finite(dtype):
     """Infinite and NaN scales and activations reach what they reach through the dequantised weights, and nothing else."""
     from sglang_security_amd import ops
