@@ -677,11 +677,21 @@ def awq_gemm(x, packed, scales, qzeros, bias=None, out=None, workspace=None):
     return out
 
 
+def _packed_weight(what, x, packed, scales, qzeros):
+    """M, N, K of x @ W; the kernels take the rows' type and length for the weight's, so both are looked at here."""
+    M, K = x.shape
+    N = scales.shape[1]
+    if x.dtype != scales.dtype:
+        raise SglkError(f"{what}: activation and scale dtypes differ")
+    if tuple(packed.shape) != (K, N // 8) or tuple(qzeros.shape) != (scales.shape[0], N // 8):
+        raise SglkError(f"{what}: rows of {K}, but a weight of {tuple(packed.shape)} words and zeros of {tuple(qzeros.shape)} for {N} columns")
+    return M, N, K
+
+
 def awq_gemm_prefill(x, packed, scales, qzeros, bias=None, out=None):
     """Large-M x @ W for a packed AWQ weight, dequantised inside the GEMM (K % 128 == 0, N % 128 == 0)."""
     _need_gpu(x, packed, scales, qzeros)
-    M, K = x.shape
-    N = scales.shape[1]
+    M, N, K = _packed_weight("awq_gemm_prefill", x, packed, scales, qzeros)
     if out is None:
         out = torch.empty(M, N, dtype=x.dtype, device=x.device)
     check(lib().sglk_awq_gemm_prefill(_ptr(x), _ptr(packed), _ptr(scales), _ptr(qzeros), _ptr(bias), _ptr(out), M, N, K,
@@ -693,8 +703,7 @@ def awq_gemm_prefill(x, packed, scales, qzeros, bias=None, out=None):
 def awq_gemm_prefill_silu_mul(x, packed, scales, qzeros, out):
     """out[M, N/2] = silu(x @ W_gate) * (x @ W_up) for many rows, on a weight interleaved by awq_interleave_gate_up."""
     _need_gpu(x, packed, scales, qzeros, out)
-    M, K = x.shape
-    N = scales.shape[1]
+    M, N, K = _packed_weight("awq_gemm_prefill_silu_mul", x, packed, scales, qzeros)
     check(lib().sglk_awq_gemm_prefill_silu_mul(_ptr(x), _ptr(packed), _ptr(scales), _ptr(qzeros), _ptr(out), M, N, K,
                                                K // scales.shape[0], x.stride(0), out.stride(0), dtype_code(x.dtype), _stream(x)),
           "awq_gemm_prefill_silu_mul")

@@ -106,6 +106,14 @@ class AWQLinearMethod:
             layer.sglk_workspace = ws
         return ws
 
+    @staticmethod
+    def _kernel_rows(layer, x: torch.Tensor) -> Optional[torch.Tensor]:
+        """x as the product that dequantises on the way takes it, or None where only the library does: another type, length or device
+        than the weight's (which it refuses)."""
+        if x.dtype != layer.scales.dtype or x.shape[1] != layer.sglk_shape[0] or x.device != layer.scales.device:
+            return None
+        return x.contiguous()
+
     def apply(self, layer: torch.nn.Module, x: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
         """awq.py:197-215."""
         k, n = layer.sglk_shape
@@ -117,10 +125,12 @@ class AWQLinearMethod:
                                self._workspace(layer, m, x.device))
             return out.reshape(out_shape)
         if m > 0 and layer.sglk_fusable and n % 128 == 0 and ops.awq_prefill_fused(m, n, k):
-            out = ops.awq_gemm_prefill(x2.contiguous(), layer.sglk_packed, layer.scales, layer.qzeros)
-            if bias is not None:
-                out.add_(bias)
-            return out.reshape(out_shape)
+            rows = self._kernel_rows(layer, x2)
+            if rows is not None:
+                out = ops.awq_gemm_prefill(rows, layer.sglk_packed, layer.scales, layer.qzeros)
+                if bias is not None:
+                    out.add_(bias)
+                return out.reshape(out_shape)
         if layer.qweight is not None:
             w = ops.awq_dequantize(layer.qweight, layer.scales, layer.qzeros)
         else:

@@ -1,7 +1,12 @@
-"""CPU: which int4 products of many rows go where: the tiles a plan cuts."""
+"""CPU: which int4 products of many rows go where -- the tiles a plan cuts, and the rows that only the library takes."""
+from types import SimpleNamespace
+
 import pytest
+import torch
 
 from sglang_security_amd import ops
+from sglang_security_amd._lib import SglkError
+from sglang_security_amd.quantization.awq import AWQLinearMethod
 
 
 @pytest.mark.parametrize("gated", [False, True])
@@ -20,3 +25,27 @@ def test_tiles_cover_a_product_once(gated):
                 else:
                     assert -256 < rest <= 0
     assert gated or ragged > 20
+
+
+def _layer(k, n, dtype):
+    return SimpleNamespace(sglk_shape=(k, n), scales=torch.ones(k // 128, n, dtype=dtype))
+
+
+def test_rows_of_another_type_or_length_are_the_librarys():
+    """(which refuses them)"""
+    layer = _layer(256, 128, torch.bfloat16)
+    for rows in (torch.randn(4, 256).half(), torch.randn(4, 256), torch.randn(4, 512).to(torch.bfloat16)):
+        assert AWQLinearMethod._kernel_rows(layer, rows) is None
+
+
+def test_a_weight_of_another_type_or_shape_is_refused():
+    """The kernel would read scales as the rows' type and words for the rows' length."""
+    w = lambda k, n: (torch.zeros(k, n // 8, dtype=torch.int32), torch.ones(k // 128, n, dtype=torch.bfloat16),
+                      torch.zeros(k // 128, n // 8, dtype=torch.int32))
+    rows = torch.zeros(3, 256, dtype=torch.bfloat16)
+    assert ops._packed_weight("product", rows, *w(256, 128)) == (3, 128, 256)
+    packed, scales, zeros = w(256, 128)
+    for args in ((rows.half(), packed, scales, zeros), (torch.zeros(3, 512, dtype=torch.bfloat16), packed, scales, zeros),
+                 (rows, packed[:, :8], scales, zeros), (rows, packed, scales, zeros[:1])):
+        with pytest.raises(SglkError):
+            ops._packed_weight("product", *args)

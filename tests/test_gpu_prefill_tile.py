@@ -132,6 +132,27 @@ def test_linear_method_of_many_rows():
         assert ((got.double() - want.double()).norm() / want.double().norm()).item() < 2 ** -8
 
 
+def _linear(M, K, N):
+    from types import SimpleNamespace
+
+    from sglang_security_amd import ops
+
+    qw, sc, qz, g = _int4(K, N, torch.bfloat16, M)
+    layer = SimpleNamespace(sglk_shape=(K, N), sglk_fusable=True, sglk_packed=ops.awq_repack(qw), scales=sc, qzeros=qz, qweight=None)
+    assert ops.awq_prefill_fused(M, N, K)
+    return layer, torch.randn(M * K + 8, device=DEV, generator=g).to(torch.bfloat16)
+
+
+def test_linear_method_refuses_rows_of_another_type_or_length():
+    from sglang_security_amd.quantization.awq import AWQLinearMethod
+
+    layer, flat = _linear(300, 4096, 28672)
+    rows = flat[: 300 * 4096].view(300, 4096)
+    for wrong in (rows.half(), rows.float(), rows[:, :2048], rows.view(150, 8192).repeat(2, 1)):
+        with pytest.raises(RuntimeError):
+            AWQLinearMethod(None).apply(layer, wrong)
+
+
 def test_rule_stays_where_it_was_measured():
     from sglang_security_amd import ops
 
