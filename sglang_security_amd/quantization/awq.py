@@ -109,10 +109,11 @@ class AWQLinearMethod:
     @staticmethod
     def _kernel_rows(layer, x: torch.Tensor) -> Optional[torch.Tensor]:
         """x as the product that dequantises on the way takes it, or None where only the library does: another type, length or device
-        than the weight's (which it refuses)."""
+        than the weight's (which it refuses), and rows off 16 bytes."""
         if x.dtype != layer.scales.dtype or x.shape[1] != layer.sglk_shape[0] or x.device != layer.scales.device:
             return None
-        return x.contiguous()
+        x = x.contiguous()
+        return x if x.data_ptr() % 16 == 0 and x.stride(0) % 8 == 0 else None
 
     def apply(self, layer: torch.nn.Module, x: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
         """awq.py:197-215."""

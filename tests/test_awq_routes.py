@@ -31,6 +31,17 @@ def _layer(k, n, dtype):
     return SimpleNamespace(sglk_shape=(k, n), scales=torch.ones(k // 128, n, dtype=dtype))
 
 
+def test_rows_that_start_off_16_bytes_are_the_librarys():
+    layer, flat = _layer(256, 128, torch.bfloat16), torch.randn(4 * 256 + 8).to(torch.bfloat16)
+    rows = flat[8:].view(4, 256)
+    assert AWQLinearMethod._kernel_rows(layer, rows) is rows
+    assert AWQLinearMethod._kernel_rows(layer, flat[1: 1 + 4 * 256].view(4, 256)) is None
+    copied = AWQLinearMethod._kernel_rows(layer, flat[1: 1 + 4 * 256].view(256, 4).t())   # a copy of its own is in place
+    assert copied.is_contiguous() and copied.data_ptr() % 16 == 0
+    one = flat[: 2 * 260].as_strided((1, 256), (260 + 1, 1))
+    assert one.is_contiguous() and AWQLinearMethod._kernel_rows(layer, one) is None       # a pitch off 16 bytes
+
+
 def test_rows_of_another_type_or_length_are_the_librarys():
     """(which refuses them)"""
     layer = _layer(256, 128, torch.bfloat16)

@@ -143,6 +143,16 @@ def _linear(M, K, N):
     return layer, torch.randn(M * K + 8, device=DEV, generator=g).to(torch.bfloat16)
 
 
+def test_linear_method_takes_rows_that_start_anywhere():
+    from sglang_security_amd.quantization.awq import AWQLinearMethod
+
+    layer, flat = _linear(300, 4096, 28672)
+    rows = lambda at: flat[at: at + 300 * 4096].view(300, 4096)
+    got = AWQLinearMethod(None).apply(layer, rows(1))
+    want = AWQLinearMethod(None).apply(layer, rows(1).clone())
+    assert ((got.double() - want.double()).norm() / want.double().norm()).item() < 2 ** -8   # a rounding each, sums in another order
+
+
 def test_linear_method_refuses_rows_of_another_type_or_length():
     from sglang_security_amd.quantization.awq import AWQLinearMethod
 
