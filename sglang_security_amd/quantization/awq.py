@@ -109,7 +109,12 @@ class AWQLinearMethod:
     @staticmethod
     def _kernel_rows(layer, x: torch.Tensor) -> Optional[torch.Tensor]:
         """x as the product that dequantises on the way takes it, or None where only the library does: another type, length or device
-        than the weight's (which it refuses), and rows off 16 bytes."""
+        than the weight's (which it refuses), rows off 16 bytes, and rows that autograd, autocast, a transform or a trace looks at."""
+        if (type(x) not in (torch.Tensor, torch.nn.Parameter) or torch._C._functorch.is_functorch_wrapped_tensor(x)
+                or torch.jit.is_tracing() or (x.requires_grad and torch.is_grad_enabled())
+                or torch.autograd.forward_ad.unpack_dual(x).tangent is not None
+                or (torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != x.dtype)):
+            return None
         if x.dtype != layer.scales.dtype or x.shape[1] != layer.sglk_shape[0] or x.device != layer.scales.device:
             return None
         x = x.contiguous()

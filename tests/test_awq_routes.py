@@ -49,6 +49,27 @@ def test_rows_of_another_type_or_length_are_the_librarys():
         assert AWQLinearMethod._kernel_rows(layer, rows) is None
 
 
+def test_rows_that_autograd_or_a_transform_looks_at_are_the_librarys():
+    layer, x = _layer(256, 128, torch.float32), torch.randn(4, 256)
+    taken = lambda t: AWQLinearMethod._kernel_rows(layer, t) is not None
+    assert taken(x)
+    with_grad = x.clone().requires_grad_()
+    assert not taken(with_grad) and not taken(with_grad * 2)
+    with torch.no_grad():
+        assert taken(with_grad)
+    with torch.autograd.forward_ad.dual_level():
+        assert not taken(torch.autograd.forward_ad.make_dual(x, x))
+    half, low = _layer(256, 128, torch.bfloat16), x.to(torch.bfloat16)
+    for dtype in (torch.bfloat16, torch.float16):
+        with torch.autocast("cuda", dtype):
+            assert (AWQLinearMethod._kernel_rows(half, low) is not None) == (dtype == torch.bfloat16)
+    seen = []
+    torch.vmap(lambda t: (seen.append(taken(t)), t)[1])(x[None])
+    torch.jit.trace(lambda t: (seen.append(taken(t)), t + 1)[1], x, check_trace=False)
+    assert seen and not any(seen)
+    assert not taken(x.as_subclass(type("Own", (torch.Tensor,), {})))
+
+
 def test_a_weight_of_another_type_or_shape_is_refused():
     """The kernel would read scales as the rows' type and words for the rows' length."""
     w = lambda k, n: (torch.zeros(k, n // 8, dtype=torch.int32), torch.ones(k // 128, n, dtype=torch.bfloat16),

@@ -163,6 +163,20 @@ def test_linear_method_refuses_rows_of_another_type_or_length():
             AWQLinearMethod(None).apply(layer, wrong)
 
 
+def test_linear_method_keeps_the_gradient_of_its_rows():
+    from sglang_security_amd import ops
+    from sglang_security_amd.quantization.awq import AWQLinearMethod
+
+    layer, flat = _linear(300, 4096, 28672)
+    rows = flat[: 300 * 4096].view(300, 4096).clone().requires_grad_()
+    out = AWQLinearMethod(None).apply(layer, rows)
+    weights = torch.randn_like(out)
+    out.backward(weights)
+    w = ops.awq_dequantize_packed_nk(layer.sglk_packed, layer.scales, layer.qzeros)
+    want = weights.float() @ w.float()
+    assert ((rows.grad.float() - want).norm() / want.norm()).item() < 2 ** -8   # one rounding to bf16
+
+
 def test_rule_stays_where_it_was_measured():
     from sglang_security_amd import ops
 
