@@ -177,6 +177,18 @@ def test_linear_method_keeps_the_gradient_of_its_rows():
     assert ((rows.grad.float() - want).norm() / want.norm()).item() < 2 ** -8   # one rounding to bf16
 
 
+def test_linear_method_follows_autocast():
+    from sglang_security_amd.quantization.awq import AWQLinearMethod
+
+    layer, flat = _linear(300, 4096, 28672)
+    rows = flat[: 300 * 4096].view(300, 4096)
+    want = AWQLinearMethod(None).apply(layer, rows)
+    for dtype in (torch.bfloat16, torch.float16):
+        with torch.autocast("cuda", dtype):
+            got = AWQLinearMethod(None).apply(layer, rows)
+        assert got.dtype == dtype and ((got.double() - want.double()).norm() / want.double().norm()).item() < 2 ** -8   # `want` has one rounding to bf16
+
+
 def test_rule_stays_where_it_was_measured():
     from sglang_security_amd import ops
 
