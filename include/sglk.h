@@ -451,8 +451,8 @@ SGLK_API int sglk_awq_dequantize_packed_nk(const int32_t* packed, const void* sc
  * buffer serves any number of consecutive calls on a stream (calls that overlap on two streams need two). */
 SGLK_API int64_t sglk_awq_gemm_workspace_bytes(int M, int N, int K);
 /* Rows a block, 96 or 128, of the kernel that dequantises a weight once for so many, if it is the one to take a product (gated:
- * sglk_awq_gemm_silu_mul, else sglk_awq_gemm), and the splits along K; else 0.  Host only. */
-SGLK_API int sglk_awq_gemm_tall_rows(int M, int N, int K, int group_size, int dtype, int gated, int* splits);
+ * sglk_awq_gemm_silu_mul, else sglk_awq_gemm; sums: with the block sums of x), and the splits along K; else 0.  Host only. */
+SGLK_API int sglk_awq_gemm_tall_rows(int M, int N, int K, int group_size, int dtype, int gated, int sums, int* splits);
 SGLK_API int sglk_awq_gemm(const void* x, const int32_t* packed, const void* scales,
                            const int32_t* qzeros, const void* bias, void* out, float* workspace,
                            int M, int N, int K, int group_size, int64_t x_stride, int64_t out_stride,

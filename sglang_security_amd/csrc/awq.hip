@@ -1626,17 +1626,17 @@ int64_t sglk_awq_gemm_workspace_bytes(int M, int N, int K) {
 
 // What awq_tall.h's kernel makes of a product, if it is the one to take it: whole sums if gated, else as many splits as the slabs of
 // sglk_awq_gemm_workspace_bytes hold.
-static TallPlan tall_plan(int M, int N, int K, int group_size, int dtype, bool gated) {
+static TallPlan tall_plan(int M, int N, int K, int group_size, int dtype, bool gated, bool sums) {
   if (M <= kGemmBM) return TallPlan{};
-  TallPlan p = plan_awq_tall(M, N, K, group_size, dtype, gated,
+  TallPlan p = plan_awq_tall(M, N, K, group_size, dtype, gated, sums,
                              gated ? 0 : sglk_awq_gemm_workspace_bytes(M, N, K) - (int64_t)kMaxTiles * 4);
   p.ok = p.ok && (gated || p.tiles <= kMaxTiles);
   return p;
 }
 
-int sglk_awq_gemm_tall_rows(int M, int N, int K, int group_size, int dtype, int gated, int* splits) {
+int sglk_awq_gemm_tall_rows(int M, int N, int K, int group_size, int dtype, int gated, int sums, int* splits) {
   if (M <= 0 || N <= 0 || K <= 0 || group_size <= 0) return 0;
-  const TallPlan p = tall_plan(M, N, K, group_size, dtype, gated != 0);
+  const TallPlan p = tall_plan(M, N, K, group_size, dtype, gated != 0, sums != 0);
   if (!p.ok) return 0;
   if (splits) *splits = p.splits;
   return 32 * p.rt;
@@ -1744,7 +1744,7 @@ int sglk_awq_gemm_silu_mul(const void* x, const int32_t* packed, const void* sca
   SGLK_CHECK(!xsum || xs_stride >= M, "awq_gemm_silu_mul: xs_stride smaller than M");
   SGLK_CHECK(!xsum_out || xs_out_stride >= M, "awq_gemm_silu_mul: xs_out_stride smaller than M");
   // the activation needs whole sums: one split, whatever the planner would pick
-  if (const TallPlan tp = tall_plan(M, N, K, group_size, dtype, true); tp.ok && x_stride < kTallMaxStride)
+  if (const TallPlan tp = tall_plan(M, N, K, group_size, dtype, true, xsum); tp.ok && x_stride < kTallMaxStride)
     return launch_awq_tall(tp,
                            AwqTallArgs{(const uint16_t*)x, packed, (const uint16_t*)scales, qzeros, nullptr, (uint16_t*)out,
                                        nullptr, nullptr, xsum, xsum_out, x_stride, out_stride, xs_stride, xs_out_stride, M, N, K,
@@ -1878,7 +1878,7 @@ int sglk_awq_gemm_xs(const void* x, const int32_t* packed, const void* scales, c
   hipStream_t s = (hipStream_t)stream;
   int* tickets = reinterpret_cast<int*>(workspace);
   float* partial = reinterpret_cast<float*>(reinterpret_cast<char*>(workspace) + (int64_t)kMaxTiles * 4);
-  if (const TallPlan tp = tall_plan(M, N, K, group_size, dtype, false); tp.ok && x_stride < kTallMaxStride)
+  if (const TallPlan tp = tall_plan(M, N, K, group_size, dtype, false, xsum); tp.ok && x_stride < kTallMaxStride)
     return launch_awq_tall(tp,
                            AwqTallArgs{(const uint16_t*)x, packed, (const uint16_t*)scales, qzeros, (const uint16_t*)bias,
                                        (uint16_t*)out, partial, tickets, xsum, nullptr, x_stride, out_stride, xs_stride, 0, M,

@@ -43,9 +43,9 @@ struct TallPlan {
   bool ok;
   int rt, tiles, splits, stages_per_split, mblocks;
 };
-// gated: the gated activation behind the product (whole sums in one block), else finished rows; slab_bytes: room for the sums
-// of a split product
-TallPlan plan_awq_tall(int M, int N, int K, int group_size, int dtype, bool gated, int64_t slab_bytes = 0);
+// gated: the gated activation behind the product (whole sums in one block), else finished rows; sums: with the block sums of x;
+// slab_bytes: room for the sums of a split product
+TallPlan plan_awq_tall(int M, int N, int K, int group_size, int dtype, bool gated, bool sums, int64_t slab_bytes = 0);
 int launch_awq_tall(const TallPlan& p, AwqTallArgs a, hipStream_t s);
 int prepare_awq_tall();
 

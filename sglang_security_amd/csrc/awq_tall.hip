@@ -7,14 +7,21 @@
 
 namespace sglk {
 
-// Which kernel takes a product of more than 64 rows, in microseconds fitted to the four projections of Llama-3-8B (bf16, cold
-// weights, captured) at 80 to 384 rows.  A launch here costs 8.4 (96 rows a block) or 9.9 (128) and 2.45 or 2.75 a stage, 3.3
-// and 4.1 where more than 192 blocks run at once; the wide kernel's rounds of 64 rows 5.5 and 1.95 or 2.4.  Within a microsecond the
-// wide kernel, whose sums are those of fewer rows to the bit.  Measured, wide and here: 4096 x 28672 with its activation
-// 96 rows 49.6 and 34.8, 128 rows 49.1 and 41.9, 192 rows 71 and 66, 255 rows 94 and 80; left to the wide one: 128 rows of
-// 4096 x 6144 14.2 and 15.3, of 14336 x 4096 22.1 and 27.4, of 4096 x 4096 11.9 and 14.2 (a launch's start and end, with twice
-// the sums to add up and to leave, outweigh few stages).
-TallPlan plan_awq_tall(int M, int N, int K, int group_size, int dtype, bool gated, int64_t slab_bytes) {
+// Which kernel takes a product of more than 64 rows, in microseconds: a round's start and end, and a stage with up to 128 and with 256
+// blocks at once; blocks of 96 and of 128 rows and the wide kernel's of 64, without and with the producer's sums.  Fitted to 780
+// products in each form (2048 to 32768 columns, 2 to 56 stages, bf16, cold weights, captured), which they tell within a tenth; the bound
+// of nineteen twentieths leaves none that is taken more than 2 % slower than on the wide kernel.  A split product's sums cost 1.5 and 0.9 a split
+// on both.  Measured, wide and here: 4096 x 28672 with its activation 96 rows 49.6 and 34.8, 128 rows 49.1 and 41.9; finished rows 5120 x
+// 15360 at 192 rows 58.6 and 42.1, 8192 x 10240 at 96 (two splits) 43.0 and 36.8; left to the wide one: 13824 x 5120 at 80 rows 30.1 and 34.5
+// (four splits), 26624 x 12160 at 255 210 and 245, 4096 x 6144 at 128 14.2 and 15.3 (a launch's start and end, with twice the sums to add
+// up and to leave, outweigh few stages).
+struct TallCost {
+  float round, few, full;
+};
+static constexpr TallCost kTallCost[2][3] = {{{7.5f, 3.08f, 3.65f}, {8.4f, 3.98f, 4.65f}, {6.4f, 1.96f, 2.3f}},
+                                             {{7.3f, 2.68f, 3.4f}, {8.2f, 3.48f, 4.15f}, {6.4f, 1.78f, 2.1f}}};
+
+TallPlan plan_awq_tall(int M, int N, int K, int group_size, int dtype, bool gated, bool sums, int64_t slab_bytes) {
   TallPlan p{};
   if (dtype != SGLK_BF16 || M <= kGemmBM || getenv("SGLK_AWQ_WIDE") || getenv("SGLK_AWQ_WIDE_SPS")) return p;  // (test hooks)
   const WidePlan wide = plan_awq_wide(M, N, K, group_size, gated);
@@ -25,22 +32,23 @@ TallPlan plan_awq_tall(int M, int N, int K, int group_size, int dtype, bool gate
   p.tiles = (N / 128) * p.mblocks;
   const int total = K / AwqTall::kStageK;
   const int64_t slab = (int64_t)p.tiles * p.rt * 32 * 128 * 4;
-  auto cost = [&](int tiles, int sps, float start, float one, float full) {
-    const int splits = (total + sps - 1) / sps, blocks = tiles * splits;
-    return start + (blocks + 255) / 256 * sps * (blocks > 192 ? full : one) + (splits > 1 ? 0.5f * splits : 0.f);
+  auto cost = [&](int tiles, int sps, const TallCost& c) {
+    const int splits = (total + sps - 1) / sps, blocks = tiles * splits, whole = blocks / 256, rest = blocks % 256;
+    const float last = rest == 0 ? 0.f : c.few + (c.full - c.few) * std::max(0, rest - 128) / 128.f;
+    return (whole + (rest > 0)) * c.round + sps * (whole * c.full + last) + (splits > 1 ? 1.5f + 0.9f * splits : 0.f);
   };
   float least = 1e30f;
   for (int sps = gated ? total : 1; sps <= total; ++sps) {
     const int splits = (total + sps - 1) / sps;
     if (splits > 1 && slab * splits > slab_bytes) continue;
-    const float c = p.rt == 3 ? cost(p.tiles, sps, 8.4f, 2.45f, 3.3f) : cost(p.tiles, sps, 9.9f, 2.75f, 4.1f);
+    const float c = cost(p.tiles, sps, kTallCost[sums][p.rt - 3]);
     if (c < least) {
       least = c;
       p.stages_per_split = sps;
       p.splits = splits;
     }
   }
-  p.ok = least + 1.f < cost(wide.tiles, gated ? total : wide.stages_per_split, 5.5f, 1.95f, 2.4f);
+  p.ok = least < 0.95f * cost(wide.tiles, gated ? total : wide.stages_per_split, kTallCost[sums][2]);
   return p;
 }
 

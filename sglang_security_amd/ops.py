@@ -648,10 +648,11 @@ def awq_gemm_workspace_bytes(M, N, K) -> int:
     return int(lib().sglk_awq_gemm_workspace_bytes(M, N, K))
 
 
-def awq_gemm_tall_rows(M, N, K, group=128, dtype=torch.bfloat16, gated=False):
-    """(rows a block, splits along K) where awq_gemm (gated: awq_gemm_silu_mul) takes blocks of 96 or 128 rows, else None."""
+def awq_gemm_tall_rows(M, N, K, group=128, dtype=torch.bfloat16, gated=False, sums=False):
+    """(rows a block, splits along K) where awq_gemm (gated: awq_gemm_silu_mul; sums: with the block sums of x) takes blocks of 96 or
+    128 rows, else None."""
     splits = C.c_int(0)
-    rows = lib().sglk_awq_gemm_tall_rows(M, N, K, group, dtype_code(dtype), int(gated), C.byref(splits))
+    rows = lib().sglk_awq_gemm_tall_rows(M, N, K, group, dtype_code(dtype), int(gated), int(sums), C.byref(splits))
     return (rows, splits.value) if rows else None
 
 

@@ -27,6 +27,17 @@ def test_tiles_cover_a_product_once(gated):
     assert gated or ragged > 20
 
 
+def test_blocks_of_96_and_128_rows_stay_where_they_were_measured():
+    """Sizes that were timed with the wide kernel ahead by 5 % or more are its, whoever forms the block sums (fp16 and up to 64 rows always)."""
+    rows = ops.awq_gemm_tall_rows
+    wide = [(80, 13824, 5120), (255, 26624, 12160), (128, 4096, 6144), (128, 14336, 4096)]
+    here = [(96, 4096, 28672), (128, 4096, 28672), (192, 5120, 15360), (96, 8192, 10240), (192, 28672, 8192), (97, 1536, 16640)]
+    for sums in (False, True):
+        assert not any(rows(m, n, k, sums=sums) for m, k, n in wide)
+        assert all(rows(m, n, k, sums=sums) for m, k, n in here)
+    assert not rows(128, 28672, 4096, dtype=torch.float16) and not rows(64, 28672, 4096) and not rows(128, 28672, 4096, group=256)
+
+
 def _layer(k, n, dtype):
     return SimpleNamespace(sglk_shape=(k, n), scales=torch.ones(k // 128, n, dtype=dtype))
 

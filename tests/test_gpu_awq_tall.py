@@ -27,15 +27,17 @@ def _wide(monkeypatch, call):
 
 
 def _takes(M, N, K, rows, splits=1, gated=False):
-    """The size is one that blocks of so many rows take, K in so many splits."""
+    """The size is one that blocks of so many rows take, K in so many splits, whoever forms the block sums."""
     from sglang_security_amd import ops
 
-    assert ops.awq_gemm_tall_rows(M, N, K, gated=gated) == (rows, splits)
+    for sums in (False, True):
+        assert ops.awq_gemm_tall_rows(M, N, K, gated=gated, sums=sums) == (rows, splits)
 
 
 @pytest.mark.parametrize("M,K,inter,block", [(65, 4096, 14336, 96), (96, 4096, 14336, 96), (97, 4096, 14336, 128), (128, 4096, 14336, 128),
-                                            (192, 4096, 14336, 96), (200, 4096, 14336, 128), (255, 4096, 14336, 128),
-                                            (65, 1024, 8320, 96), (96, 1536, 14336, 96), (97, 1536, 8320, 128), (128, 2560, 8320, 128)])
+                                             (200, 4096, 14336, 128), (255, 4096, 14336, 128), (192, 1024, 5632, 96), (65, 512, 8320, 96),
+                                             (97, 512, 8320, 128), (65, 1024, 8320, 96), (96, 1536, 14336, 96), (97, 1536, 8320, 128),
+                                             (193, 1024, 4224, 128), (128, 2560, 8320, 128)])
 def test_gated_rows_and_their_sums(monkeypatch, M, K, inter, block):
     """Every output of the gated form, ragged rows among them, with and without the producer's block sums: the unfused sequence's
     roundings, so half an ulp of bf16 twice (2^-8 each) beside the product's own 1e-6; rows behind M stay as they were.  With the
@@ -71,9 +73,11 @@ def test_gated_rows_and_their_sums(monkeypatch, M, K, inter, block):
 
 
 @pytest.mark.parametrize("M,K,N,rows,splits", [(65, 4096, 28672, 96, 1), (96, 1024, 16640, 96, 1), (97, 1536, 16640, 128, 1),
-                                               (128, 2560, 16640, 128, 1), (80, 5632, 11008, 96, 2), (192, 28672, 8192, 96, 2),
-                                               (128, 8192, 10240, 128, 2), (97, 13824, 8448, 128, 3), (65, 13824, 5120, 96, 4),
-                                               (255, 24576, 3072, 128, 4), (65, 9728, 16640, 96, 5), (96, 18432, 3072, 96, 6)])
+                                               (128, 2560, 16640, 128, 1), (193, 1024, 8448, 128, 1), (160, 4608, 5632, 96, 2),
+                                               (192, 28672, 8192, 96, 2), (97, 10240, 11008, 128, 2), (255, 10240, 5632, 128, 2),
+                                               (65, 4608, 8448, 96, 3), (97, 4608, 8448, 128, 3), (193, 4608, 4352, 128, 3),
+                                               (192, 12800, 3840, 96, 4), (80, 12800, 5632, 96, 5), (255, 12800, 2816, 128, 5),
+                                               (65, 25088, 4352, 96, 7), (97, 25088, 4352, 128, 7)])
 def test_finished_rows(monkeypatch, M, K, N, rows, splits):
     """Finished rows with a bias, whole and split along K, twice over one workspace of the size that is asked for, no further from 64
     bits than the wide kernel's: what is left after the rounding to bf16 is that rounding."""
@@ -104,9 +108,9 @@ def test_finished_rows(monkeypatch, M, K, N, rows, splits):
         assert err(got, exact) <= 1.01 * err(_wide(monkeypatch, call), exact)
 
 
-@pytest.mark.parametrize("M,K,rows", [(96, 1024, 96), (80, 1536, 96), (128, 1536, 128), (100, 2560, 128)])
+@pytest.mark.parametrize("M,K,rows", [(96, 512, 96), (100, 512, 128), (96, 1024, 96), (80, 1536, 96), (128, 1536, 128), (100, 2560, 128)])
 def test_zero_scales_and_few_stages(monkeypatch, M, K, rows):
-    """Columns whose scale is zero in the first, a middle, the last or all groups, over two, three and five stages: nothing from there,
+    """Columns whose scale is zero in the first, a middle, the last or all groups, over one to three and five stages: nothing from there,
     the rest as before; a capture replays the same bits."""
     from sglang_security_amd import ops
 
