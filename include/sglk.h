@@ -631,6 +631,8 @@ SGLK_API int sglk_awq_gemm_prefill_silu_mul(const void* x, const int32_t* packed
 SGLK_API int sglk_awq_gemm_prefill_tiles(int M, int N, int K, int gated, int* tiles);
 /* Whether sglk_awq_gemm_prefill is expected to be faster than a dequantisation to memory and a library product. */
 SGLK_API int sglk_awq_prefill_fused(int M, int N, int K);
+/* ... and sglk_awq_gemm_prefill_silu_mul than those two and sglk_act_and_mul. */
+SGLK_API int sglk_awq_prefill_silu_mul_fused(int M, int N, int K);
 SGLK_API int sglk_dense_gemm_prefill(const void* x, const void* w, const void* bias, void* out, int M, int N, int K,
                                      int64_t x_stride, int64_t w_stride, int64_t out_stride, int dtype,
                                      void* stream);

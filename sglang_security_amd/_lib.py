@@ -101,6 +101,7 @@ _SIGS = {
     "sglk_awq_gemm_tall_rows": (i32, [i32, i32, i32, i32, i32, i32, i32, p]),
     "sglk_awq_gemm_prefill_tiles": (i32, [i32, i32, i32, i32, p]),
     "sglk_awq_prefill_fused": (i32, [i32, i32, i32]),
+    "sglk_awq_prefill_silu_mul_fused": (i32, [i32, i32, i32]),
     "sglk_awq_gemm_prefill": (i32, [p, p, p, p, p, p, i32, i32, i32, i32, i64, i64, i32, p]),
     "sglk_dense_gemm_prefill": (i32, [p, p, p, p, i32, i32, i32, i64, i64, i64, i32, p]),
     "sglk_dense_repack": (i32, [p, p, i32, i32, i64, p]),

@@ -311,17 +311,35 @@ int sglk_awq_gemm_prefill_tiles(int M, int N, int K, int gated, int* tiles) {
   return SGLK_OK;
 }
 
-// The other way: the weight dequantised to memory (2.5 bytes of traffic a weight), then the library's product, which needs its
-// weights' way from memory, its operations or a chain along K, whichever is longest.  Below four million weights nothing was
-// measured, and the library keeps them.  Measured, library and here: 1152 x 28672 x 4096 300 and 254 us, 500 rows 154 and 110, 256
-// rows 125 and 67; 1152 x 6144 x 4096 70 and 64; 1152 x 4096 x 14336 164 and 155; left to the library: 640 x 4096 x 14336 139 and
-// 133, 256 rows 94 and 130.
-int sglk_awq_prefill_fused(int M, int N, int K) {
-  if (M <= 0 || N <= 0 || K <= 0 || K % 128 != 0 || N % 128 != 0 || (int64_t)N * K < (4 << 20)) return 0;
+// The other way, in microseconds: the weight dequantised to memory and the library's product, whose tiles round M up and whose chain
+// along K is never shorter than that.  Fitted to what follows, within a tenth for half of it: choices of the library's own move its
+// products by a quarter either way, so the entries below draw lines around the estimate.
+static double prefill_library(int M, int N, int K) {
   const double weights = (double)N * K;
-  const double dequantise = 2 + 2.5e-6 / 5.2 * weights;
-  const double product = 10 + std::max({2e-6 / 4.5 * weights, 2e-9 / 1.15 * weights * M, 0.0045 * K});
-  return prefill_plan(M, N, K, true).cost < dequantise + product;
+  return 14 + 0.22e-6 * weights + std::max(2e-9 / 1.52 * weights * (M + 336), 0.0049 * K);
+}
+
+// Timed both ways, one launch behind the other on weights from memory, over 28 weights of 1B to 70B models and eight of their ranks,
+// 257 to 4096 rows in bf16; captured over 32, 1 to 8192 rows, bf16 and fp16.  Of the calls that these lines take none is more than 3 % slower
+// than the library behind a dequantisation (captured, without the gap between two launches, four are, by 4 to 8 %: 4096 x 4096 at 1536
+// rows, 5120 x 5120 at 1152, 8192 x 8192 and 3584 at 640), and they take a fifth less on average: 28672 x 4096, 257 rows 136 -> 83 us, 500 rows 158 -> 105, 1152
+// rows 288 -> 244; 6144 x 4096, 500 rows 49 -> 42, 1152 rows 67 -> 62.  Left to the library: 4096 x 14336 at 640 rows 117 and here 137,
+// 7168 x 8192 at 800 116 and 124, 28672 x 4096 at 4096 675 and 781, and a long K with so few rows as other kernels take, 100 of 8192 x
+// 8192 63 and 78.
+int sglk_awq_prefill_fused(int M, int N, int K) {
+  if (M <= 0 || K <= 0 || K % 128 != 0 || N % 128 != 0 || (int64_t)N * K < (4 << 20)) return 0;
+  const bool wide = N >= 8192;
+  if (N < 4096 || M > 1700 || (M < 256 && !wide) || (K > 5120 && (M < 256 || !wide))) return 0;
+  return prefill_plan(M, N, K, true).cost < (wide ? 1.0 : 0.95) * prefill_library(M, N, K);
+}
+
+// With the activation behind it, against the library and a launch of the activation: twelve weights, 257 to 8192 rows, captured; none
+// taken is more than 3 % slower.  28672 x 4096, 2048 rows 426 -> 409 us, 27648 x 5120, 1300 rows 387 -> 352; left to the library: 16384
+// x 3072, 3000 rows 254 and here 268.
+int sglk_awq_prefill_silu_mul_fused(int M, int N, int K) {
+  if (M < 256 || M > 2112 || N < 8192 || K <= 0 || K % 128 != 0 || N % 256 != 0) return 0;
+  const double activation = 3 + 0.61e-6 * M * N;
+  return prefill_plan(M, N, K, true, true).cost < prefill_library(M, N, K) + activation;
 }
 
 int sglk_dense_gemm_prefill(const void* x, const void* w, const void* bias, void* out, int M, int N, int K,

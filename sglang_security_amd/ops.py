@@ -718,9 +718,10 @@ def awq_gemm_prefill_tiles(M, N, K, gated=False):
     return tuple(tiles)
 
 
-def awq_prefill_fused(M, N, K) -> bool:
-    """Whether awq_gemm_prefill is expected to be faster than dequantising the weight and a library product."""
-    return bool(lib().sglk_awq_prefill_fused(M, N, K))
+def awq_prefill_fused(M, N, K, gated=False) -> bool:
+    """Whether awq_gemm_prefill (gated: awq_gemm_prefill_silu_mul) is expected to be faster than dequantising the weight and a library
+    product (and act_and_mul)."""
+    return bool((lib().sglk_awq_prefill_silu_mul_fused if gated else lib().sglk_awq_prefill_fused)(M, N, K))
 
 
 def dense_gemm_prefill(x, w, bias=None, out=None):

@@ -135,15 +135,15 @@ class LlamaPrefill:
             raise NotImplementedError("prefill runner: awq and bf16 weights")
         return out
 
-    def _by_library(self, w, T):
+    def _by_library(self, w, T, gated=False):
         """Whether T rows go to a dequantised copy of an int4 weight and the library (prefill_gemm = "library")."""
-        return self.resident_bf16 or not (ops.awq_prefill_fused(T, w.N, w.K) and w.K // w.scales.shape[0] % 128 == 0)
+        return self.resident_bf16 or not (ops.awq_prefill_fused(T, w.N, w.K, gated) and w.K // w.scales.shape[0] % 128 == 0)
 
     def _gated(self, L, T):
         """Whether gate_up takes the activation along: a product that dequantises on the way, on the decoder's interleaved copy."""
         w = L["gate_up"]
         return (T >= DEQUANT_GEMM_MIN_TOKENS and "gate_up_il" in L and w.N % 256 == 0
-                and (self.prefill_gemm == "fused" and w.K % 128 == 0 or not self._by_library(w, T)))
+                and (self.prefill_gemm == "fused" and w.K % 128 == 0 or not self._by_library(w, T, True)))
 
     # -- dequantisation one projection ahead of the library product, on a second stream --------------------------------
     _RING = 3
@@ -153,11 +153,13 @@ class LlamaPrefill:
         if not (self.overlap_dequant and self.prefill_gemm == "library" and not self.resident_bf16
                 and c.quant == "awq" and T >= DEQUANT_GEMM_MIN_TOKENS):
             return
-        seq = [L[k] for L in self.dec.layers for k in ("qkv", "o", "gate_up", "down")]
+        names = ("qkv", "o", "gate_up", "down")
+        seq = [L[k] for L in self.dec.layers for k in names]
         if not all(isinstance(w, _AwqLinear) for w in seq):
             self.overlap_dequant = False
             return
-        self._seq = [w for w in seq if self._by_library(w, T)]
+        self._seq = [L[k] for L in self.dec.layers for k in names
+                     if self._by_library(L[k], T) and not (k == "gate_up" and self._gated(L, T))]
         if not self._seq:
             return
         if self._ring is None:

@@ -27,6 +27,20 @@ def test_tiles_cover_a_product_once(gated):
     assert gated or ragged > 20
 
 
+def test_rules_of_many_rows_stay_where_they_were_measured():
+    """Sizes that were timed with the library ahead by 5 % or more are the library's, and those with this package's product ahead by as much its."""
+    library = [(8192, 14336, 4096), (8192, 4096, 28672), (4096, 4096, 28672), (3000, 8192, 10240), (4096, 13824, 5120), (2500, 3072, 8192),
+               (500, 14336, 4096), (1152, 8192, 7168), (800, 4096, 6144), (1300, 11008, 4096), (640, 14336, 4096), (100, 8192, 8192),
+               (1, 28672, 8192), (64, 8192, 10240)]
+    here = [(257, 4096, 28672), (500, 4096, 28672), (1152, 4096, 28672), (257, 2560, 13824), (500, 5120, 15360), (384, 28672, 8192),
+            (257, 1024, 8192), (500, 1536, 8960), (500, 8192, 57344), (800, 1024, 8192), (64, 4096, 28672), (200, 2560, 13824)]
+    assert not any(ops.awq_prefill_fused(m, n, k) for m, k, n in library)
+    assert all(ops.awq_prefill_fused(m, n, k) for m, k, n in here)
+    gated = [(257, 4096, 28672), (1700, 4096, 28672), (1300, 5120, 27648), (2048, 8192, 57344)]
+    assert all(ops.awq_prefill_fused(m, n, k, True) for m, k, n in gated)
+    assert not any(ops.awq_prefill_fused(m, n, k, True) for m, k, n in [(4096, 4096, 28672), (8192, 3072, 16384), (1152, 8192, 7168)])
+
+
 def test_blocks_of_96_and_128_rows_stay_where_they_were_measured():
     """Sizes that were timed with the wide kernel ahead by 5 % or more are its, whoever forms the block sums (fp16 and up to 64 rows always)."""
     rows = ops.awq_gemm_tall_rows
