@@ -41,13 +41,26 @@ __global__ void __launch_bounds__(256) short_conv_kernel(ShortConv a) {
   short_conv_rows<T, R, ACT>(a, (int)(idx / nv) * R, (int)(idx % nv) * 8);
 }
 
-// 4 G rows a thread, the last ones first: those at the ends of sequences, which go four at a time, take longest.
+// Threads of short_conv_run_kernel along the rows: four of them a thread while they are sequences of one row, then 4 G.
+static __host__ __device__ __forceinline__ uint32_t short_conv_fours(int singles) { return (uint32_t)(singles + 3) / 4; }
+static __host__ __device__ __forceinline__ uint32_t short_conv_runs(int M, int singles, int G) {
+  const int64_t rest = M - 4 * (int64_t)short_conv_fours(singles);
+  return short_conv_fours(singles) + (rest > 0 ? (uint32_t)((rest + 4 * G - 1) / (4 * G)) : 0);
+}
+
+// Sequences of one row first, then 4 G rows a thread, the last ones ahead: single rows and those at the ends of sequences, which go four
+// at a time, take longest (64 of them with four prompts of 900, 5120 channels: 38 us eight a thread and last, 28 like this).
 template <typename T, int G, int ACT>
 __global__ void __launch_bounds__(256) short_conv_run_kernel(ShortConv a) {
-  const uint32_t nv = a.W / 8, runs = (a.M + 4 * G - 1) / (4 * G);
+  const uint32_t nv = a.W / 8, fours = short_conv_fours(a.singles), runs = short_conv_runs(a.M, a.singles, G);
   const uint32_t idx = blockIdx.x * 256 + threadIdx.x, run = idx / nv;
   if (run >= runs) return;
-  const int m0 = (int)(runs - 1 - run) * 4 * G, c = (int)(idx - run * nv) * 8;
+  const int c = (int)(idx - run * nv) * 8;
+  if (run < fours) {
+    short_conv_rows<T, 4, ACT>(a, (int)run * 4, c);
+    return;
+  }
+  const int m0 = (int)(fours + (runs - 1 - run) * G) * 4;
   const int s = a.seq.row_seq[m0];
   if (m0 + 4 * G <= a.M && a.seq.row_seq[m0 + 4 * G - 1] == s && m0 - a.seq.row0[s] >= 3) {
     short_conv_run<T, G, ACT>(a, m0, c);
@@ -720,7 +733,7 @@ int sglk_short_conv(const void* src, int src_f32, int splits, int64_t part_strid
   // 160 bytes beside 16 a row, so four rows cost as much in them as in rows: 7921 rows of 5120 channels 59 -> 44 us; 12 rows 44, 16
   // 48; 2164 rows, fewer blocks than that, 21 -> 22.
   constexpr int G = 2;
-  const int64_t run_threads = (int64_t)((M + 4 * G - 1) / (4 * G)) * (W / 8);
+  const int64_t run_threads = (int64_t)short_conv_runs(M, singles, G) * (W / 8);
   if (taps == 4 && !src_f32 && dtype != SGLK_F32 && run_threads >= 4 * 256 * 256 && run_threads < (1ll << 31)) {
     const dim3 run_grid((unsigned)((run_threads + 255) / 256));
     SGLK_DISPATCH_HALF(dtype, T, {

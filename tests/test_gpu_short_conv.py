@@ -17,6 +17,7 @@ def _seqs(lens, starts, slots):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("W,lens,starts", [
     (5120, [1, 1, 1500, 2, 1, 3, 7, 1801], [5, 0, 9, 1, 4, 0, 2, 0]),      # eight rows a thread; ends inside, at and across them
+    (5120, [1] * 37 + [1500, 4, 1801], [i % 6 for i in range(40)]),         # single rows, which are no multiple of four
     (65536, [8, 8, 3, 5, 240, 1], [0, 3, 0, 7, 1, 2]),                       # just enough threads, as few rows
     (65528, [1, 255], [1, 1]),                                               # just too few: four rows a thread
     (64, [1, 2, 3, 4, 5, 250], [1, 2, 3, 0, 5, 6]),
