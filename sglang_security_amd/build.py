@@ -25,9 +25,6 @@ ARCH = "gfx950"
 # no packed fp32 vector instructions: some of their forms have given wrong results on these devices
 CODEGEN = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
-# by source: accumulators in vector registers although the kernel names accumulation registers of its own
-EXTRA = {"awq_tall.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
-
 
 def _hipcc() -> str:
     for c in (shutil.which("hipcc"), "/opt/rocm/bin/hipcc"):
@@ -49,7 +46,7 @@ def _compile(src: str, force: bool) -> str:
     obj = os.path.join(OBJ, os.path.basename(src) + ".o")
     if (not force and os.path.exists(obj) and os.path.getmtime(obj) >= max(os.path.getmtime(src), _deps_mtime())):
         return obj
-    cmd = [_hipcc(), f"--offload-arch={ARCH}", *CODEGEN, *EXTRA.get(os.path.basename(src), ()), "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden",
+    cmd = [_hipcc(), f"--offload-arch={ARCH}", *CODEGEN, "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden",
            "-I" + os.path.join(ROOT, "include"), "-I" + CSRC, "-c", src, "-o", obj]
     if src.endswith(".cpp"):
         cmd.insert(1, "-x")

@@ -1,5 +1,4 @@
-// Fused int4 GEMM of more than 64 rows: plan and launches of the kernel in awq_tall.h.  A source of its own because it is compiled
-// with the sums of the matrix instructions in vector registers (the accumulation registers hold the weights on their way).
+// Fused int4 GEMM of more than 64 rows: plan and launches of the kernel in awq_tall.h.
 #include "awq_tall.h"
 
 #include <algorithm>
@@ -11,9 +10,9 @@ namespace sglk {
 // blocks at once; blocks of 96 and of 128 rows and the wide kernel's of 64, without and with the producer's sums.  Fitted to 780
 // products in each form (2048 to 32768 columns, 2 to 56 stages, bf16, cold weights, captured), which they tell within a tenth; the bound
 // of nineteen twentieths leaves none that is taken more than 2 % slower than on the wide kernel.  A split product's sums cost 1.5 and 0.9 a split
-// on both.  Measured, wide and here: 4096 x 28672 with its activation 96 rows 49.6 and 34.8, 128 rows 49.1 and 41.9; finished rows 5120 x
-// 15360 at 192 rows 58.6 and 42.1, 8192 x 10240 at 96 (two splits) 43.0 and 36.8; left to the wide one: 13824 x 5120 at 80 rows 30.1 and 34.5
-// (four splits), 26624 x 12160 at 255 210 and 245, 4096 x 6144 at 128 14.2 and 15.3 (a launch's start and end, with twice the sums to add
+// on both.  Measured, wide and here: 4096 x 28672 with its activation and the producer's sums 96 rows 42.8 and 34.1, 128 rows 42.3 and 40.3,
+// without sums 47.4 and 38.6, 46.0 and 44.3; finished rows 5120 x 15360 at 192 rows 56.8 and 41.6, 8192 x 10240 at 96 (three splits) 41.4
+// and 33.0, 28672 x 8192 at 192 (two) 134 and 115; left to the wide one: 13824 x 5120 at 80 rows 30.1 and 34.5 (four splits), 26624 x 12160 at 255 210 and 245, 4096 x 6144 at 128 14.2 and 15.3 (a launch's start and end, with twice the sums to add
 // up and to leave, outweigh few stages).
 struct TallCost {
   float round, few, full;
