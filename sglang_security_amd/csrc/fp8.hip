@@ -721,10 +721,10 @@ enum class Fp8Other { kRegister, kSplit, kStreaming };  // what a call falls bac
 // k-block of 128 for every round of blocks; the others take the lesser of an estimate by work and one by rounds (narrow outputs
 // spread K over idle units, which the tiles do not).  Measured against the register kernel, the split and the streaming one:
 //   N, K of the 8B model's projections and of the 70B model's on one of eight ranks, M = 1 .. 2048: 2048 x 28672 x 4096
-//   1190 -> 181 (streaming 788); 2048 x 4096 x 14336 593 -> 95 (349); 256 x 4096 x 14336 79 -> 37 (68); 128 x 28672 x
+//   1190 -> 199 (streaming 788); 2048 x 4096 x 14336 593 -> 97 (349); 256 x 4096 x 14336 79 -> 37 (68); 128 x 28672 x
 //   4096 83 -> 33 (57); 128 x 4096 x 4096 14.6 -> 12.9 (16.5); 64 x 28672 x 4096 without the streaming copy 50 -> 30;
 //   between the forms, the same projections at 18 sizes from 65 to 2048 rows: no choice is slower than the fastest form by more
-//   than a tenth.  Four waves against the older forms: 2048 x 6144 x 4096 50 -> 42, 2048 x 4096 x 4096 40 -> 32, 1300 x 7168 x 8192
+//   than a tenth.  Four waves against the older forms: 2048 x 6144 x 4096 50 -> 43, 2048 x 4096 x 4096 39 -> 33, 1300 x 7168 x 8192
 //   88 -> 67, 700 x 28672 x 4096 97 -> 79; eight waves stay where a full round has few k-blocks: 2048 x 8192 x 1024 20 and 21.
 //   M = 33 .. 2048, N = 32 .. 8192, K = 512 .. 14336, 1008 sizes: no call on tiles is slower than its fallback by more
 //   than 4 % (33 x 6144 x 14336), none that stays would gain more than 11 % (the same, against the split kernel).

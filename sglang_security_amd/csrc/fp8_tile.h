@@ -9,9 +9,9 @@
 // Two kernels.  fp8_tile4_kernel, four waves of 128 x 64, 128 x 96 or 128 x 128 sums, is bound by a wave's own issue and by the
 // matrix unit (busy two thirds of a wave's life; counters), a launch also by its start and by the results that all units store at once.
 // fp8_tile_kernel's smaller tiles are bound by the trip of a stage from memory, hence their deeper rings.  Measured (bf16 out,
-// weights from memory): 2048 x 28672 x 4096 212 us (eight waves) -> 181 = 2.66 PFLOP/s; 2048 x 4096 x 14336 127 (128 x 128
-// tiles) -> 95 = 2.53 PFLOP/s; 2048 x 6144 x 4096 52 -> 42, 2048 x 4096 x 4096 40 -> 32.  Of that, the rows on their way out without
-// a branch per quad for the bias are 10 to 20 us of the largest, in every form.
+// weights from memory, both on one card): 2048 x 28672 x 4096 222 us (eight waves) -> 199 = 2.42 PFLOP/s (181 to 202 from card to card);
+// 2048 x 4096 x 14336 125 (128 x 128 tiles) -> 97 = 2.48 PFLOP/s; 2048 x 6144 x 4096 50 -> 43, 2048 x 4096 x 4096 39 -> 33.  Of that, the
+// rows on their way out without a branch per quad for the bias are a twentieth to a tenth of the largest, in every form.
 #pragma once
 #include <type_traits>
 
@@ -193,8 +193,8 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) fp8_tile_kernel(Fp8TileArgs p
 // products where eight waves have it serve two to four.  Activations and weights have rings of their own, SA and SA + 1 stages
 // deep: weights come from memory and are asked for a stage earlier (256 x 256 tiles of two whole stages: 4096 columns at 512 rows, an
 // idle chip, 58 -> 44 us).  A stage's barrier lies between its two k-steps, when a wave holds the second one's operands; requests
-// are spread one by one among the products, since all waves share one address unit (in pairs at the start of a half: 223 -> 248 us
-// for 2048 x 28672 x 4096).
+// are spread one by one among the products, since all waves share one address unit (in pairs at the start of a half: a ninth more for
+// 2048 x 28672 x 4096).
 template <typename TO, int BN, int SA>
 __device__ __forceinline__ void fp8_tile4(const Fp8TileArgs& p, char* lds, int m0, int n0) {
   constexpr int BM = 256, MI = 4, NJ = BN / 64, SB = SA + 1, kA = BM * 128, kB = BN * 128, kRingB = SA * kA;
@@ -302,7 +302,7 @@ __device__ __forceinline__ void fp8_tile4(const Fp8TileArgs& p, char* lds, int m
 }
 
 // Strips of 256 columns, then narrower ones (`tail` columns) for what would be a last round that leaves units idle: 2048 x 28672
-// in three rounds and one of half strips instead of four, 232 -> 205 us; 2048 x 6144 in one of 192 columns, 57 -> 46
+// in three rounds and one of half strips instead of four, an eighth less; 2048 x 6144 in one of 192 columns, a fifth
 template <typename TO>
 __global__ void __launch_bounds__(256, 1) fp8_tile4_kernel(Fp8TileArgs p) {
   extern __shared__ __attribute__((aligned(16))) char lds[];

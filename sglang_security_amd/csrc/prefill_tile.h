@@ -9,9 +9,8 @@
 // Bound: one wave's issue.  A half stage of 128 x 128 sums is 32 matrix instructions of 32 cycles, beside which a wave issues 100
 // vector instructions for its weights, 20 for LDS and 10 requests, at 4 cycles each (8 for a matrix one): nothing may wait for the
 // instruction before, and nothing may gather.  So a pair of weights takes three steps, one behind each second product, and the
-// products are pinned where they stand.  2048 x 28672 x 4096: 16-bit weights 360 us (1.34 PFLOP/s; the library 355), int4 with each
-// step's instructions in a row 421, in three steps 391; the kernel before (256 x 128 tiles, rows through registers, a barrier
-// every 32 of K) was slower than the library behind a dequantisation, which is 418.
+// products are pinned where they stand.  2048 x 28672 x 4096, one card: 16-bit weights 374 us (1.29 PFLOP/s; the library 367), int4 395 (each
+// step's instructions in a row: a twelfth more), where the library behind a dequantisation takes 381; 1152 rows 246 and 292.
 #pragma once
 #include <type_traits>
 
