@@ -102,3 +102,37 @@ def test_a_weight_of_another_type_or_shape_is_refused():
                  (rows, packed[:, :8], scales, zeros), (rows, packed, scales, zeros[:1])):
         with pytest.raises(SglkError):
             ops._packed_weight("product", *args)
+
+
+@pytest.mark.parametrize("T", [256, 300, 700, 1152, 1600, 1900, 2112, 2500])
+def test_dequantisation_pipeline_holds_what_the_layers_ask_of_it(monkeypatch, T):
+    """Projections dequantised ahead are those, in that order, that the layers then multiply by the library: where gate_up takes its
+    activation along, on the rule of its own, it is not among them."""
+    from sglang_security_amd.decode_runner import _AwqLinear
+    from sglang_security_amd.prefill_runner import LlamaPrefill
+
+    def weight(K, N):
+        w = _AwqLinear.__new__(_AwqLinear)
+        w.K, w.N, w.packed, w.scales, w.qzeros = K, N, None, torch.empty(K // 128, 0), None
+        return w
+
+    layers = [{"qkv": weight(4096, 6144), "o": weight(4096, 4096), "gate_up": weight(4096, 28672), "down": weight(14336, 4096),
+               "gate_up_il": (None, None, None)} for _ in range(2)]
+    model = LlamaPrefill.__new__(LlamaPrefill)
+    model.prefill_gemm, model.resident_bf16, model.overlap_dequant, model._pipe = "library", False, True, None
+    model.cfg = SimpleNamespace(quant="awq")
+    model.dec = SimpleNamespace(layers=layers, device=torch.device("cpu"), dtype=torch.bfloat16)
+    model._ring, model._side = [], SimpleNamespace(wait_stream=lambda s: None)
+    asked = []
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: None)
+    monkeypatch.setattr(ops, "awq_gemm_prefill", lambda *a: None)
+    monkeypatch.setattr(LlamaPrefill, "_pipe_issue", lambda self, j: None)
+    monkeypatch.setattr(LlamaPrefill, "_pipe_matmul", lambda self, w, x, out: asked.append(w))
+    monkeypatch.setattr(ops, "awq_dequantize_packed_nk", lambda *a: pytest.fail("dequantised outside the pipeline"))
+    model._pipe_begin(T)
+    for L in layers:
+        for k in ("qkv", "o", "gate_up", "down"):
+            if k != "gate_up" or not model._gated(L, T):
+                model._linear(L[k], torch.empty(T, L[k].K, device="meta"), None)
+    assert model._gated(layers[0], T) == (T <= 2112)
+    assert asked and [id(w) for w in asked] == [id(w) for w in model._seq]
